@@ -61,111 +61,95 @@ __device__ __forceinline__ int proc_law(const CV& c, int ci, const CV& q, int qi
   }
 }
 
-__device__ __forceinline__ double ljmain(const Tis& t, const CV& a, const CV& b) {
+// Coefficient of law `law` with c1 = a, c2 = b (cell_interaction.cpp:77-285).
+//
+// Most laws are one of three forms, and neighbouring lanes meet all of them:
+//   L  4 eps Q (Q - 1) / s     ljmain, and MEMB-MEMB below cr_dist
+//   A  -(K / d) x (1 - x^2 / c) adhesion, x = Q - 1 (0 past LJ_THRESH)
+//   S  -(K / d) (Q - 1)         the FIX-MEMB anchor, and MEMB-MEMB up to contact
+// with s = d^2.  Q and the second quotient are each a numerator over a
+// denominator chosen per lane, so a wave pays for one square root and three
+// FP64 divisions whatever its lanes hold, not for every law's own; the
+// operands and their order are each law's.  The rare forms (DER-DER,
+// stretched MEMB-MEMB, the pair spring) follow in branches of their own.
+// PAIR false leaves out the pair spring, which no list entry takes.
+template <bool PAIR>
+__device__ __forceinline__ double coef_law(const Tis& t, int law, const CV& a, const CV& b, Status* st) {
   const double distSq = dist_sq(t, a.p, b.p);
   const double rad_sum = a.r + b.r;
-  const double LJ6 = POW6(rad_sum) / POW3(distSq);
-  return 4.0 * t.m_eps * LJ6 * (LJ6 - 1) / distSq;
-}
-__device__ __forceinline__ bool is_near(const Tis& t, const CV& a, const CV& b) {
-  return dist_sq(t, a.p, b.p) < (a.r + b.r) * (a.r + b.r);
-}
-__device__ __forceinline__ double adhesion(const Tis& t, const CV& a, const CV& b, double spring_const) {
-  const double distlj = sqrt(dist_sq(t, a.p, b.p));
-  const double rad_sum = a.r + b.r;
-  const double LJ2_m1 = (distlj / rad_sum) - 1;
-  return (LJ2_m1 + 1 > t.prm.LJ_THRESH ? 0.0
-          : -(spring_const / distlj) * LJ2_m1 *
-                (1 - LJ2_m1 * LJ2_m1 / ((t.prm.LJ_THRESH - 1.0) * (t.prm.LJ_THRESH - 1.0))));
-}
-
-// Coefficient of law `law` with c1 = a, c2 = b (cell_interaction.cpp:77-285).
-__device__ double coef_law(const Tis& t, int law, const CV& a, const CV& b, Status* st) {
-  switch (law) {
-    case LAW_OTHER:
-      return ljmain(t, a, b);
-    case LAW_DER_DER: {
-      const double dist = sqrt(dist_sq(t, a.p, b.p));
-      if (dist + t.prm.delta_R < a.r + b.r) {
-        const double dist2 = dist + t.prm.delta_R;
-        const double rad_sum = a.r + b.r;
-        const double LJ6 = POW6(rad_sum) / POW6(dist2);
-        return 4.0 * t.m_eps * LJ6 * (LJ6 - 1) / (dist * dist2) + t.prm.para_ljp2;
-      } else if (is_near(t, a, b)) {
-        return t.prm.para_ljp2;
-      } else {
-        const double dist2 = dist + t.prm.delta_R;
-        const double rad_sum = a.r + b.r;
-        const double LJ6 = POW6(rad_sum) / POW6(dist2);
-        return 4.0 * t.m_eps * LJ6 * (LJ6 - 1) / (dist * dist) + t.prm.para_ljp2;
-      }
-    }
-    case LAW_ALAIRDE:
-      if (is_near(t, a, b)) return ljmain(t, a, b);
-      else {
-        double spf = (t.m_kadh * t.prm.K_DESMOSOME_RATIO);
-        if (a.agek > t.prm.THRESH_SP && b.agek > t.prm.THRESH_SP) spf = t.m_kadh;
-        return adhesion(t, a, b, spf);
-      }
-    case LAW_FIXMU:
-      if (is_near(t, a, b)) return ljmain(t, a, b);
-      return adhesion(t, a, b, (t.m_kadh * t.prm.K_DESMOSOME_RATIO));
-    case LAW_MU_MEMB: {
-      if (is_near(t, a, b)) return ljmain(t, a, b);
-      // spring_force_to_memb, set at the top of _MUSUME_interaction (:613-620)
-      double spring = 0;
-      if (a.pair >= 0 && t.state[a.pair] == FIX) spring = t.m_kspring;
-      else if (a.rdt > 0) spring = t.prm.Kspring_d;
-      return adhesion(t, a, b, spring);
-    }
-    case LAW_FIX_MEMB:
-      if (is_near(t, a, b)) return ljmain(t, a, b);
-      else {
-        const double distlj = sqrt(dist_sq(t, a.p, b.p));
-        const double LJ2 = distlj / (a.r + b.r);
-        return -(t.m_kspring / distlj) * (LJ2 - 1.0);
-      }
-    case LAW_MEMB_MEMB: {
-      const double rad_sum = a.r + b.r;
-      const double rad_sum_sq = rad_sum * rad_sum;
-      double cr_dist_sq;
-      const double distSq = dist_sq(t, a.p, b.p);
-      double tmp;
-      if (distSq < (cr_dist_sq = rad_sum_sq * t.prm.P_MEMB * t.prm.P_MEMB)) {
-        const double LJ6 = POW3(cr_dist_sq) / POW3(distSq);
-        tmp = 4.0 * t.m_eps * LJ6 * (LJ6 - 1) / distSq;
-      } else if (distSq < rad_sum_sq) {
-        const double distlj = sqrt(distSq);
-        const double cr_dist = rad_sum * t.prm.P_MEMB;
-        tmp = -(t.prm.DER_DER_CONST / distlj) * (distlj / cr_dist - 1.0);
-      } else {
-        const double distlj = sqrt(distSq);
-        const double lambda_dist = (1.0 + t.prm.P_MEMB) * rad_sum;
-        const double cr_dist = rad_sum * t.prm.P_MEMB;
-        const double LJ6 = POW6(cr_dist) / POW6(lambda_dist - distlj);
-        tmp = -(t.prm.DER_DER_CONST / rad_sum) * ((1.0 - t.prm.P_MEMB) / t.prm.P_MEMB)
-              - 4 * t.m_eps * (LJ6 * (LJ6 - 1.0)) / ((lambda_dist - distlj) * distlj);
-      }
-      if (fabs(tmp) > 100) set_err(st, ERR_STRONG_INTERACTION);
-      return tmp;
-    }
-    case LAW_PAIR: {
-      const double dist = sqrt(dist_sq(t, a.p, b.p));
-      const double force = t.prm.Kspring_division * (dist - a.snl);
-      return -force / dist;
-    }
-    default:
-      return 0.0;
+  const double dist = sqrt(distSq);
+  if (PAIR && law == LAW_PAIR) {
+    const double force = t.prm.Kspring_division * (dist - a.snl);
+    return -force / dist;
   }
+  if (law == LAW_DER_DER) {
+    if (dist + t.prm.delta_R < rad_sum) {
+      const double dist2 = dist + t.prm.delta_R;
+      const double LJ6 = POW6(rad_sum) / POW6(dist2);
+      return 4.0 * t.m_eps * LJ6 * (LJ6 - 1) / (dist * dist2) + t.prm.para_ljp2;
+    }
+    if (distSq < rad_sum * rad_sum) return t.prm.para_ljp2;
+    const double dist2 = dist + t.prm.delta_R;
+    const double LJ6 = POW6(rad_sum) / POW6(dist2);
+    return 4.0 * t.m_eps * LJ6 * (LJ6 - 1) / (dist * dist) + t.prm.para_ljp2;
+  }
+  const bool memb = law == LAW_MEMB_MEMB;
+  const double rad_sum_sq = rad_sum * rad_sum;
+  const double cr_dist = rad_sum * t.prm.P_MEMB;
+  const double cr_dist_sq = rad_sum_sq * t.prm.P_MEMB * t.prm.P_MEMB;
+  if (memb && !(distSq < cr_dist_sq) && !(distSq < rad_sum_sq)) {   // stretched MEMB-MEMB
+    const double lambda_dist = (1.0 + t.prm.P_MEMB) * rad_sum;
+    const double LJ6 = POW6(cr_dist) / POW6(lambda_dist - dist);
+    const double tmp = -(t.prm.DER_DER_CONST / rad_sum) * ((1.0 - t.prm.P_MEMB) / t.prm.P_MEMB)
+                       - 4 * t.m_eps * (LJ6 * (LJ6 - 1.0)) / ((lambda_dist - dist) * dist);
+    if (fabs(tmp) > 100) set_err(st, ERR_STRONG_INTERACTION);
+    return tmp;
+  }
+  // is_near: every law but LAW_OTHER takes ljmain within contact
+  const bool L = law == LAW_OTHER || (memb ? distSq < cr_dist_sq : distSq < rad_sum * rad_sum);
+  double K = t.m_kadh * t.prm.K_DESMOSOME_RATIO;   // LAW_FIXMU, LAW_ALAIRDE
+  if (law == LAW_ALAIRDE) {
+    if (a.agek > t.prm.THRESH_SP && b.agek > t.prm.THRESH_SP) K = t.m_kadh;
+  } else if (law == LAW_MU_MEMB) {
+    // spring_force_to_memb, set at the top of _MUSUME_interaction (:613-620)
+    K = 0;
+    if (!L) {
+      if (a.pair >= 0 && t.state[a.pair] == FIX) K = t.m_kspring;
+      else if (a.rdt > 0) K = t.prm.Kspring_d;
+    }
+  } else if (law == LAW_FIX_MEMB) {
+    K = t.m_kspring;
+  } else if (memb) {
+    K = t.prm.DER_DER_CONST;
+  }
+  const double n1 = L ? (memb ? POW3(cr_dist_sq) : POW6(rad_sum)) : dist;
+  const double d1 = L ? POW3(distSq) : (memb ? cr_dist : rad_sum);
+  const double Q = n1 / d1;
+  const double x = Q - 1.0;
+  const double k2 = (L ? 4.0 * t.m_eps * Q * x : K) / (L ? distSq : dist);
+  if (L) {
+    if (memb && fabs(k2) > 100) set_err(st, ERR_STRONG_INTERACTION);
+    return k2;
+  }
+  if (law == LAW_FIX_MEMB) return -k2 * x;
+  if (memb) {
+    const double tmp = -k2 * x;
+    if (fabs(tmp) > 100) set_err(st, ERR_STRONG_INTERACTION);
+    return tmp;
+  }
+  const double c2 = (t.prm.LJ_THRESH - 1.0) * (t.prm.LJ_THRESH - 1.0);
+  return x + 1 > t.prm.LJ_THRESH ? 0.0 : -k2 * x * (1 - x * x / c2);
 }
 
 // cell_interaction_apply (:48-66): the displacement added to c1, subtracted from c2
-__device__ __forceinline__ P3 delta(const Tis& t, int law, const CV& a, const CV& b, Status* st) {
-  const double coef = coef_law(t, law, a, b, st);
+template <bool PAIR>
+__device__ __forceinline__ P3 delta_law(const Tis& t, int law, const CV& a, const CV& b, Status* st) {
+  const double coef = coef_law<PAIR>(t, law, a, b, st);
   if (fabs(coef) > 1000) set_err(st, ERR_STRONG_INTERACTION);
   const double d = t.prm.DT_Cell * coef;
   return P3{d * p_diff_x(t, a.p.x, b.p.x), d * p_diff_y(t, a.p.y, b.p.y), d * (a.p.z - b.p.z)};
 }
+__device__ P3 delta(const Tis& t, int law, const CV& a, const CV& b, Status* st) { return delta_law<true>(t, law, a, b, st); }
 
 // wall_interaction (:287-294): the z increment
 __device__ __forceinline__ double wall_dz(const Tis& t, const CV& c) {
@@ -199,23 +183,30 @@ __device__ __forceinline__ double bend_factor(double cdot) {   // :349-360
 }
 __device__ __forceinline__ P3 tri_rho(P3 n1, P3 b1) { return v_sub(b1, v_scale(v_dot(n1, b1), n1)); }
 
-__device__ P3 tri_bend_1(const Tis& t, P3 r1v, P3 a1v, P3 b1v, P3 c1v) {   // :468-474
-  P3 norm1_pre = v_cross(vpsub(t, r1v, b1v), vpsub(t, a1v, b1v));
-  P3 norm1 = v_normalize(norm1_pre);
-  P3 n2 = v_cross(vpsub(t, a1v, b1v), vpsub(t, c1v, b1v));
-  P3 norm2 = v_normalize(n2);
-  double dot1 = v_dot(norm1, norm2);
-  return v_scale(bend_factor(dot1), v_div(v_cross(vpsub(t, a1v, b1v), tri_rho(norm1, norm2)), v_norm(norm1_pre)));
+// Term i of a membrane particle's 12 dihedral terms: tri_bend_1 (:468-474) of
+// (a, b, c) for i < 6, tri_bend_2 (:476-486) for the others.  With
+//   n1 = |A1 x A2|, n2 = |B1 x B2|, both unit,
+//   1: A1 = r - b, A2 = a - b, B1 = a - b, B2 = c - b, f(n1.n2) (a - b) x rho(n1, n2) / |n1|
+//   2: A1 = r - c, A2 = b - c, B1 = r - b, B2 = a - b,
+//      f(n1.n2) ((b - c) x rho(n1, n2) / |n1| + (a - b) x rho(n2, n1) / |n2|)
+// the two differ in the vectors they take and in the second summand, so the
+// lanes of a particle run one code path for both.
+__device__ __forceinline__ P3 p3_sel(bool c, P3 a, P3 b) { return P3{c ? a.x : b.x, c ? a.y : b.y, c ? a.z : b.z}; }
+__device__ __forceinline__ P3 tri_bend(const Tis& t, bool second, P3 r1v, P3 a1v, P3 b1v, P3 c1v) {
+  const P3 ab = vpsub(t, a1v, b1v), rb = vpsub(t, r1v, b1v);
+  const P3 rc = vpsub(t, r1v, c1v);
+  // c - b of form 1, b - c of form 2 (vpsub is not antisymmetric at half a box)
+  const P3 bc = vpsub(t, p3_sel(second, b1v, c1v), p3_sel(second, c1v, b1v));
+  P3 norm1_pre = v_cross(p3_sel(second, rc, rb), p3_sel(second, bc, ab));
+  P3 norm2_pre = v_cross(p3_sel(second, rb, ab), p3_sel(second, ab, bc));
+  const P3 norm1 = v_normalize(norm1_pre), norm2 = v_normalize(norm2_pre);
+  const double dot1 = v_dot(norm1, norm2);
+  P3 s = v_div(v_cross(p3_sel(second, bc, ab), tri_rho(norm1, norm2)), v_norm(norm1_pre));
+  if (second) s = v_add(s, v_div(v_cross(ab, tri_rho(norm2, norm1)), v_norm(norm2_pre)));
+  return v_scale(bend_factor(dot1), s);
 }
-__device__ P3 tri_bend_2(const Tis& t, P3 r1v, P3 a1v, P3 b1v, P3 c1v) {   // :476-486
-  P3 norm1_pre = v_cross(vpsub(t, r1v, c1v), vpsub(t, b1v, c1v));
-  P3 norm2_pre = v_cross(vpsub(t, r1v, b1v), vpsub(t, a1v, b1v));
-  P3 norm1 = v_normalize(norm1_pre), norm2 = v_normalize(norm2_pre);
-  double dot1 = v_dot(norm1, norm2);
-  return v_scale(bend_factor(dot1),
-                 v_add(v_div(v_cross(vpsub(t, b1v, c1v), tri_rho(norm1, norm2)), v_norm(norm1_pre)),
-                       v_div(v_cross(vpsub(t, a1v, b1v), tri_rho(norm2, norm1)), v_norm(norm2_pre))));
-}
+__device__ P3 tri_bend_1(const Tis& t, P3 r1v, P3 a1v, P3 b1v, P3 c1v) { return tri_bend(t, false, r1v, a1v, b1v, c1v); }
+__device__ P3 tri_bend_2(const Tis& t, P3 r1v, P3 a1v, P3 b1v, P3 c1v) { return tri_bend(t, true, r1v, a1v, b1v, c1v); }
 
 // ---- serial form: one lane does a whole cell --------------------------------
 // Used for rows longer than the LDS slots of the cooperative kernel.
@@ -327,23 +318,32 @@ __device__ void forces_serial(const Tis& t, int pb, int cb, int X, Status* st) {
 
 // ---- cooperative form --------------------------------------------------------
 // A group of FG lanes owns one cell.  Every list entry e is handled by lane
-// e % FG, which evaluates both displacements the pair can contribute to the
-// cell: "own" (the cell's handler processes the entry, added) and "oth" (the
-// entry's handler processes the cell, subtracted).  The group leader then
-// adds them in the serial order of cell_interaction (:650-679): bending,
-// wall, lower-index handlers ascending, the cell's own list, its pair,
-// higher-index handlers ascending with a higher-index partner's spring
-// after that partner's list.  Lane 0..11 evaluate the 12 dihedral terms of a
-// membrane particle.
+// e % FG, which evaluates the displacement the pair contributes to the cell:
+// "own" (the cell's handler processes the entry, added) or "oth" (the entry's
+// handler processes the cell, subtracted).  Only a DER-DER pair has both; it
+// takes a second turn of the same code, so the laws are compiled once.  The
+// group's first three lanes then add them, one coordinate each, in the serial
+// order of cell_interaction (:650-679): bending, wall, lower-index handlers
+// ascending, the cell's own list, its pair, higher-index handlers ascending
+// with a higher-index partner's spring after that partner's list.  Lane 0..11
+// evaluate the 12 dihedral terms of a membrane particle.
 //
 // An absent "own" term is stored as -0.0 and an absent "oth" term as +0.0:
-// x + (-0.0) and x - (+0.0) are x for every x, so the leader adds and
-// subtracts every slot without flags or branches, four slots' LDS reads
-// ahead of their adds, in the same order and with the same results.
+// x + (-0.0) and x - (+0.0) are x for every x, so the sums take every slot
+// without flags or branches, four slots' LDS reads ahead of their adds, in
+// the same order and with the same results.
 //
 // Each group takes one cell, so the grid must cover all cells (a launch that
 // does not is reported as ERR_INVALID); a loop over cells would keep the
 // math's loop-invariant constants in registers and cost occupancy.
+//
+// What bounds it: FP64 issue of the laws (divergent lanes run one after the
+// other) and, on a small tissue, the chain of round trips and the ordered
+// sum.  One copy of the laws with shared divisions, one path for both
+// dihedral forms and one coordinate per summing lane, against every law and
+// form on its own and a leader summing all three: 100 steps of one tissue of
+// 3,900 cells 1490 -> 1073 us, of 24 tissues (with their reverse pass) 30.3 ->
+// 26.9 ms.
 //
 // FCAP, the LDS slots per cell, is chosen per launch from the longest list
 // built so far: 40 keeps a 128-lane block's LDS small enough for 4 waves per
@@ -353,16 +353,30 @@ constexpr int FG = 16;
 constexpr int F_BLOCK = 128;
 constexpr int F_GROUPS = F_BLOCK / FG;
 
-// a group's LDS slots, padded by 8 bytes so that the leaders of a wave's
-// groups read different banks
+// a group's LDS slots, padded by 8 bytes so that the summing lanes of a
+// wave's groups read different banks
 template <int FCAP>
 struct FRow {
   P3 v[FCAP];
   double pad;
 };
 
-__device__ __forceinline__ void p3_add(P3& a, const P3& d) { a.x += d.x; a.y += d.y; a.z += d.z; }
-__device__ __forceinline__ void p3_sub(P3& a, const P3& d) { a.x -= d.x; a.y -= d.y; a.z -= d.z; }
+// acc +- the coordinate at v[3 e] for e in [e0, e1), in order
+template <bool ADD>
+__device__ __forceinline__ double sum_slots(double acc, const double* v, int e0, int e1) {
+  int e = e0;
+#pragma unroll 1
+  for (; e + 4 <= e1; e += 4) {
+    double d[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) d[j] = v[3 * (e + j)];
+#pragma unroll
+    for (int j = 0; j < 4; j++) acc = ADD ? acc + d[j] : acc - d[j];
+  }
+  for (; e < e1; e++) acc = ADD ? acc + v[3 * e] : acc - v[3 * e];
+  return acc;
+}
+__device__ __forceinline__ double p3_at(const P3& p, int k) { return k == 0 ? p.x : k == 1 ? p.y : p.z; }
 
 template <int FCAP>
 __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, int pb, int cb) {
@@ -370,16 +384,15 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
   Status* st = t.st;
   __shared__ FRow<FCAP> s_own[F_GROUPS];
   __shared__ FRow<FCAP> s_oth[F_GROUPS];
-  __shared__ int s_idx[F_GROUPS][FCAP];
-  __shared__ uint8_t s_flag[F_GROUPS][FCAP];
+  __shared__ __align__(16) int s_idx[F_GROUPS][FCAP];
   __shared__ uint8_t s_perm[F_GROUPS][FCAP];
   __shared__ P3 s_bend[F_GROUPS][12];
   const int lane = threadIdx.x & (FG - 1);
   const int grp = threadIdx.x / FG;
   const int X = blockIdx.x * F_GROUPS + grp;
   if (X >= t.cap) return;
-  // the cell's own words (and its lane's first list word) are loaded before
-  // the cell count arrives, in one round trip with it: a cell past the count
+  // the cell's own words (and its lane's list words) are loaded before the
+  // cell count arrives, in one round trip with it: a cell past the count
   // reads allocated, stale slots and leaves once the count is in
   const int len = t.nlen[cb][X];
   const CV cx = load_cv(t, pb, X);
@@ -391,146 +404,144 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
   if (blockIdx.x == 0 && threadIdx.x == 0 && (long long)gridDim.x * F_GROUPS < n) set_err(st, ERR_INVALID);
   if (X >= n) return;
   if (len > FCAP) return;   // k_forces_long
+  bool hi = false;          // this lane's membrane slot is subtracted (its handler has the higher index)
+#pragma unroll 1
   for (int e = lane; e < len; e += FG) {
     const int q = e == lane ? q0 : row[e];
     const CV cq = load_cv(t, pb, q);
-    uint8_t f = 0;
-    P3 own = P3{-0.0, -0.0, -0.0}, oth = P3{0, 0, 0};
+    int law = LAW_NONE, law2 = LAW_NONE;
+    bool own = false;
     if (memb) {
-      if (e < MEMB_ADJ) {
-        if (cq.s == MEMB) {
-          if (X > q) { own = delta(t, LAW_MEMB_MEMB, cx, cq, st); f |= 1; }
-          else if (q > X) { oth = delta(t, LAW_MEMB_MEMB, cq, cx, st); f |= 2; }
-        }
-      } else {
-        const int law2 = proc_law(cq, q, cx, X);
-        if (law2 != LAW_NONE) { oth = delta(t, law2, cq, cx, st); f |= 2; }
+      if (e >= MEMB_ADJ) {
+        law = proc_law(cq, q, cx, X);
+      } else if (cq.s == MEMB && X != q) {
+        law = LAW_MEMB_MEMB;
+        own = X > q;
+        hi = !own;
       }
     } else {
-      const int law = proc_law(cx, X, cq, q);
-      if (law != LAW_NONE) { own = delta(t, law, cx, cq, st); f |= 1; }
-      if (e >= nA || cq.s != MEMB) {
-        const int law2 = proc_law(cq, q, cx, X);
-        if (law2 != LAW_NONE) { oth = delta(t, law2, cq, cx, st); f |= 2; }
+      law = proc_law(cx, X, cq, q);
+      if (e >= nA || cq.s != MEMB) law2 = proc_law(cq, q, cx, X);
+      own = law != LAW_NONE;
+      if (!own) {
+        law = law2;
+        law2 = LAW_NONE;
       }
     }
     s_idx[grp][e] = q;
-    s_flag[grp][e] = f;
-    s_own[grp].v[e] = own;
-    s_oth[grp].v[e] = oth;
+    s_own[grp].v[e] = P3{-0.0, -0.0, -0.0};
+    s_oth[grp].v[e] = P3{0, 0, 0};
+#pragma unroll 1
+    while (law != LAW_NONE) {
+      CV a, b;
+      a.p = p3_sel(own, cx.p, cq.p); b.p = p3_sel(own, cq.p, cx.p);
+      a.r = cx.r; b.r = cq.r;            // the sum of the two radii alone is read
+      a.agek = cx.agek; b.agek = cq.agek;   // and whether both ages pass a threshold
+      a.pair = own ? cx.pair : cq.pair;
+      a.rdt = own ? cx.rdt : cq.rdt;
+      const P3 d = delta_law<false>(t, law, a, b, st);
+      if (own) s_own[grp].v[e] = d;
+      else s_oth[grp].v[e] = d;
+      law = law2;
+      law2 = LAW_NONE;
+      own = false;
+    }
   }
   if (memb && lane < 12) {
     const int* md = t.memb6 + 6 * X;
     const int i = lane < 6 ? lane : lane - 6;
-    const P3 a = ld_pos(t, pb, md[i]);
-    const P3 b = ld_pos(t, pb, md[(i + 1) % 6]);
-    if (lane < 6)
-      s_bend[grp][lane] = tri_bend_1(t, cx.p, a, b, ld_pos(t, pb, t.memb6[6 * md[(i + 1) % 6] + i]));
-    else
-      s_bend[grp][lane] = tri_bend_2(t, cx.p, a, b, ld_pos(t, pb, md[(i + 2) % 6]));
+    const int ma = md[i], mb = md[(i + 1) % 6];
+    const int mc = lane < 6 ? t.memb6[6 * mb + i] : md[(i + 2) % 6];
+    s_bend[grp][lane] = tri_bend(t, lane >= 6, cx.p, ld_pos(t, pb, ma), ld_pos(t, pb, mb), ld_pos(t, pb, mc));
   }
   wave_sync();
-  // rank of each lower-part entry by cell index
-  for (int e = lane; e < nA; e += FG) {
-    const int v = s_idx[grp][e];
-    int r = 0;
-    for (int k = 0; k < nA; k++) r += s_idx[grp][k] < v;
-    s_perm[grp][r] = (uint8_t)e;
-  }
-  wave_sync();
-  if (lane != 0) return;
-  const P3* own = s_own[grp].v;
-  const P3* oth = s_oth[grp].v;
-  P3 acc = cx.p;
+  int nhi = 0;
   if (memb) {
-    P3 dr = P3{0, 0, 0};
-    for (int i = 0; i < 12; i++) dr = v_add(dr, s_bend[grp][i]);
-    acc.x += t.prm.DT_Cell * t.m_kbend * dr.x;
-    acc.y += t.prm.DT_Cell * t.m_kbend * dr.y;
-    acc.z += t.prm.DT_Cell * t.m_kbend * dr.z;
-    if (cx.p.z < cx.r) acc.z += wall_dz(t, cx);
-    int hi[6], nhi = 0;
-    for (int e = 0; e < MEMB_ADJ; e++) {
-      p3_add(acc, own[e]);
-      if (s_flag[grp][e] & 2) {
-        int k = nhi++;
-        const int q = s_idx[grp][e];
-        while (k > 0 && s_idx[grp][hi[k - 1]] > q) { hi[k] = hi[k - 1]; k--; }
-        hi[k] = e;
+    // the membrane slots that are subtracted, ascending by cell index
+    const unsigned m = (unsigned)(__ballot(hi) >> (threadIdx.x & 48)) & 0x3fu;
+    nhi = __popc(m);
+    if (hi) {
+      const int v = s_idx[grp][lane];
+      int r = 0;
+      for (int k = 0; k < MEMB_ADJ; k++) r += ((m >> k) & 1u) && s_idx[grp][k] < v;
+      s_perm[grp][r] = (uint8_t)lane;
+    }
+  } else {
+    // rank of each lower-part entry by cell index
+    for (int e = lane; e < nA; e += FG) {
+      const int v = s_idx[grp][e];
+      int r = 0, k = 0;
+      for (; k + 4 <= nA; k += 4) {
+        const int4 w = *reinterpret_cast<const int4*>(&s_idx[grp][k]);
+        r += (w.x < v) + (w.y < v) + (w.z < v) + (w.w < v);
       }
+      for (; k < nA; k++) r += s_idx[grp][k] < v;
+      s_perm[grp][r] = (uint8_t)e;
     }
-    for (int i = 0; i < nhi; i++) p3_sub(acc, oth[hi[i]]);
-    int e = MEMB_ADJ;
-#pragma unroll 1
-    for (; e + 4 <= len; e += 4) {
-      P3 d[4];
+  }
+  wave_sync();
+  if (lane >= 3) return;
+  const double* own = reinterpret_cast<const double*>(s_own[grp].v) + lane;
+  const double* oth = reinterpret_cast<const double*>(s_oth[grp].v) + lane;
+  double acc = p3_at(cx.p, lane);
+  if (memb) {
+    const double* bend = reinterpret_cast<const double*>(s_bend[grp]) + lane;
+    double dr = 0;
 #pragma unroll
-      for (int j = 0; j < 4; j++) d[j] = oth[e + j];
+    for (int i = 0; i < 12; i++) dr = dr + bend[3 * i];
+    acc += t.prm.DT_Cell * t.m_kbend * dr;
+    if (lane == 2 && cx.p.z < cx.r) acc += wall_dz(t, cx);
 #pragma unroll
-      for (int j = 0; j < 4; j++) p3_sub(acc, d[j]);
-    }
-    for (; e < len; e++) p3_sub(acc, oth[e]);
+    for (int e = 0; e < MEMB_ADJ; e++) acc += own[3 * e];
+    for (int i = 0; i < nhi; i++) acc -= oth[3 * s_perm[grp][i]];
+    acc = sum_slots<false>(acc, oth, MEMB_ADJ, len);
   } else {
     {
       int r = 0;
 #pragma unroll 1
       for (; r + 4 <= nA; r += 4) {
         int k[4];
-        P3 d[4];
+        double d[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) k[j] = s_perm[grp][r + j];
 #pragma unroll
-        for (int j = 0; j < 4; j++) d[j] = oth[k[j]];
+        for (int j = 0; j < 4; j++) d[j] = oth[3 * k[j]];
 #pragma unroll
-        for (int j = 0; j < 4; j++) p3_sub(acc, d[j]);
+        for (int j = 0; j < 4; j++) acc -= d[j];
       }
-      for (; r < nA; r++) p3_sub(acc, oth[s_perm[grp][r]]);
+      for (; r < nA; r++) acc -= oth[3 * s_perm[grp][r]];
     }
-    if (cx.s == DER && cx.p.z < cx.r) acc.z += wall_dz(t, cx);
-    {
-      int e = 0;
-#pragma unroll 1
-      for (; e + 4 <= len; e += 4) {
-        P3 d[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) d[j] = own[e + j];
-#pragma unroll
-        for (int j = 0; j < 4; j++) p3_add(acc, d[j]);
-      }
-      for (; e < len; e++) p3_add(acc, own[e]);
-    }
-    if (cx.pair >= 0 && X > cx.pair) p3_add(acc, delta(t, LAW_PAIR, cx, load_cv(t, pb, cx.pair), st));
-    int P = cx.pair > X ? cx.pair : -1;
-    if (P < 0) {
-      int e = nA;
-#pragma unroll 1
-      for (; e + 4 <= len; e += 4) {
-        P3 d[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) d[j] = oth[e + j];
-#pragma unroll
-        for (int j = 0; j < 4; j++) p3_sub(acc, d[j]);
-      }
-      for (; e < len; e++) p3_sub(acc, oth[e]);
+    if (lane == 2 && cx.s == DER && cx.p.z < cx.r) acc += wall_dz(t, cx);
+    acc = sum_slots<true>(acc, own, 0, len);
+    if (cx.pair < 0) {
+      acc = sum_slots<false>(acc, oth, nA, len);
     } else {
-      for (int e = nA; e < len; e++) {
-        const int p = s_idx[grp][e];
-        if (P >= 0 && P < p) {
-          p3_sub(acc, delta(t, LAW_PAIR, load_cv(t, pb, P), cx, st));
-          P = -1;
+      // the pair's spring: added after the own list when this cell has the
+      // higher index, else subtracted after the partner's list
+      const CV cp = load_cv(t, pb, cx.pair);
+      const bool up = X > cx.pair;
+      const double dp = p3_at(up ? delta(t, LAW_PAIR, cx, cp, st) : delta(t, LAW_PAIR, cp, cx, st), lane);
+      if (up) {
+        acc = sum_slots<false>(acc + dp, oth, nA, len);
+      } else {
+        int P = cx.pair;
+        for (int e = nA; e < len; e++) {
+          const int p = s_idx[grp][e];
+          if (P >= 0 && P < p) {
+            acc -= dp;
+            P = -1;
+          }
+          acc -= oth[3 * e];
+          if (p == P) {
+            acc -= dp;
+            P = -1;
+          }
         }
-        p3_sub(acc, oth[e]);
-        if (p == P) {
-          p3_sub(acc, delta(t, LAW_PAIR, load_cv(t, pb, P), cx, st));
-          P = -1;
-        }
+        if (P >= 0) acc -= dp;
       }
-      if (P >= 0) p3_sub(acc, delta(t, LAW_PAIR, load_cv(t, pb, P), cx, st));
     }
   }
-  t.pos[1 - pb][0][X] = acc.x;
-  t.pos[1 - pb][1][X] = acc.y;
-  t.pos[1 - pb][2][X] = acc.z;
+  t.pos[1 - pb][lane][X] = acc;
 }
 
 // cells whose rows exceed the LDS slots (cap) of k_forces, one lane per cell

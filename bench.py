@@ -56,7 +56,7 @@ STEP_GROUPS = (
 # the voxel maps, written once per step over the active box (cmap1 4 + cmap2
 # 1 per voxel; the B stencil's 21 bytes per point count their reads), and
 # the B stencil
-MAP_KERNELS = ("k_zz_set", "k_zzmax", "k_map_clear", "k_map_stamp", "k_map_halo")
+MAP_KERNELS = ("k_zz_set", "k_zzmax", "k_map_clear", "k_map_stamp")
 MAP_BYTES_PER_VOXEL = 5.0
 
 

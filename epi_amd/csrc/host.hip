@@ -82,7 +82,7 @@ namespace {
 const char* kKernelNames[K_COUNT] = {
     "k_forces", "k_forces_long", "k_renew_flags", "k_renew_scan", "k_renew_apply", "k_remove", "k_pair_disperse",
     "k_initialize_sc", "k_periodic_fix", "k_bucket_insert", "k_bucket_sort", "k_sweep",
-    "k_finish", "k_snapshot", "k_zz_set", "k_zzmax", "k_map_clear", "k_map_stamp", "k_map_halo",
+    "k_finish", "k_snapshot", "k_zz_set", "k_zzmax", "k_map_clear", "k_map_stamp",
     "k_ext_stim", "k_ca_begin", "k_ca_vox", "k_ca_cells", "k_atp", "k_ca_end", "k_sw_reset",
     "k_rd_snapshot", "k_rd_restore", "k_rd_put_gj", "k_rd_state", "k_rd_seed",
     "k_rd_step", "k_rd_gj0", "k_rd_own", "k_mech_state", "k_mech_seed", "k_mech_bwd_begin",
@@ -398,11 +398,6 @@ int max_nb(const epi_ctx* c) {
 long long max_gsize(const epi_ctx* c) {
   long long m = 1;
   for (auto& h : c->th) m = std::max(m, h.gsize);
-  return m;
-}
-int max_halo(const epi_ctx* c) {
-  int m = 1;
-  for (auto& h : c->th) m = std::max(m, (h.NX + 1 + h.NY + 1) * h.NZ);
   return m;
 }
 int max_nx(const epi_ctx* c) {
@@ -1114,7 +1109,7 @@ int epi_calc_zzmax(epi_ctx* c, double* zzmax) {
 
 int epi_setup_map_lat(epi_ctx* c) {
   if (!c) return EPI_ERR_INVALID;
-  launch_maps(c->stream, c->d_tis, c->T, c->pb, max_n(c), max_gsize(c), max_halo(c), c->tu);
+  launch_maps(c->stream, c->d_tis, c->T, c->pb, max_n(c), max_gsize(c), c->tu);
   HIPCHK(c, hipGetLastError());
   return EPI_OK;
 }
@@ -1242,7 +1237,7 @@ hipError_t issue_build(epi_ctx* c, int mn, int nb, int izb, bool join = true) {
   if (c->tu.side_fork) chk(hipEventRecord(c->ev_fork, c->stream));
   chk(hipStreamWaitEvent(c->side_stream, c->ev_fork, 0));
   launch_zzmax(c->side_stream, c->d_tis, c->T, c->pb, mn);
-  launch_maps(c->side_stream, c->d_tis, c->T, c->pb, mn, max_gsize(c), max_halo(c), c->tu);
+  launch_maps(c->side_stream, c->d_tis, c->T, c->pb, mn, max_gsize(c), c->tu);
   launch_ext_stim(c->side_stream, c->d_tis, c->T, c->bp, b_tiles_est(c), c->d_wl, c->tu);
   chk(hipEventRecord(c->ev_join, c->side_stream));
   if (join) chk(hipStreamWaitEvent(c->stream, c->ev_join, 0));
@@ -1262,7 +1257,7 @@ int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
       (1ull << K_RENEW_FLAGS) | (1ull << K_RENEW_SCAN) | (1ull << K_RENEW_APPLY) | (1ull << K_REMOVE) |
       (1ull << K_PAIR_DISPERSE) | (1ull << K_BUCKET_INSERT) | (1ull << K_BUCKET_SORT) | (1ull << K_SWEEP_WAVE) |
       (1ull << K_SWEEP) | (1ull << K_FINISH) | (1ull << K_SNAPSHOT) | (1ull << K_ZZ_SET) | (1ull << K_ZZMAX) |
-      (1ull << K_MAP_CLEAR) | (1ull << K_MAP_STAMP) | (1ull << K_MAP_HALO) | (1ull << K_EXT_STIM);
+      (1ull << K_MAP_CLEAR) | (1ull << K_MAP_STAMP) | (1ull << K_EXT_STIM);
   if (!c->tu.step_graph || (g_prof.mask & seg)) {
     *joined = false;
     HIPCHK(c, issue_build(c, mn, nb, izb, false));
@@ -1273,7 +1268,7 @@ int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
   for (auto& h : c->th) mcap = std::max(mcap, h.cap);
   const int mr = std::max(mn, std::min((mn + 1023) / 1024 * 1024, mcap));
   const Tuning& tu = c->tu;
-  const std::vector<long long> key = {1, c->pb, c->cb, c->cp, c->bp, nb, mr, izb, max_gsize(c), max_halo(c),
+  const std::vector<long long> key = {1, c->pb, c->cb, c->cp, c->bp, nb, mr, izb, max_gsize(c),
                                       max_nx(c), max_ny(c), tu.b_zb, tu.b_rows, tu.map_lanes, tu.sweep_wave, tu.side_fork};
   return graph_run(c, key, [&] { return issue_build(c, mr, nb, izb); });
 }

@@ -44,103 +44,108 @@ __device__ __forceinline__ int lat_wrap(long v, int N, Status* st) {
   if (i < 0 || i >= 3L * N) { set_err(st, ERR_OUT_OF_GRID); return (int)(((i % N) + N) % N); }
   return (int)(i % N);
 }
+// the same for a box index that rarely leaves [0, N): no division there
+__device__ __forceinline__ int lat_near(int v, int N, Status* st) {
+  if (v >= 0 && v < N) return v;
+  if (v < 0 && v >= -N) return v + N;
+  if (v >= N && v < 2 * N) return v - N;
+  return lat_wrap(v, N, st);
+}
 
-// set_lattice (:18-22) and the sphere stamping (:39-155); the last writer of
-// the serial loop is the highest cell index, hence atomicMax on cmap1.  One
-// lane per cell.
-// MS lanes per cell (1, 4 or 16, a launch shape) split each x slice of the
-// stamp box, its (y, z) voxels taken z fastest, round-robin: the lanes of a
-// cell touch voxels a plane apart.  The result does not depend on MS (a max
-// and idempotent stores).
+// set_lattice (:18-22), the sphere stamping (:39-155) and the periodic planes
+// x = NX and y = NY (:156-166); the last writer of the serial loop is the
+// highest cell index, hence atomicMax on cmap1.
+//
+// MS lanes per cell (1, 4 or 16, a launch shape) walk the stamp box x
+// fastest, so a group's lanes write runs of consecutive x of one or two
+// rows: a store or an atomic touches a few cache lines, where lanes a plane
+// apart touched one line each (bound by those transactions and, on a small
+// tissue, by the walk's length).  A voxel of row y = 0 or column x = 0 is
+// written to its periodic copies too, which the clear has emptied, so no
+// kernel copies the planes afterwards.  The result does not depend on MS (a
+// max and idempotent stores).  16 lanes against the z-fastest walk with its
+// default of one: 420 cells 39 -> 7.9 us, 36,000 cells 41 -> 16.5 us (23.9 with
+// 16 lanes there), 32 uneven tissues of 290,000 cells 577 -> 175 us, and no
+// copy kernel (5 to 23 us).
 template <int MS>
 __global__ void __launch_bounds__(128) k_map_stamp(const Tis* __restrict__ T, int pb) {
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;
-  const int n = st->n;
   const int zl = threadIdx.x & (MS - 1);
   const double FAC_MAP = t.prm.FAC_MAP;
+  const int NX = t.NX, NY = t.NY, NZ = t.NZ, XP = t.XP;
+  const long long PL = t.PL;
+  const double dx = t.dx, dy = t.dy, dz = t.dz;
+  int* __restrict__ cmap1 = t.cmap1;
+  uint8_t* __restrict__ cmap2 = t.cmap2;
   int ztop = 0;
-  for (int c = (blockIdx.x * blockDim.x + threadIdx.x) / MS; c < n; c += gridDim.x * blockDim.x / MS) {
-    const P3 p = ld_pos(t, pb, c);
-    const int lx = lat_wrap((long)(int)(p.x * t.inv_dx), t.NX, st);
-    const int ly = lat_wrap((long)(int)(p.y * t.inv_dy), t.NY, st);
-    const int lz = lat_wrap((long)(int)(p.z * t.inv_dz), t.NZ, st);
+  const int cap = t.cap;
+  int c = (blockIdx.x * blockDim.x + threadIdx.x) / MS;
+  // the first cell's words are loaded in one round trip with the cell count
+  // (a cell past the count reads allocated, stale slots)
+  const int c0 = c < cap ? c : cap - 1;
+  P3 p = ld_pos(t, pb, c0);
+  uint8_t s = t.state[c0];
+  double r = t.radius[c0];
+  const int n = st->n;
+  const int step = gridDim.x * blockDim.x / MS;
+  for (; c < n; c += step) {
+    const int lx = lat_wrap((long)(int)(p.x * t.inv_dx), NX, st);
+    const int ly = lat_wrap((long)(int)(p.y * t.inv_dy), NY, st);
+    const int lz = lat_wrap((long)(int)(p.z * t.inv_dz), NZ, st);
     if (zl == 0) { t.lat[3 * c] = lx; t.lat[3 * c + 1] = ly; t.lat[3 * c + 2] = lz; }
-    const uint8_t s = t.state[c];
     const bool afm = is_afm(s);
     const int irx = afm ? 2 * t.irx : t.irx, iry = afm ? 2 * t.iry : t.iry, irz = afm ? 2 * t.irz : t.irz;
-    const double r = t.radius[c];
     const double normal_radSq = r * r;
     const double crad = FAC_MAP * r;
     const double cradSq = crad * crad;
     const int z_b = lz - irz, z_u = lz + irz;
     const int zmin = z_b >= 1 ? z_b : 1;
-    const int zmax = z_u < t.NZ ? z_u : t.NZ - 1;
+    const int zmax = z_u < NZ ? z_u : NZ - 1;
     ztop = max(ztop, zmax);
     const int nzr = zmax - zmin + 1;
+    const int bx = 2 * irx + 1, by = 2 * iry + 1;
     if (nzr <= 0) {   // no plane to stamp: the box's x and y range is still checked
       if (zl == 0) {
-        for (int k = lx - irx; k <= lx + irx; k++) lat_wrap(k, t.NX, st);
-        for (int l = ly - iry; l <= ly + iry; l++) lat_wrap(l, t.NY, st);
+        for (int k = lx - irx; k <= lx + irx; k++) lat_wrap(k, NX, st);
+        for (int l = ly - iry; l <= ly + iry; l++) lat_wrap(l, NY, st);
       }
-      continue;
-    }
-    // this lane's first (y, z) voxel of a slice: the zl-th, z fastest
-    const int l_first = ly - iry + zl / nzr, m_first = zmin + zl % nzr;
-    for (int k = lx - irx; k <= lx + irx; k++) {
-      const double mx = k * t.dx;
-      const int ipx = lat_wrap(k, t.NX, st);
-      const double diffx = p_diff_x(t, mx, p.x);
-      const double diffxSq = diffx * diffx;
-      int m = m_first;
-      for (int l = l_first; l <= ly + iry;) {
-        const double my = l * t.dy;
-        const int ipy = lat_wrap(l, t.NY, st);
-        const double diffy = p_diff_y(t, my, p.y);
-        const double tmps = diffxSq + diffy * diffy;
-        for (; m <= zmax; m += MS) {
-          const double mz = m * t.dz;
-          const double diffz = mz - p.z;
-          const double distSq = tmps + diffz * diffz;
-          const long long v = gidx(t, ipx, ipy, m);
-          if (!afm) {
-            if (distSq < normal_radSq) atomicMax(&t.cmap1[v], c);
-          } else if (distSq < cradSq) {
-            t.cmap2[v] = 1;
-            if (distSq < normal_radSq) atomicMax(&t.cmap1[v], c);
+    } else {
+      // the zl-th voxel of the box, then every MS-th: (ix, iy, iz) with ix
+      // fastest, advanced by MS's own digits in that radix
+      const int sx = MS % bx, sy = MS / bx % by, sz = MS / (bx * by);
+      int ix = zl % bx, iy = zl / bx % by, iz = zl / (bx * by);
+      while (iz < nzr) {
+        const int k = lx - irx + ix, l = ly - iry + iy, m = zmin + iz;
+        const double diffx = p_diff_x(t, k * dx, p.x);
+        const double diffy = p_diff_y(t, l * dy, p.y);
+        const double diffz = m * dz - p.z;
+        const int ipx = lat_near(k, NX, st), ipy = lat_near(l, NY, st);
+        const double distSq = diffx * diffx + diffy * diffy + diffz * diffz;
+        const bool in1 = distSq < normal_radSq, in2 = afm && distSq < cradSq;
+        const bool mark = afm ? in1 && in2 : in1;
+        if (in2 || mark) {
+          const long long v = (long long)m * PL + ipy * XP + ipx;
+          // the voxel, and its copies in the planes x = NX, y = NY
+          for (int copy = 0; copy < 4; copy++) {
+            if (((copy & 1) && ipx != 0) || ((copy & 2) && ipy != 0)) continue;
+            const long long w = v + ((copy & 1) ? NX : 0) + ((copy & 2) ? (long long)NY * XP : 0);
+            if (in2) cmap2[w] = 1;
+            if (mark) atomicMax(&cmap1[w], c);
+            if (ipx != 0 && ipy != 0) break;
           }
         }
-        // carry the stride into the next rows
-        while (m > zmax) { m -= nzr; l++; }
+        ix += sx; iy += sy; iz += sz;
+        if (ix >= bx) { ix -= bx; iy++; }
+        if (iy >= by) { iy -= by; iz++; }
       }
     }
+    const int cn = c + step;
+    if (cn < n) { p = ld_pos(t, pb, cn); s = t.state[cn]; r = t.radius[cn]; }
   }
   for (int o = 32; o > 0; o >>= 1) ztop = max(ztop, __shfl_down(ztop, o, 64));
   if ((threadIdx.x & 63) == 0 && ztop > __hip_atomic_load(&st->stamp_z, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
     atomicMax(&st->stamp_z, ztop);
-}
-
-// periodic planes x = NX and y = NY for l < NZ (:156-166)
-__global__ void __launch_bounds__(256) k_map_halo(const Tis* __restrict__ T) {
-  const Tis& t = T[blockIdx.y];
-  const int NX = t.NX, NY = t.NY;
-  const int per_l = (NX + 1) + (NY + 1);
-  const long long tot = (long long)per_l * min(t.st->stamp_z + 1, t.NZ);
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot; i += (long long)gridDim.x * blockDim.x) {
-    const int l = (int)(i / per_l), r = (int)(i % per_l);
-    long long dst, src;
-    if (r <= NX) {   // y = NY row
-      const int j = r;
-      dst = gidx(t, j, NY, l);
-      src = gidx(t, j == NX ? 0 : j, 0, l);
-    } else {         // x = NX column
-      const int k = r - (NX + 1);
-      dst = gidx(t, NX, k, l);
-      src = gidx(t, 0, k == NY ? 0 : k, l);
-    }
-    t.cmap1[dst] = t.cmap1[src];
-    t.cmap2[dst] = t.cmap2[src];
-  }
 }
 
 // ---- ext_stim B: calc_ext_stim (ext_stim.cpp:18-69) ------------------------
@@ -1133,8 +1138,7 @@ void launch_ca_swap(hipStream_t s, const Tis* dT, const int* tlist, int ntis, in
   EPI_LAUNCH(K_CA_SWAP, k_ca_swap, dim3((unsigned)g, ntis), dim3(256), 0, s, dT, tlist);
 }
 
-void launch_maps(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, long long max_gsize, int max_halo,
-                 const Tuning& tu) {
+void launch_maps(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, long long max_gsize, const Tuning& tu) {
   const long long q = (max_gsize / 4 + 255) / 256;
   dim3 gg((unsigned)(q < 1 ? 1 : q < 65535 ? q : 65535), ntis);
   EPI_LAUNCH(K_MAP_CLEAR, k_map_clear, gg, dim3(256), 0, s, dT);
@@ -1144,7 +1148,6 @@ void launch_maps(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, long
     EPI_LAUNCH(K_MAP_STAMP, k_map_stamp<4>, dim3((4 * max_n + 127) / 128, ntis), dim3(128), 0, s, dT, pb);
   else
     EPI_LAUNCH(K_MAP_STAMP, k_map_stamp<1>, dim3((max_n + 127) / 128, ntis), dim3(128), 0, s, dT, pb);
-  EPI_LAUNCH(K_MAP_HALO, k_map_halo, dim3((max_halo + 255) / 256, ntis), dim3(256), 0, s, dT);
 }
 
 namespace {

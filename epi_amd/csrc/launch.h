@@ -11,7 +11,7 @@ struct Status;
 enum KernelId {
   K_FORCES, K_FORCES_LONG, K_RENEW_FLAGS, K_RENEW_SCAN, K_RENEW_APPLY, K_REMOVE, K_PAIR_DISPERSE,
   K_INIT_SC, K_PERIODIC_FIX, K_BUCKET_INSERT, K_BUCKET_SORT, K_SWEEP,
-  K_FINISH, K_SNAPSHOT, K_ZZ_SET, K_ZZMAX, K_MAP_CLEAR, K_MAP_STAMP, K_MAP_HALO,
+  K_FINISH, K_SNAPSHOT, K_ZZ_SET, K_ZZMAX, K_MAP_CLEAR, K_MAP_STAMP,
   K_EXT_STIM, K_CA_BEGIN, K_CA_VOX, K_CA_CELLS, K_ATP, K_CA_END, K_SW_RESET,
   K_RD_SNAPSHOT, K_RD_RESTORE, K_RD_PUT_GJ, K_RD_STATE, K_RD_SEED, K_RD_STEP,
   K_RD_GJ0, K_RD_OWN, K_MECH_STATE, K_MECH_SEED, K_MECH_BWD_BEGIN, K_MECH_BWD_PAIRS, K_MECH_BWD_MEMB,
@@ -35,7 +35,7 @@ struct Tuning {
   int ca_fuse = 1;            // Ca solves: ATP of a sub-step and cells of the next in one launch
                               // (0 never, 1 always, 2 for solves of at most 131072 cells)
   int ca_group_small = 8;     // k_ca_cells lanes per cell in the solves that ca_fuse 2 fuses
-  int map_lanes = 1;          // k_map_stamp: lanes per cell (1, 4 or 16; a box slice split between them)
+  int map_lanes = 16;         // k_map_stamp: lanes per cell (1, 4 or 16, along x of the stamp box)
   int step_graph = 0;         // epi_step: 1 replays the renewal and build from a captured graph
 };
 
@@ -94,7 +94,7 @@ constexpr long long out_record_bytes(long long m) { return OUT_HDR + m * (8 * OU
 // buffer pb, Ca2+ from cp, lists from cb
 void launch_out_pack(hipStream_t s, const Tis* dT, int tissue, int pb, int cp, int cb, int n, long long m, char* out);
 void launch_zz_set(hipStream_t s, const Tis* dT, int ntis, double v);
-void launch_maps(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, long long max_gsize, int max_halo,
+void launch_maps(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, long long max_gsize,
                  const Tuning& tu);
 // the B stencil over a work list of (tissue, tile) built on the device from
 // zzmax (d_wl: 2 ntis + 1 ints); tiles_est sizes the grid (any value covers

@@ -170,6 +170,20 @@ __device__ __forceinline__ long long gidx(const Tis& t, int j, int k, int l) {
   return (long long)l * t.PL + (long long)k * t.XP + j;
 }
 
+// empties the voxel maps' planes 0..stamp_z, four voxels per thread, by block
+// b of nb blocks (a plane holds PL = XP (NY + 1) voxels with XP a multiple of
+// 16, and the maps start 256-byte aligned)
+__device__ __forceinline__ void map_clear(const Tis& t, int b, int nb) {
+  const int planes = min(t.st->stamp_z, t.NZ) + 1;
+  const long long g4 = (long long)planes * t.PL / 4;
+  int4* __restrict__ m1 = reinterpret_cast<int4*>(t.cmap1);
+  unsigned* __restrict__ m2 = reinterpret_cast<unsigned*>(t.cmap2);
+  for (long long q = (long long)b * blockDim.x + threadIdx.x; q < g4; q += (long long)nb * blockDim.x) {
+    m1[q] = make_int4(-1, -1, -1, -1);
+    m2[q] = 0u;
+  }
+}
+
 __device__ __forceinline__ bool is_afm(uint8_t s) { return s == ALIVE || s == FIX || s == MUSUME; }
 
 }  // namespace epi

@@ -390,11 +390,6 @@ int max_memb(const epi_ctx* c) {
   for (auto& h : c->th) m = std::max(m, h.nmemb);
   return m;
 }
-int max_nb(const epi_ctx* c) {
-  int m = 1;
-  for (auto& h : c->th) m = std::max(m, h.nbuckets);
-  return m;
-}
 long long max_gsize(const epi_ctx* c) {
   long long m = 1;
   for (auto& h : c->th) m = std::max(m, h.gsize);
@@ -1069,7 +1064,7 @@ int epi_pos_copy(epi_ctx* c) {
 int epi_cell_state_renew(epi_ctx* c) {
   if (!c) return EPI_ERR_INVALID;
   if (c->pos_pending) return fail(c, EPI_ERR_INVALID, "pos_copy must follow cell_interaction");
-  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, max_n(c));
+  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, max_n(c), 0);
   HIPCHK(c, hipGetLastError());
   for (auto& v : c->dev_ts) v++;   // k_remove advances each tissue's timestep
   return EPI_OK;
@@ -1085,7 +1080,7 @@ int epi_cell_pos_periodic_fix(epi_ctx* c) {
 int epi_connect_cell(epi_ctx* c) {
   if (!c) return EPI_ERR_INVALID;
   const int nb = 1 - c->cb;
-  launch_connect(c->stream, c->d_tis, c->T, c->pb, nb, max_n(c), max_nb(c), 0, c->tu.sweep_wave);
+  launch_connect(c->stream, c->d_tis, c->T, c->pb, nb, max_n(c), c->tu.sweep_wave);
   c->len_known = false;
   HIPCHK(c, hipGetLastError());
   c->cb = nb;
@@ -1109,7 +1104,8 @@ int epi_calc_zzmax(epi_ctx* c, double* zzmax) {
 
 int epi_setup_map_lat(epi_ctx* c) {
   if (!c) return EPI_ERR_INVALID;
-  launch_maps(c->stream, c->d_tis, c->T, c->pb, max_n(c), max_gsize(c), c->tu);
+  launch_map_clear(c->stream, c->d_tis, c->T, max_gsize(c));
+  launch_map_stamp(c->stream, c->d_tis, c->T, c->pb, max_n(c), c->tu);
   HIPCHK(c, hipGetLastError());
   return EPI_OK;
 }
@@ -1216,10 +1212,11 @@ int epi_ca_substep(epi_ctx* c, int32_t iz_bound) {
 }
 
 // cell_state_renew (proc.cpp:153), the bucket insertion with the periodic
-// fix and the rest of connect_cell (:154), and, on the side stream forked
-// after the insertion, calc_zzmax, setup_map_lat and calc_ext_stim
-// (:155-157), which read only the fixed positions, states and radii (and the
-// B field) that the rest of the build leaves alone.  The build, the longer
+// fix, calc_zzmax (:155) and the emptying of the voxel maps, the rest of
+// connect_cell (:154), and, on the side stream forked after the insertion,
+// setup_map_lat's stamping and calc_ext_stim (:156-157), which read only the
+// fixed positions, states and radii (and the B field) that the rest of the
+// build leaves alone.  The build, the longer
 // chain, is issued first.
 // With join false the main stream does not wait for the side stream's maps
 // and B sweep: epi_step joins it after issuing the next step's forces, which
@@ -1227,8 +1224,8 @@ int epi_ca_substep(epi_ctx* c, int32_t iz_bound) {
 hipError_t issue_build(epi_ctx* c, int mn, int nb, int izb, bool join = true) {
   hipError_t e = hipSuccess;
   auto chk = [&](hipError_t r) { if (e == hipSuccess) e = r; };
-  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, mn);
-  launch_connect_insert(c->stream, c->d_tis, c->T, c->pb, mn, 1);
+  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, mn, 1);
+  launch_connect_insert(c->stream, c->d_tis, c->T, c->pb, mn, map_clear_blocks(max_gsize(c)));
   // the side stream forks after the insertion (SIDE_FORK 0: the maps run
   // beside the sweep) or after the whole build (1: the sweep runs alone and
   // the maps beside the next forces)
@@ -1236,8 +1233,7 @@ hipError_t issue_build(epi_ctx* c, int mn, int nb, int izb, bool join = true) {
   launch_connect_rest(c->stream, c->d_tis, c->T, c->pb, nb, mn, c->tu.sweep_wave, c->h_st);
   if (c->tu.side_fork) chk(hipEventRecord(c->ev_fork, c->stream));
   chk(hipStreamWaitEvent(c->side_stream, c->ev_fork, 0));
-  launch_zzmax(c->side_stream, c->d_tis, c->T, c->pb, mn);
-  launch_maps(c->side_stream, c->d_tis, c->T, c->pb, mn, max_gsize(c), c->tu);
+  launch_map_stamp(c->side_stream, c->d_tis, c->T, c->pb, mn, c->tu);
   launch_ext_stim(c->side_stream, c->d_tis, c->T, c->bp, b_tiles_est(c), c->d_wl, c->tu);
   chk(hipEventRecord(c->ev_join, c->side_stream));
   if (join) chk(hipStreamWaitEvent(c->stream, c->ev_join, 0));
@@ -1321,8 +1317,7 @@ int epi_step(epi_ctx* c, int64_t nsteps, epi_driver* drv) {
       // the read-back follows this step's main chain only: the maps and the
       // B sweep (side stream) run on beside the next forces, which read
       // neither, and what the main stream issues after those forces (the
-      // next renewal, a solve) waits for them.  Their zzmax reaches the host
-      // with a later read-back; a solve reads it again first.
+      // next renewal, a solve) waits for them.
       RCHK(sync_status_begin(c));
       forces_pb = c->pb;
       forces_cap = launch_forces_rows(c->stream, c->d_tis, c->T, c->pb, c->cb, cap_n, known_len);
@@ -1372,9 +1367,6 @@ int epi_step(epi_ctx* c, int64_t nsteps, epi_driver* drv) {
     }
     nca = (int)ca_list.size();
     if (nca) {
-      // the solve's work lists need this step's zzmax, which an early
-      // read-back may have missed
-      if (forces_issued) RCHK(sync_status(c));
       if (nsc) HIPCHK(c, hipStreamSynchronize(c->stream));
       for (int i = 0; i < nca; i++) c->h_tlist[i] = ca_list[i];
       HIPCHK(c, hipMemcpyAsync(c->d_tlist, c->h_tlist, sizeof(int) * nca, hipMemcpyHostToDevice, c->stream));

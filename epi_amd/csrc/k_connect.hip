@@ -21,15 +21,40 @@
 
 namespace epi {
 
+// calc_zzmax (proc.cpp:34-43): z values that matter are positive, where the
+// IEEE bit order is the numeric order
+__device__ __forceinline__ bool counts_zzmax(uint8_t s) { return s == DEAD || s == ALIVE || s == MUSUME || s == FIX; }
+// a lane's maximum into the tissue's, which was cleared before this launch
+// and only grows during it
+__device__ __forceinline__ void zzmax_add(Status* st, double m) {
+  for (int o = 32; o > 0; o >>= 1) {
+    const double v = __shfl_down(m, o, 64);
+    if (m < v) m = v;
+  }
+  const unsigned long long mb = (unsigned long long)__double_as_longlong(m);
+  if ((threadIdx.x & 63) == 0 && m > 0 &&
+      mb > __hip_atomic_load(&st->zzmax_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(&st->zzmax_bits, mb);
+}
+
 // grid_init (:38-62); with fix != 0 it first applies cell_pos_periodic_fix
-// (cellmanager.cpp:395-414) to the cell, which touches only that cell
-__global__ void __launch_bounds__(256) k_bucket_insert(const Tis* __restrict__ T, int pb, int fix) {
-  const Tis& t = T[blockIdx.y];
+// (cellmanager.cpp:395-414) to the cell, which touches only that cell.
+// In a step (STEP) the launch carries two more pieces of work that need only
+// what it reads or nothing, and that would otherwise be three launches on the
+// side stream before the stamping (zz_set, zzmax, clear: 12 us of a step of
+// 420 cells with their gaps): calc_zzmax over the same cells (the maximum was
+// cleared by k_remove), and, in the blocks from cell_blocks on, the emptying of
+// the voxel maps, which nothing reads between the last step's B sweep or solve
+// and this step's stamping.
+__device__ __forceinline__ void insert_cells(const Tis& t, int pb, int fix, bool step, int nblocks) {
   Status* st = t.st;
-  const int n = st->n;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
+  const int n = st->n, start = t.nmemb + t.nder;
+  double zmax = 0;
+  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += nblocks * blockDim.x) {
     double x = t.pos[pb][0][c], y = t.pos[pb][1][c];
     const double z = t.pos[pb][2][c];
+    const double r = t.radius[c];
+    if (step && c >= start && zmax < z && counts_zzmax(t.state[c])) zmax = z;
     if (fix) {
       if (x > t.LX) { x = x - t.LX; t.pos[pb][0][c] = x; }
       else if (x < 0) { x = x + t.LX; t.pos[pb][0][c] = x; }
@@ -39,7 +64,7 @@ __global__ void __launch_bounds__(256) k_bucket_insert(const Tis* __restrict__ T
     const long aix = (long)((0.5 * t.LX - p_diff_x(t, 0.5 * t.LX, x)) / AREA_GRID);
     const long aiy = (long)((0.5 * t.LY - p_diff_y(t, 0.5 * t.LY, y)) / AREA_GRID);
     const long aiz = (long)((min0(z)) / AREA_GRID);
-    t.pk[c] = make_double4(x, y, z, t.radius[c]);
+    t.pk[c] = make_double4(x, y, z, r);
     t.bcnt[c] = 0;
     t.nlo[c] = 0;
     t.bslot[c] = -1;
@@ -56,6 +81,14 @@ __global__ void __launch_bounds__(256) k_bucket_insert(const Tis* __restrict__ T
     t.bucket_cells[(size_t)b * bucket_stride(t.bcap) + slot] = c;
     t.bslot[c] = slot;
   }
+  if (step) zzmax_add(st, zmax);
+}
+
+template <bool STEP>
+__global__ void __launch_bounds__(256) k_bucket_insert(const Tis* __restrict__ T, int pb, int fix, int cell_blocks) {
+  const Tis& t = T[blockIdx.y];
+  if (STEP && (int)blockIdx.x >= cell_blocks) map_clear(t, blockIdx.x - cell_blocks, gridDim.x - cell_blocks);
+  else insert_cells(t, pb, fix, STEP, cell_blocks);
 }
 
 // each bucket in ascending cell index: every cell counts the cells of its
@@ -441,34 +474,24 @@ __global__ void __launch_bounds__(256) k_snapshot(const Tis* __restrict__ T, int
   }
 }
 
-// calc_zzmax (proc.cpp:34-43): z values that matter are positive, where the
-// IEEE bit order is the numeric order
+// calc_zzmax by itself (a step's rides with the bucket insertion)
 __global__ void __launch_bounds__(256) k_zzmax(const Tis* __restrict__ T, int pb) {
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;
   const int n = st->n;
   double m = 0;
   for (int c = t.nmemb + t.nder + blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
-    const uint8_t s = t.state[c];
-    if (s == DEAD || s == ALIVE || s == MUSUME || s == FIX) {
+    if (counts_zzmax(t.state[c])) {
       const double z = t.pos[pb][2][c];
       if (m < z) m = z;
     }
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    const double v = __shfl_down(m, o, 64);
-    if (m < v) m = v;
-  }
-  // the value was cleared by k_zz_set and only grows during this launch
-  const unsigned long long mb = (unsigned long long)__double_as_longlong(m);
-  if ((threadIdx.x & 63) == 0 && m > 0 &&
-      mb > __hip_atomic_load(&st->zzmax_bits, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-    atomicMax(&st->zzmax_bits, mb);
+  zzmax_add(st, m);
 }
 
-__global__ void k_zz_set(const Tis* __restrict__ T, int use_value, double v) {
+__global__ void k_zz_set(const Tis* __restrict__ T) {
   const Tis& t = T[blockIdx.x];
-  if (threadIdx.x == 0) t.st->zzmax_bits = use_value ? (unsigned long long)__double_as_longlong(v) : 0ull;
+  if (threadIdx.x == 0) t.st->zzmax_bits = 0ull;
 }
 
 // CellManager::output's per-cell record (cellmanager.cpp:451-538) packed for
@@ -512,9 +535,14 @@ void launch_out_pack(hipStream_t s, const Tis* dT, int tissue, int pb, int cp, i
   EPI_LAUNCH(K_OUT_PACK, k_out_pack, dim3(g), dim3(256), 0, s, dT, tissue, pb, cp, cb, n, m, out);
 }
 
-void launch_connect_insert(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, int fix) {
-  dim3 gc((max_n + 255) / 256, ntis);
-  EPI_LAUNCH(K_BUCKET_INSERT, k_bucket_insert, gc, dim3(256), 0, s, dT, pb, fix);
+void launch_connect_insert(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, unsigned clear_blocks) {
+  const unsigned gc = (max_n + 255) / 256;
+  if (clear_blocks) {
+    EPI_LAUNCH(K_BUCKET_INSERT, k_bucket_insert<true>, dim3(gc + clear_blocks, ntis), dim3(256), 0, s, dT, pb, 1,
+               (int)gc);
+  } else {
+    EPI_LAUNCH(K_BUCKET_INSERT, k_bucket_insert<false>, dim3(gc, ntis), dim3(256), 0, s, dT, pb, 0, (int)gc);
+  }
 }
 
 void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave,
@@ -531,21 +559,15 @@ void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb,
   EPI_LAUNCH(K_SNAPSHOT, k_snapshot, gc, dim3(256), 0, s, dT, pb, h_status);
 }
 
-void launch_connect(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int max_buckets, int fix,
-                    int sweep_wave) {
-  (void)max_buckets;
-  launch_connect_insert(s, dT, ntis, pb, max_n, fix);
+void launch_connect(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave) {
+  launch_connect_insert(s, dT, ntis, pb, max_n, 0);
   launch_connect_rest(s, dT, ntis, pb, nb, max_n, sweep_wave, nullptr);
 }
 
 void launch_zzmax(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n) {
-  EPI_LAUNCH(K_ZZ_SET, k_zz_set, dim3(ntis), dim3(64), 0, s, dT, 0, 0.0);
+  EPI_LAUNCH(K_ZZ_SET, k_zz_set, dim3(ntis), dim3(64), 0, s, dT);
   dim3 gc((max_n + 255) / 256, ntis);
   EPI_LAUNCH(K_ZZMAX, k_zzmax, gc, dim3(256), 0, s, dT, pb);
-}
-
-void launch_zz_set(hipStream_t s, const Tis* dT, int ntis, double v) {
-  EPI_LAUNCH(K_ZZ_SET, k_zz_set, dim3(ntis), dim3(64), 0, s, dT, 1, v);
 }
 
 }  // namespace epi

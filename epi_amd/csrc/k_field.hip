@@ -22,20 +22,9 @@ namespace epi {
 // ---- voxel maps ---------------------------------------------------------
 // Only planes 0..stamp_z can hold stamps (stamp_z never decreases), so only
 // they are cleared; the rest of the maps stays empty from the first build.
-// Four voxels per thread: a plane holds PL = XP (NY + 1) voxels with XP a
-// multiple of 16, and the maps start 256-byte aligned, so every quad is one
-// 16-byte and one 4-byte store.
+// In a step the bucket insertion's spare blocks do it (map_clear, epi_dev.h).
 __global__ void __launch_bounds__(256) k_map_clear(const Tis* __restrict__ T) {
-  const Tis& t = T[blockIdx.y];
-  const int planes = min(t.st->stamp_z, t.NZ) + 1;
-  const long long g4 = (long long)planes * t.PL / 4;
-  int4* __restrict__ m1 = reinterpret_cast<int4*>(t.cmap1);
-  unsigned* __restrict__ m2 = reinterpret_cast<unsigned*>(t.cmap2);
-  for (long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x; q < g4;
-       q += (long long)gridDim.x * blockDim.x) {
-    m1[q] = make_int4(-1, -1, -1, -1);
-    m2[q] = 0u;
-  }
+  map_clear(T[blockIdx.y], blockIdx.x, gridDim.x);
 }
 
 __device__ __forceinline__ int lat_wrap(long v, int N, Status* st) {
@@ -190,11 +179,23 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* total) {
   return before + x - v;
 }
 
-// The B stencil's list, once zzmax is on the device: per tissue
-// iz_bound = (int)((zzmax + FAC_MAP * R_max) * inv_dz) (ext_stim.cpp:22) into
-// izb[i], and ceil(NX NY / bs) ceil(iz_bound / zb) tiles.  A tissue whose
-// iz_bound lies outside [0, NZ] gets none and reports ERR_OUT_OF_GRID.  The
-// sweep's NX NY iz_bound points are added to the tissue's count.  One block.
+// The B stencil's iz_bound = (int)((zzmax + FAC_MAP * R_max) * inv_dz)
+// (ext_stim.cpp:22) from the device's zzmax.  One outside [0, NZ] sweeps
+// nothing and is reported as ERR_OUT_OF_GRID; the sweep's NX NY iz_bound
+// points are added to the tissue's count (both by the thread that counts).
+__device__ __forceinline__ int b_iz_bound(const Tis& t, bool counts) {
+  const double zzmax = __longlong_as_double((long long)t.st->zzmax_bits);
+  int izb = (int)((zzmax + t.prm.iz_margin) * t.inv_dz);
+  if (izb > t.NZ || izb < 0) {
+    if (counts) set_err(t.st, ERR_OUT_OF_GRID);
+    izb = 0;
+  }
+  if (counts) t.st->grid_b += (long long)t.NX * t.NY * izb;
+  return izb;
+}
+
+// The B stencil's list, once zzmax is on the device: per tissue iz_bound into
+// izb[i], and ceil(NX NY / bs) ceil(iz_bound / zb) tiles.  One block.
 __global__ void __launch_bounds__(256) k_wl_b(const Tis* __restrict__ T, int ntis, int bs, int zb,
                                               int* __restrict__ off, int* __restrict__ izb_out) {
   int carry = 0;
@@ -203,14 +204,8 @@ __global__ void __launch_bounds__(256) k_wl_b(const Tis* __restrict__ T, int nti
     int cnt = 0;
     if (i < ntis) {
       const Tis& t = T[i];
-      const double zzmax = __longlong_as_double((long long)t.st->zzmax_bits);
-      int izb = (int)((zzmax + t.prm.iz_margin) * t.inv_dz);
-      if (izb > t.NZ || izb < 0) {
-        set_err(t.st, ERR_OUT_OF_GRID);
-        izb = 0;
-      }
+      const int izb = b_iz_bound(t, true);
       izb_out[i] = izb;
-      t.st->grid_b += (long long)t.NX * t.NY * izb;
       cnt = ((t.NX * t.NY + bs - 1) / bs) * ((izb + zb - 1) / zb);
     }
     int tot;
@@ -408,9 +403,23 @@ __device__ __forceinline__ void b_column_roll(const Tis& t, int j, int k, int l0
   }
 }
 
+// One tile of the B stencil: one thread per (x, y) point; tiles of up to 2
+// planes load the column first (b_column), taller ones roll it
+// (b_column_roll).
+template <int ZB>
+__device__ __forceinline__ void b_tile(const Tis& t, int local, int iz_bound, int bp) {
+  const int bs = blockDim.x;
+  const int NX = t.NX, plane = NX * t.NY;
+  const int npt = (plane + bs - 1) / bs;
+  const int p = (local % npt) * bs + (int)threadIdx.x;
+  if (p >= plane) return;
+  const int l0 = (local / npt) * ZB;
+  const int l1 = min(l0 + ZB, iz_bound);
+  if (ZB >= 4) b_column_roll(t, p % NX, p / NX, l0, l1, bp);
+  else b_column<ZB>(t, p % NX, p / NX, l0, l1, bp);
+}
+
 // The B stencil over its tile list.
-// One thread per (x, y) point of a tile: tiles of up to 2 planes load the
-// column first (b_column), taller ones roll it (b_column_roll).
 template <int ZB>
 __global__ void __launch_bounds__(256) k_ext_stim(const Tis* __restrict__ T, const int* __restrict__ woff,
                                                   const int* __restrict__ wizb, int ntis, int bp, int xcd) {
@@ -425,26 +434,25 @@ __global__ void __launch_bounds__(256) k_ext_stim(const Tis* __restrict__ T, con
     __syncthreads();
   }
   auto off = [&](int i) { return lds ? s_off[i] : woff[i]; };
-  const int bs = blockDim.x;
   int ti = 0;
   for (TileWalk tw(off(ntis), xcd, blockIdx.x, gridDim.x); tw.w < tw.end; tw.w += tw.stride) {
     // the tile, hence its tissue, is the block's: held in scalar registers,
     // so the tissue's record is read with scalar loads
     ti = __builtin_amdgcn_readfirstlane(wl_find(off, ti, ntis, tw.w));
-    const Tis& t = T[ti];
-    const int iz_bound = __builtin_amdgcn_readfirstlane(lds ? s_izb[ti] : wizb[ti]);
-    const int NX = t.NX, NY = t.NY, NZ = t.NZ;
-    const int plane = NX * NY;
-    const int npt = (plane + bs - 1) / bs;
-    const int local = tw.w - __builtin_amdgcn_readfirstlane(off(ti));
-    const int p = (local % npt) * bs + (int)threadIdx.x;
-    if (p >= plane) continue;
-    const int j = p % NX, k = p / NX;
-    const int l0 = (local / npt) * ZB;
-    const int l1 = min(l0 + ZB, iz_bound);
-    if (ZB >= 4) b_column_roll(t, j, k, l0, l1, bp);
-    else b_column<ZB>(t, j, k, l0, l1, bp);
+    b_tile<ZB>(T[ti], tw.w - __builtin_amdgcn_readfirstlane(off(ti)),
+               __builtin_amdgcn_readfirstlane(lds ? s_izb[ti] : wizb[ti]), bp);
   }
+}
+
+// The B stencil of one tissue: its tiles follow from its iz_bound, which
+// every block takes from zzmax itself, so no list is built (k_wl_b, a launch
+// of one block, 4 to 5 us) nor read.  The first thread does k_wl_b's share.
+template <int ZB>
+__global__ void __launch_bounds__(256) k_ext_stim_one(const Tis* __restrict__ T, int bp, int xcd) {
+  const Tis& t = T[0];
+  const int iz_bound = __builtin_amdgcn_readfirstlane(b_iz_bound(t, blockIdx.x == 0 && threadIdx.x == 0));
+  const int total = ((t.NX * t.NY + (int)blockDim.x - 1) / (int)blockDim.x) * ((iz_bound + ZB - 1) / ZB);
+  for (TileWalk tw(total, xcd, blockIdx.x, gridDim.x); tw.w < tw.end; tw.w += tw.stride) b_tile<ZB>(t, tw.w, iz_bound, bp);
 }
 
 // ---- calc_ca2p ------------------------------------------------------------
@@ -1138,10 +1146,18 @@ void launch_ca_swap(hipStream_t s, const Tis* dT, const int* tlist, int ntis, in
   EPI_LAUNCH(K_CA_SWAP, k_ca_swap, dim3((unsigned)g, ntis), dim3(256), 0, s, dT, tlist);
 }
 
-void launch_maps(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, long long max_gsize, const Tuning& tu) {
-  const long long q = (max_gsize / 4 + 255) / 256;
-  dim3 gg((unsigned)(q < 1 ? 1 : q < 65535 ? q : 65535), ntis);
-  EPI_LAUNCH(K_MAP_CLEAR, k_map_clear, gg, dim3(256), 0, s, dT);
+unsigned map_clear_blocks(long long max_gsize) {
+  // four quads a thread, if every plane had been stamped: the stores of 32
+  // uneven tissues (72 MB of maps) took 57 us with one quad a thread
+  const long long q = (max_gsize / 16 + 255) / 256;
+  return (unsigned)(q < 1 ? 1 : q < 65535 ? q : 65535);
+}
+
+void launch_map_clear(hipStream_t s, const Tis* dT, int ntis, long long max_gsize) {
+  EPI_LAUNCH(K_MAP_CLEAR, k_map_clear, dim3(map_clear_blocks(max_gsize), ntis), dim3(256), 0, s, dT);
+}
+
+void launch_map_stamp(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, const Tuning& tu) {
   if (tu.map_lanes == 16)
     EPI_LAUNCH(K_MAP_STAMP, k_map_stamp<16>, dim3((16 * max_n + 127) / 128, ntis), dim3(128), 0, s, dT, pb);
   else if (tu.map_lanes == 4)
@@ -1176,6 +1192,10 @@ void launch_ext_stim(hipStream_t s, const Tis* dT, int ntis, int bp, long long t
   g = (g + 7) / 8 * 8;
   by_zb(tu.b_zb, [&](auto zbc) {
     constexpr int zb = decltype(zbc)::value;
+    if (ntis == 1) {
+      EPI_LAUNCH(K_EXT_STIM, k_ext_stim_one<zb>, dim3((unsigned)g), dim3(bs), 0, s, dT, bp, tu.b_xcd);
+      return;
+    }
     EPI_LAUNCH(K_WL, k_wl_b, dim3(1), dim3(256), 0, s, dT, ntis, bs, zb, d_wl, d_wl + ntis + 1);
     EPI_LAUNCH(K_EXT_STIM, k_ext_stim<zb>, dim3((unsigned)g), dim3(bs), 0, s, dT, d_wl, d_wl + ntis + 1, ntis, bp,
                tu.b_xcd);

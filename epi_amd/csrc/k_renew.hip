@@ -336,7 +336,7 @@ __global__ void __launch_bounds__(256) k_renew_apply(const Tis* __restrict__ T, 
 // live cell there): ERR_REMOVE_ALIAS.  A removed DEAD cell's cell_stat goes
 // to cst_store with k_disap = the current timestep (:343-346), in queue
 // order; the timestep then advances (one renewal per step).
-__global__ void __launch_bounds__(256) k_remove(const Tis* __restrict__ T, int pb) {
+__global__ void __launch_bounds__(256) k_remove(const Tis* __restrict__ T, int pb, int zero_zz) {
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;
   const int ndiv = st->ndiv, nrm = st->nrm;
@@ -398,6 +398,7 @@ __global__ void __launch_bounds__(256) k_remove(const Tis* __restrict__ T, int p
   if (threadIdx.x == 0) {
     st->n = N - nrm;
     st->next_uid += ndiv;
+    if (zero_zz) st->zzmax_bits = 0ull;
   }
 }
 
@@ -452,12 +453,12 @@ __global__ void __launch_bounds__(256) k_periodic_fix(const Tis* __restrict__ T,
   }
 }
 
-void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_n) {
+void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_n, int zero_zz) {
   dim3 g((max_n + 255) / 256, ntis);
   EPI_LAUNCH(K_RENEW_FLAGS, k_renew_flags, g, dim3(256), 0, s, dT, cb);
   EPI_LAUNCH(K_RENEW_SCAN, k_renew_scan, dim3(1, ntis), dim3(1024), 0, s, dT, pb, cb);
   EPI_LAUNCH(K_RENEW_APPLY, k_renew_apply, g, dim3(256), 0, s, dT, pb, cb, cpar);
-  EPI_LAUNCH(K_REMOVE, k_remove, dim3(1, ntis), dim3(256), 0, s, dT, pb);
+  EPI_LAUNCH(K_REMOVE, k_remove, dim3(1, ntis), dim3(256), 0, s, dT, pb, zero_zz);
   EPI_LAUNCH(K_PAIR_DISPERSE, k_pair_disperse, g, dim3(256), 0, s, dT, pb);
 }
 

@@ -69,17 +69,19 @@ void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int m
 // the returned number of slots (chosen from max_len), and the long rows
 int launch_forces_rows(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len);
 void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int cap);
-void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_n);
+// zero_zz: also clear zzmax, for a build whose insertion takes it
+void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_n, int zero_zz);
 void launch_initialize_sc(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int pb, int max_n);
 void launch_periodic_fix(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n);
-// the bucket insertion (with the periodic fix) and the rest of the build,
-// for callers that run the voxel maps beside the rest
-void launch_connect_insert(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, int fix);
+// the bucket insertion and the rest of the build, for callers that run the
+// voxel maps beside the rest.  With clear_blocks (a step), the insertion also
+// applies the periodic fix, takes zzmax (cleared by launch_renew) and empties
+// the voxel maps with that many more blocks
+void launch_connect_insert(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, unsigned clear_blocks);
 // with h_status, k_snapshot also copies every tissue's status there
 void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave,
                          Status* h_status);
-void launch_connect(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int max_buckets, int fix,
-                    int sweep_wave);
+void launch_connect(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave);
 void launch_zzmax(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n);
 // A snapshot's output record (CellManager::output's fields): a header of
 // OUT_HDR bytes whose first int is the device's cell count, then m >= n
@@ -93,9 +95,10 @@ constexpr long long out_record_bytes(long long m) { return OUT_HDR + m * (8 * OU
 // the output record of one tissue's first n cells into out, positions from
 // buffer pb, Ca2+ from cp, lists from cb
 void launch_out_pack(hipStream_t s, const Tis* dT, int tissue, int pb, int cp, int cb, int n, long long m, char* out);
-void launch_zz_set(hipStream_t s, const Tis* dT, int ntis, double v);
-void launch_maps(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, long long max_gsize,
-                 const Tuning& tu);
+// setup_map_lat: the maps emptied (map_clear_blocks blocks a tissue), then stamped
+unsigned map_clear_blocks(long long max_gsize);
+void launch_map_clear(hipStream_t s, const Tis* dT, int ntis, long long max_gsize);
+void launch_map_stamp(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, const Tuning& tu);
 // the B stencil over a work list of (tissue, tile) built on the device from
 // zzmax (d_wl: 2 ntis + 1 ints); tiles_est sizes the grid (any value covers
 // the list: the blocks walk it grid-stride)

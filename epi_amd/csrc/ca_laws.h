@@ -17,31 +17,28 @@ struct CaK {   // the per-cell update of a sub-step (ca2p.cpp:36-144, 156-222)
   double DT_Ca, Kpp, H0, para_k2, wd;
   double mu0, mu1, kmu, para_b, para_bb, para_k1, k_flux, gamma, kg, kbc, Cout, Hb, leak_from_storage;
 };
-__device__ __forceinline__ CaK ca_k(const Params& pm) {
+__host__ __device__ __forceinline__ CaK ca_k(const Params& pm) {
   return CaK{pm.DT_Ca, pm.Kpp, pm.H0, pm.para_k2, pm.wd, pm.mu0, pm.mu1, pm.kmu, pm.para_b, pm.para_bb, pm.para_k1,
              pm.k_flux, pm.gamma, pm.kg, pm.kbc, pm.Cout, pm.Hb, pm.leak_from_storage};
 }
 struct AtpK {   // ATP_refresh (ca2p.cpp:302-338)
   double DT_Ca, Da, STIM11, Kaa, AIR_STIM;
 };
-__device__ __forceinline__ AtpK atp_k(const Params& pm) {
+__host__ __device__ __forceinline__ AtpK atp_k(const Params& pm) {
   return AtpK{pm.DT_Ca, pm.Da, pm.STIM11, pm.Kaa, pm.AIR_STIM};
 }
 
+// ca2p_by_ext_stim (:59-63) of a cell's mean B
+__device__ __forceinline__ double ca2p_by_ext(const CaK& k, double B) {
+  return k.kbc * B * B * k.Cout / (k.Hb + B * B);
+}
 __device__ __forceinline__ double ca2p_reaction_factor(const CaK& k, double u, double ER3, double p,
-                                                       double B) {   // :36-87
+                                                       double by_ext) {   // :36-87
   const double er1 = (k.mu0 + k.mu1 * p / (p + k.kmu));
   const double er2 = (k.para_b + k.para_bb * u / (k.para_k1 + u));
   const double ca2p_from_storage = k.k_flux * er1 * er2 * ER3;
   const double into = k.gamma * u / (k.kg + u);
-  const double by_ext = k.kbc * B * B * k.Cout / (k.Hb + B * B);
   return ca2p_from_storage - into + k.leak_from_storage + by_ext;
-}
-
-__device__ __forceinline__ double grid_avg8(const Tis& t, const double* g, int ix, int iy, int iz) {   // utils.h:18-23
-  return 0.125 * (g[gidx(t, ix, iy, iz)] + g[gidx(t, ix + 1, iy, iz)] + g[gidx(t, ix, iy + 1, iz)]
-                  + g[gidx(t, ix, iy, iz + 1)] + g[gidx(t, ix + 1, iy + 1, iz)] + g[gidx(t, ix + 1, iy, iz + 1)]
-                  + g[gidx(t, ix, iy + 1, iz + 1)] + g[gidx(t, ix + 1, iy + 1, iz + 1)]);
 }
 
 __device__ __forceinline__ int ca_iz_bound(const Tis& t) {   // :386

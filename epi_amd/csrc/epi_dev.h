@@ -85,23 +85,26 @@ struct Tis {
   double* ca2p[2]; double* ip3[2];
   double *ca2p_avg, *ex_inert, *agek, *ageb, *ex_fat, *in_fat, *spr_nat_len, *diff_u;
   double *ca_th, *ca_kpa, *ca_iag;   // per-solve constants of the Ca step (agek and state are frozen)
-  // per list entry during a solve: neighbour << 2 | kind (0 skip, 1 coupled,
-  // 3 coupled ALIVE), one word for the index and the kind
-  int* ca_ent;
-  // the coupled entries alone (kind 1 or 3), in list order: (word, slot of
-  // the entry in the row, where its gj lives), and their number per cell
-  int2* ca_ce;
+  // The coupled list entries of the AFM and DEAD cells during a solve or
+  // window, packed to the front of a row of ns in list order: the word
+  // neighbour << 2 | kind (1 coupled, 3 coupled ALIVE), the entry's slot in the
+  // list row, and its gj, which lives here until k_ca_end puts it back; and
+  // their number per cell (0 for the other cells)
+  int* ca_w;
+  unsigned short* ca_sl;
+  double* ca_g;
   int* ca_cn;
-  // (ca2p, IP3) of buffer b beside the two arrays during a solve, so that a
-  // list entry reads its neighbour's pair with one 16-byte gather; every
-  // kernel that writes ca2p or IP3 inside a solve or window writes it too
+  // (ca2p, IP3) of buffer b during a solve or window, so that a list entry
+  // reads its neighbour's pair with one 16-byte gather; the arrays ca2p and
+  // ip3 follow at its end (k_ca_end)
   double2* ca_up[2];
   // diff_u of the Ca sub-steps at parity 1 (parity 0 writes diff_u itself)
   double* ca_dfu;
-  // per AFM cell and grid_avg8 ATP corner, during a solve: the corner's voxel
-  // word and the masks of its six stencil neighbours (bits 0-5; bit 31 set
-  // when a mask is not 0/1 and the corner reads the map instead)
-  uint2* ca_cq;
+  // per AFM cell and grid_avg8 corner (binary x, y, z), during a solve: the
+  // corner's point wrapped in x and y, its voxel word, the masks of its six
+  // stencil neighbours and the CQ_ flags, and the point as it lies
+  uint4* ca_cq;
+  double* ca_bx;   // ca2p_by_ext_stim per AFM cell (B does not change during a solve)
   long long* uid; long long* old_uid; int* src_row;
   // cell_stat (define.h:198-202): per cell k_aging_start, k_cornified,
   // k_disap (-1 = never set); cst_store (cellmanager.h:106): the records of
@@ -166,7 +169,8 @@ __device__ __forceinline__ double dist_sq(const Tis& t, P3 a, P3 b) {
 }
 
 // grid index of (x, y, z) lattice point in the device layout
-__device__ __forceinline__ long long gidx(const Tis& t, int j, int k, int l) {
+template <class G>   // a Tis, or what a launch carries of one (CaArg)
+__device__ __forceinline__ long long gidx(const G& t, int j, int k, int l) {
   return (long long)l * t.PL + (long long)k * t.XP + j;
 }
 

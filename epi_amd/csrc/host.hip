@@ -168,6 +168,7 @@ struct epi_ctx {
     unsigned long long used = 0;
   };
   std::vector<StepGraph> graphs;
+  long long tis_version = 0;   // counts changes of the descriptors (captured solves hold copies)
   unsigned long long graph_tick = 0;
   // frozen reaction-diffusion window (epi_rd_*)
   struct Rd {
@@ -281,12 +282,14 @@ void carve_tissue(Carver& cv, TH& h, Tis& t) {
   t.ca_th = cv.take<double>(cap);
   t.ca_kpa = cv.take<double>(cap);
   t.ca_iag = cv.take<double>(cap);
-  t.ca_ent = cv.take<int>(cap * ns);
-  t.ca_ce = cv.take<int2>(cap * ns);
+  t.ca_w = cv.take<int>(cap * ns);
+  t.ca_sl = cv.take<unsigned short>(cap * ns);
+  t.ca_g = cv.take<double>(cap * ns);
   t.ca_cn = cv.take<int>(cap);
   for (int b = 0; b < 2; b++) t.ca_up[b] = cv.take<double2>(cap);
   t.ca_dfu = cv.take<double>(cap);
-  t.ca_cq = cv.take<uint2>(cap * 8);
+  t.ca_cq = cv.take<uint4>(cap * 8);
+  t.ca_bx = cv.take<double>(cap);
   t.uid = cv.take<long long>(cap);
   t.old_uid = cv.take<long long>(cap);
   t.cst = cv.take<long long>(3 * cap);
@@ -535,7 +538,7 @@ int ca_list(epi_ctx* c, const int* ids, int ntis, int cg, int bs, int zb, CaList
     c->cal_key = key;
     c->cal = CaList{c->d_cal, c->d_cal + ntis + 1, c->d_cal + 2 * ntis + 1,
                     reinterpret_cast<const int4*>(c->d_cal + hdr), ntis, (int)ncb, (int)tiles, bs,
-                    ids ? ids[0] : 0, izb[0]};
+                    ids ? ids[0] : 0, izb[0], &c->tis[ids ? ids[0] : 0]};
   }
   *out = c->cal;
   return EPI_OK;
@@ -578,6 +581,30 @@ int graph_run(epi_ctx* c, const std::vector<long long>& key, F issue) {
   return EPI_OK;
 }
 
+// the launch shapes of a solve or window over tissues ids[0..ntis) (nullptr =
+// all), ca_fuse resolved to 0 or 1.  ca_fuse 2 fuses those of at most
+// FUSE_AUTO_CELLS cells (a gated solve of a few tissues is latency-bound,
+// where one launch per sub-step wins; a solve of a whole large batch is
+// throughput-bound, where two leaner ones do)
+Tuning ca_shapes(const epi_ctx* c, const int* ids, int ntis) {
+  constexpr long long FUSE_AUTO_CELLS = 131072;
+  long long cells = 0;
+  for (int i = 0; i < ntis; i++) cells += c->th[ids ? ids[i] : i].n_est;
+  Tuning tu = c->tu;
+  if (tu.ca_fuse == 2 && cells <= FUSE_AUTO_CELLS) {
+    // a small, latency-bound solve: fused, with its own lanes per cell
+    tu.ca_fuse = 1;
+    tu.ca_group = tu.ca_group_small;
+  } else {
+    tu.ca_fuse = tu.ca_fuse == 1;
+  }
+  // a fused launch's ATP tiles are one or two planes: taller ones roll their
+  // planes through one thread, which the cells beside them wait for (14.1
+  // against 10.1 us per sub-step of the large tissue)
+  if (tu.ca_fuse && tu.a_zb > 2) tu.a_zb = 1;
+  return tu;
+}
+
 // calc_ca2p (ca2p.cpp:380-402) for the tissues in tlist (nullptr = all)
 // (with d_tlist, c->h_tlist holds the same ntis ids), n_sub sub-steps.  The
 // list covers the solving tissues only: a gated solve of one small tissue in
@@ -593,27 +620,10 @@ int run_ca_n(epi_ctx* c, const int* d_tlist, int ntis, int n_sub) {
     mn = std::max(mn, h.n_est + 64);
     box = std::max(box, (long long)h.NX * h.NY * iz);
   }
-  // ca_fuse 2: fuse the solves of at most FUSE_AUTO_CELLS cells (a gated solve
-  // of a few tissues is latency-bound, where one launch per sub-step wins; a
-  // solve of a whole large batch is throughput-bound, where two leaner ones do)
-  constexpr long long FUSE_AUTO_CELLS = 131072;
-  long long cells = 0;
-  for (int i = 0; i < ntis; i++) cells += c->th[d_tlist ? c->h_tlist[i] : i].n_est;
-  Tuning tu = c->tu;
-  if (tu.ca_fuse == 2 && cells <= FUSE_AUTO_CELLS) {
-    // a small, latency-bound solve: fused, with its own lanes per cell, and
-    // one-plane ATP tiles (the planes per thread chosen for the batch-wide
-    // grid kernel roll 8 or 16 planes through one thread, which a
-    // latency-bound solve waits for)
-    tu.ca_fuse = 1;
-    tu.ca_group = tu.ca_group_small;
-    if (tu.a_zb > 2) tu.a_zb = 1;
-  } else {
-    tu.ca_fuse = tu.ca_fuse == 1;
-  }
+  const Tuning tu = ca_shapes(c, d_tlist ? c->h_tlist : nullptr, ntis);
   CaList cl;
-  RCHK(ca_list(c, d_tlist ? c->h_tlist : nullptr, ntis, tu.ca_group, ca_list_bs(tu, tu.ca_fuse && n_sub >= 2),
-               tu.a_zb, &cl));
+  RCHK(ca_list(c, d_tlist ? c->h_tlist : nullptr, ntis, ca_lanes(tu.ca_group),
+               ca_list_bs(tu, tu.ca_fuse && n_sub >= 2), tu.a_zb, &cl));
   constexpr unsigned long long seg = (1ull << K_CA_BEGIN) | (1ull << K_CA_VOX) | (1ull << K_CA_CORNERS) |
                                      (1ull << K_CA_CELLS) | (1ull << K_ATP) | (1ull << K_CA_FUSED) |
                                      (1ull << K_CA_END) | (1ull << K_SW_RESET);
@@ -623,22 +633,22 @@ int run_ca_n(epi_ctx* c, const int* d_tlist, int ntis, int n_sub) {
     int mcap = 1;
     for (int i = 0; i < ntis; i++) mcap = std::max(mcap, c->th[d_tlist ? c->h_tlist[i] : i].cap);
     const int mr = std::max(mn, std::min((mn + 1023) / 1024 * 1024, mcap));
-    std::vector<long long> key = {2, d_tlist != nullptr, ntis, n_sub, mr, box, c->cb, c->cp, c->ap, c->bp,
-                                  tu.ca_fuse, tu.ca_group, tu.a_zb, tu.a_rows, tu.xcd};
+    std::vector<long long> key = {2, c->tis_version, d_tlist != nullptr, ntis, n_sub, mr, box, c->cb, c->cp, c->ap,
+                                  c->bp, tu.ca_fuse, tu.ca_group, tu.a_zb, tu.a_rows, tu.xcd};
     key.insert(key.end(), c->cal_key.begin(), c->cal_key.end());
     RCHK(graph_run(c, key, [&] {
       int cp = c->cp, ap = c->ap;
-      launch_ca_begin(c->stream, c->d_tis, d_tlist, ntis, c->cb, mr, box);
-      launch_ca_substeps(c->stream, c->d_tis, cl, c->cb, cp, ap, c->bp, n_sub, tu);
-      launch_ca_end(c->stream, c->d_tis, d_tlist, ntis, mr);
+      launch_ca_begin(c->stream, c->d_tis, d_tlist, ntis, c->cb, c->bp, mr, box, 1);
+      launch_ca_substeps(c->stream, c->d_tis, cl, cp, ap, n_sub, tu);
+      launch_ca_end(c->stream, c->d_tis, d_tlist, ntis, c->cb, mr, CA_END_SOLVE);
       return hipGetLastError();
     }));
     c->cp ^= n_sub & 1;
     c->ap ^= n_sub & 1;
   } else {
-    launch_ca_begin(c->stream, c->d_tis, d_tlist, ntis, c->cb, mn, box);
-    launch_ca_substeps(c->stream, c->d_tis, cl, c->cb, c->cp, c->ap, c->bp, n_sub, tu);
-    launch_ca_end(c->stream, c->d_tis, d_tlist, ntis, mn);
+    launch_ca_begin(c->stream, c->d_tis, d_tlist, ntis, c->cb, c->bp, mn, box, 1);
+    launch_ca_substeps(c->stream, c->d_tis, cl, c->cp, c->ap, n_sub, tu);
+    launch_ca_end(c->stream, c->d_tis, d_tlist, ntis, c->cb, mn, CA_END_SOLVE);
   }
   if ((n_sub & 1) && d_tlist && ntis < c->T) {
     // the parities name the same buffer for every tissue: an odd count
@@ -913,6 +923,7 @@ int epi_load_cells(epi_ctx* c, int32_t t, const epi_cell_input* in) {
     }
   h.nder = in->nder;
   ti.nder = in->nder;
+  c->tis_version++;
   HIPCHK(c, hipMemcpy(c->d_tis + t, &ti, sizeof(Tis), hipMemcpyHostToDevice));
   RCHK(upload(c, ti.state, st.data(), n));
   RCHK(upload(c, ti.is_malignant, mal.data(), n));
@@ -1201,12 +1212,10 @@ int epi_ca_substep(epi_ctx* c, int32_t iz_bound) {
   long long box = 1;
   for (auto& h : c->th) box = std::max(box, (long long)h.NX * h.NY * (iz_bound + 1));
   CaList cl;
-  RCHK(ca_list(c, nullptr, c->T, c->tu.ca_group, ca_list_bs(c->tu, false), c->tu.a_zb, &cl));
-  launch_ca_touch(c->stream, c->d_tis, nullptr, c->T, c->cb, mn, box);
-  launch_ca_substep(c->stream, c->d_tis, cl, c->cb, c->cp, c->ap, c->bp, c->tu);
-  c->cp ^= 1;
-  c->ap ^= 1;
-  launch_ca_diffu_zero(c->stream, c->d_tis, nullptr, c->T, mn);
+  RCHK(ca_list(c, nullptr, c->T, ca_lanes(c->tu.ca_group), ca_list_bs(c->tu, false), c->tu.a_zb, &cl));
+  launch_ca_begin(c->stream, c->d_tis, nullptr, c->T, c->cb, c->bp, mn, box, 0);
+  launch_ca_substeps(c->stream, c->d_tis, cl, c->cp, c->ap, 1, c->tu);
+  launch_ca_end(c->stream, c->d_tis, nullptr, c->T, c->cb, mn, CA_END_SUBSTEP);
   HIPCHK(c, hipGetLastError());
   return sync_status(c);
 }
@@ -1391,6 +1400,7 @@ int epi_set_params(epi_ctx* c, int32_t t, const epi_params* p) {
   derive_params(*p, ti.prm);
   ti.prm.outputdir[sizeof(ti.prm.outputdir) - 1] = 0;
   window_values_from_params(ti);
+  c->tis_version++;
   HIPCHK(c, hipMemcpy(c->d_tis + t, &ti, sizeof(Tis), hipMemcpyHostToDevice));
   return EPI_OK;
 }
@@ -1791,6 +1801,7 @@ long long rd_max_box(const epi_ctx* c) {
 
 // du/dp into the device descriptors, kpa (or its snapshot) and gj0 staged
 int rd_params(epi_ctx* c, const epi_rd_params* prm) {
+  c->tis_version++;
   std::vector<double> g0(c->T);
   for (int t = 0; t < c->T; t++) {
     c->tis[t].ca_du = prm[t].du;
@@ -1809,14 +1820,14 @@ int rd_params(epi_ctx* c, const epi_rd_params* prm) {
   return EPI_OK;
 }
 
-// one window sub-step; with sv the state before it is saved into segment
-// slot `slot` by the cell kernel (cells_only: only that, no ATP update)
-int rd_substep(epi_ctx* c, const RdTis* sv = nullptr, int slot = 0, bool cells_only = false) {
+// n window sub-steps; with sv the state before each is saved by the cell kernel
+// into segment slots 0, 1, ... (last_cells_only: of the last one only that, no
+// ATP update)
+int rd_substeps(epi_ctx* c, int n, const RdTis* sv = nullptr, bool last_cells_only = false) {
+  const Tuning tu = ca_shapes(c, nullptr, c->T);
   CaList cl;
-  RCHK(ca_list(c, nullptr, c->T, c->tu.ca_group, ca_list_bs(c->tu, false), c->tu.a_zb, &cl));
-  launch_ca_substep(c->stream, c->d_tis, cl, c->cb, c->cp, c->ap, c->bp, c->tu, sv, slot, cells_only);
-  c->cp ^= 1;
-  c->ap ^= 1;
+  RCHK(ca_list(c, nullptr, c->T, ca_lanes(tu.ca_group), ca_list_bs(tu, tu.ca_fuse && n >= 2), tu.a_zb, &cl));
+  launch_ca_substeps(c->stream, c->d_tis, cl, c->cp, c->ap, n, tu, sv, 0, last_cells_only);
   return EPI_OK;
 }
 
@@ -1853,7 +1864,7 @@ int epi_rd_begin(epi_ctx* c, const double* zzmax) {
   // per-solve maps: entry kinds, th/Kpa/IAG, voxel owners (init_ca2p_map)
   long long box = 1;
   for (int t = 0; t < c->T; t++) box = std::max(box, (long long)c->th[t].NX * c->th[t].NY * (rd.izb[t] + 1));
-  launch_ca_touch(c->stream, c->d_tis, nullptr, c->T, c->cb, max_n(c), box);
+  launch_ca_begin(c->stream, c->d_tis, nullptr, c->T, c->cb, c->bp, max_n(c), box, 0);
   // arena: snapshot + adjoint arrays per tissue
   rd.h.assign(c->T, RdTis{});
   Carver dry{nullptr, 0, true};
@@ -1900,7 +1911,9 @@ int epi_rd_forward(epi_ctx* c, const epi_rd_params* prm, int32_t n_sub) {
   if (!c->rd.active) return fail(c, EPI_ERR_INVALID, "no reaction-diffusion window is open");
   RCHK(rd_params(c, prm));
   launch_rd_restore(c->stream, c->d_tis, c->rd.d, c->rd.d_gj0, c->T, c->cb, c->cp, c->ap, 1, rd_items(c));
-  for (int s = 0; s < n_sub; s++) RCHK(rd_substep(c));
+  launch_ca_corners(c->stream, c->d_tis, nullptr, c->T, c->bp, max_n(c));   // B may have been set since
+  RCHK(rd_substeps(c, n_sub));
+  launch_ca_end(c->stream, c->d_tis, nullptr, c->T, c->cb, max_n(c), CA_END_PUT);
   HIPCHK(c, hipGetLastError());
   return sync_status(c);
 }
@@ -1954,24 +1967,22 @@ int epi_rd_adjoint(epi_ctx* c, const epi_rd_params* prm, int32_t n_sub, int32_t 
   RCHK(rd_params(c, prm));
   const long long items = rd_items(c);
   launch_rd_restore(c->stream, c->d_tis, rd.d, rd.d_gj0, c->T, c->cb, c->cp, c->ap, 1, items);
+  launch_ca_corners(c->stream, c->d_tis, nullptr, c->T, c->bp, max_n(c));   // B may have been set since
   // forward, checkpoint every K sub-steps; the last segment saves its states
   // straight into the slots, so the reverse pass starts without a recompute
   std::vector<int> ck_cp(nck), ck_ap(nck);
-  const int last0 = (nck - 1) * K;
-  for (int s = 0; s < n_sub; s++) {
-    if (s >= last0) {
-      RCHK(rd_substep(c, rd.d, s - last0));
-      continue;
+  for (int k = 0; k < nck; k++) {
+    if (k == nck - 1) {
+      RCHK(rd_substeps(c, n_sub - k * K, rd.d));
+      break;
     }
-    if (s % K == 0) {
-      ck_cp[s / K] = c->cp;
-      ck_ap[s / K] = c->ap;
-      launch_rd_state(c->stream, c->d_tis, rd.d, c->T, s / K, 2, c->cb, c->cp, c->ap, items);
-    }
-    RCHK(rd_substep(c));
+    ck_cp[k] = c->cp;
+    ck_ap[k] = c->ap;
+    launch_rd_state(c->stream, c->d_tis, rd.d, c->T, k, 1, c->cp, c->ap, items);
+    RCHK(rd_substeps(c, K));
   }
   int q = 0, qa = 0;
-  launch_rd_seed(c->stream, c->d_tis, rd.d, c->T, c->cp, c->cb, q, items);
+  launch_rd_seed(c->stream, c->d_tis, rd.d, c->T, c->cp, q, items);
   const int mn = max_n(c);
   const long long mb = rd_max_box(c);
   for (int k = nck - 1; k >= 0; k--) {
@@ -1979,19 +1990,20 @@ int epi_rd_adjoint(epi_ctx* c, const epi_rd_params* prm, int32_t n_sub, int32_t 
     if (k < nck - 1) {
       c->cp = ck_cp[k];
       c->ap = ck_ap[k];
-      launch_rd_state(c->stream, c->d_tis, rd.d, c->T, k, 3, c->cb, c->cp, c->ap, items);
+      launch_rd_state(c->stream, c->d_tis, rd.d, c->T, k, 0, c->cp, c->ap, items);
       // the states before sub-steps s0 .. s1 - 1, saved by the sub-steps'
       // cell kernels; the state after s1 - 1 is the next checkpoint, so the
-      // last sub-step runs its cell kernel only, for the save
-      for (int s = s0; s < s1; s++) RCHK(rd_substep(c, rd.d, s - s0, s + 1 == s1));
+      // last sub-step runs its cells only, for the save
+      RCHK(rd_substeps(c, s1 - s0, rd.d, true));
     }
     for (int s = s1 - 1; s >= s0; s--) {
-      launch_rd_backward_substep(c->stream, c->d_tis, rd.d, c->T, s - s0, c->cb, c->bp, q, qa, mn, mb, c->tu.rd_group);
+      launch_rd_backward_substep(c->stream, c->d_tis, rd.d, c->T, s - s0, q, qa, mn, mb, c->tu.rd_group);
       q ^= 1;
       qa = qa == 2 ? 0 : qa + 1;
     }
   }
-  launch_rd_gj0(c->stream, c->d_tis, rd.d, c->T, c->cb, q, items);
+  launch_rd_gj0(c->stream, c->d_tis, rd.d, c->T, q, items);
+  launch_ca_end(c->stream, c->d_tis, nullptr, c->T, c->cb, mn, CA_END_PUT);
   HIPCHK(c, hipGetLastError());
   RCHK(sync_status(c));
   for (int t = 0; t < c->T; t++) {
@@ -2013,6 +2025,7 @@ int epi_rd_end(epi_ctx* c) {
   if (!c) return EPI_ERR_INVALID;
   auto& rd = c->rd;
   if (!rd.active) return EPI_OK;
+  c->tis_version++;
   std::vector<double> g0(c->T);
   for (int t = 0; t < c->T; t++) {
     window_values_from_params(c->tis[t]);

@@ -3,7 +3,8 @@
 // frozen) and its reverse pass.
 //
 // Forward: the window restores a snapshot of the tissue and runs the plain
-// sub-step kernels (k_ca_cells, k_atp) with the runtime coefficients in Tis.
+// sub-step kernels (k_ca_cells, k_atp, k_ca_fused) with the runtime
+// coefficients in Tis.
 // Reverse: for the loss L = mean over AFM cells of (ca2p_T - target)^2 each
 // sub-step is differentiated with respect to its state (ca2p, IP3, ex_inert,
 // per-edge gj, ATP) and the parameters.  Values a sub-step never writes
@@ -20,12 +21,13 @@ namespace epi {
 namespace {
 constexpr int RL = 16;   // lanes per cell for row-wise copies
 
-// every (cell, list entry) of the rows of buffer cb, RL lanes per cell
-#define RD_FOR_ROW_ENTRIES(t, cb, n, c, i)                                                      \
+// every (cell, entry) of rows of lens[c] entries, RL lanes per cell: the list
+// rows of a buffer (nlen[cb]) or the packed coupled entries (ca_cn)
+#define RD_FOR_ROW_ENTRIES(t, lens, n, c, i)                                                    \
   for (int c = (int)((blockIdx.x * (long long)blockDim.x + threadIdx.x) / RL); c < (n);          \
        c += (int)((long long)gridDim.x * blockDim.x / RL))                                       \
     for (long long i = (long long)c * (t).ns + (threadIdx.x & (RL - 1)),                         \
-                   i##_end = (long long)c * (t).ns + (t).nlen[cb][c];                            \
+                   i##_end = (long long)c * (t).ns + (lens)[c];                                  \
          i < i##_end; i += RL)
 
 __device__ __forceinline__ long long box_end(const Tis& t, const RdTis& r) { return (long long)r.izb * t.PL; }
@@ -49,7 +51,8 @@ __global__ void __launch_bounds__(256) k_rd_restore(const Tis* __restrict__ T, R
   const int n = t.st->n;
   const double g0 = gj0[blockIdx.y];
   const long long stride = (long long)gridDim.x * blockDim.x;
-  RD_FOR_ROW_ENTRIES(t, cb, n, c, i) t.gj[cb][i] = g0;
+  RD_FOR_ROW_ENTRIES(t, t.nlen[cb], n, c, i) t.gj[cb][i] = g0;
+  RD_FOR_ROW_ENTRIES(t, t.ca_cn, n, c, i) t.ca_g[i] = g0;
   for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += stride) {
     t.ca2p[cp][c] = r.u0[0][c]; t.ca2p[1 - cp][c] = r.u0[1][c];
     t.ip3[cp][c] = r.p0[0][c]; t.ip3[1 - cp][c] = r.p0[1][c];
@@ -72,7 +75,7 @@ __global__ void __launch_bounds__(256) k_rd_snapshot(const Tis* __restrict__ T, 
   const int start = t.nmemb + t.nder;
   const long long stride = (long long)gridDim.x * blockDim.x;
   int nafm = 0;
-  RD_FOR_ROW_ENTRIES(t, cb, n, c, i) r.g0[i] = t.gj[cb][i];
+  RD_FOR_ROW_ENTRIES(t, t.nlen[cb], n, c, i) r.g0[i] = t.gj[cb][i];
   for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += stride) {
     r.u0[0][c] = t.ca2p[cp][c]; r.u0[1][c] = t.ca2p[1 - cp][c];
     r.p0[0][c] = t.ip3[cp][c]; r.p0[1][c] = t.ip3[1 - cp][c];
@@ -91,54 +94,37 @@ __global__ void __launch_bounds__(256) k_rd_put_gj(const Tis* __restrict__ T, Rd
   const Tis& t = T[blockIdx.y];
   const RdTis& r = R[blockIdx.y];
   const int n = t.st->n;
-  RD_FOR_ROW_ENTRIES(t, cb, n, c, i) t.gj[cb][i] = r.g0[i];
+  RD_FOR_ROW_ENTRIES(t, t.nlen[cb], n, c, i) t.gj[cb][i] = r.g0[i];
 }
 
-// copy the state between the tissue and a segment slot (dir 0: save,
-// 1: restore; of the ATP grid a slot keeps only the cells' grid_avg8, so a
-// restore from it leaves the grid as it is) or a checkpoint (both buffers;
-// dir 2: save, 3: restore)
+// copy the state (both buffers) between the tissue and checkpoint `slot`
+// (save 1: to it, 0: back)
 __global__ void __launch_bounds__(256) k_rd_state(const Tis* __restrict__ T, RdTis* __restrict__ R, int slot,
-                                                   int dir, int cb, int cp, int ap) {
+                                                   int save, int cp, int ap) {
   const Tis& t = T[blockIdx.y];
   const RdTis& r = R[blockIdx.y];
   const int n = t.st->n;
   const long long cap = t.cap, ns = t.ns;
   const long long stride = (long long)gridDim.x * blockDim.x;
-  const bool ck = dir >= 2, save = (dir & 1) == 0;
-  double* gs = (ck ? r.cg : r.sg) + slot * cap * ns;
-  RD_FOR_ROW_ENTRIES(t, cb, n, c, i) {
-    if (save) gs[i] = t.gj[cb][i];
-    else t.gj[cb][i] = gs[i];
+  double* gs = r.cg + slot * cap * ns;
+  RD_FOR_ROW_ENTRIES(t, t.ca_cn, n, c, i) {
+    if (save) gs[i] = t.ca_g[i];
+    else t.ca_g[i] = gs[i];
   }
-  const int nb = ck ? 2 : 1;
-  const int start = t.nmemb + t.nder;
+  double* hs = r.ch + slot * cap;
   for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += stride) {
-    double* hs = (ck ? r.ch : r.sh) + slot * cap;
     if (save) hs[c] = t.ex_inert[c];
     else t.ex_inert[c] = hs[c];
-    if (!ck && save) {
-      // grid_avg8 of the ATP buffer at the cell's lattice corner
-      double av = 0;
-      if (c >= start && is_afm(t.state[c])) {
-        const double* A = t.atp[ap];
-        const long long b0 = gidx(t, t.lat[3 * c], t.lat[3 * c + 1], t.lat[3 * c + 2]);
-        av = 0.125 * (A[b0] + A[b0 + 1] + A[b0 + t.XP] + A[b0 + t.PL] + A[b0 + t.XP + 1] + A[b0 + t.PL + 1]
-                      + A[b0 + t.PL + t.XP] + A[b0 + t.PL + t.XP + 1]);
-      }
-      r.sAv[slot * cap + c] = av;
-    }
-    for (int b = 0; b < nb; b++) {
-      const int buf = b ? 1 - cp : cp;
-      double* us = (ck ? r.cu + (2 * slot + b) * cap : r.su + slot * cap);
-      double* ps = (ck ? r.cp_ + (2 * slot + b) * cap : r.sp + slot * cap);
-      if (save) { us[c] = t.ca2p[buf][c]; ps[c] = t.ip3[buf][c]; }
-      else { t.ca2p[buf][c] = us[c]; t.ip3[buf][c] = ps[c]; t.ca_up[buf][c] = make_double2(us[c], ps[c]); }
+    for (int b = 0; b < 2; b++) {
+      double2* up = t.ca_up[b ? 1 - cp : cp];
+      double* us = r.cu + (2 * slot + b) * cap;
+      double* ps = r.cp_ + (2 * slot + b) * cap;
+      if (save) { const double2 w = up[c]; us[c] = w.x; ps[c] = w.y; }
+      else up[c] = make_double2(us[c], ps[c]);
     }
   }
-  if (!ck) return;   // a segment state keeps grid_avg8 per cell, not the grid
   for (long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x; v < r.box; v += stride) {
-    for (int b = 0; b < nb; b++) {
+    for (int b = 0; b < 2; b++) {
       const int buf = b ? 1 - ap : ap;
       double* as = r.cA + (2 * slot + b) * r.box;
       if (save) as[v] = t.atp[buf][v];
@@ -150,8 +136,7 @@ __global__ void __launch_bounds__(256) k_rd_state(const Tis* __restrict__ T, RdT
 // the loss and the seed of the reverse pass.  Every adjoint buffer starts at
 // zero; the sub-steps keep them so (a cell's group clears the cell adjoints
 // it has read, the grid part the ATP buffer the next sub-step scatters into).
-__global__ void __launch_bounds__(256) k_rd_seed(const Tis* __restrict__ T, RdTis* __restrict__ R, int cp, int cb,
-                                                  int q) {
+__global__ void __launch_bounds__(256) k_rd_seed(const Tis* __restrict__ T, RdTis* __restrict__ R, int cp, int q) {
   const Tis& t = T[blockIdx.y];
   const RdTis& r = R[blockIdx.y];
   const int n = t.st->n;
@@ -161,14 +146,14 @@ __global__ void __launch_bounds__(256) k_rd_seed(const Tis* __restrict__ T, RdTi
   for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < n; c += stride) {
     double s = 0;
     if (c >= start && is_afm(t.state[c])) {
-      const double d = t.ca2p[cp][c] - r.target[c];
+      const double d = t.ca_up[cp][c].x - r.target[c];
       part += d * d;
       s = 2.0 * d / r.nafm;
     }
     r.lu[q][c] = s; r.lp[q][c] = 0; r.lh[q][c] = 0; r.gkpa[c] = 0;
     r.lu[1 - q][c] = 0; r.lp[1 - q][c] = 0; r.lh[1 - q][c] = 0;
   }
-  RD_FOR_ROW_ENTRIES(t, cb, n, c, i) r.lg[q][i] = 0;
+  RD_FOR_ROW_ENTRIES(t, t.ca_cn, n, c, i) r.lg[q][i] = 0;
   for (long long v = (long long)blockIdx.x * blockDim.x + threadIdx.x; v < r.box; v += stride) {
     r.lA[0][v] = 0; r.lA[1][v] = 0; r.lA[2][v] = 0;
   }
@@ -178,9 +163,8 @@ __global__ void __launch_bounds__(256) k_rd_seed(const Tis* __restrict__ T, RdTi
 
 // reverse of dead_IP3_calc and supra_calc for one sub-step, the state before
 // the sub-step from slot `slot`.  A group of RG lanes (8 or 16, a launch
-// shape) owns one cell: lanes take the coupled list entries (the per-solve
-// compact (word, slot) list; gj and its adjoint live at the slot), their partial sums are
-// reduced over the group (a gradient need not follow the forward's summation
+// shape) owns one cell: lanes take the packed coupled entries (gj and its
+// adjoint lie at the same place), their partial sums are reduced over the group (a gradient need not follow the forward's summation
 // order), and each lane scatters its entries' contributions.  A lane keeps
 // its first 32 / RG entries (and their neighbour values) in registers for
 // both passes, every load of them issued up front; entries past 32 take the
@@ -227,8 +211,8 @@ __device__ __forceinline__ void rd_entry_bwd(const RdEntry& k, int kd, int o, do
 }  // namespace
 
 template <int RG>
-__device__ __forceinline__ void rd_cells_part(const Tis& t, const RdTis& r, int bid, int nblk, int slot, int cb,
-                                              int bp, int q, int qa) {
+__device__ __forceinline__ void rd_cells_part(const Tis& t, const RdTis& r, int bid, int nblk, int slot, int q,
+                                              int qa) {
   constexpr int REP = 32 / RG;
   const int start = t.nmemb + t.nder;
   const long long cap = t.cap, ns = t.ns;
@@ -264,16 +248,16 @@ __device__ __forceinline__ void rd_cells_part(const Tis& t, const RdTis& r, int 
   if (bid == 0 && threadIdx.x == 0 && start + (long long)groups < n) set_err(t.st, ERR_INVALID);
   if (c < n) do {   // "continue" below leaves the cell
     const uint8_t s = s0;
-    // the coupled entries only, (word, slot of the entry in the row)
+    // the coupled entries only
     const int len = len0;
     const double lpc = lpc0;
     const double uc = uc0, pc = pc0;
-    const int2* ent = t.ca_ce + (size_t)c * ns;
+    const int* ent = t.ca_w + (size_t)c * ns;
     if (s == DEAD) {
       double cnt = 0, sum = 0;
       for (int e = lane; e < len; e += RG)
-        if ((ent[e].x & 3) == 3) {
-          const int o = ent[e].x >> 2;
+        if ((ent[e] & 3) == 3) {
+          const int o = ent[e] >> 2;
           sum += p[o];
           cnt += 1;
           atomicAdd(&np[o], lpc * DT_Ca * dp);
@@ -294,26 +278,27 @@ __device__ __forceinline__ void rd_cells_part(const Tis& t, const RdTis& r, int 
     // the lane's first REP entries: packed neighbour and kind, gj, edge
     // adjoint, then the neighbours' state, Ca2+ and IP3, all in flight together
     const int m0 = min(len, RG * REP);
-    int o[REP], sl[REP];
+    int o[REP];
     uint8_t kd[REP], so[REP];
     double gv[REP], lgv[REP], uo[REP], po[REP];
     // every load unconditional (a row holds ns >= 32 slots; a masked entry
-    // reads slot 0 and cell 0), masked with integer masks afterwards, so that
-    // no load sits in a branch that waits for it
-    int2 x[REP];
-#pragma unroll
-    for (int i = 0; i < REP; i++) x[i] = ent[lane + i * RG];
+    // reads cell 0), masked with integer masks afterwards, so that no load
+    // sits in a branch that waits for it
+    int x[REP];
 #pragma unroll
     for (int i = 0; i < REP; i++) {
-      const int msk = -(int)(lane + i * RG < m0);
-      o[i] = (x[i].x & msk) >> 2;
-      kd[i] = (uint8_t)(x[i].x & msk & 3);
-      sl[i] = x[i].y & msk;
+      x[i] = ent[lane + i * RG];
+      gv[i] = gr[lane + i * RG];
+      lgv[i] = lgr[lane + i * RG];
     }
 #pragma unroll
     for (int i = 0; i < REP; i++) {
-      gv[i] = gr[sl[i]];
-      lgv[i] = lgr[sl[i]];
+      const int msk = -(int)(lane + i * RG < m0);
+      o[i] = (x[i] & msk) >> 2;
+      kd[i] = (uint8_t)(x[i] & msk & 3);
+    }
+#pragma unroll
+    for (int i = 0; i < REP; i++) {
       uo[i] = u[o[i]];
       po[i] = p[o[i]];
       so[i] = t.state[o[i]];
@@ -350,9 +335,8 @@ __device__ __forceinline__ void rd_cells_part(const Tis& t, const RdTis& r, int 
         gsum += gv[i];
       }
     for (int e = RG * REP + lane; e < len; e += RG) {
-      const int2 en = ent[e];
-      const int oe = en.x >> 2;
-      const double ge = gr[en.y];
+      const int oe = ent[e] >> 2;
+      const double ge = gr[e];
       su += ge * (u[oe] - uc);
       sp += ge * (p[oe] - pc);
       gsum += ge;
@@ -361,21 +345,18 @@ __device__ __forceinline__ void rd_cells_part(const Tis& t, const RdTis& r, int 
     sp = group_sum<RG>(sp);
     gsum = group_sum<RG>(gsum);
     acc_own = group_sum<RG>(acc_own);
-    const double Bavg = grid_avg8(t, t.bf[bp], ix, iy, iz);
     const double Aavg = r.sAv[slot * cap + c];
-    const double diffu = ca2p_reaction_factor(ck, uc, hc, pc, Bavg) + du * iag * su;
+    const double diffu = ca2p_reaction_factor(ck, uc, hc, pc, t.ca_bx[c]) + du * iag * su;
     const double abar = DT_Ca * luc + (diffu > 0 ? acc_own * DT_Ca * STIM11 : 0.0);
     const RdEntry k{abar * du * iag, lpc * DT_Ca * dp * iag, uc, pc, DT_Ca, ck.wd};
     double own_u = 0;
 #pragma unroll
     for (int i = 0; i < REP; i++)
-      if (kd[i]) rd_entry_bwd(k, kd[i], o[i], gv[i], uo[i], po[i], lgv[i], so[i], &ng[(size_t)c * ns + sl[i]],
-                              nu, np, own_u);
+      if (kd[i]) rd_entry_bwd(k, kd[i], o[i], gv[i], uo[i], po[i], lgv[i], so[i],
+                              &ng[(size_t)c * ns + lane + i * RG], nu, np, own_u);
     for (int e = RG * REP + lane; e < len; e += RG) {
-      const int2 en = ent[e];
-      const int oe = en.x >> 2;
-      rd_entry_bwd(k, en.x & 3, oe, gr[en.y], u[oe], p[oe], lgr[en.y], t.state[oe], &ng[(size_t)c * ns + en.y], nu,
-                   np, own_u);
+      const int en = ent[e], oe = en >> 2;
+      rd_entry_bwd(k, en & 3, oe, gr[e], u[oe], p[oe], lgr[e], t.state[oe], &ng[(size_t)c * ns + e], nu, np, own_u);
     }
     own_u = group_sum<RG>(own_u);
     if (lane < 8) {   // the eight grid_avg8 corners of the IP3 production term
@@ -455,23 +436,23 @@ __device__ __forceinline__ void rd_grid_part(const Tis& t, const RdTis& r, int b
 
 // one reverse sub-step: blocks [0, ncb) take the cells, the rest the box
 template <int RG>
-__global__ void __launch_bounds__(256) k_rd_step(const Tis* __restrict__ T, RdTis* __restrict__ R, int slot, int cb,
-                                                  int bp, int q, int qa, int ncb) {
+__global__ void __launch_bounds__(256) k_rd_step(const Tis* __restrict__ T, RdTis* __restrict__ R, int slot, int q,
+                                                  int qa, int ncb) {
   const Tis& t = T[blockIdx.y];
   const RdTis& r = R[blockIdx.y];
-  if ((int)blockIdx.x < ncb) rd_cells_part<RG>(t, r, blockIdx.x, ncb, slot, cb, bp, q, qa);
+  if ((int)blockIdx.x < ncb) rd_cells_part<RG>(t, r, blockIdx.x, ncb, slot, q, qa);
   else rd_grid_part(t, r, blockIdx.x - ncb, gridDim.x - ncb, qa);
 }
 
 // dL/dgj0: the adjoints of every coupled edge at the window's start
-__global__ void __launch_bounds__(256) k_rd_gj0(const Tis* __restrict__ T, RdTis* __restrict__ R, int cb, int q) {
+__global__ void __launch_bounds__(256) k_rd_gj0(const Tis* __restrict__ T, RdTis* __restrict__ R, int q) {
   const Tis& t = T[blockIdx.y];
   RdTis& r = R[blockIdx.y];
   const int n = t.st->n;
   const int start = t.nmemb + t.nder;
   double part = 0;
-  RD_FOR_ROW_ENTRIES(t, cb, n, c, i)
-    if (c >= start && is_afm(t.state[c]) && (t.ca_ent[i] & 3)) part += r.lg[q][i];
+  RD_FOR_ROW_ENTRIES(t, t.ca_cn, n, c, i)
+    if (c >= start && is_afm(t.state[c])) part += r.lg[q][i];
   for (int o = 32; o > 0; o >>= 1) part += __shfl_down(part, o, 64);
   if ((threadIdx.x & 63) == 0 && part != 0) atomicAdd(&r.scal[3], part);
 }
@@ -532,24 +513,24 @@ void launch_rd_restore(hipStream_t s, const Tis* dT, RdTis* dR, const double* gj
 void launch_rd_put_gj(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int cb, long long items) {
   EPI_LAUNCH(K_RD_PUT_GJ, k_rd_put_gj, cells_grid(items, ntis), dim3(256), 0, s, dT, dR, cb);
 }
-void launch_rd_state(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int slot, int dir, int cb, int cp, int ap,
+void launch_rd_state(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int slot, int save, int cp, int ap,
                      long long items) {
-  EPI_LAUNCH(K_RD_STATE, k_rd_state, cells_grid(items, ntis), dim3(256), 0, s, dT, dR, slot, dir, cb, cp, ap);
+  EPI_LAUNCH(K_RD_STATE, k_rd_state, cells_grid(items, ntis), dim3(256), 0, s, dT, dR, slot, save, cp, ap);
 }
-void launch_rd_seed(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int cp, int cb, int q, long long items) {
-  EPI_LAUNCH(K_RD_SEED, k_rd_seed, cells_grid(items, ntis), dim3(256), 0, s, dT, dR, cp, cb, q);
+void launch_rd_seed(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int cp, int q, long long items) {
+  EPI_LAUNCH(K_RD_SEED, k_rd_seed, cells_grid(items, ntis), dim3(256), 0, s, dT, dR, cp, q);
 }
-void launch_rd_backward_substep(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int slot, int cb, int bp, int q,
-                                int qa, int max_n, long long max_box, int rg) {
+void launch_rd_backward_substep(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int slot, int q, int qa, int max_n,
+                                long long max_box, int rg) {
   const int ncb = (int)(((long long)max_n * rg + 255) / 256);   // one cell per group: no cap
   const dim3 g(ncb + cells_grid(max_box, ntis).x, ntis);
   if (rg == 16)
-    EPI_LAUNCH(K_RD_STEP, k_rd_step<16>, g, dim3(256), 0, s, dT, dR, slot, cb, bp, q, qa, ncb);
+    EPI_LAUNCH(K_RD_STEP, k_rd_step<16>, g, dim3(256), 0, s, dT, dR, slot, q, qa, ncb);
   else
-    EPI_LAUNCH(K_RD_STEP, k_rd_step<8>, g, dim3(256), 0, s, dT, dR, slot, cb, bp, q, qa, ncb);
+    EPI_LAUNCH(K_RD_STEP, k_rd_step<8>, g, dim3(256), 0, s, dT, dR, slot, q, qa, ncb);
 }
-void launch_rd_gj0(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int cb, int q, long long items) {
-  EPI_LAUNCH(K_RD_GJ0, k_rd_gj0, cells_grid(items, ntis), dim3(256), 0, s, dT, dR, cb, q);
+void launch_rd_gj0(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int q, long long items) {
+  EPI_LAUNCH(K_RD_GJ0, k_rd_gj0, cells_grid(items, ntis), dim3(256), 0, s, dT, dR, q);
 }
 
 }  // namespace epi

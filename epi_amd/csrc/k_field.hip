@@ -456,51 +456,64 @@ __global__ void __launch_bounds__(256) k_ext_stim_one(const Tis* __restrict__ T,
 }
 
 // ---- calc_ca2p ------------------------------------------------------------
-// init_ca2p_avg (:20-27) and the per-cell "touches AIR" flag used by
-// init_ca2p_map (:262-268)
+// init_ca2p_avg (:20-27), the per-cell "touches AIR" flag used by
+// init_ca2p_map (:262-268), the (ca2p, IP3) pairs, the packed coupled entries
+// and the constants of the Ca laws.  BL lanes per cell take its list BL
+// entries at a time: the neighbours' states in one gather, the coupled entries
+// placed by a ballot (one lane walking the list waited for two round trips per
+// entry: 27 us for lists of up to 40).
+constexpr int BL = 16;
 __global__ void __launch_bounds__(256) k_ca_begin(const Tis* __restrict__ T, const int* tlist, int cb, int zero_avg) {
   const Tis& t = T[tlist ? tlist[blockIdx.y] : blockIdx.y];
   const int n = t.st->n;
   const int start = t.nmemb + t.nder;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
+  const int lane = threadIdx.x & (BL - 1);
+  // the constants are read before any store (see CaK)
+  const Params& pm = t.prm;
+  const double thgra = pm.thgra, thpri = pm.thpri, delta_th = pm.delta_th, TSP = pm.THRESH_SP;
+  const double kpa = pm.kpa, Kpri = pm.Kpri, delta_K = pm.delta_K, delta_I = pm.delta_I, ik = pm.iage_kitei;
+  for (int c = (blockIdx.x * blockDim.x + threadIdx.x) / BL; c < n; c += gridDim.x * blockDim.x / BL) {
     const int* row = t.col[cb] + (size_t)c * t.ns;
     const int len = t.nlen[cb][c];
-    uint8_t air = 0;
-    for (int e = 0; e < len; e++)
-      if (t.state[row[e]] == AIR) { air = 1; break; }
-    t.touch_air[c] = air;
     const uint8_t s = t.state[c];
-    t.ca_up[0][c] = make_double2(t.ca2p[0][c], t.ip3[0][c]);
-    t.ca_up[1][c] = make_double2(t.ca2p[1][c], t.ip3[1][c]);
-    if (c >= start && (s == DEAD || is_afm(s))) {
+    const bool afm = c >= start && is_afm(s), takes = afm || (c >= start && s == DEAD);
+    const double* g = t.gj[cb] + (size_t)c * t.ns;
+    const size_t at = (size_t)c * t.ns;
+    bool air = false;
+    int k = 0;
+    for (int e0 = 0; e0 < len; e0 += BL) {
+      const int e = e0 + lane;
+      const int o = e < len ? row[e] : -1;
+      const uint8_t so = o >= 0 ? t.state[o] : MEMB;
+      const double gv = o >= 0 && takes ? g[e] : 0.0;
+      air = air || so == AIR;
       // which entries take part in the gap-junction sums (supra_calc
       // :201-209; dead_IP3_calc :160-165 counts the ALIVE ones)
-      int* ent = t.ca_ent + (size_t)c * t.ns;
-      int2* ce = t.ca_ce + (size_t)c * t.ns;
-      int k = 0;
-      for (int e = 0; e < len; e++) {
-        const int o = row[e];
-        const uint8_t so = t.state[o];
-        const int w = (o << 2) | ((so == ALIVE) ? 3 : (so == DEAD || so == FIX || so == MUSUME) ? 1 : 0);
-        ent[e] = w;
-        if (w & 3) ce[k++] = make_int2(w, e);
+      const int kd = so == ALIVE ? 3 : (so == DEAD || so == FIX || so == MUSUME) ? 1 : 0;
+      const unsigned m = (unsigned)(__ballot(takes && kd) >> (threadIdx.x & 48)) & 0xffffu;
+      if (takes && kd) {
+        const size_t i = at + k + __popc(m & ((1u << lane) - 1));
+        t.ca_w[i] = (o << 2) | kd;
+        t.ca_sl[i] = (unsigned short)e;
+        t.ca_g[i] = gv;
       }
-      t.ca_cn[c] = k;
+      k += __popc(m);
     }
-    if (c >= start && is_afm(s)) {
-      // calc_th, calc_Kpa, calc_IAG (ca2p.cpp:90-126): agek and state do
-      // not change during a solve
-      const bool is_alive = s == ALIVE;
-      const double agek = t.agek[c];
-      // the constants are read before this cell's stores (see CaK)
-      const Params& pm = t.prm;
-      const double thgra = pm.thgra, thpri = pm.thpri, delta_th = pm.delta_th, TSP = pm.THRESH_SP;
-      const double kpa = pm.kpa, Kpri = pm.Kpri, delta_K = pm.delta_K, delta_I = pm.delta_I, ik = pm.iage_kitei;
-      if (zero_avg) t.ca2p_avg[c] = 0;
-      t.ca_th[c] = is_alive ? thgra + ((thpri - thgra) * 0.5) * (1.0 + tanh((TSP - agek) / delta_th)) : thpri;
-      t.ca_kpa[c] = is_alive ? kpa + ((Kpri - kpa) * 0.5) * (1.0 + tanh((TSP - agek) / delta_K)) : Kpri;
-      t.ca_iag[c] = is_alive ? 0.5 * (1.0 + tanh((agek - TSP) / delta_I)) : ik;
-    }
+    const bool any_air = ((__ballot(air) >> (threadIdx.x & 48)) & 0xffffu) != 0;
+    if (lane != 0) continue;
+    t.touch_air[c] = any_air;
+    t.ca_cn[c] = k;
+    t.ca_up[0][c] = make_double2(t.ca2p[0][c], t.ip3[0][c]);
+    t.ca_up[1][c] = make_double2(t.ca2p[1][c], t.ip3[1][c]);
+    if (!afm) continue;
+    // calc_th, calc_Kpa, calc_IAG (ca2p.cpp:90-126): agek and state do
+    // not change during a solve
+    const bool is_alive = s == ALIVE;
+    const double agek = t.agek[c];
+    if (zero_avg) t.ca2p_avg[c] = 0;
+    t.ca_th[c] = is_alive ? thgra + ((thpri - thgra) * 0.5) * (1.0 + tanh((TSP - agek) / delta_th)) : thpri;
+    t.ca_kpa[c] = is_alive ? kpa + ((Kpri - kpa) * 0.5) * (1.0 + tanh((TSP - agek) / delta_K)) : Kpri;
+    t.ca_iag[c] = is_alive ? 0.5 * (1.0 + tanh((agek - TSP) / delta_I)) : ik;
   }
 }
 
@@ -550,317 +563,345 @@ __device__ __forceinline__ double atp_new(const AtpK& k, double catp, double cxm
 
 // diff_u of a sub-step by Ca parity: the sub-step at parity cp writes it and
 // its ATP update reads it, so a fused launch (ATP of one sub-step beside the
-// cells of the next) reads one buffer while it writes the other
-__device__ __forceinline__ double* dfu_buf(const Tis& t, int cp) { return cp ? t.ca_dfu : t.diff_u; }
+// cells of the next) reads one buffer while it writes the other.
 
-// The voxel map, the masks and iz_bound do not change during a solve, so
-// each AFM cell's eight ATP corners keep their voxel word and neighbour masks
-// for all of its sub-steps (used when the corners are computed, not read).
-// One thread per (cell, corner), after k_ca_vox.
-__global__ void __launch_bounds__(256) k_ca_corners(const Tis* __restrict__ T, const int* tlist) {
+// What a launch of the Ca kernels reads and writes of one tissue, resolved from
+// its descriptor and the parities.  A one-tissue launch carries it by value,
+// as kernel arguments: its waves then start on the cells' words without first
+// fetching pointers through the descriptor (a round trip of the five a
+// sub-step's cells wait for).  The laws' constants stay in the descriptor: they
+// are needed late, and by value they would be held in scalar registers from
+// the start, more of them than a wave has.
+struct CaArg {
+  const Status* st;
+  const uint8_t* state;
+  const int* cn;
+  const int* w;
+  double* g;
+  const double2* up;      // (ca2p, IP3) before the sub-step
+  double2* upn;           // and after it
+  const double* dfo;      // diff_u that the ATP update and the recomputed corners read
+  double* dfn;            // diff_u that the cells write
+  const uint4* cq;
+  const double *th, *kpa, *iag, *bx;
+  double *exi, *avg;
+  const double* A0;       // ATP before the launch's ATP update
+  double* A1;             // and after it
+  const uint8_t* cm2;
+  const unsigned* vox;
+  long long PL;
+  int start, cap, ns, NX, NY, NZ, XP;
+};
+// cells at Ca parity cpc; the ATP update of the sub-step at Ca parity cpa from
+// ATP buffer ap
+__host__ __device__ __forceinline__ CaArg ca_arg(const Tis& t, int cpc, int cpa, int ap) {
+  CaArg a;
+  a.st = t.st; a.state = t.state; a.cn = t.ca_cn; a.w = t.ca_w; a.g = t.ca_g;
+  a.up = t.ca_up[cpc]; a.upn = t.ca_up[1 - cpc];
+  a.dfo = cpa ? t.ca_dfu : t.diff_u; a.dfn = cpc ? t.ca_dfu : t.diff_u;
+  a.cq = t.ca_cq; a.th = t.ca_th; a.kpa = t.ca_kpa; a.iag = t.ca_iag; a.bx = t.ca_bx;
+  a.exi = t.ex_inert; a.avg = t.ca2p_avg; a.A0 = t.atp[ap]; a.A1 = t.atp[1 - ap];
+  a.cm2 = t.cmap2; a.vox = t.vox; a.PL = t.PL;
+  a.start = t.nmemb + t.nder; a.cap = t.cap; a.ns = t.ns;
+  a.NX = t.NX; a.NY = t.NY; a.NZ = t.NZ; a.XP = t.XP;
+  return a;
+}
+
+// The voxel map, the masks, B and iz_bound do not change during a solve, so
+// each AFM cell keeps, for all of its sub-steps, its ca2p_by_ext_stim and, of
+// its eight grid_avg8 corners, the point, its voxel word, neighbour masks and
+// where the stencil wraps.  One lane per (cell, corner), after k_ca_vox.
+constexpr unsigned CQ_XM = 1u << 6, CQ_XP = 1u << 7, CQ_YM = 1u << 8, CQ_YP = 1u << 9;   // x = 0, x = NX - 1, ...
+constexpr unsigned CQ_ZM = 1u << 10, CQ_ZP = 1u << 11;   // z = 0 (mirror), z = NZ - 1 (self)
+constexpr unsigned CQ_PLAIN = 1u << 30;   // not updated inside the solve: read as it is
+constexpr unsigned CQ_SLOW = 1u << 31;    // a mask byte above 1: word and masks come from the maps
+
+__global__ void __launch_bounds__(256) k_ca_corners(const Tis* __restrict__ T, const int* tlist, int bp) {
   const Tis& t = T[tlist ? tlist[blockIdx.y] : blockIdx.y];
   const int n = t.st->n;
   const int start = t.nmemb + t.nder;
   const int izb = ca_iz_bound(t);
   const int NX = t.NX, NY = t.NY, NZ = t.NZ;
+  const CaK ck = ca_k(t.prm);
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < 8LL * n;
        i += (long long)gridDim.x * blockDim.x) {
     const int c = (int)(i >> 3), k = (int)(i & 7);
     if (c < start || !is_afm(t.state[c])) continue;
-    int j = t.lat[3 * c] + ((k == 1 || k == 4 || k == 5 || k == 7) ? 1 : 0);
-    int kk = t.lat[3 * c + 1] + ((k == 2 || k == 4 || k == 6 || k == 7) ? 1 : 0);
-    const int l = t.lat[3 * c + 2] + ((k == 3 || k == 5 || k == 6 || k == 7) ? 1 : 0);
+    int j = t.lat[3 * c] + (k & 1), kk = t.lat[3 * c + 1] + ((k >> 1) & 1);
+    const int l = t.lat[3 * c + 2] + (k >> 2);
+    const long long raw = gidx(t, j, kk, l);
+    const double b = t.bf[bp][raw];
     if (j == NX) j = 0;
     if (kk == NY) kk = 0;
-    uint2 pre = make_uint2(0u, 0x80000000u);
+    const long long v = gidx(t, j, kk, l);
+    unsigned word = 0, bits = CQ_PLAIN;
     if (l < izb && izb <= NZ) {
       const int px = j == 0 ? NX - 1 : j - 1, nx = j == NX - 1 ? 0 : j + 1;
       const int py = kk == 0 ? NY - 1 : kk - 1, ny = kk == NY - 1 ? 0 : kk + 1;
       const int pz = l == 0 ? 1 : l - 1, nz = l + 1 == NZ ? NZ - 1 : l + 1;
       const uint8_t m[6] = {t.cmap2[gidx(t, px, kk, l)], t.cmap2[gidx(t, nx, kk, l)], t.cmap2[gidx(t, j, py, l)],
                             t.cmap2[gidx(t, j, ny, l)], t.cmap2[gidx(t, j, kk, pz)], t.cmap2[gidx(t, j, kk, nz)]};
-      unsigned bits = 0;
-      for (int b = 0; b < 6; b++) {
-        if (m[b] > 1) bits |= 0x80000000u;
-        bits |= (unsigned)(m[b] & 1) << b;
+      bits = (j == 0 ? CQ_XM : 0) | (j == NX - 1 ? CQ_XP : 0) | (kk == 0 ? CQ_YM : 0) | (kk == NY - 1 ? CQ_YP : 0) |
+             (l == 0 ? CQ_ZM : 0) | (l + 1 == NZ ? CQ_ZP : 0);
+      for (int q = 0; q < 6; q++) {
+        if (m[q] > 1) bits |= CQ_SLOW;
+        bits |= (unsigned)(m[q] & 1) << q;
       }
-      pre = make_uint2(t.vox[gidx(t, j, kk, l)], bits);
+      word = t.vox[v];
     }
-    t.ca_cq[i] = pre;
+    t.ca_cq[i] = make_uint4((unsigned)v, word, bits, (unsigned)raw);
+    // grid_avg8 (utils.h:18-23) of B in its order: 000 100 010 001 110 101 011 111
+    const double sum = __shfl(b, 0, 8) + __shfl(b, 1, 8) + __shfl(b, 2, 8) + __shfl(b, 4, 8) + __shfl(b, 3, 8) +
+                       __shfl(b, 5, 8) + __shfl(b, 6, 8) + __shfl(b, 7, 8);
+    if (k == 0) t.ca_bx[c] = ca2p_by_ext(ck, 0.125 * sum);
   }
 }
 
-// The new value of interior point (j, k, l), l < iz_bound, from buffer carr
-// and the sub-step's diff_u, with the point's voxel word and neighbour masks
-// from k_ca_corners.  The seven ATP loads do not depend on them; a point whose
-// top bit is set (a mask byte above 1) reads the word and masks itself.
-__device__ __forceinline__ double atp_point_pre(const Tis& t, const AtpK& ak, const double* __restrict__ carr,
-                                                const double* __restrict__ dfu, int j, int k, int l, uint2 pre) {
-  const int NX = t.NX, NY = t.NY, NZ = t.NZ;
-  const int px = j == 0 ? NX - 1 : j - 1, nx = j == NX - 1 ? 0 : j + 1;
-  const int py = k == 0 ? NY - 1 : k - 1, ny = k == NY - 1 ? 0 : k + 1;
-  const int pz = l == 0 ? 1 : l - 1, nz = l + 1 == NZ ? NZ - 1 : l + 1;
-  const long long v = gidx(t, j, k, l);
-  const long long vxm = gidx(t, px, k, l), vxp = gidx(t, nx, k, l);
-  const long long vym = gidx(t, j, py, l), vyp = gidx(t, j, ny, l);
-  const long long vzm = gidx(t, j, k, pz), vzp = gidx(t, j, k, nz);
-  const double c0 = carr[v], cxm = carr[vxm], cxp = carr[vxp], cym = carr[vym], cyp = carr[vyp], czm = carr[vzm],
-               czp = carr[vzp];
-  unsigned w;
+// The ATP value of a cell's corner `k` (binary x, y, z; its lane is k) after
+// the ATP update that runs beside this launch, computed from the buffer before
+// it (the grid kernel's expression, atp_new).  The corners of a cell are the
+// points of a cube, so three of a corner's six stencil neighbours are the
+// cube's other corners and come from their lanes; the other three, the point
+// itself and the owner's diff_u are loaded, without branches, so that the
+// loads of the cell's entries can be issued behind them.  A corner that the
+// update leaves alone takes its value from the buffer after it, in `ox`.
+struct Corner { double c0, ox, oy, oz, diffu; };
+__device__ __forceinline__ Corner corner_load(const CaArg& a, int k, uint4 q) {
+  const double* __restrict__ A = a.A0;
+  const long long v = q.x;
+  const unsigned f = q.z;
+  const bool hx = k & 1, hy = k & 2, hz = k & 4;
+  const int dx = hx ? ((f & CQ_XP) ? 1 - a.NX : 1) : ((f & CQ_XM) ? a.NX - 1 : -1);
+  const int wy = (a.NY - 1) * a.XP;   // a plane has fewer than 2^31 points (epi_create)
+  const int dy = hy ? ((f & CQ_YP) ? -wy : a.XP) : ((f & CQ_YM) ? wy : -a.XP);
+  const long long dz = hz ? ((f & CQ_ZP) ? 0 : a.PL) : ((f & CQ_ZM) ? a.PL : -a.PL);
+  const bool plain = f & CQ_PLAIN;
+  const unsigned cell1 = q.y & 0x7fffffffu;
+  Corner r;
+  r.c0 = A[v];
+  r.ox = *(plain ? a.A1 + v : A + v + dx);
+  r.oy = A[plain ? v : v + dy];
+  r.oz = A[plain ? v : v + dz];
+  r.diffu = a.dfo[cell1 ? cell1 - 1 : 0];
+  return r;
+}
+__device__ __forceinline__ double corner_value(const Tis& t, const CaArg& a, int k, uint4 q, const Corner& r) {
+  const unsigned f = q.z;
+  const bool hx = k & 1, hy = k & 2, hz = k & 4;
+  const double c0 = r.c0;
+  const double ix = __shfl_xor(c0, 1, 64), iy = __shfl_xor(c0, 2, 64), iz = __shfl_xor(c0, 4, 64);
+  // next_z(NZ - 1) is the point itself (utils.cpp:32-72); such a point is the
+  // upper corner (oz above) or, with its cell at the grid's top, the lower one
+  const double izn = !hz && (f & CQ_ZP) ? c0 : iz;
+  unsigned word = q.y;
+  double diffu = (word & 0x7fffffffu) ? r.diffu : 0.0;
   double m[6];
-  if (pre.y & 0x80000000u) {
-    const uint8_t* __restrict__ cm2 = t.cmap2;
-    w = t.vox[v];
-    m[0] = cm2[vxm]; m[1] = cm2[vxp]; m[2] = cm2[vym]; m[3] = cm2[vyp]; m[4] = cm2[vzm]; m[5] = cm2[vzp];
-  } else {
-    w = pre.x;
 #pragma unroll
-    for (int b = 0; b < 6; b++) m[b] = (double)((pre.y >> b) & 1);
+  for (int b = 0; b < 6; b++) m[b] = (double)((f >> b) & 1);
+  if (f & CQ_SLOW) {
+    const uint8_t* __restrict__ cm2 = a.cm2;
+    const long long v = q.x, wy = (long long)(a.NY - 1) * a.XP;
+    m[0] = cm2[v + ((f & CQ_XM) ? a.NX - 1 : -1)];
+    m[1] = cm2[v + ((f & CQ_XP) ? 1 - a.NX : 1)];
+    m[2] = cm2[v + ((f & CQ_YM) ? wy : -(long long)a.XP)];
+    m[3] = cm2[v + ((f & CQ_YP) ? -wy : a.XP)];
+    m[4] = cm2[v + ((f & CQ_ZM) ? a.PL : -a.PL)];
+    m[5] = cm2[v + ((f & CQ_ZP) ? 0 : a.PL)];
   }
-  const unsigned cell1 = w & 0x7fffffffu;
-  const double diffu = cell1 ? dfu[cell1 - 1] : 0.0;
-  return atp_new(ak, c0, cxm, cxp, cym, cyp, czm, czp, m[0], m[1], m[2], m[3], m[4], m[5], diffu, (double)(w >> 31),
-                 t.inv_dx);
+  const double nv = atp_new(atp_k(t.prm), c0, hx ? ix : r.ox, hx ? r.ox : ix, hy ? iy : r.oy, hy ? r.oy : iy,
+                            hz ? iz : r.oz, hz ? r.oz : izn, m[0], m[1], m[2], m[3], m[4], m[5], diffu,
+                            (double)(word >> 31), t.inv_dx);
+  return (f & CQ_PLAIN) ? r.ox : nv;
 }
 
-// dead_IP3_calc (:156-173) and supra_calc (:182-222).  A group of CG lanes
-// (4, 8 or 16, set by the autotuner) owns one cell: lanes evaluate the
-// gap-junction terms of the list entries (and update gj toward ALIVE
-// neighbours) 16 (CG 16: 32) entries at a time and load the 16 grid corners
-// of the two grid_avg8; the leader sums them in list / corner order.  Each
-// group takes one cell, so the grid must cover every cell past the membrane
-// and dermis (a launch that does not is reported as ERR_INVALID); a loop over
-// cells would keep loop-invariant constants of the math in registers for
-// the whole kernel and cost a wave per SIMD.  Every lane issues
-// all loads of its entries of a chunk (list word, gj, then the neighbours'
-// Ca2+ and IP3 pair) before it uses any of them.  With carr_prev set, the ATP
-// corners are not read but computed from the previous sub-step's buffer
-// (atp_point_pre), the ATP update of that sub-step running beside this one.
-// With sv set (a reaction-diffusion window's reverse pass), the cell also
+// dead_IP3_calc (:156-173) and supra_calc (:182-222).  A group of CG lanes (8
+// or 16) owns one cell: lanes evaluate the gap-junction terms of the packed
+// coupled entries (and update gj toward ALIVE neighbours) 32 at a time, and the
+// first eight take one grid_avg8 corner of ATP each; two lanes sum the
+// terms in list order, one the Ca2+ and one the IP3 side.  Each group takes
+// one cell, so the grid must cover every cell past the membrane and dermis (a
+// launch that does not is reported as ERR_INVALID); a loop over cells would
+// keep loop-invariant constants of the math in registers for the whole kernel
+// and cost a wave per SIMD.
+//
+// What bounds it: the chain of round trips through the Infinity Cache (what
+// the other XCDs wrote is in no local L2 after a launch) and, on a large
+// tissue, the cache lines its gathers touch.  So everything that depends on
+// the cell alone is loaded in the first round trip (a lane each for the six
+// per-cell values), the entries' pairs and the corners' neighbours in the
+// second, and nothing after them; gj sits beside the entries instead of in the
+// list row's slots; the quotients of the reaction terms that depend on the
+// cell alone are one division, a lane each, while the gathers fly, and the two
+// that do not are another one.  Per fused sub-step, against the same split
+// with the row's slots, B read anew, all corners read by every lane and a
+// leader's own loads and divisions (8 lanes, one-plane tiles): 17,500 AFM
+// cells 11.3 -> 10.2 us, 700 cells 7.1 -> 5.7 us (with 16 lanes 6.4 -> 5.6, and
+// 11.3 on the large tissue, so 8 is the default).
+//
+// With REC, the ATP corners are computed from the buffer before the ATP update
+// that runs beside this launch (corner_recomputed), else read.
+// With SAVE (a reaction-diffusion window's reverse pass), the cell also
 // writes what the reverse sub-step reads of the state before it into segment
 // slot `slot`: ca2p and IP3 (AFM and DEAD cells), ex_inert, the ATP
 // grid_avg8 and the gj of its coupled entries (AFM cells).
 constexpr int C_BLOCK = 128;
 
-template <int CG, int NT>
-__device__ __forceinline__ void ca_cells_part(const Tis& t, unsigned bx, unsigned nbx, int cb, int cp, int ap, int bp,
-                                              const double* __restrict__ carr_prev,
-                                              const double* __restrict__ dfu_prev,
-                                              const RdTis* __restrict__ sv = nullptr, int slot = 0) {
-  constexpr int C_GROUPS = NT / CG;
-  constexpr int EPL = CG >= 8 ? 2 : 4;   // entries per lane per chunk
-  constexpr int CCAP = EPL * CG;    // list entries per chunk
-  constexpr int NQ = 16 / CG;       // grid corners per lane
-  // per-entry terms for the leader; rows padded by 16 bytes so that the
-  // leaders of a wave's groups read different LDS banks
+template <int CG, bool REC, bool SAVE>
+__device__ __forceinline__ void ca_cells_part(const Tis& t, const CaArg& a, unsigned bx, unsigned nbx,
+                                              const RdTis* __restrict__ sv, int slot) {
+  constexpr int C_GROUPS = C_BLOCK / CG;
+  constexpr int CCAP = 32;          // entries per chunk: more than nearly every cell has
+  constexpr int EPL = CCAP / CG;    // of them per lane
+  // per-entry terms for the summing lanes, corners, and the per-cell values
+  // and quotients; rows padded so that the groups of a wave read different banks
   __shared__ double2 s_a[C_GROUPS][CCAP + 1];
-  __shared__ double s_g[C_GROUPS][17];
+  __shared__ double s_g[C_GROUPS][9];
+  __shared__ double s_v[C_GROUPS][11];
   const int lane = threadIdx.x & (CG - 1);
   const int grp = threadIdx.x / CG;
-  const double2* __restrict__ up = t.ca_up[cp];
-  double2* __restrict__ up_next = t.ca_up[1 - cp];
-  double* __restrict__ dfu_out = dfu_buf(t, cp);
-  const int start = t.nmemb + t.nder;
-  const int c = start + bx * C_GROUPS + grp;
-  if (c >= t.cap) return;
+  const int c = a.start + bx * C_GROUPS + grp;
+  if (c >= a.cap) return;
+  // First round trip: the cell's own words, its first chunk's entries and its
+  // corners' words, beside the cell count (a device value).  A cell past the
+  // count reads allocated, stale slots and leaves once the count is in; a row
+  // holds ns >= CCAP slots, and entries past len are masked.
+  const uint8_t s = a.state[c];
+  const int len = a.cn[c];
+  const double2 uc = a.up[c];
+  const size_t row = (size_t)c * a.ns;
+  int en[EPL];
+  double gv[EPL];
+#pragma unroll
+  for (int i = 0; i < EPL; i++) { en[i] = a.w[row + lane + i * CG]; gv[i] = a.g[row + lane + i * CG]; }
+  uint4 q = a.cq[8 * (size_t)c + (lane & 7)];
+  const double* __restrict__ vp =
+      lane == 0 ? a.th : lane == 1 ? a.kpa : lane == 2 ? a.iag : lane == 3 ? a.bx : lane == 4 ? a.exi : a.avg;
+  const double val = vp[c];
+  const int n = a.st->n;
+  if (bx == 0 && threadIdx.x == 0 && a.start + (long long)nbx * C_GROUPS < n) set_err(t.st, ERR_INVALID);
+  if (c >= n) return;
+  const bool dead = s == DEAD;
+  if (!dead && !is_afm(s)) return;
+  // Second round trip: the corners' points and the entries' pairs.  A DEAD
+  // cell has no corners (its words may never have been written): point 0, as
+  // it lies.
+  if (dead) q = make_uint4(0u, 0u, CQ_PLAIN, 0u);
+  Corner cr;
+  double raw = 0;
+  if (REC) cr = corner_load(a, lane & 7, q);
+  else raw = a.A0[q.w];
+  double2 w[EPL];
+#pragma unroll
+  for (int i = 0; i < EPL; i++) w[i] = a.up[lane + i * CG < len ? en[i] >> 2 : c];
   const CaK ck = ca_k(t.prm);
-  const AtpK ak = atp_k(t.prm);
-  {
-    // The cell's own words are loaded before the cell count and iz_bound
-    // (device values) arrive, in one round trip with them: a cell past the
-    // count reads allocated, stale slots and leaves once the count is in.
-    const uint8_t s = t.state[c];
-    // the coupled entries only, in list order: an entry that is skipped
-    // would add +0.0 to the sums, which leaves them as they are
-    const int len = t.ca_cn[c];
-    const double2 uc = up[c];
-    const double u = uc.x, p = uc.y;
-    // the first chunk's entries do not wait for len: a row holds ns >= CCAP
-    // slots, and slots past len are masked once len has arrived
-    const int2* ent = t.ca_ce + (size_t)c * t.ns;
-    double* g = t.gj[cb] + (size_t)c * t.ns;
-    int2 en0[EPL];
+  const double ca_du = t.ca_du, ca_dp = t.ca_dp;
+  const double u = uc.x, p = uc.y;
+  // meanwhile, the quotients that depend on the cell alone (:36-87, :128-136),
+  // a lane each
+  const double k2 = ck.para_k2 * ck.para_k2;
+  const double num = lane == 0 ? ck.mu1 * p : lane == 1 ? ck.para_bb * u : lane == 2 ? ck.gamma * u : k2;
+  const double den = lane == 0 ? p + ck.kmu : lane == 1 ? ck.para_k1 + u : lane == 2 ? ck.kg + u : k2 + u * u;
+  const double quo = num / den;
+  if (lane < 6) s_v[grp][lane] = val;
+  if (lane < 4) s_v[grp][6 + lane] = quo;
+  const double cv = REC ? corner_value(t, a, lane & 7, q, cr) : raw;
+  if (lane < 8) s_g[grp][lane] = cv;
+  double acc = 0;   // lane 0: the Ca2+ sum, lane 1: the IP3 sum (DEAD: lane 1 IP3, lane 0 the ALIVE count)
+  for (int e0 = 0; e0 < len; e0 += CCAP) {
+    const int m = min(CCAP, len - e0);
+    if (e0 > 0) {
 #pragma unroll
-    for (int i = 0; i < EPL; i++) en0[i] = ent[lane + i * CG];
-    // the lattice position is fetched now too, so the corner gathers start
-    // one round trip earlier
-    const int lx = t.lat[3 * c], ly = t.lat[3 * c + 1], lz = t.lat[3 * c + 2];
-    // the corners' per-solve words depend on c only
-    uint2 pre[NQ];
-#pragma unroll
-    for (int j = 0; j < NQ; j++) {
-      const int q = lane + j * CG;
-      pre[j] = q >= 8 ? t.ca_cq[8 * (size_t)c + (q & 7)] : make_uint2(0u, 0u);
-    }
-    const int n = t.st->n;
-    const int izb = carr_prev ? ca_iz_bound(t) : 0;
-    const bool recompute = carr_prev && izb <= t.NZ;
-    if (bx == 0 && threadIdx.x == 0 && start + (long long)nbx * C_GROUPS < n) set_err(t.st, ERR_INVALID);
-    if (c >= n) return;
-    const bool dead = s == DEAD;
-    if (!dead && !is_afm(s)) return;
-    if (dead) {
-      int count = 0;
-      double tmp = 0;
-      for (int e0 = 0; e0 < len; e0 += CCAP) {
-        const int m = min(CCAP, len - e0);
-        int en[EPL];
-        double po[EPL];
-#pragma unroll
-        for (int i = 0; i < EPL; i++) {
-          const int e = lane + i * CG;
-          en[i] = e < m ? (e0 == 0 ? en0[i] : ent[e0 + e]).x : 0;
-        }
-#pragma unroll
-        for (int i = 0; i < EPL; i++) po[i] = (en[i] & 3) == 3 ? up[en[i] >> 2].y : 0.0;
-#pragma unroll
-        for (int i = 0; i < EPL; i++) {
-          const int e = lane + i * CG;
-          if (e < m) s_a[grp][e] = make_double2(po[i], (en[i] & 3) == 3 ? 1.0 : 0.0);
-        }
-        wave_sync();
-        // adding the +0.0 of an entry that is not ALIVE leaves tmp as it is
-        // (tmp starts at +0.0, so it is never -0.0)
-        if (lane == 0) {
-          int e = 0;
-          for (; e + 4 <= m; e += 4) {
-            double2 a[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) a[j] = s_a[grp][e + j];
-#pragma unroll
-            for (int j = 0; j < 4; j++) { tmp += a[j].x; count += a[j].y != 0.0; }
-          }
-          for (; e < m; e++) { const double2 a = s_a[grp][e]; tmp += a.x; count += a.y != 0.0; }
-        }
-        wave_sync();
+      for (int i = 0; i < EPL; i++) {
+        const int e = lane + i * CG;
+        en[i] = e < m ? a.w[row + e0 + e] : 0;
+        gv[i] = e < m ? a.g[row + e0 + e] : 0.0;
       }
-      if (lane == 0) {
-        if (sv) {
-          sv->su[slot * (size_t)t.cap + c] = u;
-          sv->sp[slot * (size_t)t.cap + c] = p;
-        }
-        const double np = p + ck.DT_Ca * (t.ca_dp * (tmp - count * p) - ck.Kpp * p);
-        t.ip3[1 - cp][c] = np;
-        reinterpret_cast<double*>(up_next + c)[1] = np;   // ca2p of a DEAD cell stays as it is
-      }
-      return;
-    }
-    // the corners of grid_avg8 (utils.h:18-23; slots 0-7 B, 8-15 ATP) are
-    // fetched now, beside the list loads
-    double cq[NQ];
-    {
 #pragma unroll
-      for (int j = 0; j < NQ; j++) {
-        const int q = lane + j * CG;
-        const int k = q & 7;
-        const int ix = lx + ((k == 1 || k == 4 || k == 5 || k == 7) ? 1 : 0);
-        const int iy = ly + ((k == 2 || k == 4 || k == 6 || k == 7) ? 1 : 0);
-        const int iz = lz + ((k == 3 || k == 5 || k == 6 || k == 7) ? 1 : 0);
-        if (q < 8) {
-          cq[j] = t.bf[bp][gidx(t, ix, iy, iz)];
-        } else if (recompute && iz < izb) {
-          // the periodic copies x = NX, y = NY hold the values of x = 0, y = 0
-          cq[j] = atp_point_pre(t, ak, carr_prev, dfu_prev, ix == t.NX ? 0 : ix, iy == t.NY ? 0 : iy, iz, pre[j]);
-        } else if (recompute) {
-          // plane iz_bound is never updated inside a solve; its copies are
-          // written beside this launch, so read the value they copy
-          cq[j] = t.atp[ap][gidx(t, ix == t.NX ? 0 : ix, iy == t.NY ? 0 : iy, iz)];
+      for (int i = 0; i < EPL; i++) w[i] = a.up[lane + i * CG < m ? en[i] >> 2 : c];
+    }
+#pragma unroll
+    for (int i = 0; i < EPL; i++) {
+      const int e = lane + i * CG;
+      if (e < m) {
+        const bool alive = (en[i] & 3) == 3;
+        if (dead) {
+          // adding the +0.0 of an entry that is not ALIVE leaves the sums as
+          // they are (they start at +0.0, so neither is ever -0.0)
+          s_a[grp][e] = alive ? make_double2(1.0, w[i].y) : make_double2(0.0, 0.0);
         } else {
-          cq[j] = t.atp[ap][gidx(t, ix, iy, iz)];
+          s_a[grp][e] = make_double2(gv[i] * (w[i].x - u), gv[i] * (w[i].y - p));
+          if (SAVE) sv->sg[(size_t)slot * a.cap * a.ns + row + e0 + e] = gv[i];
+          if (alive) a.g[row + e0 + e] = gv[i] + ck.DT_Ca * fw_term(ck.wd, fabs(w[i].x - u), gv[i]);
         }
       }
     }
-    double tmp_diffu = 0, tmp_IP3 = 0;
-    for (int e0 = 0; e0 < len; e0 += CCAP) {
-      const int m = min(CCAP, len - e0);
-      int en[EPL], sl[EPL];
-      double gv[EPL];
-      double2 w[EPL];
-#pragma unroll
-      for (int i = 0; i < EPL; i++) {
-        const int e = lane + i * CG;
-        const int2 x = e < m ? (e0 == 0 ? en0[i] : ent[e0 + e]) : make_int2(0, 0);
-        en[i] = x.x;
-        sl[i] = x.y;
-      }
-#pragma unroll
-      for (int i = 0; i < EPL; i++) {
-        gv[i] = (en[i] & 3) ? g[sl[i]] : 0.0;
-        w[i] = (en[i] & 3) ? up[en[i] >> 2] : make_double2(0.0, 0.0);
-      }
-#pragma unroll
-      for (int i = 0; i < EPL; i++) {
-        const int e = lane + i * CG;
-        if (e < m) {
-          const int kd = en[i] & 3;
-          double a1 = 0, a2 = 0;
-          if (kd) {
-            if (sv) sv->sg[(slot * (size_t)t.cap + c) * t.ns + sl[i]] = gv[i];
-            a1 = gv[i] * (w[i].x - u);
-            a2 = gv[i] * (w[i].y - p);
-            if (kd == 3) g[sl[i]] = gv[i] + ck.DT_Ca * fw_term(ck.wd, fabs(w[i].x - u), gv[i]);
-          }
-          s_a[grp][e] = make_double2(a1, a2);
-        }
-      }
-      wave_sync();
-      // the leader adds in list order, four entries' LDS reads ahead of their
-      // adds.  A skipped entry adds +0.0, which leaves the sums as they are
-      // (they start at +0.0, so neither is ever -0.0).
-      if (lane == 0) {
-        int e = 0;
-        for (; e + 4 <= m; e += 4) {
-          double2 a[4];
-#pragma unroll
-          for (int j = 0; j < 4; j++) a[j] = s_a[grp][e + j];
-#pragma unroll
-          for (int j = 0; j < 4; j++) { tmp_diffu += a[j].x; tmp_IP3 += a[j].y; }
-        }
-        for (; e < m; e++) { const double2 a = s_a[grp][e]; tmp_diffu += a.x; tmp_IP3 += a.y; }
-      }
-      wave_sync();
-    }
-#pragma unroll
-    for (int j = 0; j < NQ; j++) s_g[grp][lane + j * CG] = cq[j];
     wave_sync();
-    if (lane == 0) {
-      const double exi = t.ex_inert[c], avg = t.ca2p_avg[c], _th = t.ca_th[c], _Kpa = t.ca_kpa[c],
-                   IAGv = t.ca_iag[c];
-      const double ca2p_du = t.ca_du;
-      const double* q = s_g[grp];
-      const double Bavg = 0.125 * (q[0] + q[1] + q[2] + q[3] + q[4] + q[5] + q[6] + q[7]);
-      const double Aavg = 0.125 * (q[8] + q[9] + q[10] + q[11] + q[12] + q[13] + q[14] + q[15]);
-      if (sv) {
-        const size_t k = slot * (size_t)t.cap + c;
-        sv->su[k] = u;
-        sv->sp[k] = p;
-        sv->sh[k] = exi;
-        sv->sAv[k] = Aavg;
+    // in list order, four entries' LDS reads ahead of their adds
+    if (lane < 2) {
+      const double* v = reinterpret_cast<const double*>(s_a[grp]) + lane;
+      int e = 0;
+      for (; e + 4 <= m; e += 4) {
+        double d[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) d[j] = v[2 * (e + j)];
+#pragma unroll
+        for (int j = 0; j < 4; j++) acc += d[j];
       }
-      const double diff_u = ca2p_reaction_factor(ck, u, exi, p, Bavg) + ca2p_du * IAGv * tmp_diffu;
-      dfu_out[c] = diff_u;
-      const double H0 = ck.H0, DT_Ca = ck.DT_Ca;
-      const double np = p + DT_Ca * ((_Kpa * Aavg / (H0 + Aavg) - ck.Kpp * p) + t.ca_dp * IAGv * tmp_IP3);
-      t.ip3[1 - cp][c] = np;
-      const double cs = u + DT_Ca * diff_u;
-      t.ca2p[1 - cp][c] = cs;
-      up_next[c] = make_double2(cs, np);
-      t.ca2p_avg[c] = avg + cs;
-      const double para_k2 = ck.para_k2;
-      t.ex_inert[c] = exi + DT_Ca * ((para_k2 * para_k2 / (para_k2 * para_k2 + u * u) - exi) / _th);
+      for (; e < m; e++) acc += v[2 * e];
     }
     wave_sync();
   }
+  if (dead) {
+    const double count = __shfl(acc, 0, CG);
+    if (lane == 1) {
+      if (SAVE) {
+        sv->su[slot * (size_t)a.cap + c] = u;
+        sv->sp[slot * (size_t)a.cap + c] = p;
+      }
+      // ca2p of a DEAD cell stays as it is
+      reinterpret_cast<double*>(a.upn + c)[1] = p + ck.DT_Ca * (ca_dp * (acc - count * p) - ck.Kpp * p);
+    }
+    return;
+  }
+  wave_sync();
+  if (lane >= 3) return;
+  const double* g = s_g[grp];
+  const double* v = s_v[grp];
+  // grid_avg8 in its order: 000 100 010 001 110 101 011 111
+  const double Aavg = 0.125 * (g[0] + g[1] + g[2] + g[4] + g[3] + g[5] + g[6] + g[7]);
+  const double exi = v[4];
+  const double late = (lane == 2 ? v[9] - exi : v[1] * Aavg) / (lane == 2 ? v[0] : ck.H0 + Aavg);
+  if (lane == 0) {
+    const double er1 = ck.mu0 + v[6], er2 = ck.para_b + v[7];
+    const double diff_u = ck.k_flux * er1 * er2 * exi - v[8] + ck.leak_from_storage + v[3] + ca_du * v[2] * acc;
+    a.dfn[c] = diff_u;
+    const double cs = u + ck.DT_Ca * diff_u;
+    a.upn[c].x = cs;
+    a.avg[c] = v[5] + cs;
+  } else if (lane == 1) {
+    a.upn[c].y = p + ck.DT_Ca * ((late - ck.Kpp * p) + ca_dp * v[2] * acc);
+  } else {
+    a.exi[c] = exi + ck.DT_Ca * late;
+    if (SAVE) {
+      const size_t k = slot * (size_t)a.cap + c;
+      sv->su[k] = u;
+      sv->sp[k] = p;
+      sv->sh[k] = exi;
+      sv->sAv[k] = Aavg;
+    }
+  }
 }
 
-template <int CG>
-__global__ void __launch_bounds__(C_BLOCK) k_ca_cells(const Tis* __restrict__ T, CaList cl, int cb, int cp,
-                                                      int ap, int bp, int xcd, const RdTis* __restrict__ sv,
-                                                      int slot) {
+template <int CG, bool ONE, bool SAVE>
+__global__ void __launch_bounds__(C_BLOCK) k_ca_cells(const Tis* __restrict__ T, CaList cl, CaArg one, int cp, int ap,
+                                                      int xcd, const RdTis* __restrict__ sv, int slot) {
   const unsigned b = xcd_order(blockIdx.x, gridDim.x, xcd);
-  const int4 e = cl.ntis == 1 ? make_int4(cl.t0, (int)b, cl.ncb, 0) : cl.cmap[b];
-  const Tis& t = T[e.x];
-  ca_cells_part<CG, C_BLOCK>(t, e.y, e.z, cb, cp, ap, bp, nullptr, nullptr, sv ? sv + e.x : nullptr, slot);
+  if (ONE) {
+    ca_cells_part<CG, false, SAVE>(T[cl.t0], one, b, cl.ncb, SAVE ? sv + cl.t0 : nullptr, slot);
+  } else {
+    const int4 e = cl.cmap[b];
+    ca_cells_part<CG, false, SAVE>(T[e.x], ca_arg(T[e.x], cp, cp, ap), e.y, e.z, SAVE ? sv + e.x : nullptr, slot);
+  }
 }
 
 // ATP_refresh (:302-338) with the periodic copies of planes 0..iz_bound,
@@ -871,13 +912,13 @@ __global__ void __launch_bounds__(C_BLOCK) k_ca_cells(const Tis* __restrict__ T,
 // each plane's voxel word), then the owners' diff_u, then ATP_refresh's
 // point update (atp_new) per plane.
 template <int ZB>
-__device__ __forceinline__ void atp_column(const Tis& t, int j, int k, int l0, int l1, int ap, int cp) {
+__device__ __forceinline__ void atp_column(const Tis& ti, const CaArg& t, int j, int k, int l0, int l1) {
   const int NX = t.NX, NY = t.NY, NZ = t.NZ;
-  const AtpK ak = atp_k(t.prm);
-  const double* __restrict__ carr = t.atp[ap];
-  double* __restrict__ narr = t.atp[1 - ap];
-  const double* __restrict__ dfu = dfu_buf(t, cp);
-  const uint8_t* __restrict__ cm2 = t.cmap2;
+  const AtpK ak = atp_k(ti.prm);
+  const double* __restrict__ carr = t.A0;
+  double* __restrict__ narr = t.A1;
+  const double* __restrict__ dfu = t.dfo;
+  const uint8_t* __restrict__ cm2 = t.cm2;
   const int prev_x = j == 0 ? NX - 1 : j - 1, next_x = j == NX - 1 ? 0 : j + 1;
   const int prev_y = k == 0 ? NY - 1 : k - 1, next_y = k == NY - 1 ? 0 : k + 1;
   const long long PL = t.PL;
@@ -919,7 +960,7 @@ __device__ __forceinline__ void atp_column(const Tis& t, int j, int k, int l0, i
     const unsigned cell1 = w[q] & 0x7fffffffu;
     diffu[q] = cell1 ? dfu[cell1 - 1] : 0.0;
   }
-  const double inv_dx = t.inv_dx;
+  const double inv_dx = ti.inv_dx;
 #pragma unroll
   for (int q = 0; q < ZB; q++) {
     if (q < nl) {
@@ -938,16 +979,16 @@ __device__ __forceinline__ void atp_column(const Tis& t, int j, int k, int l0, i
 // The same column rolling through registers plane by plane (as
 // b_column_roll), for tall tiles; the voxel word is read one plane ahead, so
 // a plane waits for one round trip (its owner's diff_u), not two.
-__device__ __forceinline__ void atp_column_roll(const Tis& t, int j, int k, int l0, int l1, int ap, int cp) {
+__device__ __forceinline__ void atp_column_roll(const Tis& ti, const CaArg& t, int j, int k, int l0, int l1) {
   const int NX = t.NX, NY = t.NY, NZ = t.NZ;
-  const AtpK ak = atp_k(t.prm);
-  const double* __restrict__ carr = t.atp[ap];
-  double* __restrict__ narr = t.atp[1 - ap];
-  const double* __restrict__ dfu = dfu_buf(t, cp);
-  const uint8_t* __restrict__ cm2 = t.cmap2;
+  const AtpK ak = atp_k(ti.prm);
+  const double* __restrict__ carr = t.A0;
+  double* __restrict__ narr = t.A1;
+  const double* __restrict__ dfu = t.dfo;
+  const uint8_t* __restrict__ cm2 = t.cm2;
   const int prev_x = j == 0 ? NX - 1 : j - 1, next_x = j == NX - 1 ? 0 : j + 1;
   const int prev_y = k == 0 ? NY - 1 : k - 1, next_y = k == NY - 1 ? 0 : k + 1;
-  const double inv_dx = t.inv_dx;
+  const double inv_dx = ti.inv_dx;
   const long long PL = t.PL;
   const long long cxy = gidx(t, j, k, 0);
   const int pz = l0 == 0 ? 1 : l0 - 1;   // mirror z (utils.cpp:32-72)
@@ -995,7 +1036,7 @@ __device__ __forceinline__ void atp_column_roll(const Tis& t, int j, int k, int 
 // one tile of a solve's list: blockDim.x consecutive points of the (x, y)
 // plane times ZB planes (atp_column up to 2 planes, atp_column_roll above).
 template <int ZB>
-__device__ __forceinline__ void atp_tile(const Tis& t, int local, int izb, int ap, int cp) {
+__device__ __forceinline__ void atp_tile(const Tis& ti, const CaArg& t, int local, int izb) {
   const int NX = t.NX, NY = t.NY;
   const int bs = blockDim.x;
   const int plane = NX * NY;
@@ -1004,12 +1045,12 @@ __device__ __forceinline__ void atp_tile(const Tis& t, int local, int izb, int a
   if (p >= plane) return;
   const int j = p % NX, k = p / NX;
   const int l0 = (local / npt) * ZB;
-  if (ZB >= 4) atp_column_roll(t, j, k, l0, min(l0 + ZB, izb), ap, cp);
-  else atp_column<ZB>(t, j, k, l0, min(l0 + ZB, izb), ap, cp);
+  if (ZB >= 4) atp_column_roll(ti, t, j, k, l0, min(l0 + ZB, izb));
+  else atp_column<ZB>(ti, t, j, k, l0, min(l0 + ZB, izb));
   // plane l = iz_bound: copies of values left in the next buffer (:334-337);
   // the corner (NX, NY) ends as a copy of (0, 0)
   if (l0 == 0) {
-    double* __restrict__ narr = t.atp[1 - ap];
+    double* __restrict__ narr = t.A1;
     if (k == 0) narr[gidx(t, j, NY, izb)] = narr[gidx(t, j, 0, izb)];
     if (j == 0) narr[gidx(t, NX, k, izb)] = narr[gidx(t, 0, k, izb)];
     if (j == 0 && k == 0) narr[gidx(t, NX, NY, izb)] = narr[gidx(t, 0, 0, izb)];
@@ -1021,15 +1062,16 @@ __device__ __forceinline__ void atp_tile(const Tis& t, int local, int izb, int a
 // and tissue ids of up to CA_LDS_T tissues are staged in LDS (kept small: the
 // fused kernel's cell blocks hold LDS of their own)
 constexpr int CA_LDS_T = 256;
-template <int ZB>
-__device__ __forceinline__ void atp_walk(const Tis* __restrict__ T, const CaList& cl, int b, int nb, int xcd,
-                                         int ap, int cp) {
-  const int nt = cl.ntis;
-  if (nt == 1) {   // one tissue: its id and iz_bound come with the list
+template <int ZB, bool ONE>
+__device__ __forceinline__ void atp_walk(const Tis* __restrict__ T, const CaList& cl, int b, int nb, int xcd, int ap,
+                                         int cp) {
+  if (ONE) {   // one tissue: its id and iz_bound come with the list
     const Tis& t = T[cl.t0];
-    for (TileWalk tw(cl.atiles, xcd, b, nb); tw.w < tw.end; tw.w += tw.stride) atp_tile<ZB>(t, tw.w, cl.izb0, ap, cp);
+    const CaArg a = ca_arg(t, cp, cp, ap);
+    for (TileWalk tw(cl.atiles, xcd, b, nb); tw.w < tw.end; tw.w += tw.stride) atp_tile<ZB>(t, a, tw.w, cl.izb0);
     return;
   }
+  const int nt = cl.ntis;
   __shared__ int s_off[CA_LDS_T + 1];
   __shared__ int2 s_ti[CA_LDS_T];
   const bool lds = nt <= CA_LDS_T;
@@ -1046,14 +1088,14 @@ __device__ __forceinline__ void atp_walk(const Tis* __restrict__ T, const CaList
     // uniform over the block (see k_ext_stim)
     ti = __builtin_amdgcn_readfirstlane(wl_find(off, ti, nt, tw.w));
     const int2 q = lds ? s_ti[ti] : make_int2(cl.atis[ti], cl.aizb[ti]);
-    atp_tile<ZB>(T[__builtin_amdgcn_readfirstlane(q.x)], tw.w - __builtin_amdgcn_readfirstlane(off(ti)),
-                 __builtin_amdgcn_readfirstlane(q.y), ap, cp);
+    const Tis* t = T + __builtin_amdgcn_readfirstlane(q.x);
+    atp_tile<ZB>(*t, ca_arg(*t, cp, cp, ap), tw.w - __builtin_amdgcn_readfirstlane(off(ti)), __builtin_amdgcn_readfirstlane(q.y));
   }
 }
 
-template <int ZB>
+template <int ZB, bool ONE>
 __global__ void __launch_bounds__(256) k_atp(const Tis* __restrict__ T, CaList cl, int ap, int cp, int xcd) {
-  atp_walk<ZB>(T, cl, blockIdx.x, gridDim.x, xcd, ap, cp);
+  atp_walk<ZB, ONE>(T, cl, blockIdx.x, gridDim.x, xcd, ap, cp);
 }
 
 // one launch for the ATP update of sub-step i (parities cp, ap) and the cells
@@ -1067,9 +1109,9 @@ __global__ void __launch_bounds__(256) k_atp(const Tis* __restrict__ T, CaList c
 // unevenly loaded).  Results do not depend on it.
 constexpr int F_BLOCK = 128;
 
-template <int CG, int ZB>
-__global__ void __launch_bounds__(F_BLOCK) k_ca_fused(const Tis* __restrict__ T, CaList cl, int cb, int cp,
-                                                      int ap, int bp, int ncb, int xcd) {
+template <int CG, int ZB, bool ONE, bool SAVE>
+__global__ void __launch_bounds__(F_BLOCK) k_ca_fused(const Tis* __restrict__ T, CaList cl, CaArg one, int cp, int ap,
+                                                      int ncb, int xcd, const RdTis* __restrict__ sv, int slot) {
   int cbk = -1;   // this block's cell block, or -1 for an ATP block
   int ab = 0, an = 0;
   if (xcd) {
@@ -1087,29 +1129,49 @@ __global__ void __launch_bounds__(F_BLOCK) k_ca_fused(const Tis* __restrict__ T,
     ab = (int)blockIdx.x - ncb;
     an = (int)gridDim.x - ncb;
   }
-  if (cbk >= 0) {
-    const int4 e = cl.ntis == 1 ? make_int4(cl.t0, cbk, ncb, 0) : cl.cmap[cbk];
-    const Tis& t = T[e.x];
-    ca_cells_part<CG, F_BLOCK>(t, e.y, e.z, cb, 1 - cp, 1 - ap, bp, t.atp[ap], dfu_buf(t, cp));
+  if (cbk < 0) {
+    atp_walk<ZB, ONE>(T, cl, ab, an, xcd, ap, cp);
+  } else if (ONE) {
+    ca_cells_part<CG, true, SAVE>(T[cl.t0], one, cbk, ncb, SAVE ? sv + cl.t0 : nullptr, slot);
   } else {
-    atp_walk<ZB>(T, cl, ab, an, xcd, ap, cp);
+    const int4 e = cl.cmap[cbk];
+    ca_cells_part<CG, true, SAVE>(T[e.x], ca_arg(T[e.x], 1 - cp, cp, ap), e.y, e.z, SAVE ? sv + e.x : nullptr, slot);
   }
 }
 
-__global__ void __launch_bounds__(256) k_ca_end(const Tis* __restrict__ T, const int* tlist, int full) {
+// The packed gj back into the list rows and the (ca2p, IP3) pairs into their
+// arrays; at the end of a solve (ca2p.cpp:400-402) also the averages divided
+// and the cells past the membrane and dermis that are not AFM cleared.
+__global__ void __launch_bounds__(256) k_ca_end(const Tis* __restrict__ T, const int* tlist, int cb, int what) {
   const Tis& t = T[tlist ? tlist[blockIdx.y] : blockIdx.y];
   const int n = t.st->n;
   const int Ca_ITR = t.prm.Ca_ITR;
-  for (int c = t.nmemb + t.nder + blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
-    if (!full) {
-    } else if (is_afm(t.state[c])) {
-      t.ca2p_avg[c] = t.ca2p_avg[c] / Ca_ITR;
-    } else {
-      t.ca2p_avg[c] = 0;
-      t.ca2p[0][c] = 0;
-      t.ca2p[1][c] = 0;
+  const int lane = threadIdx.x & (BL - 1);
+  for (int c = t.nmemb + t.nder + (blockIdx.x * blockDim.x + threadIdx.x) / BL; c < n;
+       c += gridDim.x * blockDim.x / BL) {
+    const size_t at = (size_t)c * t.ns;
+    const uint8_t s = t.state[c];
+    const int k = t.ca_cn[c];
+    for (int e = lane; e < k; e += BL) t.gj[cb][at + t.ca_sl[at + e]] = t.ca_g[at + e];
+    if (lane != 0) continue;
+    const bool afm = is_afm(s);
+    if (afm || s == DEAD) {
+      for (int b = 0; b < 2; b++) {
+        const double2 w = t.ca_up[b][c];
+        t.ca2p[b][c] = w.x;
+        t.ip3[b][c] = w.y;
+      }
     }
-    t.diff_u[c] = 0;
+    if (what == CA_END_SOLVE) {
+      if (afm) {
+        t.ca2p_avg[c] = t.ca2p_avg[c] / Ca_ITR;
+      } else {
+        t.ca2p_avg[c] = 0;
+        t.ca2p[0][c] = 0;
+        t.ca2p[1][c] = 0;
+      }
+    }
+    if (what != CA_END_PUT) t.diff_u[c] = 0;
   }
 }
 
@@ -1202,39 +1264,58 @@ void launch_ext_stim(hipStream_t s, const Tis* dT, int ntis, int bp, long long t
   });
 }
 
-static void ca_maps(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int max_n, long long max_box,
-                    int zero_avg) {
-  EPI_LAUNCH(K_CA_BEGIN, k_ca_begin, dim3((max_n + 255) / 256, ntis), dim3(256), 0, s, dT, tlist, cb, zero_avg);
+static unsigned ca_lane_blocks(int max_n) { return ((unsigned)max_n * BL + 255) / 256; }
+
+void launch_ca_corners(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int bp, int max_n) {
+  EPI_LAUNCH(K_CA_CORNERS, k_ca_corners, dim3((8 * max_n + 255) / 256, ntis), dim3(256), 0, s, dT, tlist, bp);
+}
+
+void launch_ca_begin(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int bp, int max_n,
+                     long long max_box, int zero_avg) {
+  EPI_LAUNCH(K_CA_BEGIN, k_ca_begin, dim3(ca_lane_blocks(max_n), ntis), dim3(256), 0, s, dT, tlist, cb, zero_avg);
   unsigned gb = (unsigned)((max_box + 255) / 256);
   if (gb < 1) gb = 1;
   if (gb > 65535) gb = 65535;
   EPI_LAUNCH(K_CA_VOX, k_ca_vox, dim3(gb, ntis), dim3(256), 0, s, dT, tlist);
-  EPI_LAUNCH(K_CA_CORNERS, k_ca_corners, dim3((8 * max_n + 255) / 256, ntis), dim3(256), 0, s, dT, tlist);
+  launch_ca_corners(s, dT, tlist, ntis, bp, max_n);
 }
 
-void launch_ca_begin(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int max_n, long long max_box) {
-  ca_maps(s, dT, tlist, ntis, cb, max_n, max_box, 1);
-}
-
-void launch_ca_touch(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int max_n, long long max_box) {
-  ca_maps(s, dT, tlist, ntis, cb, max_n, max_box, 0);
-}
-
-void launch_ca_diffu_zero(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int max_n) {
-  EPI_LAUNCH(K_CA_END, k_ca_end, dim3((max_n + 255) / 256, ntis), dim3(256), 0, s, dT, tlist, 0);
+void launch_ca_end(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int max_n, int what) {
+  EPI_LAUNCH(K_CA_END, k_ca_end, dim3(ca_lane_blocks(max_n), ntis), dim3(256), 0, s, dT, tlist, cb, what);
+  if (what == CA_END_SOLVE) EPI_LAUNCH(K_SW_RESET, k_sw_reset, dim3(ntis), dim3(64), 0, s, dT, tlist);
 }
 
 namespace {
-void launch_cells(hipStream_t s, const Tis* dT, const CaList& cl, int cb, int cp, int ap, int bp, const Tuning& tu,
-                  const RdTis* sv = nullptr, int slot = 0) {
-  const int cg = tu.ca_group;
-  const dim3 gc((unsigned)std::max(cl.ncb, 1));
-  if (cg == 4)
-    EPI_LAUNCH(K_CA_CELLS, k_ca_cells<4>, gc, dim3(C_BLOCK), 0, s, dT, cl, cb, cp, ap, bp, tu.xcd, sv, slot);
-  else if (cg == 8)
-    EPI_LAUNCH(K_CA_CELLS, k_ca_cells<8>, gc, dim3(C_BLOCK), 0, s, dT, cl, cb, cp, ap, bp, tu.xcd, sv, slot);
-  else
-    EPI_LAUNCH(K_CA_CELLS, k_ca_cells<16>, gc, dim3(C_BLOCK), 0, s, dT, cl, cb, cp, ap, bp, tu.xcd, sv, slot);
+// the launch's by-value tissue: a one-tissue list's, or nothing that is read
+CaArg one_arg(const CaList& cl, int cpc, int cpa, int ap) {
+  return cl.ntis == 1 ? ca_arg(*cl.h0, cpc, cpa, ap) : CaArg{};
+}
+
+// f with true or false as a type, by b
+template <class F>
+void by_bool(bool b, F f) {
+  if (b) f(std::true_type());
+  else f(std::false_type());
+}
+// f with the lanes per cell, whether the list has one tissue and whether the
+// launch saves, as types
+template <class F>
+void by_cells(const CaList& cl, const Tuning& tu, const RdTis* sv, F f) {
+  by_bool(cl.ntis == 1, [&](auto one) {
+    by_bool(sv != nullptr, [&](auto save) {
+      if (ca_lanes(tu.ca_group) == 8) f(std::integral_constant<int, 8>(), one, save);
+      else f(std::integral_constant<int, 16>(), one, save);
+    });
+  });
+}
+
+void launch_cells(hipStream_t s, const Tis* dT, const CaList& cl, int cp, int ap, const Tuning& tu, const RdTis* sv,
+                  int slot) {
+  by_cells(cl, tu, sv, [&](auto cg, auto one, auto save) {
+    const auto kfn = k_ca_cells<decltype(cg)::value, decltype(one)::value, decltype(save)::value>;
+    EPI_LAUNCH(K_CA_CELLS, kfn, dim3((unsigned)std::max(cl.ncb, 1)), dim3(C_BLOCK), 0, s, dT, cl,
+               one_arg(cl, cp, cp, ap), cp, ap, tu.xcd, sv, slot);
+  });
 }
 
 // blocks that walk a list of `tiles` tiles: one per tile (as launch_ext_stim),
@@ -1247,63 +1328,46 @@ unsigned walk_blocks(long long tiles, int bs) {
 }
 
 void launch_atp(hipStream_t s, const Tis* dT, const CaList& cl, int cp, int ap, const Tuning& tu) {
+  const dim3 g(walk_blocks(cl.atiles, cl.abs));
   by_zb(tu.a_zb, [&](auto zbc) {
     constexpr int zb = decltype(zbc)::value;
-    EPI_LAUNCH(K_ATP, k_atp<zb>, dim3(walk_blocks(cl.atiles, cl.abs)), dim3(cl.abs), 0, s, dT, cl, ap, cp, tu.xcd);
+    const auto k1 = k_atp<zb, true>, kn = k_atp<zb, false>;
+    if (cl.ntis == 1) EPI_LAUNCH(K_ATP, k1, g, dim3(cl.abs), 0, s, dT, cl, ap, cp, tu.xcd);
+    else EPI_LAUNCH(K_ATP, kn, g, dim3(cl.abs), 0, s, dT, cl, ap, cp, tu.xcd);
   });
 }
 
-template <int CG>
-void launch_fused_cg(hipStream_t s, const Tis* dT, const CaList& cl, int cb, int cp, int ap, int bp,
-                     const Tuning& tu) {
-  by_zb(tu.a_zb, [&](auto zbc) {
-    constexpr int zb = decltype(zbc)::value;
-    const unsigned cblocks = tu.xcd ? (unsigned)(cl.ncb + 7) / 8 * 8 : (unsigned)cl.ncb;
-    const dim3 g(cblocks + walk_blocks(cl.atiles, F_BLOCK));
-    const auto kfn = k_ca_fused<CG, zb>;
-    EPI_LAUNCH(K_CA_FUSED, kfn, g, dim3(F_BLOCK), 0, s, dT, cl, cb, cp, ap, bp, cl.ncb, tu.xcd);
+// the ATP update of the sub-step at (cp, ap) beside the cells of the next one
+void launch_fused(hipStream_t s, const Tis* dT, const CaList& cl, int cp, int ap, const Tuning& tu, const RdTis* sv,
+                  int slot) {
+  const unsigned cblocks = tu.xcd ? (unsigned)(cl.ncb + 7) / 8 * 8 : (unsigned)cl.ncb;
+  const dim3 g(cblocks + walk_blocks(cl.atiles, F_BLOCK));
+  by_cells(cl, tu, sv, [&](auto cg, auto one, auto save) {
+    constexpr int CG = decltype(cg)::value;
+    constexpr bool ONE = decltype(one)::value, SAVE = decltype(save)::value;
+    const auto k1 = k_ca_fused<CG, 1, ONE, SAVE>, k2 = k_ca_fused<CG, 2, ONE, SAVE>;
+    EPI_LAUNCH(K_CA_FUSED, (tu.a_zb == 2 ? k2 : k1), g, dim3(F_BLOCK), 0, s, dT, cl, one_arg(cl, 1 - cp, cp, ap), cp, ap,
+               cl.ncb, tu.xcd, sv, slot);
   });
 }
 }  // namespace
 
 int ca_list_bs(const Tuning& tu, bool fused) { return fused ? F_BLOCK : 64 * tu.a_rows; }
 
-void launch_ca_substep(hipStream_t s, const Tis* dT, const CaList& cl, int cb, int cp, int ap, int bp,
-                       const Tuning& tu, const RdTis* sv, int slot, bool cells_only) {
-  launch_cells(s, dT, cl, cb, cp, ap, bp, tu, sv, slot);
-  if (!cells_only) launch_atp(s, dT, cl, cp, ap, tu);
-}
-
-void launch_ca_substeps(hipStream_t s, const Tis* dT, const CaList& cl, int cb, int& cp, int& ap, int bp,
-                        int n_sub, const Tuning& tu) {
-  if (!tu.ca_fuse || n_sub < 2) {
-    for (int i = 0; i < n_sub; i++) {
-      launch_ca_substep(s, dT, cl, cb, cp, ap, bp, tu);
-      cp ^= 1;
-      ap ^= 1;
+void launch_ca_substeps(hipStream_t s, const Tis* dT, const CaList& cl, int& cp, int& ap, int n_sub, const Tuning& tu,
+                        const RdTis* sv, int slot, bool last_cells_only) {
+  const bool fuse = tu.ca_fuse && n_sub >= 2;
+  // fused: cells of sub-step 0; then (ATP of i, cells of i + 1); then ATP of the last
+  for (int i = 0; i < n_sub; i++) {
+    if (i == 0 || !fuse) launch_cells(s, dT, cl, cp, ap, tu, sv, slot + i);
+    if (i + 1 < n_sub && fuse) {
+      launch_fused(s, dT, cl, cp, ap, tu, sv, slot + i + 1);
+    } else if (i + 1 < n_sub || !last_cells_only) {
+      launch_atp(s, dT, cl, cp, ap, tu);
     }
-    return;
-  }
-  // cells of sub-step 0; then (ATP of i, cells of i + 1); then ATP of the last
-  launch_cells(s, dT, cl, cb, cp, ap, bp, tu);
-  for (int i = 0; i + 1 < n_sub; i++) {
-    if (tu.ca_group == 4)
-      launch_fused_cg<4>(s, dT, cl, cb, cp, ap, bp, tu);
-    else if (tu.ca_group == 8)
-      launch_fused_cg<8>(s, dT, cl, cb, cp, ap, bp, tu);
-    else
-      launch_fused_cg<16>(s, dT, cl, cb, cp, ap, bp, tu);
     cp ^= 1;
     ap ^= 1;
   }
-  launch_atp(s, dT, cl, cp, ap, tu);
-  cp ^= 1;
-  ap ^= 1;
-}
-
-void launch_ca_end(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int max_n) {
-  EPI_LAUNCH(K_CA_END, k_ca_end, dim3((max_n + 255) / 256, ntis), dim3(256), 0, s, dT, tlist, 1);
-  EPI_LAUNCH(K_SW_RESET, k_sw_reset, dim3(ntis), dim3(64), 0, s, dT, tlist);
 }
 
 }  // namespace epi

@@ -26,7 +26,7 @@ constexpr long long WL_INTS(int ntis) { return 8LL * (ntis + 1); }
 struct Tuning {
   int b_zb = 4, b_rows = 4;   // k_ext_stim: z planes per tile, 64-lane rows per block (points per tile)
   int a_zb = 4, a_rows = 4;   // k_atp: the same (a fused solve's tiles are 128 points)
-  int ca_group = 16;          // k_ca_cells: lanes per cell
+  int ca_group = 8;           // Ca cell kernels: lanes per cell (8, or 16; 4 takes 8)
   int xcd = 0;                // k_ca_cells, k_atp: XCD-contiguous workgroup order
   int b_xcd = 0;              // k_ext_stim: its tile list in one contiguous run per XCD
   int sweep_wave = 0;         // k_sweep: 1, one wave per cell (k_sweep_wave)
@@ -104,7 +104,12 @@ void launch_map_stamp(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n,
 // the list: the blocks walk it grid-stride)
 void launch_ext_stim(hipStream_t s, const Tis* dT, int ntis, int bp, long long tiles_est, int* d_wl,
                      const Tuning& tu);
-void launch_ca_begin(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int max_n, long long max_box);
+// a solve's or window's set-up: packed entries, pairs, laws' constants (and
+// ca2p_avg cleared with zero_avg), voxel words, corners.  launch_ca_corners
+// alone renews what depends on B (buffer bp)
+void launch_ca_begin(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int bp, int max_n,
+                     long long max_box, int zero_avg);
+void launch_ca_corners(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int bp, int max_n);
 struct RdTis;
 // A Ca solve's work, flattened over its tissues (built on the host once per
 // solve, device pointers): blocks of the cell kernels map to (tissue, block
@@ -121,21 +126,24 @@ struct CaList {
   const int4* cmap;
   int ntis, ncb, atiles, abs;
   int t0, izb0;
+  const Tis* h0;   // host: that tissue's descriptor, passed to the kernels by value
 };
 // points per ATP tile of a solve: the fused kernel's block, or the ATP
 // kernel's 64 a_rows
 int ca_list_bs(const Tuning& tu, bool fused);
-// sv: a reaction-diffusion window's reverse-pass storage; the cell kernel
-// then also saves the state before the sub-step into its segment slot
-// `slot`; cells_only skips the ATP update (the last state of a segment)
-void launch_ca_substep(hipStream_t s, const Tis* dT, const CaList& cl, int cb, int cp, int ap, int bp,
-                       const Tuning& tu, const RdTis* sv = nullptr, int slot = 0, bool cells_only = false);
-// n_sub sub-steps (fused when tu.ca_fuse), flipping cp and ap after each
-void launch_ca_substeps(hipStream_t s, const Tis* dT, const CaList& cl, int cb, int& cp, int& ap, int bp,
-                        int n_sub, const Tuning& tu);
-void launch_ca_touch(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int max_n, long long max_box);
-void launch_ca_diffu_zero(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int max_n);
-void launch_ca_end(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int max_n);
+// lanes per cell that a CA_GROUP value asks for (8 serves 4 too: a cell's
+// eight corners take eight lanes)
+constexpr int ca_lanes(int ca_group) { return ca_group <= 8 ? 8 : 16; }
+// n_sub sub-steps (fused when tu.ca_fuse), flipping cp and ap after each.
+// sv: a reaction-diffusion window's reverse-pass storage; the cells then also
+// save the state before each sub-step into segment slots slot, slot + 1, ...;
+// last_cells_only skips the ATP update of the last one
+void launch_ca_substeps(hipStream_t s, const Tis* dT, const CaList& cl, int& cp, int& ap, int n_sub, const Tuning& tu,
+                        const RdTis* sv = nullptr, int slot = 0, bool last_cells_only = false);
+// packed gj and pairs back into the cells' arrays (CA_END_PUT), with diff_u
+// cleared (CA_END_SUBSTEP), and the rest of a solve's end (CA_END_SOLVE)
+enum { CA_END_PUT = 0, CA_END_SUBSTEP = 1, CA_END_SOLVE = 2 };
+void launch_ca_end(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int max_n, int what);
 // the listed tissues' two Ca, IP3 and ATP buffers trade contents (after a
 // solve of part of a context with an odd sub-step count, whose buffer
 // parities are shared by every tissue)
@@ -146,11 +154,11 @@ void launch_rd_own(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int max_n)
 void launch_rd_restore(hipStream_t s, const Tis* dT, RdTis* dR, const double* gj0, int ntis, int cb, int cp, int ap,
                        int use_kpa, long long items);
 void launch_rd_put_gj(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int cb, long long items);
-void launch_rd_state(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int slot, int dir, int cb, int cp, int ap,
+void launch_rd_state(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int slot, int save, int cp, int ap,
                      long long items);
-void launch_rd_seed(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int cp, int cb, int q, long long items);
-void launch_rd_backward_substep(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int slot, int cb, int bp, int q,
-                                int qa, int max_n, long long max_box, int rg);
+void launch_rd_seed(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int cp, int q, long long items);
+void launch_rd_backward_substep(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int slot, int q, int qa, int max_n,
+                                long long max_box, int rg);
 // frozen mechanics window (k_mech.hip)
 struct MechTis;
 void launch_mech_state(hipStream_t s, const Tis* dT, const MechTis* dM, int ntis, int slot, int dir, int pb,
@@ -158,5 +166,5 @@ void launch_mech_state(hipStream_t s, const Tis* dT, const MechTis* dM, int ntis
 void launch_mech_seed(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int q, int max_n);
 void launch_mech_backward_step(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int slot, int pb, int cb, int q,
                                int max_n);
-void launch_rd_gj0(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int cb, int q, long long items);
+void launch_rd_gj0(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int q, long long items);
 }  // namespace epi

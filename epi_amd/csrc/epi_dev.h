@@ -41,6 +41,27 @@ constexpr double AREA_GRID = 2.0 + 1e-7;   // cell_connection.cpp:16-19 (the buc
 enum : int { LAW_NONE = 0, LAW_OTHER, LAW_DER_DER, LAW_FIXMU, LAW_FIX_MEMB,
              LAW_MU_MEMB, LAW_ALAIRDE, LAW_MEMB_MEMB, LAW_PAIR };
 
+// A pointer into device memory that a kernel reads from a descriptor.  The
+// compiler cannot know where a pointer loaded from memory leads and would
+// reach it with flat instructions, which also wait as LDS accesses do, cannot
+// take a scalar base and return in no order; this one says that it is global.
+// The layout is a pointer's; files without kernels see a plain one.
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(EPI_NO_KERNELS)
+template <class T>
+struct GPtr {
+  __attribute__((address_space(1))) T* p;
+  __host__ __device__ __forceinline__ GPtr& operator=(T* q) {
+    p = (__attribute__((address_space(1))) T*)q;
+    return *this;
+  }
+  __host__ __device__ __forceinline__ operator T*() const { return (T*)p; }
+  __host__ __device__ __forceinline__ T* operator->() const { return (T*)p; }
+};
+#else
+template <class T>
+using GPtr = T*;
+#endif
+
 // ---- per-tissue device status (changes on device) ---------------------
 struct Status {
   int n;                  // live cells
@@ -70,67 +91,71 @@ struct Tis {
   long long gsize;            // XP*(NY+1)*(NZ+1)
   double LX, LY, LZ, dx, dy, dz, inv_dx, inv_dy, inv_dz;
   int ANX, ANY, ANZ, bcap;
-  int irx, iry, irz, pad1;
+  int irx, iry, irz;
+  unsigned mg_nx;             // div_magic(NX, NX NY)
   // ca2p_du (ca2p.cpp:183), dp (ca2p.cpp:17), eps_m, K_TOTAL, Kspring and
   // KBEND (cell_interaction.cpp:21-28) as the kernels use them: prm's
   // values, or a window's while one is open
   double ca_du, ca_dp;
   double m_eps, m_kadh, m_kspring, m_kbend;
-  Status* st;
+  GPtr<Status> st;
   // cells
-  uint8_t* state; uint8_t* is_malignant; uint8_t* touch_air;
-  int* fix_origin; int* rest_div_times; int* pair; int* dermis; int* lat;  // lat: 3/cell
-  double* pos[2][3];          // [buffer][axis]
-  double *radius, *div_age_thresh;
-  double* ca2p[2]; double* ip3[2];
-  double *ca2p_avg, *ex_inert, *agek, *ageb, *ex_fat, *in_fat, *spr_nat_len, *diff_u;
-  double *ca_th, *ca_kpa, *ca_iag;   // per-solve constants of the Ca step (agek and state are frozen)
+  GPtr<uint8_t> state; GPtr<uint8_t> is_malignant; GPtr<uint8_t> touch_air;
+  GPtr<int> fix_origin; GPtr<int> rest_div_times; GPtr<int> pair; GPtr<int> dermis; GPtr<int> lat;  // lat: 3/cell
+  GPtr<double> pos[2][3];          // [buffer][axis]
+  GPtr<double> radius, div_age_thresh;
+  GPtr<double> ca2p[2]; GPtr<double> ip3[2];
+  GPtr<double> ca2p_avg, ex_inert, agek, ageb, ex_fat, in_fat, spr_nat_len, diff_u;
+  GPtr<double> ca_th, ca_kpa, ca_iag;   // per-solve constants of the Ca step (agek and state are frozen)
   // The coupled list entries of the AFM and DEAD cells during a solve or
   // window, packed to the front of a row of ns in list order: the word
   // neighbour << 2 | kind (1 coupled, 3 coupled ALIVE), the entry's slot in the
   // list row, and its gj, which lives here until k_ca_end puts it back; and
   // their number per cell (0 for the other cells)
-  int* ca_w;
-  unsigned short* ca_sl;
-  double* ca_g;
-  int* ca_cn;
+  GPtr<int> ca_w;
+  GPtr<unsigned short> ca_sl;
+  GPtr<double> ca_g;
+  GPtr<int> ca_cn;
   // (ca2p, IP3) of buffer b during a solve or window, so that a list entry
   // reads its neighbour's pair with one 16-byte gather; the arrays ca2p and
   // ip3 follow at its end (k_ca_end)
-  double2* ca_up[2];
+  GPtr<double2> ca_up[2];
   // diff_u of the Ca sub-steps at parity 1 (parity 0 writes diff_u itself)
-  double* ca_dfu;
+  GPtr<double> ca_dfu;
   // per AFM cell and grid_avg8 corner (binary x, y, z), during a solve: the
   // corner's point wrapped in x and y, its voxel word, the masks of its six
   // stencil neighbours and the CQ_ flags, and the point as it lies
-  uint4* ca_cq;
-  double* ca_bx;   // ca2p_by_ext_stim per AFM cell (B does not change during a solve)
-  long long* uid; long long* old_uid; int* src_row;
+  GPtr<uint4> ca_cq;
+  GPtr<double> ca_bx;   // ca2p_by_ext_stim per AFM cell (B does not change during a solve)
+  GPtr<long long> uid; GPtr<long long> old_uid; GPtr<int> src_row;
   // cell_stat (define.h:198-202): per cell k_aging_start, k_cornified,
   // k_disap (-1 = never set); cst_store (cellmanager.h:106): the records of
   // removed DEAD cells, up to cap of them, Status::nstat in use
-  long long* cst; long long* cst_store;
+  GPtr<long long> cst; GPtr<long long> cst_store;
   // neighbour rows (two buffers: current and previous build)
-  int* nlen[2]; int* col[2]; double* gj[2];
-  int* nlo;                   // entries of the row below the cell index
-  int* btmp; int* bcnt;       // upper partners gathered during the sweep
-  int* memb6;                 // triangular adjacency, 6 per membrane cell
+  GPtr<int> nlen[2]; GPtr<int> col[2]; GPtr<double> gj[2];
+  GPtr<int> nlo;                   // entries of the row below the cell index
+  GPtr<int> btmp; GPtr<int> bcnt;       // upper partners gathered during the sweep
+  GPtr<int> memb6;                 // triangular adjacency, 6 per membrane cell
   // buckets
-  int* bucket_of; int* bslot; int* bucket_n; int* bucket_cells;
-  int* bucket_sorted;   // the buckets in ascending cell index, written by k_bucket_sort for the sweep
+  GPtr<int> bucket_of; GPtr<int> bslot; GPtr<int> bucket_n; GPtr<int> bucket_cells;
+  GPtr<int> bucket_sorted;   // the buckets in ascending cell index, written by k_bucket_sort for the sweep
   // (x, y, z, radius) of every cell after the periodic fix, written by the
   // bucket insertion: the sweep and the row assembly gather a candidate's
   // position and radius with one 32-byte load instead of four
-  double4* pk;
+  GPtr<double4> pk;
   // state renewal
-  int* div_slot; double* div_dir;  // per division: parent, direction
-  int* div_parent; int* rm_list;
-  uint8_t* rflag; int* chunk_any;   // renewal flags and per-1024-cell chunk marks
+  GPtr<int> div_slot; GPtr<double> div_dir;  // per division: parent, direction
+  GPtr<int> div_parent; GPtr<int> rm_list;
+  GPtr<uint8_t> rflag; GPtr<int> chunk_any;   // renewal flags and per-1024-cell chunk marks
   // grids
-  double* atp[2]; double* bf[2];
-  int* cmap1; uint8_t* cmap2; unsigned* vox;
+  GPtr<double> atp[2]; GPtr<double> bf[2];
+  // vox, vmk: during a solve or window, per voxel of the active box, the AFM
+  // owner and air flag (k_ca_vox) and the masks of its six neighbours in one
+  // byte (bits 0-5: x-, x+, y-, y+, z-, z+; VMK_SLOW when one is above 1)
+  GPtr<int> cmap1; GPtr<uint8_t> cmap2; GPtr<unsigned> vox; GPtr<uint8_t> vmk;
   // replay stream
-  const double* rng; long long rng_n;
+  GPtr<const double> rng; long long rng_n;
   // the tissue's runtime parameters (epi_set_params)
   Params prm;
 };
@@ -174,14 +199,27 @@ __device__ __forceinline__ long long gidx(const G& t, int j, int k, int l) {
   return (long long)l * t.PL + (long long)k * t.XP + j;
 }
 
+constexpr unsigned VMK_SLOW = 0x80u;
+
+// n / d for n below the limit the magic was made for (0: none was)
+__device__ __forceinline__ unsigned div_by(unsigned n, unsigned d, unsigned magic) {
+  return magic ? __umulhi(n, magic) : n / d;
+}
+// ceil(2^32 / d) if n * that / 2^32 rounds down to n / d for every n < limit
+// (the excess e = magic d - 2^32 < d adds n e / (d 2^32) < 1 / d), else 0
+inline unsigned div_magic(unsigned d, unsigned long long limit) {
+  const unsigned long long m = ((1ull << 32) + d - 1) / d, e = m * d - (1ull << 32);
+  return d > 1 && limit * e < (1ull << 32) ? (unsigned)m : 0u;
+}
+
 // empties the voxel maps' planes 0..stamp_z, four voxels per thread, by block
 // b of nb blocks (a plane holds PL = XP (NY + 1) voxels with XP a multiple of
 // 16, and the maps start 256-byte aligned)
 __device__ __forceinline__ void map_clear(const Tis& t, int b, int nb) {
   const int planes = min(t.st->stamp_z, t.NZ) + 1;
   const long long g4 = (long long)planes * t.PL / 4;
-  int4* __restrict__ m1 = reinterpret_cast<int4*>(t.cmap1);
-  unsigned* __restrict__ m2 = reinterpret_cast<unsigned*>(t.cmap2);
+  int4* __restrict__ m1 = reinterpret_cast<int4*>(static_cast<int*>(t.cmap1));
+  unsigned* __restrict__ m2 = reinterpret_cast<unsigned*>(static_cast<uint8_t*>(t.cmap2));
   for (long long q = (long long)b * blockDim.x + threadIdx.x; q < g4; q += (long long)nb * blockDim.x) {
     m1[q] = make_int4(-1, -1, -1, -1);
     m2[q] = 0u;

@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../include/epi_amd.h"
+#define EPI_NO_KERNELS   // plain pointers in the descriptors (epi_dev.h)
 #include "epi_dev.h"
 #include "launch.h"
 #include "rd_dev.h"
@@ -320,6 +321,7 @@ void carve_tissue(Carver& cv, TH& h, Tis& t) {
   t.cmap1 = cv.take<int>(h.gsize);
   t.cmap2 = cv.take<uint8_t>(h.gsize);
   t.vox = cv.take<unsigned>(h.gsize);
+  t.vmk = cv.take<uint8_t>(h.gsize);
 }
 
 int check_tissue(epi_ctx* c, int t) {
@@ -396,6 +398,11 @@ int max_memb(const epi_ctx* c) {
 long long max_gsize(const epi_ctx* c) {
   long long m = 1;
   for (auto& h : c->th) m = std::max(m, h.gsize);
+  return m;
+}
+long long max_plane(const epi_ctx* c) {
+  long long m = 1;
+  for (auto& h : c->th) m = std::max(m, (long long)h.NX * h.NY);
   return m;
 }
 int max_nx(const epi_ctx* c) {
@@ -484,6 +491,13 @@ int set_zz(epi_ctx* c, const double* zzmax) {
   return EPI_OK;
 }
 
+// whether a plane of one of the tissues is past 32-bit byte offsets
+bool any_wide_plane(const epi_ctx* c, const int* ids, int ntis) {
+  for (int i = 0; i < ntis; i++)
+    if (c->th[ids ? ids[i] : i].PL * 8 > (1LL << 32)) return true;
+  return false;
+}
+
 // The list of a Ca solve (or window) over tissues ids[0..ntis) (nullptr:
 // all of them), for cg lanes per cell and ATP tiles of bs points by zb
 // planes, from what the host holds: the cell counts of the last status
@@ -538,7 +552,10 @@ int ca_list(epi_ctx* c, const int* ids, int ntis, int cg, int bs, int zb, CaList
     c->cal_key = key;
     c->cal = CaList{c->d_cal, c->d_cal + ntis + 1, c->d_cal + 2 * ntis + 1,
                     reinterpret_cast<const int4*>(c->d_cal + hdr), ntis, (int)ncb, (int)tiles, bs,
-                    ids ? ids[0] : 0, izb[0], &c->tis[ids ? ids[0] : 0]};
+                    ids ? ids[0] : 0, izb[0], &c->tis[ids ? ids[0] : 0], 0u, any_wide_plane(c, ids, ntis)};
+    const TH& h0 = c->th[c->cal.t0];
+    const int npt = (h0.NX * h0.NY + bs - 1) / bs;
+    c->cal.mg_npt = div_magic((unsigned)npt, (unsigned long long)std::max(tiles, 1LL));
   }
   *out = c->cal;
   return EPI_OK;
@@ -600,7 +617,9 @@ Tuning ca_shapes(const epi_ctx* c, const int* ids, int ntis) {
   }
   // a fused launch's ATP tiles are one or two planes: taller ones roll their
   // planes through one thread, which the cells beside them wait for (14.1
-  // against 10.1 us per sub-step of the large tissue)
+  // against 10.1 us per sub-step of the large tissue).  They address a plane
+  // with 32-bit byte offsets; a tissue of larger planes takes two launches.
+  if (any_wide_plane(c, ids, ntis)) tu.ca_fuse = 0;
   if (tu.ca_fuse && tu.a_zb > 2) tu.a_zb = 1;
   return tu;
 }
@@ -611,14 +630,16 @@ Tuning ca_shapes(const epi_ctx* c, const int* ids, int ntis) {
 // a large batch launches that tissue's blocks, not the batch's largest.
 int run_ca_n(epi_ctx* c, const int* d_tlist, int ntis, int n_sub) {
   int mn = 1;
-  long long box = 1;
+  long long plane = 1;
+  int planes = 1;
   for (int i = 0; i < ntis; i++) {
     const int t = d_tlist ? c->h_tlist[i] : i;
     const TH& h = c->th[t];
     const double zz = c->h_st[t].zzmax;
     const int iz = std::min((int)((zz + c->tis[t].prm.iz_margin) / c->tis[t].dz) + 2, h.NZ + 1);
     mn = std::max(mn, h.n_est + 64);
-    box = std::max(box, (long long)h.NX * h.NY * iz);
+    plane = std::max(plane, (long long)h.NX * h.NY);
+    planes = std::max(planes, iz);
   }
   const Tuning tu = ca_shapes(c, d_tlist ? c->h_tlist : nullptr, ntis);
   CaList cl;
@@ -633,12 +654,12 @@ int run_ca_n(epi_ctx* c, const int* d_tlist, int ntis, int n_sub) {
     int mcap = 1;
     for (int i = 0; i < ntis; i++) mcap = std::max(mcap, c->th[d_tlist ? c->h_tlist[i] : i].cap);
     const int mr = std::max(mn, std::min((mn + 1023) / 1024 * 1024, mcap));
-    std::vector<long long> key = {2, c->tis_version, d_tlist != nullptr, ntis, n_sub, mr, box, c->cb, c->cp, c->ap,
+    std::vector<long long> key = {2, c->tis_version, d_tlist != nullptr, ntis, n_sub, mr, plane, planes, c->cb, c->cp, c->ap,
                                   c->bp, tu.ca_fuse, tu.ca_group, tu.a_zb, tu.a_rows, tu.xcd};
     key.insert(key.end(), c->cal_key.begin(), c->cal_key.end());
     RCHK(graph_run(c, key, [&] {
       int cp = c->cp, ap = c->ap;
-      launch_ca_begin(c->stream, c->d_tis, d_tlist, ntis, c->cb, c->bp, mr, box, 1);
+      launch_ca_begin(c->stream, c->d_tis, d_tlist, ntis, c->cb, c->bp, mr, plane, planes, 1);
       launch_ca_substeps(c->stream, c->d_tis, cl, cp, ap, n_sub, tu);
       launch_ca_end(c->stream, c->d_tis, d_tlist, ntis, c->cb, mr, CA_END_SOLVE);
       return hipGetLastError();
@@ -646,7 +667,7 @@ int run_ca_n(epi_ctx* c, const int* d_tlist, int ntis, int n_sub) {
     c->cp ^= n_sub & 1;
     c->ap ^= n_sub & 1;
   } else {
-    launch_ca_begin(c->stream, c->d_tis, d_tlist, ntis, c->cb, c->bp, mn, box, 1);
+    launch_ca_begin(c->stream, c->d_tis, d_tlist, ntis, c->cb, c->bp, mn, plane, planes, 1);
     launch_ca_substeps(c->stream, c->d_tis, cl, c->cp, c->ap, n_sub, tu);
     launch_ca_end(c->stream, c->d_tis, d_tlist, ntis, c->cb, mn, CA_END_SOLVE);
   }
@@ -766,6 +787,7 @@ int epi_create(int32_t ntissues, const epi_geometry* geos, epi_ctx** out) {
     ti.irx = (int)(Rad * g.nx / g.lx);
     ti.iry = (int)(Rad * g.ny / g.ly);
     ti.irz = (int)(Rad * g.nz / g.lz);
+    ti.mg_nx = div_magic((unsigned)g.nx, (unsigned long long)g.nx * g.ny);
     // epi5_MT's parameters with this geometry's grid and box
     epi_params dp;
     epi_params_default(&dp);
@@ -1209,11 +1231,9 @@ int epi_ca_substep(epi_ctx* c, int32_t iz_bound) {
     if ((int)((zz[t] + c->tis[t].prm.iz_margin) / c->tis[t].dz) != iz_bound)
       return fail(c, EPI_ERR_INVALID, "iz_bound");
   const int mn = max_n(c);
-  long long box = 1;
-  for (auto& h : c->th) box = std::max(box, (long long)h.NX * h.NY * (iz_bound + 1));
   CaList cl;
   RCHK(ca_list(c, nullptr, c->T, ca_lanes(c->tu.ca_group), ca_list_bs(c->tu, false), c->tu.a_zb, &cl));
-  launch_ca_begin(c->stream, c->d_tis, nullptr, c->T, c->cb, c->bp, mn, box, 0);
+  launch_ca_begin(c->stream, c->d_tis, nullptr, c->T, c->cb, c->bp, mn, max_plane(c), iz_bound, 0);
   launch_ca_substeps(c->stream, c->d_tis, cl, c->cp, c->ap, 1, c->tu);
   launch_ca_end(c->stream, c->d_tis, nullptr, c->T, c->cb, mn, CA_END_SUBSTEP);
   HIPCHK(c, hipGetLastError());
@@ -1862,9 +1882,8 @@ int epi_rd_begin(epi_ctx* c, const double* zzmax) {
   }
   RCHK(set_zz(c, zzmax));
   // per-solve maps: entry kinds, th/Kpa/IAG, voxel owners (init_ca2p_map)
-  long long box = 1;
-  for (int t = 0; t < c->T; t++) box = std::max(box, (long long)c->th[t].NX * c->th[t].NY * (rd.izb[t] + 1));
-  launch_ca_begin(c->stream, c->d_tis, nullptr, c->T, c->cb, c->bp, max_n(c), box, 0);
+  launch_ca_begin(c->stream, c->d_tis, nullptr, c->T, c->cb, c->bp, max_n(c), max_plane(c),
+                  *std::max_element(rd.izb.begin(), rd.izb.end()), 0);
   // arena: snapshot + adjoint arrays per tissue
   rd.h.assign(c->T, RdTis{});
   Carver dry{nullptr, 0, true};

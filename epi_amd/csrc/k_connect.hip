@@ -464,7 +464,7 @@ __global__ void __launch_bounds__(256) k_snapshot(const Tis* __restrict__ T, int
   static_assert(sizeof(Status) % 8 == 0 && sizeof(Status) / 8 <= 256, "status copied in 8-byte words");
   if (h_out && blockIdx.x == 0 && threadIdx.x < sizeof(Status) / 8)
     reinterpret_cast<unsigned long long*>(h_out + blockIdx.y)[threadIdx.x] =
-        reinterpret_cast<const unsigned long long*>(t.st)[threadIdx.x];
+        reinterpret_cast<const unsigned long long*>(static_cast<const Status*>(t.st))[threadIdx.x];
   const int n = t.st->n;
   for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
     t.src_row[c] = c;

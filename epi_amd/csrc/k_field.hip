@@ -518,24 +518,34 @@ __global__ void __launch_bounds__(256) k_ca_begin(const Tis* __restrict__ T, con
 }
 
 // init_ca2p_map (:238-278): per voxel of the active box the AFM owner
-// (+1, 0 = the dummy zero) and the air flag in bit 31
+// (+1, 0 = the dummy zero) and the air flag in bit 31; and the masks of its
+// neighbours (ATP_refresh's, :302-338), which do not change during a solve
 __global__ void __launch_bounds__(256) k_ca_vox(const Tis* __restrict__ T, const int* tlist) {
   const Tis& t = T[tlist ? tlist[blockIdx.y] : blockIdx.y];
   const int izb = ca_iz_bound(t);
-  if (izb > t.NZ || izb < 0) {
+  const int NX = t.NX, NY = t.NY, NZ = t.NZ;
+  if (izb > NZ || izb < 0) {
     if (blockIdx.x == 0 && threadIdx.x == 0) set_err(t.st, ERR_OUT_OF_GRID);
     return;
   }
-  const long long tot = (long long)t.NX * t.NY * izb;
-  for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < tot; i += (long long)gridDim.x * blockDim.x) {
-    const int j = (int)(i % t.NX);
-    const long long r = i / t.NX;
-    const int k = (int)(r % t.NY), l = (int)(r / t.NY);
-    const long long v = gidx(t, j, k, l);
-    const int c = t.cmap1[v];
-    unsigned w = 0;
-    if (c >= 0) w = (is_afm(t.state[c]) ? (unsigned)(c + 1) : 0u) | ((unsigned)t.touch_air[c] << 31);
-    t.vox[v] = w;
+  const unsigned plane = (unsigned)NX * NY;
+  for (int l = blockIdx.z; l < izb; l += gridDim.z) {
+    const int pz = l == 0 ? 1 : l - 1, nz = l + 1 == NZ ? NZ - 1 : l + 1;
+    for (unsigned p = blockIdx.x * blockDim.x + threadIdx.x; p < plane; p += gridDim.x * blockDim.x) {
+      const int k = (int)div_by(p, NX, t.mg_nx), j = (int)(p - (unsigned)k * NX);
+      const long long v = gidx(t, j, k, l);
+      const int c = t.cmap1[v];
+      unsigned w = 0;
+      if (c >= 0) w = (is_afm(t.state[c]) ? (unsigned)(c + 1) : 0u) | ((unsigned)t.touch_air[c] << 31);
+      t.vox[v] = w;
+      const uint8_t* __restrict__ m2 = t.cmap2;
+      const uint8_t m[6] = {m2[gidx(t, j == 0 ? NX - 1 : j - 1, k, l)], m2[gidx(t, j == NX - 1 ? 0 : j + 1, k, l)],
+                            m2[gidx(t, j, k == 0 ? NY - 1 : k - 1, l)], m2[gidx(t, j, k == NY - 1 ? 0 : k + 1, l)],
+                            m2[gidx(t, j, k, pz)], m2[gidx(t, j, k, nz)]};
+      unsigned bits = 0;
+      for (int q = 0; q < 6; q++) bits |= m[q] > 1 ? VMK_SLOW : (unsigned)m[q] << q;
+      t.vmk[v] = (uint8_t)bits;
+    }
   }
 }
 
@@ -589,8 +599,10 @@ struct CaArg {
   double* A1;             // and after it
   const uint8_t* cm2;
   const unsigned* vox;
+  const uint8_t* vmk;
   long long PL;
   int start, cap, ns, NX, NY, NZ, XP;
+  unsigned mg_nx;
 };
 // cells at Ca parity cpc; the ATP update of the sub-step at Ca parity cpa from
 // ATP buffer ap
@@ -601,7 +613,7 @@ __host__ __device__ __forceinline__ CaArg ca_arg(const Tis& t, int cpc, int cpa,
   a.dfo = cpa ? t.ca_dfu : t.diff_u; a.dfn = cpc ? t.ca_dfu : t.diff_u;
   a.cq = t.ca_cq; a.th = t.ca_th; a.kpa = t.ca_kpa; a.iag = t.ca_iag; a.bx = t.ca_bx;
   a.exi = t.ex_inert; a.avg = t.ca2p_avg; a.A0 = t.atp[ap]; a.A1 = t.atp[1 - ap];
-  a.cm2 = t.cmap2; a.vox = t.vox; a.PL = t.PL;
+  a.cm2 = t.cmap2; a.vox = t.vox; a.vmk = t.vmk; a.PL = t.PL; a.mg_nx = t.mg_nx;
   a.start = t.nmemb + t.nder; a.cap = t.cap; a.ns = t.ns;
   a.NX = t.NX; a.NY = t.NY; a.NZ = t.NZ; a.XP = t.XP;
   return a;
@@ -904,152 +916,154 @@ __global__ void __launch_bounds__(C_BLOCK) k_ca_cells(const Tis* __restrict__ T,
   }
 }
 
-// ATP_refresh (:302-338) with the periodic copies of planes 0..iz_bound,
-// one tile of a solve's list: blockDim.x consecutive points of the (x, y)
-// plane times ZB planes; the z column rolls through registers.
-// One (x, y) column of an ATP tile, planes l0 .. l1 - 1 (at most ZB): as
-// b_column, every load first (the column, the lateral neighbours and masks,
-// each plane's voxel word), then the owners' diff_u, then ATP_refresh's
-// point update (atp_new) per plane.
-template <int ZB>
+// ATP_refresh (:302-338) with the periodic copies of planes 0..iz_bound.
+//
+// One (x, y) column of a tile, planes l0 .. l1 - 1 (at most ZB), atp_new per
+// point.  What bounds it: the instructions of a point more than its bytes (a
+// wave's FP64 and address work at four cycles each; 6,900 waves a sub-step on
+// the large tissue).  So the six neighbours' masks come as one byte of the
+// solve's vmk, every address is a plane's base, the same for the whole wave,
+// plus an offset within the plane kept in bytes (type Off: 32 bits, or 64 for
+// planes of 4 GB), and the divisions of the tile's index are multiplications
+// (div_by): about 120 instructions a point instead of 400.
+//
+// Tiles of up to 2 planes load everything first: the column, the lateral
+// neighbours, masks and voxel words, then the owners' diff_u.  Taller ones
+// roll the column through registers, the voxel word read one plane ahead, so
+// that a plane waits for one round trip and few values are live at a time.
+template <class Off>
+struct AtpAddr {   // byte offsets of a column's points within a plane of doubles
+  Off c, xm, xp, ym, yp;
+  __device__ AtpAddr(const CaArg& t, int j, int k) {
+    const Off wx = (Off)(t.NX - 1) * 8, wy = (Off)(t.NY - 1) * t.XP * 8, row = (Off)t.XP * 8;
+    c = ((Off)k * t.XP + j) * 8;
+    xm = j == 0 ? c + wx : c - 8;
+    xp = j == t.NX - 1 ? c - wx : c + 8;
+    ym = k == 0 ? c + wy : c - row;
+    yp = k == t.NY - 1 ? c - wy : c + row;
+  }
+};
+template <class Off>
+__device__ __forceinline__ double at_f64(const double* plane, Off o) {
+  return *reinterpret_cast<const double*>(reinterpret_cast<const char*>(plane) + o);
+}
+// atp_new of one point with its mask byte and voxel word; plane l of the maps
+template <class Off>
+__device__ __forceinline__ double atp_point(const AtpK& ak, const CaArg& t, const AtpAddr<Off>& o, int l, double c0,
+                                            double xm, double xp, double ym, double yp, double zm, double zp,
+                                            unsigned mk, unsigned w, double diffu, double inv_dx) {
+  double m[6];
+#pragma unroll
+  for (int b = 0; b < 6; b++) m[b] = (double)((mk >> b) & 1);
+  if (mk & VMK_SLOW) {
+    const uint8_t* __restrict__ cm2 = t.cm2;
+    const long long p = (long long)l * t.PL;
+    m[0] = cm2[p + o.xm / 8]; m[1] = cm2[p + o.xp / 8]; m[2] = cm2[p + o.ym / 8]; m[3] = cm2[p + o.yp / 8];
+    m[4] = cm2[(long long)(l == 0 ? 1 : l - 1) * t.PL + o.c / 8];
+    m[5] = cm2[(long long)(l + 1 == t.NZ ? l : l + 1) * t.PL + o.c / 8];
+  }
+  return atp_new(ak, c0, xm, xp, ym, yp, zm, zp, m[0], m[1], m[2], m[3], m[4], m[5], diffu, (double)(w >> 31), inv_dx);
+}
+// a point's new value and its periodic copies (:334-337)
+template <class Off>
+__device__ __forceinline__ void atp_store(const CaArg& t, double* plane, Off c, int j, int k, double nv) {
+  char* p = reinterpret_cast<char*>(plane);
+  *reinterpret_cast<double*>(p + c) = nv;
+  if (j == 0 || k == 0) {
+    const Off wx = (Off)t.NX * 8, wy = (Off)t.NY * t.XP * 8;
+    if (k == 0) *reinterpret_cast<double*>(p + c + wy) = nv;
+    if (j == 0) *reinterpret_cast<double*>(p + c + wx) = nv;
+    if (j == 0 && k == 0) *reinterpret_cast<double*>(p + wx + wy) = nv;
+  }
+}
+
+template <int ZB, class Off>
 __device__ __forceinline__ void atp_column(const Tis& ti, const CaArg& t, int j, int k, int l0, int l1) {
-  const int NX = t.NX, NY = t.NY, NZ = t.NZ;
   const AtpK ak = atp_k(ti.prm);
-  const double* __restrict__ carr = t.A0;
-  double* __restrict__ narr = t.A1;
-  const double* __restrict__ dfu = t.dfo;
-  const uint8_t* __restrict__ cm2 = t.cm2;
-  const int prev_x = j == 0 ? NX - 1 : j - 1, next_x = j == NX - 1 ? 0 : j + 1;
-  const int prev_y = k == 0 ? NY - 1 : k - 1, next_y = k == NY - 1 ? 0 : k + 1;
-  const long long PL = t.PL;
-  const long long cxy = gidx(t, j, k, 0);
+  const double inv_dx = ti.inv_dx;
+  const AtpAddr<Off> o(t, j, k);
   const int nl = l1 - l0;
-  double cz[ZB + 2];
-  uint8_t mz[ZB + 2];
+  const double* __restrict__ A = t.A0;
+  double cz[ZB + 2], xm[ZB], xp[ZB], ym[ZB], yp[ZB], diffu[ZB];
+  unsigned mk[ZB], w[ZB];
 #pragma unroll
   for (int q = 0; q < ZB + 2; q++) {
     int l = q == 0 ? (l0 == 0 ? 1 : l0 - 1) : l0 + q - 1;   // mirror z boundary (utils.cpp:32-72)
-    if (l > NZ - 1) l = NZ - 1;
-    cz[q] = 0;
-    mz[q] = 0;
-    if (q <= nl + 1) {
-      cz[q] = carr[cxy + l * PL];
-      mz[q] = cm2[cxy + l * PL];
-    }
+    if (l > t.NZ - 1) l = t.NZ - 1;
+    cz[q] = q <= nl + 1 ? at_f64(A + l * t.PL, o.c) : 0.0;
   }
-  double xm[ZB], xp[ZB], ym[ZB], yp[ZB];
-  uint8_t mxm[ZB], mxp[ZB], mym[ZB], myp[ZB];
-  unsigned w[ZB];
 #pragma unroll
   for (int q = 0; q < ZB; q++) {
     xm[q] = xp[q] = ym[q] = yp[q] = 0;
-    mxm[q] = mxp[q] = mym[q] = myp[q] = 0;
-    w[q] = 0;
+    mk[q] = w[q] = 0;
     if (q < nl) {
-      const int l = l0 + q;
-      const long long vxm = gidx(t, prev_x, k, l), vxp = gidx(t, next_x, k, l);
-      const long long vym = gidx(t, j, prev_y, l), vyp = gidx(t, j, next_y, l);
-      xm[q] = carr[vxm]; xp[q] = carr[vxp]; ym[q] = carr[vym]; yp[q] = carr[vyp];
-      mxm[q] = cm2[vxm]; mxp[q] = cm2[vxp]; mym[q] = cm2[vym]; myp[q] = cm2[vyp];
-      w[q] = t.vox[cxy + l * PL];
+      const long long pl = (l0 + q) * t.PL;
+      w[q] = *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(t.vox + pl) + o.c / 2);
+      mk[q] = t.vmk[pl + o.c / 8];
+      xm[q] = at_f64(A + pl, o.xm); xp[q] = at_f64(A + pl, o.xp);
+      ym[q] = at_f64(A + pl, o.ym); yp[q] = at_f64(A + pl, o.yp);
     }
   }
-  double diffu[ZB];
 #pragma unroll
   for (int q = 0; q < ZB; q++) {
     const unsigned cell1 = w[q] & 0x7fffffffu;
-    diffu[q] = cell1 ? dfu[cell1 - 1] : 0.0;
+    diffu[q] = cell1 ? t.dfo[cell1 - 1] : 0.0;
   }
-  const double inv_dx = ti.inv_dx;
 #pragma unroll
-  for (int q = 0; q < ZB; q++) {
+  for (int q = 0; q < ZB; q++)
     if (q < nl) {
-      const int l = l0 + q;
-      const double nv = atp_new(ak, cz[q + 1], xm[q], xp[q], ym[q], yp[q], cz[q], cz[q + 2], (double)mxm[q],
-                                (double)mxp[q], (double)mym[q], (double)myp[q], (double)mz[q], (double)mz[q + 2],
-                                diffu[q], (double)(w[q] >> 31), inv_dx);
-      narr[cxy + l * PL] = nv;
-      if (k == 0) narr[gidx(t, j, NY, l)] = nv;
-      if (j == 0) narr[gidx(t, NX, k, l)] = nv;
-      if (j == 0 && k == 0) narr[gidx(t, NX, NY, l)] = nv;
+      const double nv = atp_point(ak, t, o, l0 + q, cz[q + 1], xm[q], xp[q], ym[q], yp[q], cz[q], cz[q + 2], mk[q], w[q],
+                                  diffu[q], inv_dx);
+      atp_store(t, t.A1 + (l0 + q) * t.PL, o.c, j, k, nv);
     }
-  }
 }
 
-// The same column rolling through registers plane by plane (as
-// b_column_roll), for tall tiles; the voxel word is read one plane ahead, so
-// a plane waits for one round trip (its owner's diff_u), not two.
+template <class Off>
 __device__ __forceinline__ void atp_column_roll(const Tis& ti, const CaArg& t, int j, int k, int l0, int l1) {
-  const int NX = t.NX, NY = t.NY, NZ = t.NZ;
   const AtpK ak = atp_k(ti.prm);
-  const double* __restrict__ carr = t.A0;
-  double* __restrict__ narr = t.A1;
-  const double* __restrict__ dfu = t.dfo;
-  const uint8_t* __restrict__ cm2 = t.cm2;
-  const int prev_x = j == 0 ? NX - 1 : j - 1, next_x = j == NX - 1 ? 0 : j + 1;
-  const int prev_y = k == 0 ? NY - 1 : k - 1, next_y = k == NY - 1 ? 0 : k + 1;
   const double inv_dx = ti.inv_dx;
+  const AtpAddr<Off> o(t, j, k);
+  const double* __restrict__ A = t.A0;
   const long long PL = t.PL;
-  const long long cxy = gidx(t, j, k, 0);
-  const int pz = l0 == 0 ? 1 : l0 - 1;   // mirror z (utils.cpp:32-72)
-  double czm = carr[cxy + pz * PL];
-  int mzm = cm2[cxy + pz * PL];
-  double cc = carr[cxy + l0 * PL];
-  int mc = cm2[cxy + l0 * PL];
-  // x - 1 and x + 1 lie in the lanes beside this one (the lanes of a wave
-  // hold consecutive points of a row) except at a row's ends and the wave's
-  // edges, where they are loaded.  (The same exchange in b_column_roll
-  // measured 3 % slower; here 1.6 % faster on the 256-tissue batch.)
-  const int wl = threadIdx.x & 63;
-  const bool lane_xm = j > 0 && wl != 0, lane_xp = j < NX - 1 && wl != 63;
-  const unsigned* __restrict__ vox = t.vox;
-  unsigned w = l0 < l1 ? vox[cxy + l0 * PL] : 0u;
+  auto vox = [&](int l) {
+    return *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(t.vox + l * PL) + o.c / 2);
+  };
+  double zm = at_f64(A + (l0 == 0 ? 1 : l0 - 1) * PL, o.c);   // mirror z (utils.cpp:32-72)
+  double c0 = at_f64(A + l0 * PL, o.c);
+  unsigned w = l0 < l1 ? vox(l0) : 0u;
   for (int l = l0; l < l1; l++) {
-    const int next_z = l + 1 == NZ ? NZ - 1 : l + 1;
-    const long long v = cxy + l * PL;
-    const long long vzp = cxy + next_z * PL;
-    const double czp = carr[vzp];
-    const int mzp = cm2[vzp];
-    const unsigned w_next = l + 1 < l1 ? vox[v + PL] : 0u;
+    const long long pl = l * PL;
+    const double zp = at_f64(A + (l + 1 == t.NZ ? pl : pl + PL), o.c);
+    const unsigned wn = l + 1 < l1 ? vox(l + 1) : 0u;
+    const unsigned mk = t.vmk[pl + o.c / 8];
     const unsigned cell1 = w & 0x7fffffffu;
-    const double diffu = cell1 ? dfu[cell1 - 1] : 0.0;
-    const long long vxm = gidx(t, prev_x, k, l), vxp = gidx(t, next_x, k, l);
-    const long long vym = gidx(t, j, prev_y, l), vyp = gidx(t, j, next_y, l);
-    const double sxm = __shfl_up(cc, 1, 64), sxp = __shfl_down(cc, 1, 64);
-    const int smxm = __shfl_up(mc, 1, 64), smxp = __shfl_down(mc, 1, 64);
-    const double axm = lane_xm ? sxm : carr[vxm], axp = lane_xp ? sxp : carr[vxp];
-    const int mxm = lane_xm ? smxm : cm2[vxm], mxp = lane_xp ? smxp : cm2[vxp];
-    const double nv = atp_new(ak, cc, axm, axp, carr[vym], carr[vyp], czm, czp, (double)mxm, (double)mxp,
-                              (double)cm2[vym], (double)cm2[vyp], (double)mzm, (double)mzp, diffu,
-                              (double)(w >> 31), inv_dx);
-    narr[v] = nv;
-    if (k == 0) narr[gidx(t, j, NY, l)] = nv;
-    if (j == 0) narr[gidx(t, NX, k, l)] = nv;
-    if (j == 0 && k == 0) narr[gidx(t, NX, NY, l)] = nv;
-    czm = cc; mzm = mc;
-    cc = czp; mc = mzp;
-    w = w_next;
+    const double diffu = cell1 ? t.dfo[cell1 - 1] : 0.0;
+    const double xm = at_f64(A + pl, o.xm), xp = at_f64(A + pl, o.xp), ym = at_f64(A + pl, o.ym),
+                 yp = at_f64(A + pl, o.yp);
+    atp_store(t, t.A1 + pl, o.c, j, k, atp_point(ak, t, o, l, c0, xm, xp, ym, yp, zm, zp, mk, w, diffu, inv_dx));
+    zm = c0;
+    c0 = zp;
+    w = wn;
   }
 }
 
-// ATP_refresh (:302-338) with the periodic copies of planes 0..iz_bound,
 // one tile of a solve's list: blockDim.x consecutive points of the (x, y)
-// plane times ZB planes (atp_column up to 2 planes, atp_column_roll above).
-template <int ZB>
-__device__ __forceinline__ void atp_tile(const Tis& ti, const CaArg& t, int local, int izb) {
+// plane times ZB planes; mg_npt: div_by's magic for its tiles per plane
+template <int ZB, class Off>
+__device__ __forceinline__ void atp_tile(const Tis& ti, const CaArg& t, unsigned local, unsigned mg_npt, int izb) {
   const int NX = t.NX, NY = t.NY;
-  const int bs = blockDim.x;
-  const int plane = NX * NY;
-  const int npt = (plane + bs - 1) / bs;
-  const int p = (local % npt) * bs + (int)threadIdx.x;
+  const unsigned bs = blockDim.x, plane = (unsigned)NX * NY;
+  const unsigned npt = (plane + bs - 1) / bs;
+  const unsigned zt = div_by(local, npt, mg_npt);
+  const unsigned p = (local - zt * npt) * bs + threadIdx.x;
   if (p >= plane) return;
-  const int j = p % NX, k = p / NX;
-  const int l0 = (local / npt) * ZB;
-  if (ZB >= 4) atp_column_roll(ti, t, j, k, l0, min(l0 + ZB, izb));
-  else atp_column<ZB>(ti, t, j, k, l0, min(l0 + ZB, izb));
+  const int k = (int)div_by(p, NX, t.mg_nx), j = (int)(p - (unsigned)k * NX);
+  const int l0 = (int)zt * ZB;
+  if (ZB >= 4) atp_column_roll<Off>(ti, t, j, k, l0, min(l0 + ZB, izb));
+  else atp_column<ZB, Off>(ti, t, j, k, l0, min(l0 + ZB, izb));
   // plane l = iz_bound: copies of values left in the next buffer (:334-337);
   // the corner (NX, NY) ends as a copy of (0, 0)
-  if (l0 == 0) {
+  if (l0 == 0 && (j == 0 || k == 0)) {
     double* __restrict__ narr = t.A1;
     if (k == 0) narr[gidx(t, j, NY, izb)] = narr[gidx(t, j, 0, izb)];
     if (j == 0) narr[gidx(t, NX, k, izb)] = narr[gidx(t, 0, k, izb)];
@@ -1062,13 +1076,13 @@ __device__ __forceinline__ void atp_tile(const Tis& ti, const CaArg& t, int loca
 // and tissue ids of up to CA_LDS_T tissues are staged in LDS (kept small: the
 // fused kernel's cell blocks hold LDS of their own)
 constexpr int CA_LDS_T = 256;
-template <int ZB, bool ONE>
+template <int ZB, bool ONE, class Off>
 __device__ __forceinline__ void atp_walk(const Tis* __restrict__ T, const CaList& cl, int b, int nb, int xcd, int ap,
                                          int cp) {
   if (ONE) {   // one tissue: its id and iz_bound come with the list
     const Tis& t = T[cl.t0];
     const CaArg a = ca_arg(t, cp, cp, ap);
-    for (TileWalk tw(cl.atiles, xcd, b, nb); tw.w < tw.end; tw.w += tw.stride) atp_tile<ZB>(t, a, tw.w, cl.izb0);
+    for (TileWalk tw(cl.atiles, xcd, b, nb); tw.w < tw.end; tw.w += tw.stride) atp_tile<ZB, Off>(t, a, tw.w, cl.mg_npt, cl.izb0);
     return;
   }
   const int nt = cl.ntis;
@@ -1089,13 +1103,14 @@ __device__ __forceinline__ void atp_walk(const Tis* __restrict__ T, const CaList
     ti = __builtin_amdgcn_readfirstlane(wl_find(off, ti, nt, tw.w));
     const int2 q = lds ? s_ti[ti] : make_int2(cl.atis[ti], cl.aizb[ti]);
     const Tis* t = T + __builtin_amdgcn_readfirstlane(q.x);
-    atp_tile<ZB>(*t, ca_arg(*t, cp, cp, ap), tw.w - __builtin_amdgcn_readfirstlane(off(ti)), __builtin_amdgcn_readfirstlane(q.y));
+    atp_tile<ZB, Off>(*t, ca_arg(*t, cp, cp, ap), tw.w - __builtin_amdgcn_readfirstlane(off(ti)), 0u,
+                      __builtin_amdgcn_readfirstlane(q.y));
   }
 }
 
-template <int ZB, bool ONE>
+template <int ZB, bool ONE, class Off>
 __global__ void __launch_bounds__(256) k_atp(const Tis* __restrict__ T, CaList cl, int ap, int cp, int xcd) {
-  atp_walk<ZB, ONE>(T, cl, blockIdx.x, gridDim.x, xcd, ap, cp);
+  atp_walk<ZB, ONE, Off>(T, cl, blockIdx.x, gridDim.x, xcd, ap, cp);
 }
 
 // one launch for the ATP update of sub-step i (parities cp, ap) and the cells
@@ -1130,7 +1145,7 @@ __global__ void __launch_bounds__(F_BLOCK) k_ca_fused(const Tis* __restrict__ T,
     an = (int)gridDim.x - ncb;
   }
   if (cbk < 0) {
-    atp_walk<ZB, ONE>(T, cl, ab, an, xcd, ap, cp);
+    atp_walk<ZB, ONE, unsigned>(T, cl, ab, an, xcd, ap, cp);
   } else if (ONE) {
     ca_cells_part<CG, true, SAVE>(T[cl.t0], one, cbk, ncb, SAVE ? sv + cl.t0 : nullptr, slot);
   } else {
@@ -1271,12 +1286,10 @@ void launch_ca_corners(hipStream_t s, const Tis* dT, const int* tlist, int ntis,
 }
 
 void launch_ca_begin(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int bp, int max_n,
-                     long long max_box, int zero_avg) {
+                     long long max_plane, int max_izb, int zero_avg) {
   EPI_LAUNCH(K_CA_BEGIN, k_ca_begin, dim3(ca_lane_blocks(max_n), ntis), dim3(256), 0, s, dT, tlist, cb, zero_avg);
-  unsigned gb = (unsigned)((max_box + 255) / 256);
-  if (gb < 1) gb = 1;
-  if (gb > 65535) gb = 65535;
-  EPI_LAUNCH(K_CA_VOX, k_ca_vox, dim3(gb, ntis), dim3(256), 0, s, dT, tlist);
+  const unsigned gb = (unsigned)std::max<long long>(1, std::min<long long>((max_plane + 255) / 256, 65535));
+  EPI_LAUNCH(K_CA_VOX, k_ca_vox, dim3(gb, ntis, (unsigned)std::max(1, std::min(max_izb, 65535))), dim3(256), 0, s, dT, tlist);
   launch_ca_corners(s, dT, tlist, ntis, bp, max_n);
 }
 
@@ -1331,9 +1344,9 @@ void launch_atp(hipStream_t s, const Tis* dT, const CaList& cl, int cp, int ap, 
   const dim3 g(walk_blocks(cl.atiles, cl.abs));
   by_zb(tu.a_zb, [&](auto zbc) {
     constexpr int zb = decltype(zbc)::value;
-    const auto k1 = k_atp<zb, true>, kn = k_atp<zb, false>;
-    if (cl.ntis == 1) EPI_LAUNCH(K_ATP, k1, g, dim3(cl.abs), 0, s, dT, cl, ap, cp, tu.xcd);
-    else EPI_LAUNCH(K_ATP, kn, g, dim3(cl.abs), 0, s, dT, cl, ap, cp, tu.xcd);
+    const auto k1 = k_atp<zb, true, unsigned>, kn = k_atp<zb, false, unsigned>,
+               kw = k_atp<zb, false, unsigned long long>;
+    EPI_LAUNCH(K_ATP, (cl.wide ? kw : cl.ntis == 1 ? k1 : kn), g, dim3(cl.abs), 0, s, dT, cl, ap, cp, tu.xcd);
   });
 }
 

@@ -108,7 +108,7 @@ void launch_ext_stim(hipStream_t s, const Tis* dT, int ntis, int bp, long long t
 // ca2p_avg cleared with zero_avg), voxel words, corners.  launch_ca_corners
 // alone renews what depends on B (buffer bp)
 void launch_ca_begin(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int cb, int bp, int max_n,
-                     long long max_box, int zero_avg);
+                     long long max_plane, int max_izb, int zero_avg);
 void launch_ca_corners(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int bp, int max_n);
 struct RdTis;
 // A Ca solve's work, flattened over its tissues (built on the host once per
@@ -127,6 +127,8 @@ struct CaList {
   int ntis, ncb, atiles, abs;
   int t0, izb0;
   const Tis* h0;   // host: that tissue's descriptor, passed to the kernels by value
+  unsigned mg_npt; // its tiles per plane, for div_by
+  bool wide;       // a plane of some tissue is past 32-bit byte offsets
 };
 // points per ATP tile of a solve: the fused kernel's block, or the ATP
 // kernel's 64 a_rows

@@ -11,12 +11,12 @@
 namespace epi {
 
 struct MechTis {
-  double* x0[2];      // snapshot of both position buffers, [0] = current
-  double* slot;       // positions of the states of one segment (slot-major, 3 * cap each)
-  double* ck;         // checkpoints (3 * cap each)
-  double* lam[2];     // position adjoints (3 * cap each)
-  double* target;     // 3 * cap: x, y, z
-  double* scal;       // [0] loss, [1] dL/deps, [2] dL/dK_TOTAL, [3] dL/dKspring, [4] dL/dKBEND
+  GPtr<double> x0[2];      // snapshot of both position buffers, [0] = current
+  GPtr<double> slot;       // positions of the states of one segment (slot-major, 3 * cap each)
+  GPtr<double> ck;         // checkpoints (3 * cap each)
+  GPtr<double> lam[2];     // position adjoints (3 * cap each)
+  GPtr<double> target;     // 3 * cap: x, y, z
+  GPtr<double> scal;       // [0] loss, [1] dL/deps, [2] dL/dK_TOTAL, [3] dL/dKspring, [4] dL/dKBEND
 };
 
 }  // namespace epi

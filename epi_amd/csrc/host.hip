@@ -86,7 +86,7 @@ const char* kKernelNames[K_COUNT] = {
     "k_finish", "k_snapshot", "k_zz_set", "k_zzmax", "k_map_clear", "k_map_stamp",
     "k_ext_stim", "k_ca_begin", "k_ca_vox", "k_ca_cells", "k_atp", "k_ca_end", "k_sw_reset",
     "k_rd_snapshot", "k_rd_restore", "k_rd_put_gj", "k_rd_state", "k_rd_seed",
-    "k_rd_step", "k_rd_gj0", "k_rd_own", "k_mech_state", "k_mech_seed", "k_mech_bwd_begin",
+    "k_rd_step", "k_rd_sums", "k_rd_own", "k_mech_state", "k_mech_seed", "k_mech_bwd_begin",
     "k_mech_bwd_pairs", "k_mech_bwd_memb", "k_ca_fused", "k_ca_corners", "k_sweep_wave", "k_wl", "k_ca_swap",
     "k_out_pack"};
 
@@ -1901,7 +1901,7 @@ int epi_rd_begin(epi_ctx* c, const double* zzmax) {
       r.h0 = cv.take<double>(cap); r.avg0 = cv.take<double>(cap); r.kpa0 = cv.take<double>(cap);
       r.g0 = cv.take<double>(cap * ns);
       for (int b = 0; b < 3; b++) r.lA[b] = cv.take<double>((size_t)r.box);
-      r.gkpa = cv.take<double>(cap); r.target = cv.take<double>(cap);
+      r.gkpa = cv.take<double>(cap); r.gdu = cv.take<double>(cap); r.gdp = cv.take<double>(cap); r.target = cv.take<double>(cap);
       r.kpa_in = cv.take<double>(cap); r.scal = cv.take<double>(4);
       const Tis& ti = c->tis[t];
       r.oc = (4 * ti.irx + 1) * (4 * ti.iry + 1) * (4 * ti.irz + 1);
@@ -2021,7 +2021,7 @@ int epi_rd_adjoint(epi_ctx* c, const epi_rd_params* prm, int32_t n_sub, int32_t 
       qa = qa == 2 ? 0 : qa + 1;
     }
   }
-  launch_rd_gj0(c->stream, c->d_tis, rd.d, c->T, q, items);
+  launch_rd_sums(c->stream, c->d_tis, rd.d, c->T, q, items);
   launch_ca_end(c->stream, c->d_tis, nullptr, c->T, c->cb, mn, CA_END_PUT);
   HIPCHK(c, hipGetLastError());
   RCHK(sync_status(c));

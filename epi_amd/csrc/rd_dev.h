@@ -28,7 +28,7 @@ struct RdTis {
   // ATP adjoint in three rotating buffers: [a] after the sub-step, [a+1]
   // before it, [a+2] dead (cleared for the next sub-step), a = step mod 3
   GPtr<double> lA[3];
-  GPtr<double> gkpa;                // dL/dkpa per cell
+  GPtr<double> gkpa, gdu, gdp;      // dL/dkpa per cell; each cell's share of dL/ddu and dL/ddp
   // the voxels each AFM cell owns in the window's frozen voxel map (its fa
   // source), up to oc per cell, in stamp-box order
   GPtr<int> own;

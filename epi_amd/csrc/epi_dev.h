@@ -32,9 +32,12 @@ enum { OK = 0, ERR_CAPACITY = 1, ERR_STRONG_INTERACTION = 2, ERR_NO_DERMIS = 3,
 constexpr int MEMB_ADJ = 6;                // define.h:147-153 (TRI_MEMB)
 constexpr int MAX_CONN = 400;              // define.h:80, cell_connection.cpp:30
 constexpr int N3 = 200;                    // cell_connection.cpp:28
-// slots between two buckets: the capacity rounded up to a multiple of 4, so
-// the sweep can read a bucket's indices four at a time (16-byte aligned)
-__host__ __device__ constexpr int bucket_stride(int bcap) { return (bcap + 3) & ~3; }
+// A bucket is a head of eight words, its count and its first seven cells (two
+// 16-byte loads), and the rest of its slots elsewhere: the five heads that a
+// sweep reads of a column lie in two or three cache lines.  Words between two
+// buckets' further slots: a multiple of 4, for 16-byte loads of four cells.
+constexpr int BUCKET_HEAD = 8;
+__host__ __device__ constexpr int bucket_more(int bcap) { return bcap < BUCKET_HEAD ? 4 : (bcap - (BUCKET_HEAD - 1) + 3) & ~3; }
 constexpr double AREA_GRID = 2.0 + 1e-7;   // cell_connection.cpp:16-19 (the bucket edge)
 
 // force laws (cell_interaction.cpp:68-76)
@@ -78,7 +81,7 @@ struct Status {
   double zzmax;
   long long timestep;     // CellManager::current_timestep; k_remove advances it once per renewal
   int nstat;              // records in cst_store
-  int pad_st;
+  int force_err;          // first error code of the force kernels, which run ahead of the status read-back
   long long grid_b;       // sum of nx*ny*iz_bound over the B sweeps (k_wl_b)
 };
 
@@ -127,7 +130,7 @@ struct Tis {
   // stencil neighbours and the CQ_ flags, and the point as it lies
   GPtr<uint4> ca_cq;
   GPtr<double> ca_bx;   // ca2p_by_ext_stim per AFM cell (B does not change during a solve)
-  GPtr<long long> uid; GPtr<long long> old_uid; GPtr<int> src_row;
+  GPtr<long long> uid; GPtr<long long> old_uid[2]; GPtr<int> src_row;
   // cell_stat (define.h:198-202): per cell k_aging_start, k_cornified,
   // k_disap (-1 = never set); cst_store (cellmanager.h:106): the records of
   // removed DEAD cells, up to cap of them, Status::nstat in use
@@ -138,8 +141,7 @@ struct Tis {
   GPtr<int> btmp; GPtr<int> bcnt;       // upper partners gathered during the sweep
   GPtr<int> memb6;                 // triangular adjacency, 6 per membrane cell
   // buckets
-  GPtr<int> bucket_of; GPtr<int> bslot; GPtr<int> bucket_n; GPtr<int> bucket_cells;
-  GPtr<int> bucket_sorted;   // the buckets in ascending cell index, written by k_bucket_sort for the sweep
+  GPtr<int> bucket_of; GPtr<int> bucket; GPtr<int> bucket_rest;
   // (x, y, z, radius) of every cell after the periodic fix, written by the
   // bucket insertion: the sweep and the row assembly gather a candidate's
   // position and radius with one 32-byte load instead of four
@@ -161,6 +163,9 @@ struct Tis {
 };
 
 __device__ __forceinline__ void set_err(Status* st, int e) { atomicCAS(&st->err, 0, e); }
+// of a force kernel: kept apart until the next renewal takes it over, so that
+// a step's status never shows an error of the step after it
+__device__ __forceinline__ void set_force_err(Status* st, int e) { atomicCAS(&st->force_err, 0, e); }
 
 // ---- geometry helpers: utils.h:25-53 ----------------------------------
 __device__ __forceinline__ double p_diff_x(const Tis& t, double x1, double x2) {

@@ -82,8 +82,8 @@ namespace {
 
 const char* kKernelNames[K_COUNT] = {
     "k_forces", "k_forces_long", "k_renew_flags", "k_renew_scan", "k_renew_apply", "k_remove", "k_pair_disperse",
-    "k_initialize_sc", "k_periodic_fix", "k_bucket_insert", "k_bucket_sort", "k_sweep",
-    "k_finish", "k_snapshot", "k_zz_set", "k_zzmax", "k_map_clear", "k_map_stamp",
+    "k_initialize_sc", "k_periodic_fix", "k_bucket_insert", "k_sweep",
+    "k_finish", "k_zz_set", "k_zzmax", "k_map_clear", "k_map_stamp",
     "k_ext_stim", "k_ca_begin", "k_ca_vox", "k_ca_cells", "k_atp", "k_ca_end", "k_sw_reset",
     "k_rd_snapshot", "k_rd_restore", "k_rd_put_gj", "k_rd_state", "k_rd_seed",
     "k_rd_step", "k_rd_sums", "k_rd_own", "k_mech_state", "k_mech_seed", "k_mech_bwd_begin",
@@ -156,7 +156,10 @@ struct epi_ctx {
   // join events order it with the main stream
   hipStream_t side_stream = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  hipEvent_t ev_st = nullptr;   // the status copy of a step, waited on alone
+  // a step's status read-back: the next step's force kernel writes h_st and
+  // then seq into every tissue's h_seq
+  unsigned long long* h_seq = nullptr;
+  unsigned long long seq = 0;
   int pb = 0, cb = 0, cp = 0, ap = 0, bp = 0;
   bool pos_pending = false;
   Tuning tu;
@@ -292,7 +295,7 @@ void carve_tissue(Carver& cv, TH& h, Tis& t) {
   t.ca_cq = cv.take<uint4>(cap * 8);
   t.ca_bx = cv.take<double>(cap);
   t.uid = cv.take<long long>(cap);
-  t.old_uid = cv.take<long long>(cap);
+  for (int b = 0; b < 2; b++) t.old_uid[b] = cv.take<long long>(cap);
   t.cst = cv.take<long long>(3 * cap);
   t.cst_store = cv.take<long long>(3 * cap);
   t.src_row = cv.take<int>(cap);
@@ -306,10 +309,8 @@ void carve_tissue(Carver& cv, TH& h, Tis& t) {
   t.bcnt = cv.take<int>(cap);
   t.memb6 = cv.take<int>((size_t)h.nmemb * 6);
   t.bucket_of = cv.take<int>(cap);
-  t.bslot = cv.take<int>(cap);
-  t.bucket_n = cv.take<int>(h.nbuckets);
-  t.bucket_cells = cv.take<int>((size_t)h.nbuckets * bucket_stride(h.bcap));
-  t.bucket_sorted = cv.take<int>((size_t)h.nbuckets * bucket_stride(h.bcap));
+  t.bucket = cv.take<int>((size_t)h.nbuckets * BUCKET_HEAD);
+  t.bucket_rest = cv.take<int>((size_t)h.nbuckets * bucket_more(h.bcap));
   t.pk = cv.take<double4>(cap);
   t.div_slot = cv.take<int>(cap);
   t.div_dir = cv.take<double>(3 * cap);
@@ -330,30 +331,44 @@ int check_tissue(epi_ctx* c, int t) {
   return EPI_OK;
 }
 
-// the status read-back, split so that work issued after the copy can run
-// while the host waits for the copy alone (sync_status_end with the stream
-// still busy leaves the timing events for a later read-back to resolve)
-// after issue_build: its k_snapshot has copied the statuses into h_st
-int sync_status_begin(epi_ctx* c) {
-  HIPCHK(c, hipEventRecord(c->ev_st, c->stream));
-  return EPI_OK;
-}
-int status_check(epi_ctx* c);
-int sync_status_end(epi_ctx* c) {
-  HIPCHK(c, hipEventSynchronize(c->ev_st));
+// The status read-back while the step's last force kernel is in the stream:
+// that kernel's first blocks write the statuses into h_st and then seq into
+// h_seq (system scope), and the host waits for those words alone, with no
+// event between the build and the forces.  A stream that ends or fails
+// without writing them ends the wait.  (The timing events of a stream still
+// busy are left for a later read-back to resolve.)
+int status_check(epi_ctx* c, bool early);
+int sync_status_early(epi_ctx* c) {
+  for (int t = 0; t < c->T; t++) {
+    const auto seen = [&] { return __atomic_load_n(c->h_seq + t, __ATOMIC_ACQUIRE) == c->seq; };
+    for (unsigned spin = 1; !seen(); spin++) {
+      __builtin_ia32_pause();
+      if (spin % 4096) continue;
+      const hipError_t e = hipStreamQuery(c->stream);
+      if (e == hipErrorNotReady) {
+        (void)hipGetLastError();   // not an error of a call
+        continue;
+      }
+      HIPCHK(c, e);
+      if (!seen()) return fail(c, EPI_ERR_HIP, "the status read-back did not arrive");
+    }
+  }
   if (!g_prof.pending.empty()) prof_resolve(true);
-  return status_check(c);
+  return status_check(c, true);
 }
 
 int sync_status(epi_ctx* c) {
   HIPCHK(c, hipMemcpyAsync(c->h_st, c->d_st, sizeof(Status) * c->T, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (!g_prof.pending.empty()) prof_resolve();
-  return status_check(c);
+  return status_check(c, false);
 }
 
-int status_check(epi_ctx* c) {
+// early: the next step's forces may be running; their errors are the next
+// read-back's
+int status_check(epi_ctx* c, bool early) {
   for (int t = 0; t < c->T; t++) {
+    if (!early && !c->h_st[t].err) c->h_st[t].err = c->h_st[t].force_err;
     c->th[t].n_est = c->h_st[t].n;
     // the device holds zzmax as bits (k_zzmax, set_zz); the host's double
     // follows them, so the Ca lists' iz_bound is the device's
@@ -811,7 +826,6 @@ int epi_create(int32_t ntissues, const epi_geometry* geos, epi_ctx** out) {
   if (hipStreamCreate(&c->side_stream) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&c->ev_st, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->ev_cal, hipEventDisableTiming) != hipSuccess) {
     epi_destroy(c);
     return EPI_ERR_HIP;
@@ -823,7 +837,8 @@ int epi_create(int32_t ntissues, const epi_geometry* geos, epi_ctx** out) {
       hipMalloc(&c->d_wl, sizeof(int) * WL_INTS(ntissues)) != hipSuccess ||
       hipMalloc(&c->d_cal, sizeof(int) * c->cal_ints) != hipSuccess ||
       hipHostMalloc(&c->h_cal, sizeof(int) * c->cal_ints, hipHostMallocDefault) != hipSuccess ||
-      hipHostMalloc(&c->h_st, sizeof(Status) * ntissues, hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc(&c->h_st, sizeof(Status) * ntissues, hipHostMallocCoherent) != hipSuccess ||
+      hipHostMalloc(&c->h_seq, sizeof(unsigned long long) * ntissues, hipHostMallocCoherent) != hipSuccess ||
       hipHostMalloc(&c->h_zz, sizeof(double) * ntissues, hipHostMallocDefault) != hipSuccess ||
       hipHostMalloc(&c->h_tlist, sizeof(int) * ntissues, hipHostMallocDefault) != hipSuccess) {
     epi_destroy(c);
@@ -835,6 +850,7 @@ int epi_create(int32_t ntissues, const epi_geometry* geos, epi_ctx** out) {
     return EPI_ERR_HIP;
   }
   memset(c->h_st, 0, sizeof(Status) * ntissues);
+  memset(c->h_seq, 0, sizeof(unsigned long long) * ntissues);
   Carver real{c->arena, 0, false};
   for (int t = 0; t < ntissues; t++) {
     carve_tissue(real, c->th[t], c->tis[t]);
@@ -887,13 +903,13 @@ void epi_destroy(epi_ctx* c) {
   if (c->h_cal) (void)hipHostFree(c->h_cal);
   if (c->ev_cal) (void)hipEventDestroy(c->ev_cal);
   if (c->h_st) (void)hipHostFree(c->h_st);
+  if (c->h_seq) (void)hipHostFree(c->h_seq);
   if (c->h_zz) (void)hipHostFree(c->h_zz);
   if (c->h_tlist) (void)hipHostFree(c->h_tlist);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   if (c->side_stream) (void)hipStreamDestroy(c->side_stream);
   if (c->ev_fork) (void)hipEventDestroy(c->ev_fork);
   if (c->ev_join) (void)hipEventDestroy(c->ev_join);
-  if (c->ev_st) (void)hipEventDestroy(c->ev_st);
   for (auto& g : c->graphs) (void)hipGraphExecDestroy(g.exec);
   delete c;
 }
@@ -957,7 +973,7 @@ int epi_load_cells(epi_ctx* c, int32_t t, const epi_cell_input* in) {
   RCHK(upload(c, ti.nlen[0], nl.data(), n));
   RCHK(upload(c, ti.nlen[1], nl.data(), n));
   RCHK(upload(c, ti.uid, uid.data(), n));
-  RCHK(upload(c, ti.old_uid, uid.data(), n));
+  for (int b = 0; b < 2; b++) RCHK(upload(c, ti.old_uid[b], uid.data(), n));
   for (int b = 0; b < 2; b++) {
     RCHK(upload(c, ti.pos[b][0], in->x, n));
     RCHK(upload(c, ti.pos[b][1], in->y, n));
@@ -1259,7 +1275,7 @@ hipError_t issue_build(epi_ctx* c, int mn, int nb, int izb, bool join = true) {
   // beside the sweep) or after the whole build (1: the sweep runs alone and
   // the maps beside the next forces)
   if (!c->tu.side_fork) chk(hipEventRecord(c->ev_fork, c->stream));
-  launch_connect_rest(c->stream, c->d_tis, c->T, c->pb, nb, mn, c->tu.sweep_wave, c->h_st);
+  launch_connect_rest(c->stream, c->d_tis, c->T, c->pb, nb, mn, c->tu.sweep_wave);
   if (c->tu.side_fork) chk(hipEventRecord(c->ev_fork, c->stream));
   chk(hipStreamWaitEvent(c->side_stream, c->ev_fork, 0));
   launch_map_stamp(c->side_stream, c->d_tis, c->T, c->pb, mn, c->tu);
@@ -1280,8 +1296,8 @@ hipError_t issue_build(epi_ctx* c, int mn, int nb, int izb, bool join = true) {
 int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
   constexpr unsigned long long seg =
       (1ull << K_RENEW_FLAGS) | (1ull << K_RENEW_SCAN) | (1ull << K_RENEW_APPLY) | (1ull << K_REMOVE) |
-      (1ull << K_PAIR_DISPERSE) | (1ull << K_BUCKET_INSERT) | (1ull << K_BUCKET_SORT) | (1ull << K_SWEEP_WAVE) |
-      (1ull << K_SWEEP) | (1ull << K_FINISH) | (1ull << K_SNAPSHOT) | (1ull << K_ZZ_SET) | (1ull << K_ZZMAX) |
+      (1ull << K_PAIR_DISPERSE) | (1ull << K_BUCKET_INSERT) | (1ull << K_SWEEP_WAVE) |
+      (1ull << K_SWEEP) | (1ull << K_FINISH) | (1ull << K_ZZ_SET) | (1ull << K_ZZMAX) |
       (1ull << K_MAP_CLEAR) | (1ull << K_MAP_STAMP) | (1ull << K_EXT_STIM);
   if (!c->tu.step_graph || (g_prof.mask & seg)) {
     *joined = false;
@@ -1347,14 +1363,14 @@ int epi_step(epi_ctx* c, int64_t nsteps, epi_driver* drv) {
       // B sweep (side stream) run on beside the next forces, which read
       // neither, and what the main stream issues after those forces (the
       // next renewal, a solve) waits for them.
-      RCHK(sync_status_begin(c));
       forces_pb = c->pb;
-      forces_cap = launch_forces_rows(c->stream, c->d_tis, c->T, c->pb, c->cb, cap_n, known_len);
+      forces_cap = launch_forces_rows(c->stream, c->d_tis, c->T, c->pb, c->cb, cap_n, known_len,
+                                      StatusOut{c->h_st, c->h_seq, ++c->seq});
       c->pb ^= 1;
       forces_issued = true;
       if (!joined) HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
       HIPCHK(c, hipGetLastError());
-      RCHK(sync_status_end(c));
+      RCHK(sync_status_early(c));
     } else {
       if (!joined) HIPCHK(c, hipStreamWaitEvent(c->stream, c->ev_join, 0));
       HIPCHK(c, hipGetLastError());
@@ -1773,7 +1789,7 @@ int epi_set_lists(epi_ctx* c, int32_t t, const int32_t* ptr, const int32_t* conn
   RCHK(upload(c, ti.nlen[c->cb], nl.data(), n));
   RCHK(upload(c, ti.nlo, nlo.data(), n));
   RCHK(upload(c, ti.src_row, srow.data(), n));
-  RCHK(upload(c, ti.old_uid, u.data(), n));
+  RCHK(upload(c, ti.old_uid[c->cb], u.data(), n));
   return EPI_OK;
 }
 

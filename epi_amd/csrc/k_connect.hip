@@ -5,15 +5,13 @@
 //   [6 membrane neighbours if MEMB] ++ [partners o < X found by X's own
 //   5x5x5 bucket sweep, in sweep order] ++ [partners c > X, ascending c].
 // k_bucket_insert  places cells in fixed-capacity buckets (grid_init :38-62),
-// k_bucket_sort    ranks each cell in its bucket by cell index (the serial
-//                  insertion order) and writes it to that slot of a second
-//                  copy of the buckets,
 // k_sweep          runs connect_proc (:70-129) for every non-membrane cell:
 //                  the lower part of its own row is written directly, the
 //                  upper parts of its partners are appended with atomics,
 // k_finish         sorts the upper parts, carries gap-junction
 //                  values over from the previous rows by cell uid
-//                  (gj_refresh :133-152) and picks the dermis (:158-185).
+//                  (gj_refresh :133-152), picks the dermis (:158-185) and
+//                  leaves the buckets empty for the next build.
 #include "epi_dev.h"
 #include "launch.h"
 #include "epi_group.h"
@@ -67,7 +65,6 @@ __device__ __forceinline__ void insert_cells(const Tis& t, int pb, int fix, bool
     t.pk[c] = make_double4(x, y, z, r);
     t.bcnt[c] = 0;
     t.nlo[c] = 0;
-    t.bslot[c] = -1;
     if (aix >= t.ANX || aiy >= t.ANY || aiz >= t.ANZ || aix < 0 || aiy < 0 || aiz < 0) {
       set_err(st, ERR_OUT_OF_GRID);
       t.bucket_of[c] = -1;
@@ -75,11 +72,12 @@ __device__ __forceinline__ void insert_cells(const Tis& t, int pb, int fix, bool
     }
     const int b = (int)((aix * t.ANY + aiy) * t.ANZ + aiz);
     t.bucket_of[c] = b;
-    const int slot = atomicAdd(&t.bucket_n[b], 1);
+    int* const head = t.bucket + (size_t)b * BUCKET_HEAD;
+    const int slot = atomicAdd(head, 1);
     // the reference asserts fewer than N3 = 200 cells per bucket (:59)
     if (slot + 1 >= N3 || slot >= t.bcap) { set_err(st, ERR_CAPACITY); continue; }
-    t.bucket_cells[(size_t)b * bucket_stride(t.bcap) + slot] = c;
-    t.bslot[c] = slot;
+    if (slot < BUCKET_HEAD - 1) head[1 + slot] = c;
+    else t.bucket_rest[(size_t)b * bucket_more(t.bcap) + slot - (BUCKET_HEAD - 1)] = c;
   }
   if (step) zzmax_add(st, zmax);
 }
@@ -91,44 +89,30 @@ __global__ void __launch_bounds__(256) k_bucket_insert(const Tis* __restrict__ T
   else insert_cells(t, pb, fix, STEP, cell_blocks);
 }
 
-// each bucket in ascending cell index: every cell counts the cells of its
-// bucket with a smaller index (its rank, kept in bslot) and writes itself to
-// that slot of bucket_sorted, the copy the sweep reads.  A bucket holds
-// distinct cells, so the ranks of its m cells are 0 .. m - 1.
-__global__ void __launch_bounds__(256) k_bucket_sort(const Tis* __restrict__ T) {
-  const Tis& t = T[blockIdx.y];
-  const int n = t.st->n;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
-    if (t.bslot[c] < 0) continue;
-    const int b = t.bucket_of[c];
-    const int m = min(t.bucket_n[b], t.bcap);
-    const size_t base = (size_t)b * bucket_stride(t.bcap);
-    const int* a = t.bucket_cells + base;
-    int rank = 0;
-    // four slots per 16-byte load (a bucket's slots start 16-byte aligned and
-    // its stride is a multiple of 4); slots from m on are not counted
-    for (int i = 0; i < m; i += 4) {
-      const int4 q = *reinterpret_cast<const int4*>(a + i);
-      rank += (q.x < c) + (i + 1 < m && q.y < c) + (i + 2 < m && q.z < c) + (i + 3 < m && q.w < c);
-    }
-    t.bslot[c] = rank;
-    t.bucket_sorted[base + rank] = c;
-  }
-}
-
 // connect_proc (:70-129): the 5x5x5 sweep, periodic in x, y and z, buckets
 // in ascending (j, k, l) with cells in ascending index inside a bucket.
-// A group of 32 lanes takes one cell; lane g < 25 sweeps the column
-// (j, k) = (g / 5, g % 5) over its 5 z buckets.  Lanes count their partners
-// (keeping the first SWEEP_H of them in LDS), an exclusive scan over the
-// group gives each lane its place in the row, and the lane writes its
-// partners there -- the row comes out in sweep order.  A lane with more than
-// SWEEP_H partners sweeps its column a second time.
-constexpr int SWEEP_G = 32;
-constexpr int SWEEP_H = 8;
+// A group of G = 32 lanes (64: a launch shape for few cells) takes one cell.
+//
+// What bounds it is the chain of memory round trips where the GPU is mostly
+// idle and the instructions where it is full, so the group works on a flat
+// list of candidates: a lane asks for the heads of 128 / G consecutive buckets
+// of the 125 in sweep order at once (bucket q is (j, k, l) = (q / 25,
+// q / 5 % 5, q % 5); a head is its count and seven cells), the cells below the group's own go to a list in LDS with their bucket, and
+// the lanes take the list's entries in turn, so a position is read and tested
+// only for a real candidate and no lane waits for a full column.  The hits
+// are put in sweep order by rank of (bucket, cell), which needs no order in
+// the buckets, and the lanes take them in turn again for the appends to the
+// partners' rows (an atomic whose result the store needs).  More candidates
+// or hits than the lists hold go through sweep_crowded.
+// Measured against buckets sorted by a launch of their own and one column of
+// five buckets per lane, walked one after the other, sort and sweep: 16.1 ->
+// 9.5 us (a tissue of 420 cells), 26.7 -> 12.2 (4,300), 45.2 -> 35.8 (36,400),
+// 290 -> 280 (32 tissues, 292,000 cells).
+constexpr int SWEEP_C = 384;   // candidates of a cell
+constexpr int SWEEP_H = 64;    // hits of a cell
+constexpr int SWEEP_Q = 36;    // a hit's key: its bucket above the cell index
 
-__device__ __forceinline__ bool sweep_hit(const Tis& t, const P3& pc, double rc, int o) {
-  const double4 po = t.pk[o];
+__device__ __forceinline__ bool sweep_hit(const Tis& t, const P3& pc, double rc, const double4& po) {
   const double diffx = p_diff_x(t, pc.x, po.x);
   const double diffy = p_diff_y(t, pc.y, po.y);
   const double diffz = pc.z - po.z;
@@ -137,210 +121,199 @@ __device__ __forceinline__ bool sweep_hit(const Tis& t, const P3& pc, double rc,
   return diffx * diffx + diffy * diffy + diffz * diffz <= lj * lj * rad_sum * rad_sum;
 }
 
-__global__ void __launch_bounds__(256) k_sweep(const Tis* __restrict__ T, int pb, int nb) {
-  const Tis& t = T[blockIdx.y];
-  Status* st = t.st;
-  const int n = st->n;
-  const int ANX = t.ANX, ANY = t.ANY, ANZ = t.ANZ;
-  const int lane = threadIdx.x & (SWEEP_G - 1);
-  const int groups = gridDim.x * (blockDim.x / SWEEP_G);
-  __shared__ int s_hit[256][SWEEP_H];
-  int* const hits = s_hit[threadIdx.x];
-  int* const col = t.col[nb];
-  for (int c = t.nmemb + blockIdx.x * (blockDim.x / SWEEP_G) + threadIdx.x / SWEEP_G; c < n; c += groups) {
-    const double4 pq = t.pk[c];
-    const P3 pc{pq.x, pq.y, pq.z};
-    const double rc = pq.w;
-    const long anx = (long)(pc.x / AREA_GRID);
-    const long any = (long)(pc.y / AREA_GRID);
-    const long anz = (long)(pc.z / AREA_GRID);
-    const bool bad = anx >= ANX || any >= ANY || anz >= ANZ || anx < 0 || any < 0 || anz < 0;
-    if (bad) {
-      if (lane == 0) set_err(st, ERR_OUT_OF_GRID);
-      continue;
-    }
-    const bool act = lane < 25;
-    const long aix = (anx - 2 + lane / 5 + ANX) % ANX;
-    const long aiy = (any - 2 + lane % 5 + ANY) % ANY;
-    const long bxy = (aix * ANY + aiy) * ANZ;
-    int cnt = 0;
-    if (act) {
-      int sz[5];
-#pragma unroll
-      for (int i = 0; i < 5; i++) sz[i] = min(t.bucket_n[bxy + (anz - 2 + i + ANZ) % ANZ], t.bcap);
-      // a bucket's indices four at a time (one 16-byte load: a bucket's
-      // slots start 16-byte aligned and its stride is a multiple of 4), then those
-      // candidates' positions together; the walk stops at the first index
-      // >= c (ascending within the bucket)
-#pragma unroll
-      for (int i = 0; i < 5; i++) {
-        const int* cells = t.bucket_sorted + (size_t)(bxy + (anz - 2 + i + ANZ) % ANZ) * bucket_stride(t.bcap);
-        bool done = false;
-        for (int m0 = 0; m0 < sz[i] && !done; m0 += 4) {
-          const int4 q = *reinterpret_cast<const int4*>(cells + m0);
-          const int o4[4] = {q.x, q.y, q.z, q.w};
-          bool hit[4];
-#pragma unroll
-          for (int u = 0; u < 4; u++) hit[u] = m0 + u < sz[i] && o4[u] < c && sweep_hit(t, pc, rc, o4[u]);
-#pragma unroll
-          for (int u = 0; u < 4; u++) {
-            if (done || m0 + u >= sz[i]) continue;
-            if (c <= o4[u]) { done = true; continue; }
-            if (hit[u]) {
-              if (cnt < SWEEP_H) hits[cnt] = o4[u];
-              cnt++;
-            }
-          }
-        }
-      }
-    }
-    int total;
-    int off = group_exclusive_scan<SWEEP_G>(cnt, lane, &total);
-    if (cnt) {
-      int* const row = col + (size_t)c * t.ns;
-      if (cnt <= SWEEP_H) {
-        for (int i = 0; i < cnt; i++, off++) {
-          const int o = hits[i];
-          if (off < t.ns) row[off] = o;
-          const int slot = atomicAdd(&t.bcnt[o], 1);
-          if (slot < t.ns) t.btmp[(size_t)o * t.ns + slot] = c;
-        }
-      } else {
-        for (long l = anz - 2 + ANZ; l <= anz + 2 + ANZ; l++) {
-          const long b = bxy + l % ANZ;
-          const int sz = min(t.bucket_n[b], t.bcap);
-          const int* cells = t.bucket_sorted + (size_t)b * bucket_stride(t.bcap);
-          for (int m = 0; m < sz; ++m) {
-            const int o = cells[m];
-            if (c <= o) break;
-            if (sweep_hit(t, pc, rc, o)) {
-              if (off < t.ns) row[off] = o;
-              off++;
-              const int slot = atomicAdd(&t.bcnt[o], 1);
-              if (slot < t.ns) t.btmp[(size_t)o * t.ns + slot] = c;
-            }
-          }
-        }
-      }
-    }
-    if (lane == 0) t.nlo[c] = total;
-  }
+// v mod A for the indices a sweep meets: 0 <= v < 2 A + 2, or any v where A = 1
+__device__ __forceinline__ int wrap_index(int v, int A) {
+  v -= v >= A ? A : 0;
+  v -= v >= A ? A : 0;
+  return A == 1 ? 0 : v;
+}
+struct SweepAt { int x, y, z; };   // the bucket a sweep is around
+__device__ __forceinline__ int sweep_bucket(const Tis& t, const SweepAt& at, int q) {
+  const int bx = wrap_index(at.x - 2 + q / 25 + t.ANX, t.ANX), by = wrap_index(at.y - 2 + q / 5 % 5 + t.ANY, t.ANY),
+            bz = wrap_index(at.z - 2 + q % 5 + t.ANZ, t.ANZ);
+  return (bx * t.ANY + by) * t.ANZ + bz;
 }
 
-// The same sweep with one wave per cell, for small tissues, whose few cells
-// leave the GPU mostly idle: lane g takes the buckets 2g and 2g + 1 of the
-// 125 in sweep order (bucket q is (j, k, l) = (q / 25, q / 5 % 5, q % 5)).
-// A lane issues both bucket counts, then both buckets' first four indices,
-// then those eight candidates' positions, so a sweep waits for three memory
-// round trips; buckets of more than four cells walk on four at a time.  The
-// wave's scan places each lane's partners, so the row is the same.  Twice
-// the lanes per cell cost more where the GPU is full (a launch shape chosen
-// by the tuner).
-constexpr int SWEEP_W = 64;
+__device__ __forceinline__ void sweep_append(const Tis& t, int c, int o) {
+  const int slot = atomicAdd(&t.bcnt[o], 1);
+  if (slot < t.ns) t.btmp[(size_t)o * t.ns + slot] = c;
+}
 
-__global__ void __launch_bounds__(256) k_sweep_wave(const Tis* __restrict__ T, int pb, int nb) {
+// a sweep of any size, without lists: each lane counts its buckets' hits, and
+// writes them in order, each time the least cell above the last one
+template <int G>
+__device__ __forceinline__ int sweep_crowded(const Tis& t, int c, const P3& pc, double rc, const SweepAt& at, int lane,
+                                             int* row) {
+  constexpr int NB = 128 / G;
+  const int q1 = min(NB * lane + NB, 125);
+  auto cell = [&](int b, int m) -> int {
+    return m < BUCKET_HEAD - 1 ? t.bucket[(size_t)b * BUCKET_HEAD + 1 + m]
+                               : t.bucket_rest[(size_t)b * bucket_more(t.bcap) + m - (BUCKET_HEAD - 1)];
+  };
+  int cnt = 0;
+  for (int q = NB * lane; q < q1; q++) {
+    const int b = sweep_bucket(t, at, q);
+    const int sz = min(t.bucket[(size_t)b * BUCKET_HEAD], t.bcap);
+    for (int m = 0; m < sz; m++) {
+      const int o = cell(b, m);
+      cnt += o < c && sweep_hit(t, pc, rc, t.pk[o]);
+    }
+  }
+  int total;
+  int off = group_exclusive_scan<G>(cnt, lane, &total);
+  if (cnt)
+    for (int q = NB * lane; q < q1; q++) {
+      const int b = sweep_bucket(t, at, q);
+      const int sz = min(t.bucket[(size_t)b * BUCKET_HEAD], t.bcap);
+      for (int last = -1;;) {
+        int best = c;
+        for (int m = 0; m < sz; m++) {
+          const int o = cell(b, m);
+          if (o > last && o < best && sweep_hit(t, pc, rc, t.pk[o])) best = o;
+        }
+        if (best == c) break;
+        if (off < t.ns) row[off] = best;
+        off++;
+        sweep_append(t, c, best);
+        last = best;
+      }
+    }
+  return total;
+}
+
+template <int G>
+__global__ void __launch_bounds__(256) k_sweep(const Tis* __restrict__ T, int pb, int nb) {
+  constexpr int NB = 128 / G;   // buckets of a lane
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;
   const int n = st->n;
-  const int ANX = t.ANX, ANY = t.ANY, ANZ = t.ANZ;
-  const int lane = threadIdx.x & (SWEEP_W - 1);
-  const int groups = gridDim.x * (blockDim.x / SWEEP_W);
-  __shared__ int s_hit[256][SWEEP_H];
-  int* const hits = s_hit[threadIdx.x];
+  const int ANX = t.ANX, ANY = t.ANY, ANZ = t.ANZ, bcap = t.bcap, ns = t.ns;
+  const int lane = threadIdx.x & (G - 1);
+  const int groups = gridDim.x * (blockDim.x / G);
+  __shared__ int s_cand[256 / G][SWEEP_C];
+  __shared__ uint8_t s_cq[256 / G][SWEEP_C];
+  __shared__ unsigned long long s_hit[256 / G][SWEEP_H];
+  int* const cand = s_cand[threadIdx.x / G];
+  uint8_t* const cq = s_cq[threadIdx.x / G];
+  unsigned long long* const hits = s_hit[threadIdx.x / G];
+  const unsigned long long below = (1ull << lane) - 1;   // lanes of the group before this one
+  // a ballot's bits of this group
+  auto group_bits = [&](bool p) {
+    const unsigned long long b = __ballot(p);
+    return G == 64 ? b : b >> (threadIdx.x & 32) & 0xffffffffull;
+  };
   int* const col = t.col[nb];
-  const int bstride = bucket_stride(t.bcap);
-  for (int c = t.nmemb + blockIdx.x * (blockDim.x / SWEEP_W) + threadIdx.x / SWEEP_W; c < n; c += groups) {
+  for (int c = t.nmemb + blockIdx.x * (blockDim.x / G) + threadIdx.x / G; c < n; c += groups) {
     const double4 pq = t.pk[c];
     const P3 pc{pq.x, pq.y, pq.z};
     const double rc = pq.w;
-    const long anx = (long)(pc.x / AREA_GRID);
-    const long any = (long)(pc.y / AREA_GRID);
-    const long anz = (long)(pc.z / AREA_GRID);
-    const bool bad = anx >= ANX || any >= ANY || anz >= ANZ || anx < 0 || any < 0 || anz < 0;
+    const long lx = (long)(pc.x / AREA_GRID);
+    const long ly = (long)(pc.y / AREA_GRID);
+    const long lz = (long)(pc.z / AREA_GRID);
+    const bool bad = lx >= ANX || ly >= ANY || lz >= ANZ || lx < 0 || ly < 0 || lz < 0;
     if (bad) {
       if (lane == 0) set_err(st, ERR_OUT_OF_GRID);
       continue;
     }
-    long bk[2];
-    int sz[2];
+    const SweepAt at{(int)lx, (int)ly, (int)lz};
+    int bk[NB];
+    int4 w4[NB][2];
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-      const int q = 2 * lane + u;
-      bk[u] = ((((anx - 2 + q / 25) + ANX) % ANX) * ANY + ((any - 2 + q / 5 % 5) + ANY) % ANY) * ANZ +
-              ((anz - 2 + q % 5) + ANZ) % ANZ;
-      sz[u] = q < 125 ? min(t.bucket_n[bk[u]], t.bcap) : 0;
+    for (int u = 0; u < NB; u++) {
+      bk[u] = sweep_bucket(t, at, min(NB * lane + u, 124));   // past the last: its head again, counted empty below
+      const int4* const head = reinterpret_cast<const int4*>(t.bucket + (size_t)bk[u] * BUCKET_HEAD);
+      w4[u][0] = head[0];
+      w4[u][1] = head[1];
     }
-    int4 q4[2];
+    int sz[NB], cnt = 0, most = 0;
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-      q4[u] = make_int4(0x7fffffff, 0x7fffffff, 0x7fffffff, 0x7fffffff);
-      if (sz[u] > 0) q4[u] = *reinterpret_cast<const int4*>(t.bucket_sorted + (size_t)bk[u] * bstride);
+    for (int u = 0; u < NB; u++) {
+      sz[u] = NB * lane + u < 125 ? min(w4[u][0].x, bcap) : 0;
+      most = max(most, sz[u]);
+      const int w[7] = {w4[u][0].y, w4[u][0].z, w4[u][0].w, w4[u][1].x, w4[u][1].y, w4[u][1].z, w4[u][1].w};
+#pragma unroll
+      for (int v = 0; v < 7; v++) cnt += v < sz[u] && w[v] < c;   // a slot past the count holds a past build's cell
     }
-    bool hit[2][4];
+    int nc;
+    int at_c = group_exclusive_scan<G>(cnt, lane, &nc);
+    if (nc <= SWEEP_C) {
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-      const int o4[4] = {q4[u].x, q4[u].y, q4[u].z, q4[u].w};
+      for (int u = 0; u < NB; u++) {
+        const int w[7] = {w4[u][0].y, w4[u][0].z, w4[u][0].w, w4[u][1].x, w4[u][1].y, w4[u][1].z, w4[u][1].w};
 #pragma unroll
-      for (int v = 0; v < 4; v++) hit[u][v] = v < sz[u] && o4[v] < c && sweep_hit(t, pc, rc, o4[v]);
-    }
-    int cnt = 0;
-#pragma unroll
-    for (int u = 0; u < 2; u++) {
-      const int o4[4] = {q4[u].x, q4[u].y, q4[u].z, q4[u].w};
-#pragma unroll
-      for (int v = 0; v < 4; v++)
-        if (hit[u][v]) {
-          if (cnt < SWEEP_H) hits[cnt] = o4[v];
-          cnt++;
-        }
-      // the rest of a bucket of more than four cells whose first four lie below c
-      if (sz[u] > 4 && q4[u].w < c) {
-        const int* cells = t.bucket_sorted + (size_t)bk[u] * bstride;
-        bool done = false;
-        for (int m0 = 4; m0 < sz[u] && !done; m0 += 4) {
-          const int4 q = *reinterpret_cast<const int4*>(cells + m0);
-          const int o4b[4] = {q.x, q.y, q.z, q.w};
-          bool h[4];
-#pragma unroll
-          for (int v = 0; v < 4; v++) h[v] = m0 + v < sz[u] && o4b[v] < c && sweep_hit(t, pc, rc, o4b[v]);
-#pragma unroll
-          for (int v = 0; v < 4; v++) {
-            if (done || m0 + v >= sz[u]) continue;
-            if (c <= o4b[v]) { done = true; continue; }
-            if (h[v]) {
-              if (cnt < SWEEP_H) hits[cnt] = o4b[v];
-              cnt++;
-            }
+        for (int v = 0; v < 7; v++)
+          if (v < sz[u] && w[v] < c) {
+            cand[at_c] = w[v];
+            cq[at_c++] = (uint8_t)(NB * lane + u);
           }
+      }
+    }
+    // buckets of more than seven cells: four more of each at a time
+    for (int m0 = BUCKET_HEAD - 1; nc <= SWEEP_C && group_bits(m0 < most); m0 += 4) {
+#pragma unroll
+      for (int u = 0; u < NB; u++)
+        w4[u][0] = *reinterpret_cast<const int4*>(t.bucket_rest + (size_t)bk[u] * bucket_more(bcap) +
+                                                  (m0 < sz[u] ? m0 - (BUCKET_HEAD - 1) : 0));
+      int more = 0;
+#pragma unroll
+      for (int u = 0; u < NB; u++) {
+        const int w[4] = {w4[u][0].x, w4[u][0].y, w4[u][0].z, w4[u][0].w};
+#pragma unroll
+        for (int v = 0; v < 4; v++) more += m0 + v < sz[u] && w[v] < c;
+      }
+      int add;
+      int at_m = nc + group_exclusive_scan<G>(more, lane, &add);
+      nc += add;
+      if (nc > SWEEP_C) break;
+#pragma unroll
+      for (int u = 0; u < NB; u++) {
+        const int w[4] = {w4[u][0].x, w4[u][0].y, w4[u][0].z, w4[u][0].w};
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          if (m0 + v < sz[u] && w[v] < c) {
+            cand[at_m] = w[v];
+            cq[at_m++] = (uint8_t)(NB * lane + u);
+          }
+      }
+    }
+    int total = 0;
+    if (nc <= SWEEP_C) {
+      wave_sync();
+      // 2 G candidates at a time, both positions asked for together
+      for (int i0 = 0; i0 < nc; i0 += 2 * G) {
+        int o[2], q[2];
+        double4 po[2];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+          const int i = i0 + k * G + lane;
+          o[k] = i < nc ? cand[i] : c;
+          q[k] = i < nc ? cq[i] : 0;
+          po[k] = t.pk[o[k]];
+        }
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+          const bool hit = o[k] != c && sweep_hit(t, pc, rc, po[k]);
+          const unsigned long long hb = group_bits(hit);
+          const int i = total + __popcll(hb & below);
+          if (hit && i < SWEEP_H) hits[i] = (unsigned long long)q[k] << SWEEP_Q | (unsigned)o[k];
+          total += __popcll(hb);
         }
       }
     }
-    int total;
-    int off = group_exclusive_scan<SWEEP_W>(cnt, lane, &total);
-    if (cnt) {
-      int* const row = col + (size_t)c * t.ns;
-      if (cnt <= SWEEP_H) {
-        for (int i = 0; i < cnt; i++, off++) {
-          const int o = hits[i];
-          if (off < t.ns) row[off] = o;
-          const int slot = atomicAdd(&t.bcnt[o], 1);
-          if (slot < t.ns) t.btmp[(size_t)o * t.ns + slot] = c;
-        }
-      } else {
-        for (int u = 0; u < 2; u++) {
-          const int* cells = t.bucket_sorted + (size_t)bk[u] * bstride;
-          for (int m = 0; m < sz[u]; ++m) {
-            const int o = cells[m];
-            if (c <= o) break;
-            if (sweep_hit(t, pc, rc, o)) {
-              if (off < t.ns) row[off] = o;
-              off++;
-              const int slot = atomicAdd(&t.bcnt[o], 1);
-              if (slot < t.ns) t.btmp[(size_t)o * t.ns + slot] = c;
-            }
-          }
-        }
+    int* const row = col + (size_t)c * ns;
+    if (nc > SWEEP_C || total > SWEEP_H) {
+      total = sweep_crowded<G>(t, c, pc, rc, at, lane, row);
+    } else {
+      wave_sync();
+      for (int i = lane; i < total; i += G) {
+        const unsigned long long key = hits[i];
+        const int o = (int)key;   // the key's low 32 bits
+        int rk = 0;
+        for (int k = 0; k < total; k++) rk += hits[k] < key;
+        if (rk < ns) row[rk] = o;
+        sweep_append(t, c, o);
       }
+      wave_sync();   // the lists are the next cell's from here
     }
     if (lane == 0) t.nlo[c] = total;
   }
@@ -349,16 +322,24 @@ __global__ void __launch_bounds__(256) k_sweep_wave(const Tis* __restrict__ T, i
 // Row assembly, gj carry-over and dermis.  A group of KG lanes owns one
 // cell.  Rows of at most KCAP entries are assembled in LDS: the lower part
 // (written by k_sweep in sweep order) and the upper partners (gathered in
-// k_sweep in arbitrary order, placed here by rank since they are distinct).
-// The previous row's uids and gj values are staged in LDS too and each lane resolves the
-// gap junction of its entries there (gj_refresh :133-152: a directed edge
-// keeps its value while it stays in the list, a new edge starts at gj_init).
+// k_sweep in arbitrary order, placed here by rank since they are distinct),
+// each entry with its uid.  The previous row's uids and gj values are staged
+// in LDS too and each lane resolves the gap junction of its entries there
+// (gj_refresh :133-152: a directed edge keeps its value while it stays in the
+// list, a new edge starts at gj_init).
 // The dermis (find_dermis :158-172: the first MEMB entry of minimal distance
 // in list order, strictly below LX^2) is a lexicographic (distance, entry)
 // minimum over the group.  Longer rows take the same steps through global
 // memory.
+// The time is the chain of round trips: the cell's words; the rows' first
+// KPRE entries (unconditional: a row holds at least 32 slots) with the
+// previous row's length and values; the uids of both.  The launch also does
+// what the next build needs of this one (every cell's row is its own from
+// here, the uids are kept beside the rows they number, the buckets are
+// emptied): a launch of its own for that took 2.5 to 4.4 us and its gap.
 constexpr int KG = 16;
 constexpr int KCAP = 64;   // rows (and previous rows) longer than this take the global-memory path
+constexpr int KPRE = 2;    // entries of each row a lane asks for before it knows the lengths
 constexpr int K_BLOCK = 128;
 constexpr int K_GROUPS = K_BLOCK / KG;
 
@@ -369,6 +350,7 @@ __global__ void __launch_bounds__(K_BLOCK) k_finish(const Tis* __restrict__ T, i
   const int ob = 1 - nb;
   __shared__ int s_row[K_GROUPS][KCAP];
   __shared__ int s_bt[K_GROUPS][KCAP];
+  __shared__ long long s_ru[K_GROUPS][KCAP];
   __shared__ long long s_ou[K_GROUPS][KCAP];
   __shared__ double s_og[K_GROUPS][KCAP];
   const int lane = threadIdx.x & (KG - 1);
@@ -379,56 +361,111 @@ __global__ void __launch_bounds__(K_BLOCK) k_finish(const Tis* __restrict__ T, i
   for (int c = blockIdx.x * K_GROUPS + grp; c < n; c += stride) {
     const bool memb = c < t.nmemb;
     const int base = memb ? MEMB_ADJ : 0;
-    const int na = memb ? 0 : t.nlo[c];
+    const int na0 = t.nlo[c];
     const int nbh = t.bcnt[c];
     const int src = t.src_row[c];
+    const int bkt = t.bucket_of[c];
+    const long long my_uid = t.uid[c];
+    const uint8_t s = t.state[c];
+    const P3 pc = ld_pos(t, pb, c);
+    const int na = memb ? 0 : na0;
     const int len = base + na + nbh;
+    int* const row = t.col[nb] + (size_t)c * t.ns;
+    const int* bt = t.btmp + (size_t)c * t.ns;
+    const int osrc = src >= 0 ? src : c;
+    const int* orow = t.col[ob] + (size_t)osrc * t.ns;
+    const double* og = t.gj[ob] + (size_t)osrc * t.ns;
+    const int* const lo = memb ? t.memb6 + 6 * c : row;   // the row's first part: base + na entries
+    const int nl = base + na;
+    int lo_e[KPRE], bt_e[KPRE], or_e[KPRE];
+    double og_e[KPRE];
+#pragma unroll
+    for (int k = 0; k < KPRE; k++) {
+      const int i = lane + k * KG;
+      lo_e[k] = lo[i < nl ? i : 0];
+      bt_e[k] = bt[i];
+      or_e[k] = orow[i];
+      og_e[k] = og[i];
+    }
+    const int olen = src >= 0 ? t.nlen[ob][src] : 0;
+    if (lane == 0) {
+      t.src_row[c] = c;
+      t.old_uid[nb][c] = my_uid;
+      if (bkt >= 0) t.bucket[(size_t)bkt * BUCKET_HEAD] = 0;
+    }
     // the reference asserts a list shorter than N2 = 400 (:122)
     if (len >= MAX_CONN || len > t.ns) {
       if (lane == 0) { set_err(st, ERR_CAPACITY); t.nlen[nb][c] = 0; }
       continue;
     }
     mylen = max(mylen, len);
-    const int olen = src >= 0 ? t.nlen[ob][src] : 0;
-    const int* orow = src >= 0 ? t.col[ob] + (size_t)src * t.ns : nullptr;
-    const double* og = src >= 0 ? t.gj[ob] + (size_t)src * t.ns : nullptr;
-    int* const row = t.col[nb] + (size_t)c * t.ns;
-    const int* bt = t.btmp + (size_t)c * t.ns;
     const bool fits = len <= KCAP;
     const bool staged = olen <= KCAP;
-    int* const r = fits ? s_row[grp] : row;
     if (lane == 0) t.nlen[nb][c] = len;
-    if (memb && lane < MEMB_ADJ) r[lane] = t.memb6[6 * c + lane];
-    if (fits) {
-      for (int i = lane; i < na; i += KG) r[i] = row[i];
-      for (int i = lane; i < nbh; i += KG) s_bt[grp][i] = bt[i];
+    // the uids: entries past a row's end read cell 0's and are not kept
+    long long lo_u[KPRE], bt_u[KPRE], or_u[KPRE];
+#pragma unroll
+    for (int k = 0; k < KPRE; k++) {
+      const int i = lane + k * KG;
+      lo_u[k] = t.uid[i < nl ? lo_e[k] : 0];
+      bt_u[k] = t.uid[i < nbh ? bt_e[k] : 0];
+      or_u[k] = t.old_uid[ob][i < olen ? or_e[k] : 0];
     }
-    if (staged)
-      for (int f = lane; f < olen; f += KG) {
-        s_ou[grp][f] = t.old_uid[orow[f]];
+    if (fits) {
+#pragma unroll
+      for (int k = 0; k < KPRE; k++) {
+        const int i = lane + k * KG;
+        if (i < nl) { s_row[grp][i] = lo_e[k]; s_ru[grp][i] = lo_u[k]; }
+        if (i < nbh) s_bt[grp][i] = bt_e[k];
+      }
+      for (int i = lane + KPRE * KG; i < nl; i += KG) {
+        const int o = lo[i];
+        s_row[grp][i] = o;
+        s_ru[grp][i] = t.uid[o];
+      }
+      for (int i = lane + KPRE * KG; i < nbh; i += KG) s_bt[grp][i] = bt[i];
+    } else if (memb) {
+      if (lane < MEMB_ADJ) row[lane] = lo[lane];
+    }
+    if (staged) {
+#pragma unroll
+      for (int k = 0; k < KPRE; k++) {
+        const int i = lane + k * KG;
+        if (i < olen) { s_ou[grp][i] = or_u[k]; s_og[grp][i] = og_e[k]; }
+      }
+      for (int f = lane + KPRE * KG; f < olen; f += KG) {
+        s_ou[grp][f] = t.old_uid[ob][orow[f]];
         s_og[grp][f] = og[f];
       }
-    wave_sync();
-    const int* const b = fits ? s_bt[grp] : bt;
-    for (int i = lane; i < nbh; i += KG) {
-      const int v = b[i];
-      int rk = 0;
-      for (int k = 0; k < nbh; k++) rk += b[k] < v;
-      r[base + na + rk] = v;
     }
     wave_sync();
-    const uint8_t s = t.state[c];
+    {
+      const int* const b = fits ? s_bt[grp] : bt;
+      int k = 0;
+      for (int i = lane; i < nbh; i += KG, k++) {
+        const int v = b[i];
+        int rk = 0;
+        for (int m = 0; m < nbh; m++) rk += b[m] < v;
+        if (fits) {
+          s_row[grp][nl + rk] = v;
+          s_ru[grp][nl + rk] = k == 0 ? bt_u[0] : k == 1 ? bt_u[1] : t.uid[v];
+        } else {
+          row[nl + rk] = v;
+        }
+      }
+    }
+    wave_sync();
     const bool want_dermis = !memb && c >= t.nmemb + t.nder && (s == FIX || s == MUSUME);
-    const P3 pc = ld_pos(t, pb, c);
+    const int* const r = fits ? s_row[grp] : row;
     double bd = t.LX * t.LX;
     int be = 0x7fffffff;
     double* const g = t.gj[nb] + (size_t)c * t.ns;
     for (int e = lane; e < len; e += KG) {
       const int o = r[e];
-      if (fits && (e < base || e >= base + na)) row[e] = o;
-      const long long u = t.uid[o];
+      if (fits && (e < base || e >= nl)) row[e] = o;
+      const long long u = fits ? s_ru[grp][e] : t.uid[o];
       const long long* const ou = s_ou[grp];
-      const int q = gj_carry_slot(e, olen, u, [&](int k) { return staged ? ou[k] : t.old_uid[orow[k]]; });
+      const int q = gj_carry_slot(e, olen, u, [&](int k) { return staged ? ou[k] : t.old_uid[ob][orow[k]]; });
       g[e] = q < 0 ? gj_init : staged ? s_og[grp][q] : og[q];
       if (want_dermis && t.state[o] == MEMB) {
         const double d = dist_sq(t, pc, ld_pos(t, pb, o));
@@ -453,28 +490,6 @@ __global__ void __launch_bounds__(K_BLOCK) k_finish(const Tis* __restrict__ T, i
     atomicMax(&st->maxlen, mylen);
 }
 
-// after a build: every cell's row is its own, uids snapshot the numbering,
-// and the buckets are emptied for the next build
-// With h_out (pinned host memory), block 0 of each tissue first copies the
-// tissue's status there: the status is final once the build's row assembly
-// is done, so the step's read-back needs no copy launch of its own.
-__global__ void __launch_bounds__(256) k_snapshot(const Tis* __restrict__ T, int pb, Status* h_out) {
-  (void)pb;
-  const Tis& t = T[blockIdx.y];
-  static_assert(sizeof(Status) % 8 == 0 && sizeof(Status) / 8 <= 256, "status copied in 8-byte words");
-  if (h_out && blockIdx.x == 0 && threadIdx.x < sizeof(Status) / 8)
-    reinterpret_cast<unsigned long long*>(h_out + blockIdx.y)[threadIdx.x] =
-        reinterpret_cast<const unsigned long long*>(static_cast<const Status*>(t.st))[threadIdx.x];
-  const int n = t.st->n;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
-    t.src_row[c] = c;
-    t.old_uid[c] = t.uid[c];
-    const int b = t.bucket_of[c];
-    if (b >= 0) t.bucket_n[b] = 0;
-  }
-}
-
-// calc_zzmax by itself (a step's rides with the bucket insertion)
 __global__ void __launch_bounds__(256) k_zzmax(const Tis* __restrict__ T, int pb) {
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;
@@ -545,23 +560,19 @@ void launch_connect_insert(hipStream_t s, const Tis* dT, int ntis, int pb, int m
   }
 }
 
-void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave,
-                         Status* h_status) {
-  dim3 gc((max_n + 255) / 256, ntis);
-  EPI_LAUNCH(K_BUCKET_SORT, k_bucket_sort, gc, dim3(256), 0, s, dT);
+void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave) {
   if (sweep_wave) {
-    EPI_LAUNCH(K_SWEEP_WAVE, k_sweep_wave, dim3((max_n + 3) / 4, ntis), dim3(256), 0, s, dT, pb, nb);
+    EPI_LAUNCH(K_SWEEP_WAVE, k_sweep<64>, dim3((max_n + 3) / 4, ntis), dim3(256), 0, s, dT, pb, nb);
   } else {
-    EPI_LAUNCH(K_SWEEP, k_sweep, dim3((max_n + 7) / 8, ntis), dim3(256), 0, s, dT, pb, nb);
+    EPI_LAUNCH(K_SWEEP, k_sweep<32>, dim3((max_n + 7) / 8, ntis), dim3(256), 0, s, dT, pb, nb);
   }
   dim3 gk((max_n + K_GROUPS - 1) / K_GROUPS, ntis);
   EPI_LAUNCH(K_FINISH, k_finish, gk, dim3(K_BLOCK), 0, s, dT, pb, nb);
-  EPI_LAUNCH(K_SNAPSHOT, k_snapshot, gc, dim3(256), 0, s, dT, pb, h_status);
 }
 
 void launch_connect(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave) {
   launch_connect_insert(s, dT, ntis, pb, max_n, 0);
-  launch_connect_rest(s, dT, ntis, pb, nb, max_n, sweep_wave, nullptr);
+  launch_connect_rest(s, dT, ntis, pb, nb, max_n, sweep_wave);
 }
 
 void launch_zzmax(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n) {

@@ -102,7 +102,7 @@ __device__ __forceinline__ double coef_law(const Tis& t, int law, const CV& a, c
     const double LJ6 = POW6(cr_dist) / POW6(lambda_dist - dist);
     const double tmp = -(t.prm.DER_DER_CONST / rad_sum) * ((1.0 - t.prm.P_MEMB) / t.prm.P_MEMB)
                        - 4 * t.m_eps * (LJ6 * (LJ6 - 1.0)) / ((lambda_dist - dist) * dist);
-    if (fabs(tmp) > 100) set_err(st, ERR_STRONG_INTERACTION);
+    if (fabs(tmp) > 100) set_force_err(st, ERR_STRONG_INTERACTION);
     return tmp;
   }
   // is_near: every law but LAW_OTHER takes ljmain within contact
@@ -128,13 +128,13 @@ __device__ __forceinline__ double coef_law(const Tis& t, int law, const CV& a, c
   const double x = Q - 1.0;
   const double k2 = (L ? 4.0 * t.m_eps * Q * x : K) / (L ? distSq : dist);
   if (L) {
-    if (memb && fabs(k2) > 100) set_err(st, ERR_STRONG_INTERACTION);
+    if (memb && fabs(k2) > 100) set_force_err(st, ERR_STRONG_INTERACTION);
     return k2;
   }
   if (law == LAW_FIX_MEMB) return -k2 * x;
   if (memb) {
     const double tmp = -k2 * x;
-    if (fabs(tmp) > 100) set_err(st, ERR_STRONG_INTERACTION);
+    if (fabs(tmp) > 100) set_force_err(st, ERR_STRONG_INTERACTION);
     return tmp;
   }
   const double c2 = (t.prm.LJ_THRESH - 1.0) * (t.prm.LJ_THRESH - 1.0);
@@ -145,7 +145,7 @@ __device__ __forceinline__ double coef_law(const Tis& t, int law, const CV& a, c
 template <bool PAIR>
 __device__ __forceinline__ P3 delta_law(const Tis& t, int law, const CV& a, const CV& b, Status* st) {
   const double coef = coef_law<PAIR>(t, law, a, b, st);
-  if (fabs(coef) > 1000) set_err(st, ERR_STRONG_INTERACTION);
+  if (fabs(coef) > 1000) set_force_err(st, ERR_STRONG_INTERACTION);
   const double d = t.prm.DT_Cell * coef;
   return P3{d * p_diff_x(t, a.p.x, b.p.x), d * p_diff_y(t, a.p.y, b.p.y), d * (a.p.z - b.p.z)};
 }
@@ -378,10 +378,25 @@ __device__ __forceinline__ double sum_slots(double acc, const double* v, int e0,
 }
 __device__ __forceinline__ double p3_at(const P3& p, int k) { return k == 0 ? p.x : k == 1 ? p.y : p.z; }
 
+// the tissue's status into pinned host memory, then the number the host waits
+// for.  The kernel follows the build in the stream, so the status is final but
+// for what runs beside it (the force kernel's own errors have their own word).
+__device__ __forceinline__ void status_out(const Tis& t, const StatusOut& out) {
+  static_assert(sizeof(Status) % 8 == 0 && sizeof(Status) / 8 <= 64, "status copied in 8-byte words by one wave");
+  if (threadIdx.x >= 64) return;
+  if (threadIdx.x < sizeof(Status) / 8)
+    reinterpret_cast<unsigned long long*>(out.host + blockIdx.y)[threadIdx.x] =
+        reinterpret_cast<const unsigned long long*>(static_cast<const Status*>(t.st))[threadIdx.x];
+  __threadfence_system();
+  if (threadIdx.x == 0)
+    __hip_atomic_store(out.seq + blockIdx.y, out.value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 template <int FCAP>
-__global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, int pb, int cb) {
+__global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, int pb, int cb, StatusOut out) {
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;
+  if (out.host && blockIdx.x == 0) status_out(t, out);
   __shared__ FRow<FCAP> s_own[F_GROUPS];
   __shared__ FRow<FCAP> s_oth[F_GROUPS];
   __shared__ __align__(16) int s_idx[F_GROUPS][FCAP];
@@ -401,7 +416,7 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
   const int* row = t.col[cb] + (size_t)X * t.ns;
   const int q0 = row[lane];   // a row holds ns >= 64 > FG slots
   const int n = st->n;
-  if (blockIdx.x == 0 && threadIdx.x == 0 && (long long)gridDim.x * F_GROUPS < n) set_err(st, ERR_INVALID);
+  if (blockIdx.x == 0 && threadIdx.x == 0 && (long long)gridDim.x * F_GROUPS < n) set_force_err(st, ERR_INVALID);
   if (X >= n) return;
   if (len > FCAP) return;   // k_forces_long
   bool hi = false;          // this lane's membrane slot is subtracted (its handler has the higher index)
@@ -552,18 +567,19 @@ __global__ void __launch_bounds__(256) k_forces_long(const Tis* __restrict__ T, 
     if (t.nlen[cb][X] > cap) forces_serial(t, pb, cb, X, t.st);
 }
 
-int launch_forces_rows(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len) {
+int launch_forces_rows(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len,
+                       const StatusOut& out) {
   dim3 g((max_other + F_GROUPS - 1) / F_GROUPS, ntis);
   int cap;
   if (max_len <= 40) {
     cap = 40;
-    EPI_LAUNCH(K_FORCES, k_forces<40>, g, dim3(F_BLOCK), 0, s, dT, pb, cb);
+    EPI_LAUNCH(K_FORCES, k_forces<40>, g, dim3(F_BLOCK), 0, s, dT, pb, cb, out);
   } else if (max_len <= 48) {
     cap = 48;
-    EPI_LAUNCH(K_FORCES, k_forces<48>, g, dim3(F_BLOCK), 0, s, dT, pb, cb);
+    EPI_LAUNCH(K_FORCES, k_forces<48>, g, dim3(F_BLOCK), 0, s, dT, pb, cb, out);
   } else {
     cap = FORCES_ROW_CAP;
-    EPI_LAUNCH(K_FORCES, k_forces<FORCES_ROW_CAP>, g, dim3(F_BLOCK), 0, s, dT, pb, cb);
+    EPI_LAUNCH(K_FORCES, k_forces<FORCES_ROW_CAP>, g, dim3(F_BLOCK), 0, s, dT, pb, cb, out);
   }
   return cap;
 }
@@ -576,7 +592,7 @@ void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, 
 void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_memb, int max_other,
                    int max_len) {
   (void)max_memb;
-  const int cap = launch_forces_rows(s, dT, ntis, pb, cb, max_other, max_len);
+  const int cap = launch_forces_rows(s, dT, ntis, pb, cb, max_other, max_len, StatusOut{});
   if (max_len > cap) launch_forces_long(s, dT, ntis, pb, cb, max_other, cap);
 }
 

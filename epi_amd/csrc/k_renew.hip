@@ -98,6 +98,7 @@ __global__ void __launch_bounds__(1024) k_renew_scan(const Tis* __restrict__ T, 
   const int n_old = st->n;
   const RenewK rk = renew_k(t.prm);
   if (tid == 0) { s_cursor = st->rng_pos; s_ndiv = 0; s_nrm_base = 0; st->n_old = n_old; }
+  if (tid == 64 && st->force_err) set_err(st, st->force_err);
   __syncthreads();
   for (int base = start; base < n_old; base += RCHUNK) {
     const int chunk = (base - start) / RCHUNK;

@@ -10,8 +10,8 @@ struct Status;
 
 enum KernelId {
   K_FORCES, K_FORCES_LONG, K_RENEW_FLAGS, K_RENEW_SCAN, K_RENEW_APPLY, K_REMOVE, K_PAIR_DISPERSE,
-  K_INIT_SC, K_PERIODIC_FIX, K_BUCKET_INSERT, K_BUCKET_SORT, K_SWEEP,
-  K_FINISH, K_SNAPSHOT, K_ZZ_SET, K_ZZMAX, K_MAP_CLEAR, K_MAP_STAMP,
+  K_INIT_SC, K_PERIODIC_FIX, K_BUCKET_INSERT, K_SWEEP,
+  K_FINISH, K_ZZ_SET, K_ZZMAX, K_MAP_CLEAR, K_MAP_STAMP,
   K_EXT_STIM, K_CA_BEGIN, K_CA_VOX, K_CA_CELLS, K_ATP, K_CA_END, K_SW_RESET,
   K_RD_SNAPSHOT, K_RD_RESTORE, K_RD_PUT_GJ, K_RD_STATE, K_RD_SEED, K_RD_STEP,
   K_RD_SUMS, K_RD_OWN, K_MECH_STATE, K_MECH_SEED, K_MECH_BWD_BEGIN, K_MECH_BWD_PAIRS, K_MECH_BWD_MEMB,
@@ -29,7 +29,7 @@ struct Tuning {
   int ca_group = 8;           // Ca cell kernels: lanes per cell (8, or 16; 4 takes 8)
   int xcd = 0;                // k_ca_cells, k_atp: XCD-contiguous workgroup order
   int b_xcd = 0;              // k_ext_stim: its tile list in one contiguous run per XCD
-  int sweep_wave = 0;         // k_sweep: 1, one wave per cell (k_sweep_wave)
+  int sweep_wave = 0;         // k_sweep: 1, one wave per cell (64 lanes instead of 32)
   int side_fork = 0;          // 1: the side stream forks after the whole build
   int rd_group = 8;           // k_rd_step: lanes per cell
   int ca_fuse = 1;            // Ca solves: ATP of a sub-step and cells of the next in one launch
@@ -60,6 +60,15 @@ void prof_add(int k, hipEvent_t a, hipEvent_t b, bool counted);
     }                                                                                         \
   } while (0)
 
+// where a force kernel leaves the statuses for a waiting host (pinned,
+// coherent memory; host == nullptr: nowhere): a Status per tissue, then value
+// into every tissue's seq
+struct StatusOut {
+  Status* host = nullptr;
+  unsigned long long* seq = nullptr;
+  unsigned long long value = 0;
+};
+
 // Rows of up to FORCES_ROW_CAP entries go to the cooperative kernel (whose
 // LDS slots per cell, 40, 48 or 64, follow max_len), longer ones to a
 // one-lane-per-cell kernel, launched only when max_len exceeds the slots.
@@ -67,7 +76,8 @@ constexpr int FORCES_ROW_CAP = 64;
 void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_memb, int max_other, int max_len);
 // the two halves of launch_forces: the cooperative kernel for rows of up to
 // the returned number of slots (chosen from max_len), and the long rows
-int launch_forces_rows(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len);
+int launch_forces_rows(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len,
+                       const StatusOut& out);
 void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int cap);
 // zero_zz: also clear zzmax, for a build whose insertion takes it
 void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_n, int zero_zz);
@@ -78,9 +88,7 @@ void launch_periodic_fix(hipStream_t s, const Tis* dT, int ntis, int pb, int max
 // applies the periodic fix, takes zzmax (cleared by launch_renew) and empties
 // the voxel maps with that many more blocks
 void launch_connect_insert(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, unsigned clear_blocks);
-// with h_status, k_snapshot also copies every tissue's status there
-void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave,
-                         Status* h_status);
+void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave);
 void launch_connect(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave);
 void launch_zzmax(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n);
 // A snapshot's output record (CellManager::output's fields): a header of

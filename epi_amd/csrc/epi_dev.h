@@ -148,8 +148,10 @@ struct Tis {
   GPtr<double4> pk;
   // state renewal
   GPtr<int> div_slot; GPtr<double> div_dir;  // per division: parent, direction
-  GPtr<int> div_parent; GPtr<int> rm_list;
-  GPtr<uint8_t> rflag; GPtr<int> chunk_any;   // renewal flags and per-1024-cell chunk marks
+  GPtr<int> rm_list;
+  // per block of 256 cells past the dermis: the cells that need a draw and
+  // those that go, and how many
+  GPtr<int> rd_list; GPtr<int> rm_pack; GPtr<int> rd_n; GPtr<int> rm_n;
   // grids
   GPtr<double> atp[2]; GPtr<double> bf[2];
   // vox, vmk: during a solve or window, per voxel of the active box, the AFM

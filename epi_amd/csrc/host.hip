@@ -88,7 +88,7 @@ const char* kKernelNames[K_COUNT] = {
     "k_rd_snapshot", "k_rd_restore", "k_rd_put_gj", "k_rd_state", "k_rd_seed",
     "k_rd_step", "k_rd_sums", "k_rd_own", "k_mech_state", "k_mech_seed", "k_mech_bwd_begin",
     "k_mech_bwd_pairs", "k_mech_bwd_memb", "k_ca_fused", "k_ca_corners", "k_sweep_wave", "k_wl", "k_ca_swap",
-    "k_out_pack"};
+    "k_out_pack", "k_renew_one"};
 
 // with ready_only, only the pairs whose kernels have finished (the rest stay
 // pending for a later read-back)
@@ -314,10 +314,11 @@ void carve_tissue(Carver& cv, TH& h, Tis& t) {
   t.pk = cv.take<double4>(cap);
   t.div_slot = cv.take<int>(cap);
   t.div_dir = cv.take<double>(3 * cap);
-  t.div_parent = cv.take<int>(cap);
   t.rm_list = cv.take<int>(cap);
-  t.rflag = cv.take<uint8_t>(cap);
-  t.chunk_any = cv.take<int>(cap / 1024 + 2);
+  t.rd_list = cv.take<int>(cap + 256);
+  t.rm_pack = cv.take<int>(cap + 256);
+  t.rd_n = cv.take<int>(cap / 256 + 1);
+  t.rm_n = cv.take<int>(cap / 256 + 1);
   for (int b = 0; b < 2; b++) { t.atp[b] = cv.take<double>(h.gsize); t.bf[b] = cv.take<double>(h.gsize); }
   t.cmap1 = cv.take<int>(h.gsize);
   t.cmap2 = cv.take<uint8_t>(h.gsize);
@@ -403,6 +404,12 @@ int max_list_len(const epi_ctx* c) {
 int max_n(const epi_ctx* c) {
   int m = 1;
   for (auto& h : c->th) m = std::max(m, h.n_est + 64);
+  return m;
+}
+// cells past the membrane and the dermis
+int max_free(const epi_ctx* c) {
+  int m = 1;
+  for (auto& h : c->th) m = std::max(m, h.n_est + 64 - h.nmemb - h.nder);
   return m;
 }
 int max_memb(const epi_ctx* c) {
@@ -1113,7 +1120,7 @@ int epi_pos_copy(epi_ctx* c) {
 int epi_cell_state_renew(epi_ctx* c) {
   if (!c) return EPI_ERR_INVALID;
   if (c->pos_pending) return fail(c, EPI_ERR_INVALID, "pos_copy must follow cell_interaction");
-  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, max_n(c), 0);
+  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, max_n(c), max_free(c), 0);
   HIPCHK(c, hipGetLastError());
   for (auto& v : c->dev_ts) v++;   // k_remove advances each tissue's timestep
   return EPI_OK;
@@ -1266,10 +1273,10 @@ int epi_ca_substep(epi_ctx* c, int32_t iz_bound) {
 // With join false the main stream does not wait for the side stream's maps
 // and B sweep: epi_step joins it after issuing the next step's forces, which
 // read neither.
-hipError_t issue_build(epi_ctx* c, int mn, int nb, int izb, bool join = true) {
+hipError_t issue_build(epi_ctx* c, int mn, int mfree, int nb, int izb, bool join = true) {
   hipError_t e = hipSuccess;
   auto chk = [&](hipError_t r) { if (e == hipSuccess) e = r; };
-  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, mn, 1);
+  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, mn, mfree, 1);
   launch_connect_insert(c->stream, c->d_tis, c->T, c->pb, mn, map_clear_blocks(max_gsize(c)));
   // the side stream forks after the insertion (SIDE_FORK 0: the maps run
   // beside the sweep) or after the whole build (1: the sweep runs alone and
@@ -1295,13 +1302,13 @@ hipError_t issue_build(epi_ctx* c, int mn, int nb, int izb, bool join = true) {
 // *joined tells whether the main stream already waits for the side stream.
 int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
   constexpr unsigned long long seg =
-      (1ull << K_RENEW_FLAGS) | (1ull << K_RENEW_SCAN) | (1ull << K_RENEW_APPLY) | (1ull << K_REMOVE) |
+      (1ull << K_RENEW_ONE) | (1ull << K_RENEW_FLAGS) | (1ull << K_RENEW_SCAN) | (1ull << K_RENEW_APPLY) | (1ull << K_REMOVE) |
       (1ull << K_PAIR_DISPERSE) | (1ull << K_BUCKET_INSERT) | (1ull << K_SWEEP_WAVE) |
       (1ull << K_SWEEP) | (1ull << K_FINISH) | (1ull << K_ZZ_SET) | (1ull << K_ZZMAX) |
       (1ull << K_MAP_CLEAR) | (1ull << K_MAP_STAMP) | (1ull << K_EXT_STIM);
   if (!c->tu.step_graph || (g_prof.mask & seg)) {
     *joined = false;
-    HIPCHK(c, issue_build(c, mn, nb, izb, false));
+    HIPCHK(c, issue_build(c, mn, max_free(c), nb, izb, false));
     return EPI_OK;
   }
   *joined = true;   // a captured graph rejoins its forked stream
@@ -1309,9 +1316,11 @@ int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
   for (auto& h : c->th) mcap = std::max(mcap, h.cap);
   const int mr = std::max(mn, std::min((mn + 1023) / 1024 * 1024, mcap));
   const Tuning& tu = c->tu;
-  const std::vector<long long> key = {1, c->pb, c->cb, c->cp, c->bp, nb, mr, izb, max_gsize(c),
+  // the renewal's form: a replay's grids do not depend on the count otherwise
+  const int mfree = max_free(c) <= RENEW_ONE ? RENEW_ONE : max_free(c) <= RENEW_FEW ? RENEW_FEW : mr;
+  const std::vector<long long> key = {1, std::min(mfree, RENEW_FEW + 1), c->pb, c->cb, c->cp, c->bp, nb, mr, izb, max_gsize(c),
                                       max_nx(c), max_ny(c), tu.b_zb, tu.b_rows, tu.map_lanes, tu.sweep_wave, tu.side_fork};
-  return graph_run(c, key, [&] { return issue_build(c, mr, nb, izb); });
+  return graph_run(c, key, [&] { return issue_build(c, mr, mfree, nb, izb); });
 }
 
 int epi_step(epi_ctx* c, int64_t nsteps, epi_driver* drv) {

@@ -15,7 +15,7 @@ enum KernelId {
   K_EXT_STIM, K_CA_BEGIN, K_CA_VOX, K_CA_CELLS, K_ATP, K_CA_END, K_SW_RESET,
   K_RD_SNAPSHOT, K_RD_RESTORE, K_RD_PUT_GJ, K_RD_STATE, K_RD_SEED, K_RD_STEP,
   K_RD_SUMS, K_RD_OWN, K_MECH_STATE, K_MECH_SEED, K_MECH_BWD_BEGIN, K_MECH_BWD_PAIRS, K_MECH_BWD_MEMB,
-  K_CA_FUSED, K_CA_CORNERS, K_SWEEP_WAVE, K_WL, K_CA_SWAP, K_OUT_PACK, K_COUNT
+  K_CA_FUSED, K_CA_CORNERS, K_SWEEP_WAVE, K_WL, K_CA_SWAP, K_OUT_PACK, K_RENEW_ONE, K_COUNT
 };
 
 // ints of a context's work-list buffer: the offsets and per-tissue iz_bound
@@ -79,8 +79,18 @@ void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int m
 int launch_forces_rows(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len,
                        const StatusOut& out);
 void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int cap);
-// zero_zz: also clear zzmax, for a build whose insertion takes it
-void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_n, int zero_zz);
+// zero_zz: also clear zzmax, for a build whose insertion takes it.  max_free:
+// the most cells past membrane and dermis of any tissue.  Up to RENEW_ONE the
+// renewal is one launch, a workgroup per tissue: with 160 cells 9.6 us against
+// 12.6 and two gaps for the three launches of RENEW_FEW, with 2,000 cells 20.1
+// (the lipid laws' tanh on one CU) against 17.3.  Up to RENEW_FEW the flags
+// and the ordered walk are one launch and so are the removal and the pairs:
+// with 2,000 cells 10.4 + 3.1 us against 11.6 + 4.7 and two gaps; the walk
+// takes 2.8 us more for each 1,024 cells, and with 7,000 cells 30 against 18.
+constexpr int RENEW_ONE = 768;
+constexpr int RENEW_FEW = 3072;
+void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_n, int max_free,
+                  int zero_zz);
 void launch_initialize_sc(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int pb, int max_n);
 void launch_periodic_fix(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n);
 // the bucket insertion and the rest of the build, for callers that run the

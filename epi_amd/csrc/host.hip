@@ -451,15 +451,16 @@ int izb_est(const epi_ctx* c, bool ca) {
 
 // tiles of the B stencil's work list (k_ext_stim) from the last known
 // zzmax, one plane more than it gives, for sizing the grid
+// tiles of bs points of the B stencil in tissue t, from the last known zzmax
+long long b_tiles_of(const epi_ctx* c, int t, int bs) {
+  const Tis& ti = c->tis[t];
+  const double zz = c->h_st ? c->h_st[t].zzmax : 0.0;
+  const int zb = c->tu.b_zb, izb = std::min((int)((zz + ti.prm.iz_margin) * ti.inv_dz) + 1, c->th[t].NZ);
+  return (long long)((ti.NX * ti.NY + bs - 1) / bs) * ((std::max(izb, 1) + zb - 1) / zb);
+}
 long long b_tiles_est(const epi_ctx* c) {
-  const int bs = 64 * c->tu.b_rows, zb = c->tu.b_zb;
   long long n = 0;
-  for (int t = 0; t < c->T; t++) {
-    const Tis& ti = c->tis[t];
-    const double zz = c->h_st ? c->h_st[t].zzmax : 0.0;
-    const int izb = std::min((int)((zz + ti.prm.iz_margin) * ti.inv_dz) + 1, c->th[t].NZ);
-    n += (long long)((ti.NX * ti.NY + bs - 1) / bs) * ((std::max(izb, 1) + zb - 1) / zb);
-  }
+  for (int t = 0; t < c->T; t++) n += b_tiles_of(c, t, 64 * c->tu.b_rows);
   return n;
 }
 
@@ -1270,14 +1271,26 @@ int epi_ca_substep(epi_ctx* c, int32_t iz_bound) {
 // fixed positions, states and radii (and the B field) that the rest of the
 // build leaves alone.  The build, the longer
 // chain, is issued first.
+// Up to BUILD_FIELD_TISSUES tissues there is no side stream (unless `side`):
+// the stamping is further blocks of the sweep and the B sweep further blocks of
+// k_finish.  Recording and waiting for the two events took the host 25 us a
+// step, and such a step is bound by what the host issues.
 // With join false the main stream does not wait for the side stream's maps
 // and B sweep: epi_step joins it after issuing the next step's forces, which
 // read neither.
-hipError_t issue_build(epi_ctx* c, int mn, int mfree, int nb, int izb, bool join = true) {
+constexpr int BUILD_FIELD_TISSUES = 1;
+hipError_t issue_build(epi_ctx* c, int mn, int mfree, int nb, int izb, bool side, bool join = true) {
   hipError_t e = hipSuccess;
   auto chk = [&](hipError_t r) { if (e == hipSuccess) e = r; };
   launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, mn, mfree, 1);
   launch_connect_insert(c->stream, c->d_tis, c->T, c->pb, mn, map_clear_blocks(max_gsize(c)));
+  if (!side) {
+    long long tiles = 1;
+    for (int t = 0; t < c->T; t++) tiles = std::max(tiles, b_tiles_of(c, t, BUILD_FIELD_BS));
+    launch_connect_field(c->stream, c->d_tis, c->T, c->pb, nb, c->bp, mn, tiles, c->tu);
+    chk(hipGetLastError());
+    return e;
+  }
   // the side stream forks after the insertion (SIDE_FORK 0: the maps run
   // beside the sweep) or after the whole build (1: the sweep runs alone and
   // the maps beside the next forces)
@@ -1306,9 +1319,11 @@ int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
       (1ull << K_PAIR_DISPERSE) | (1ull << K_BUCKET_INSERT) | (1ull << K_SWEEP_WAVE) |
       (1ull << K_SWEEP) | (1ull << K_FINISH) | (1ull << K_ZZ_SET) | (1ull << K_ZZMAX) |
       (1ull << K_MAP_CLEAR) | (1ull << K_MAP_STAMP) | (1ull << K_EXT_STIM);
+  // kernels that are timed one by one stay apart
+  const bool side = c->T > BUILD_FIELD_TISSUES || (g_prof.mask & seg);
   if (!c->tu.step_graph || (g_prof.mask & seg)) {
-    *joined = false;
-    HIPCHK(c, issue_build(c, mn, max_free(c), nb, izb, false));
+    *joined = !side;
+    HIPCHK(c, issue_build(c, mn, max_free(c), nb, izb, side, false));
     return EPI_OK;
   }
   *joined = true;   // a captured graph rejoins its forked stream
@@ -1320,7 +1335,7 @@ int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
   const int mfree = max_free(c) <= RENEW_ONE ? RENEW_ONE : max_free(c) <= RENEW_FEW ? RENEW_FEW : mr;
   const std::vector<long long> key = {1, std::min(mfree, RENEW_FEW + 1), c->pb, c->cb, c->cp, c->bp, nb, mr, izb, max_gsize(c),
                                       max_nx(c), max_ny(c), tu.b_zb, tu.b_rows, tu.map_lanes, tu.sweep_wave, tu.side_fork};
-  return graph_run(c, key, [&] { return issue_build(c, mr, mfree, nb, izb); });
+  return graph_run(c, key, [&] { return issue_build(c, mr, mfree, nb, izb, side); });
 }
 
 int epi_step(epi_ctx* c, int64_t nsteps, epi_driver* drv) {

@@ -16,6 +16,7 @@
 #include "launch.h"
 #include "epi_group.h"
 #include "gj_carry.h"
+#include "field_step.h"
 
 namespace epi {
 
@@ -182,14 +183,13 @@ __device__ __forceinline__ int sweep_crowded(const Tis& t, int c, const P3& pc, 
 }
 
 template <int G>
-__global__ void __launch_bounds__(256) k_sweep(const Tis* __restrict__ T, int pb, int nb) {
+__device__ __forceinline__ void sweep_part(const Tis& t, int nb, int nblk) {
   constexpr int NB = 128 / G;   // buckets of a lane
-  const Tis& t = T[blockIdx.y];
   Status* st = t.st;
   const int n = st->n;
   const int ANX = t.ANX, ANY = t.ANY, ANZ = t.ANZ, bcap = t.bcap, ns = t.ns;
   const int lane = threadIdx.x & (G - 1);
-  const int groups = gridDim.x * (blockDim.x / G);
+  const int groups = nblk * (blockDim.x / G);
   __shared__ int s_cand[256 / G][SWEEP_C];
   __shared__ uint8_t s_cq[256 / G][SWEEP_C];
   __shared__ unsigned long long s_hit[256 / G][SWEEP_H];
@@ -319,6 +319,21 @@ __global__ void __launch_bounds__(256) k_sweep(const Tis* __restrict__ T, int pb
   }
 }
 
+// Blocks [0, sweep_blocks) sweep; with MS lanes per cell the rest stamp the
+// voxel maps (MS = 0: there is none), which like the sweep needs only what the
+// insertion left.
+template <int G, int MS>
+__global__ void __launch_bounds__(256) k_sweep(const Tis* __restrict__ T, int pb, int nb, int sweep_blocks) {
+  const Tis& t = T[blockIdx.y];
+  if constexpr (MS > 0) {
+    if ((int)blockIdx.x >= sweep_blocks) {
+      map_stamp_part<MS>(t, pb, blockIdx.x - sweep_blocks, gridDim.x - sweep_blocks);
+      return;
+    }
+  }
+  sweep_part<G>(t, nb, sweep_blocks);
+}
+
 // Row assembly, gj carry-over and dermis.  A group of KG lanes owns one
 // cell.  Rows of at most KCAP entries are assembled in LDS: the lower part
 // (written by k_sweep in sweep order) and the upper partners (gathered in
@@ -343,8 +358,7 @@ constexpr int KPRE = 2;    // entries of each row a lane asks for before it know
 constexpr int K_BLOCK = 128;
 constexpr int K_GROUPS = K_BLOCK / KG;
 
-__global__ void __launch_bounds__(K_BLOCK) k_finish(const Tis* __restrict__ T, int pb, int nb) {
-  const Tis& t = T[blockIdx.y];
+__device__ __forceinline__ void finish_part(const Tis& t, int pb, int nb, int nblk) {
   Status* st = t.st;
   const int n = st->n;
   const int ob = 1 - nb;
@@ -357,7 +371,7 @@ __global__ void __launch_bounds__(K_BLOCK) k_finish(const Tis* __restrict__ T, i
   const int grp = threadIdx.x / KG;
   const double gj_init = t.prm.gj_init;   // read before any store (a store could alias the descriptor)
   int mylen = 0;
-  const int stride = gridDim.x * K_GROUPS;
+  const int stride = nblk * K_GROUPS;
   for (int c = blockIdx.x * K_GROUPS + grp; c < n; c += stride) {
     const bool memb = c < t.nmemb;
     const int base = memb ? MEMB_ADJ : 0;
@@ -490,6 +504,22 @@ __global__ void __launch_bounds__(K_BLOCK) k_finish(const Tis* __restrict__ T, i
     atomicMax(&st->maxlen, mylen);
 }
 
+// Blocks [0, finish_blocks) finish the rows; with ZB planes per tile the rest
+// take the B stencil (ZB = 0: there is none), which needs the maps that the
+// sweep's launch stamped.
+template <int ZB>
+__global__ void __launch_bounds__(K_BLOCK) k_finish(const Tis* __restrict__ T, int pb, int nb, int finish_blocks, int bp,
+                                                    int xcd) {
+  const Tis& t = T[blockIdx.y];
+  if constexpr (ZB > 0) {
+    if ((int)blockIdx.x >= finish_blocks) {
+      ext_stim_part<ZB>(t, bp, xcd, blockIdx.x - finish_blocks, gridDim.x - finish_blocks);
+      return;
+    }
+  }
+  finish_part(t, pb, nb, finish_blocks);
+}
+
 __global__ void __launch_bounds__(256) k_zzmax(const Tis* __restrict__ T, int pb) {
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;
@@ -560,14 +590,38 @@ void launch_connect_insert(hipStream_t s, const Tis* dT, int ntis, int pb, int m
   }
 }
 
-void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave) {
+namespace {
+unsigned sweep_blocks(int max_n, int sweep_wave) { return sweep_wave ? (max_n + 3) / 4 : (max_n + 7) / 8; }
+template <int MS>
+void launch_sweep(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave) {
+  const unsigned gs = sweep_blocks(max_n, sweep_wave), gm = ((unsigned)max_n * MS + 255) / 256;
   if (sweep_wave) {
-    EPI_LAUNCH(K_SWEEP_WAVE, k_sweep<64>, dim3((max_n + 3) / 4, ntis), dim3(256), 0, s, dT, pb, nb);
+    EPI_LAUNCH(K_SWEEP_WAVE, (k_sweep<64, MS>), dim3(gs + gm, ntis), dim3(256), 0, s, dT, pb, nb, (int)gs);
   } else {
-    EPI_LAUNCH(K_SWEEP, k_sweep<32>, dim3((max_n + 7) / 8, ntis), dim3(256), 0, s, dT, pb, nb);
+    EPI_LAUNCH(K_SWEEP, (k_sweep<32, MS>), dim3(gs + gm, ntis), dim3(256), 0, s, dT, pb, nb, (int)gs);
   }
-  dim3 gk((max_n + K_GROUPS - 1) / K_GROUPS, ntis);
-  EPI_LAUNCH(K_FINISH, k_finish, gk, dim3(K_BLOCK), 0, s, dT, pb, nb);
+}
+}  // namespace
+
+void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave) {
+  launch_sweep<0>(s, dT, ntis, pb, nb, max_n, sweep_wave);
+  const unsigned gk = (max_n + K_GROUPS - 1) / K_GROUPS;
+  EPI_LAUNCH(K_FINISH, k_finish<0>, dim3(gk, ntis), dim3(K_BLOCK), 0, s, dT, pb, nb, (int)gk, 0, 0);
+}
+
+void launch_connect_field(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int bp, int max_n, long long b_tiles,
+                          const Tuning& tu) {
+  static_assert(K_BLOCK == BUILD_FIELD_BS, "the caller counts tiles of this many points");
+  if (tu.map_lanes == 16) launch_sweep<16>(s, dT, ntis, pb, nb, max_n, tu.sweep_wave);
+  else if (tu.map_lanes == 4) launch_sweep<4>(s, dT, ntis, pb, nb, max_n, tu.sweep_wave);
+  else launch_sweep<1>(s, dT, ntis, pb, nb, max_n, tu.sweep_wave);
+  // a multiple of 8 blocks, so that the XCD split applies
+  const unsigned gk = (max_n + K_GROUPS - 1) / K_GROUPS;
+  const unsigned gb = (unsigned)((std::min(std::max(b_tiles, 1LL), 1LL << 24) + 7) / 8 * 8);
+  by_zb(tu.b_zb, [&](auto zbc) {
+    EPI_LAUNCH(K_FINISH, k_finish<decltype(zbc)::value>, dim3(gk + gb, ntis), dim3(K_BLOCK), 0, s, dT, pb, nb, (int)gk, bp,
+               tu.b_xcd);
+  });
 }
 
 void launch_connect(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave) {

@@ -1,6 +1,7 @@
 // launch.h -- host-side launchers of the kernel families (one per .hip file)
 // and the optional per-kernel event timer.
 #pragma once
+#include <type_traits>
 #include <hip/hip_runtime.h>
 #include <hip/hip_ext.h>
 
@@ -60,6 +61,18 @@ void prof_add(int k, hipEvent_t a, hipEvent_t b, bool counted);
     }                                                                                         \
   } while (0)
 
+// f with a z chunk as a compile-time constant
+template <class F>
+inline void by_zb(int zb, F f) {
+  switch (zb) {
+    case 1: f(std::integral_constant<int, 1>()); break;
+    case 2: f(std::integral_constant<int, 2>()); break;
+    case 8: f(std::integral_constant<int, 8>()); break;
+    case 16: f(std::integral_constant<int, 16>()); break;
+    default: f(std::integral_constant<int, 4>()); break;
+  }
+}
+
 // where a force kernel leaves the statuses for a waiting host (pinned,
 // coherent memory; host == nullptr: nowhere): a Status per tissue, then value
 // into every tissue's seq
@@ -99,6 +112,12 @@ void launch_periodic_fix(hipStream_t s, const Tis* dT, int ntis, int pb, int max
 // the voxel maps with that many more blocks
 void launch_connect_insert(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, unsigned clear_blocks);
 void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave);
+// the rest of the build of a step with the stamping of the voxel maps as
+// further blocks of the sweep and the B stencil as further blocks of k_finish:
+// up to b_tiles tiles of BUILD_FIELD_BS points per tissue
+constexpr int BUILD_FIELD_BS = 128;
+void launch_connect_field(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int bp, int max_n, long long b_tiles,
+                          const Tuning& tu);
 void launch_connect(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave);
 void launch_zzmax(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n);
 // A snapshot's output record (CellManager::output's fields): a header of

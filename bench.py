@@ -47,8 +47,7 @@ MODELED = ("k_ca_cells", "k_atp", "k_ext_stim", "k_ca_fused", "k_forces")
 # written and read 8 k.  Split over the kernels that do each part:
 STEP_GROUPS = (
     ("forces", ("k_forces", "k_forces_long"), "88 + 4 k per cell", lambda kb: 88.0 + 4.0 * kb),
-    ("renewal", ("k_renew_one", "k_renew_flags", "k_renew_scan", "k_renew_apply", "k_remove", "k_pair_disperse",
-                 "k_initialize_sc"), "16 per cell", lambda kb: 16.0),
+    ("renewal", ("k_renew_one", "k_renew_cells", "k_renew_tail", "k_initialize_sc"), "16 per cell", lambda kb: 16.0),
     ("buckets", ("k_bucket_insert", "k_periodic_fix"),
      "16 per cell", lambda kb: 16.0),
     ("lists", ("k_sweep", "k_sweep_wave", "k_finish"), "4 k per cell", lambda kb: 4.0 * kb),

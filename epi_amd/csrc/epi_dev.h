@@ -79,7 +79,7 @@ struct Status {
   long long next_uid;
   unsigned long long zzmax_bits;  // calc_zzmax result (non-negative double bits)
   double zzmax;
-  long long timestep;     // CellManager::current_timestep; k_remove advances it once per renewal
+  long long timestep;     // CellManager::current_timestep; advanced once per renewal
   int nstat;              // records in cst_store
   int force_err;          // first error code of the force kernels, which run ahead of the status read-back
   long long grid_b;       // sum of nx*ny*iz_bound over the B sweeps (k_wl_b)
@@ -147,7 +147,7 @@ struct Tis {
   // position and radius with one 32-byte load instead of four
   GPtr<double4> pk;
   // state renewal
-  GPtr<int> div_slot; GPtr<double> div_dir;  // per division: parent, direction
+  GPtr<double> div_dir;   // per division: its direction
   GPtr<int> rm_list;
   // per block of 256 cells past the dermis: the cells that need a draw and
   // those that go, and how many

@@ -81,7 +81,7 @@ void prof_add(int k, hipEvent_t a, hipEvent_t b, bool counted) { g_prof.pending.
 namespace {
 
 const char* kKernelNames[K_COUNT] = {
-    "k_forces", "k_forces_long", "k_renew_flags", "k_renew_scan", "k_renew_apply", "k_remove", "k_pair_disperse",
+    "k_forces", "k_forces_long", "k_renew_cells", "k_renew_tail",
     "k_initialize_sc", "k_periodic_fix", "k_bucket_insert", "k_sweep",
     "k_finish", "k_zz_set", "k_zzmax", "k_map_clear", "k_map_stamp",
     "k_ext_stim", "k_ca_begin", "k_ca_vox", "k_ca_cells", "k_atp", "k_ca_end", "k_sw_reset",
@@ -312,7 +312,6 @@ void carve_tissue(Carver& cv, TH& h, Tis& t) {
   t.bucket = cv.take<int>((size_t)h.nbuckets * BUCKET_HEAD);
   t.bucket_rest = cv.take<int>((size_t)h.nbuckets * bucket_more(h.bcap));
   t.pk = cv.take<double4>(cap);
-  t.div_slot = cv.take<int>(cap);
   t.div_dir = cv.take<double>(3 * cap);
   t.rm_list = cv.take<int>(cap);
   t.rd_list = cv.take<int>(cap + 256);
@@ -1121,7 +1120,7 @@ int epi_pos_copy(epi_ctx* c) {
 int epi_cell_state_renew(epi_ctx* c) {
   if (!c) return EPI_ERR_INVALID;
   if (c->pos_pending) return fail(c, EPI_ERR_INVALID, "pos_copy must follow cell_interaction");
-  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, max_n(c), max_free(c), 0);
+  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, max_free(c), 0);
   HIPCHK(c, hipGetLastError());
   for (auto& v : c->dev_ts) v++;   // k_remove advances each tissue's timestep
   return EPI_OK;
@@ -1282,7 +1281,7 @@ constexpr int BUILD_FIELD_TISSUES = 1;
 hipError_t issue_build(epi_ctx* c, int mn, int mfree, int nb, int izb, bool side, bool join = true) {
   hipError_t e = hipSuccess;
   auto chk = [&](hipError_t r) { if (e == hipSuccess) e = r; };
-  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, mn, mfree, 1);
+  launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, mfree, 1);
   launch_connect_insert(c->stream, c->d_tis, c->T, c->pb, mn, map_clear_blocks(max_gsize(c)));
   if (!side) {
     long long tiles = 1;
@@ -1315,8 +1314,7 @@ hipError_t issue_build(epi_ctx* c, int mn, int mfree, int nb, int izb, bool side
 // *joined tells whether the main stream already waits for the side stream.
 int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
   constexpr unsigned long long seg =
-      (1ull << K_RENEW_ONE) | (1ull << K_RENEW_FLAGS) | (1ull << K_RENEW_SCAN) | (1ull << K_RENEW_APPLY) | (1ull << K_REMOVE) |
-      (1ull << K_PAIR_DISPERSE) | (1ull << K_BUCKET_INSERT) | (1ull << K_SWEEP_WAVE) |
+      (1ull << K_RENEW_ONE) | (1ull << K_RENEW_CELLS) | (1ull << K_RENEW_TAIL) | (1ull << K_BUCKET_INSERT) | (1ull << K_SWEEP_WAVE) |
       (1ull << K_SWEEP) | (1ull << K_FINISH) | (1ull << K_ZZ_SET) | (1ull << K_ZZMAX) |
       (1ull << K_MAP_CLEAR) | (1ull << K_MAP_STAMP) | (1ull << K_EXT_STIM);
   // kernels that are timed one by one stay apart
@@ -1332,8 +1330,8 @@ int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
   const int mr = std::max(mn, std::min((mn + 1023) / 1024 * 1024, mcap));
   const Tuning& tu = c->tu;
   // the renewal's form: a replay's grids do not depend on the count otherwise
-  const int mfree = max_free(c) <= RENEW_ONE ? RENEW_ONE : max_free(c) <= RENEW_FEW ? RENEW_FEW : mr;
-  const std::vector<long long> key = {1, std::min(mfree, RENEW_FEW + 1), c->pb, c->cb, c->cp, c->bp, nb, mr, izb, max_gsize(c),
+  const int mfree = max_free(c) <= RENEW_ONE ? RENEW_ONE : mr;
+  const std::vector<long long> key = {1, mfree > RENEW_ONE, c->pb, c->cb, c->cp, c->bp, nb, mr, izb, max_gsize(c),
                                       max_nx(c), max_ny(c), tu.b_zb, tu.b_rows, tu.map_lanes, tu.sweep_wave, tu.side_fork};
   return graph_run(c, key, [&] { return issue_build(c, mr, mfree, nb, izb, side); });
 }

@@ -3,18 +3,17 @@
 // The reference walks the non-membrane cells in one loop; each cell only
 // changes itself and the daughter it appends, but the replayed random draws
 // are consumed in loop order and a division consumes extra draws.  So:
-//   k_renew_flags  every cell's need of a draw or removal, packed in index
+//   k_renew_cells  every cell that needs no draw applies its own rule; the
+//                  cells that need one, and those that go, are packed in index
 //                  order per block of 256 cells;
-//   k_renew_scan   one workgroup per tissue places the packed lists behind
-//                  each other and decides the divisions 64 ready cells at a
-//                  time (a ballot finds the first division of a batch; draws
-//                  after it shift by its direction draws);
-//   k_renew_apply  every cell applies its own rule in parallel; daughters are
-//                  written at n_old + division rank (parent order);
-//   k_remove       remove_exec's swap-with-tail, one workgroup per tissue;
-//   k_pair_disperse pair_disperse from the higher-index partner.
-// Smaller tissues take fewer launches (launch_renew): k_renew_one does all of
-// it, k_renew_walk the first two and k_remove_pairs the last two.
+//   k_renew_tail   one workgroup per tissue places the packed lists behind
+//                  each other, decides the divisions 256 ready cells a round (a
+//                  ballot finds the first division; draws after it shift by
+//                  its direction draws), applies the ready cells' rule
+//                  (daughters are written at n_old + division rank, parent
+//                  order), and then takes remove_exec's swap-with-tail and
+//                  pair_disperse from the higher-index partner.
+// k_renew_one does both in one launch where the tissues are small.
 #include "epi_dev.h"
 #include "launch.h"
 #include "epi_group.h"
@@ -25,6 +24,9 @@ namespace epi {
 // (Tis::prm); these two are fixed by the reference's code
 constexpr double stoch_corr_coef = 1;
 constexpr double PI_D = 3.14159265358979323846;
+
+// an error of the renewal; one of the forces before it comes first
+__device__ __forceinline__ void renew_err(Status* st, int e) { set_err(st, st->force_err ? st->force_err : e); }
 
 // The constants of the renewal laws, copied out of the tissue's record once,
 // before a kernel's first store: the compiler cannot tell a cell store from
@@ -46,13 +48,13 @@ __device__ __forceinline__ double weighted_eps_kb(const RenewK& k, uint8_t malig
 
 // what the renewal reads of a cell, loaded in one round trip
 struct RCell {
-  double ageb, agek, div_age_thresh;
+  double ageb, agek, div_age_thresh, ca2p_avg, in_fat, ex_fat;
   int dermis, pair, rest_div_times, nlen;
-  uint8_t s;
+  uint8_t s, is_malignant;
 };
 __device__ __forceinline__ RCell load_rcell(const Tis& t, int cb, int c) {
-  return RCell{t.ageb[c], t.agek[c], t.div_age_thresh[c], t.dermis[c], t.pair[c], t.rest_div_times[c], t.nlen[cb][c],
-               t.state[c]};
+  return RCell{t.ageb[c], t.agek[c], t.div_age_thresh[c], t.ca2p_avg[c], t.in_fat[c], t.ex_fat[c], t.dermis[c], t.pair[c],
+               t.rest_div_times[c], t.nlen[cb][c], t.state[c], t.is_malignant[c]};
 }
 
 // is_divide_ready without the draw (:147-155), with the MUSUME/FIX guards of
@@ -71,269 +73,6 @@ __device__ __forceinline__ bool needs_draw(const RenewK& k, const RCell& r) {
 
 __device__ __forceinline__ bool to_remove(const RenewK& k, const RCell& r) {
   return (r.s == DEAD || r.s == AIR) && r.agek >= k.ADHE_CONST && (double)r.nlen <= k.DISA;
-}
-
-// The cells of each block of 256 that need a draw, and those that go, in
-// index order at the block's place of rd_list and rm_pack.
-constexpr int RBLOCK = 256;
-
-__global__ void __launch_bounds__(RBLOCK) k_renew_flags(const Tis* __restrict__ T, int cb) {
-  const Tis& t = T[blockIdx.y];
-  Status* st = t.st;
-  __shared__ int s_rd[4], s_rm[4];
-  const RenewK rk = renew_k(t.prm);
-  const int start = t.nmemb + t.nder;
-  const int n = st->n;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  for (int b = blockIdx.x; start + b * RBLOCK < n; b += gridDim.x) {
-    const int c = start + b * RBLOCK + tid;
-    const RCell r = load_rcell(t, cb, c < n ? c : n - 1);
-    const bool rd = c < n && needs_draw(rk, r), rm = c < n && to_remove(rk, r);
-    const unsigned long long mr = __ballot(rd), mm = __ballot(rm);
-    if (lane == 0) { s_rd[wv] = __popcll(mr); s_rm[wv] = __popcll(mm); }
-    __syncthreads();
-    int at_r = b * RBLOCK, at_m = b * RBLOCK, nr = 0, nm = 0;
-#pragma unroll
-    for (int w = 0; w < 4; w++) {
-      if (w < wv) { at_r += s_rd[w]; at_m += s_rm[w]; }
-      nr += s_rd[w]; nm += s_rm[w];
-    }
-    const unsigned long long below = (1ull << lane) - 1;
-    if (rd) t.rd_list[at_r + __popcll(mr & below)] = c;
-    if (rm) t.rm_pack[at_m + __popcll(mm & below)] = c;
-    if (tid == 0) { t.rd_n[b] = nr; t.rm_n[b] = nm; }
-    __syncthreads();   // the counts are the next block's from here
-  }
-}
-
-// the ordered part: one workgroup of RCHUNK lanes decides the divisions of up
-// to RCHUNK ready cells at a time
-constexpr int RCHUNK = 1024;
-struct RenewSh {
-  int ready[RCHUNK], der[RCHUNK];
-  double thr[RCHUNK], rhs[RCHUNK];
-  double rng[2 * RCHUNK];
-  int off_r[RCHUNK], off_m[RCHUNK];
-  int wcnt[16], wrm[16];
-  int ndiv;
-  long long cursor;
-};
-
-// the replay window for the next decisions (the caller synchronises)
-__device__ __forceinline__ void renew_window(const Tis& t, RenewSh& sh, long long cur0) {
-  for (int i = threadIdx.x; i < 2 * RCHUNK; i += RCHUNK) {
-    const long long q = cur0 + i;
-    sh.rng[i] = q < t.rng_n ? t.rng[q] : 2.0;
-  }
-}
-
-// the first wave decides sh.ready[0 .. tot_r) in index order, RENEW_U * 64
-// ready cells per round as long as none of them divides; draws past the window
-// come from memory.  A round is a chain of LDS reads and a ballot, whatever it
-// holds; a division adds its cell's positions and direction.
-constexpr int RENEW_U = 4;
-__device__ __forceinline__ void renew_decide(const Tis& t, RenewSh& sh, int pb, Status* st, int tot_r) {
-  const int lane = threadIdx.x;
-  const long long cur0 = sh.cursor;
-  long long cur = cur0;
-  int ndiv = sh.ndiv;
-  auto draw = [&](long long dpos) {
-    const long long wi = dpos - cur0;
-    return wi < 2 * RCHUNK ? sh.rng[wi] : t.rng[dpos];
-  };
-  int i = 0;
-  while (i < tot_r) {
-    bool act[RENEW_U], dv[RENEW_U];
-    int cell[RENEW_U];
-#pragma unroll
-    for (int u = 0; u < RENEW_U; u++) {
-      const int idx = i + 64 * u + lane;
-      const long long dpos = cur + 64 * u + lane;
-      act[u] = idx < tot_r;
-      cell[u] = sh.ready[act[u] ? idx : 0];
-      dv[u] = act[u] && dpos < t.rng_n && draw(dpos) * sh.thr[idx] <= sh.rhs[idx];
-    }
-    int f0 = -1;   // the first division's place in the round
-    int cf = 0;
-#pragma unroll
-    for (int u = RENEW_U - 1; u >= 0; u--) {
-      const unsigned long long md = __ballot(dv[u]);
-      if (md) { f0 = 64 * u + __ffsll((long long)md) - 1; cf = cell[u]; }
-    }
-    const int k = f0 < 0 ? min(64 * RENEW_U, tot_r - i) : f0;   // cells of the round that do not divide
-    // the cells up to the first division took their draws
-    if (cur + min(k + (f0 >= 0), tot_r - i) > t.rng_n && lane == 0) set_err(st, ERR_RNG_EXHAUSTED);
-#pragma unroll
-    for (int u = 0; u < RENEW_U; u++)
-      if (64 * u + lane < k) t.div_slot[cell[u]] = -1;
-    cur += k;
-    i += k;
-    if (f0 < 0) continue;
-    int att = 0;
-    if (lane == (f0 & 63)) {
-      // div_direction (:192-217) with draws after the decision draw
-      const P3 me = ld_pos(t, pb, cf), dm = ld_pos(t, pb, sh.der[i]);
-      const double nvx = p_diff_x(t, me.x, dm.x);
-      const double nvy = p_diff_y(t, me.y, dm.y);
-      const double nvz = me.z - dm.z;
-      const double norm = sqrt(nvx * nvx + nvy * nvy + nvz * nvz);
-      const double nx = nvx / norm, ny = nvy / norm, nz = nvz / norm;
-      double ox, oy, oz, sum;
-      long long dp = cur + 1;
-      do {
-        if (dp + 1 >= t.rng_n) { set_err(st, ERR_RNG_EXHAUSTED); ox = 1; oy = 0; oz = 0; att++; break; }
-        const double rand_theta = PI_D * draw(dp);
-        const double cr1 = cos(rand_theta);
-        const double sr1 = sin(rand_theta);
-        const double rand_phi = 2 * PI_D * draw(dp + 1);
-        const double cr2 = cos(rand_phi);
-        const double sr2 = sin(rand_phi);
-        const double rvx = sr1 * cr2;
-        const double rvy = sr1 * sr2;
-        const double rvz = cr1;
-        ox = ny * rvz - nz * rvy;
-        oy = nz * rvx - nx * rvz;
-        oz = nx * rvy - ny * rvx;
-        dp += 2;
-        att++;
-      } while ((sum = ox * ox + oy * oy + oz * oz) < 1.0e-14);
-      sum = sqrt(sum);
-      t.div_slot[cf] = ndiv;
-      t.div_dir[3 * ndiv + 0] = ox / sum;
-      t.div_dir[3 * ndiv + 1] = oy / sum;
-      t.div_dir[3 * ndiv + 2] = oz / sum;
-    }
-    att = __shfl(att, f0 & 63, 64);
-    ndiv++;
-    cur += 1 + 2 * att;
-    i++;
-  }
-  if (lane == 0) { sh.cursor = cur; sh.ndiv = ndiv; }
-}
-
-// a ready cell, its dermis and the two sides of its division test
-__device__ __forceinline__ void renew_ready(const Tis& t, RenewSh& sh, const RenewK& rk, int k, int c) {
-  sh.ready[k] = c;
-  sh.der[k] = t.dermis[c];
-  sh.thr[k] = t.div_age_thresh[c] * rk.stoch_div_time_ratio;
-  sh.rhs[k] = stoch_corr_coef * rk.DT_Cell * weighted_eps_kb(rk, t.is_malignant[c]) * rk.S2;
-}
-
-// exclusive offsets of the block's values a and b, and their sums
-__device__ __forceinline__ void renew_offsets(RenewSh& sh, int a, int b, int* off_a, int* off_b, int* sum_a, int* sum_b) {
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  int ta, tb;
-  int oa = group_exclusive_scan<64>(a, lane, &ta), ob = group_exclusive_scan<64>(b, lane, &tb);
-  if (lane == 0) { sh.wcnt[wv] = ta; sh.wrm[wv] = tb; }
-  __syncthreads();
-  int sa = 0, sb = 0;
-#pragma unroll
-  for (int w = 0; w < 16; w++) {
-    if (w < wv) { oa += sh.wcnt[w]; ob += sh.wrm[w]; }
-    sa += sh.wcnt[w]; sb += sh.wrm[w];
-  }
-  *off_a = oa; *off_b = ob; *sum_a = sa; *sum_b = sb;
-}
-
-// the last block whose offset is not past i (off ascends over m blocks)
-__device__ __forceinline__ int renew_block_of(const int* off, int m, int i) {
-  int lo = 0;
-  for (int step = RCHUNK / 2; step > 0; step >>= 1)
-    if (lo + step < m && off[lo + step] <= i) lo += step;
-  return lo;
-}
-
-// flags and ordered part of a tissue in one workgroup, RCHUNK cells at a time;
-// the cells to remove go to rm_list, their number is returned
-__device__ __forceinline__ int renew_walk(const Tis& t, RenewSh& sh, const RenewK& rk, int pb, int cb, int n_old) {
-  Status* st = t.st;
-  const int tid = threadIdx.x, start = t.nmemb + t.nder;
-  const long long cur0 = st->rng_pos;
-  if (tid == 0) { sh.cursor = cur0; sh.ndiv = 0; }
-  renew_window(t, sh, cur0);
-  int nrm = 0;
-  for (int base = start; base < n_old; base += RCHUNK) {
-    const int c = base + tid;
-    const RCell r = load_rcell(t, cb, min(c, n_old - 1));
-    const bool rd = c < n_old && needs_draw(rk, r), rm = c < n_old && to_remove(rk, r);
-    int off_r, off_m, tot_r, tot_m;
-    renew_offsets(sh, rd, rm, &off_r, &off_m, &tot_r, &tot_m);
-    if (base > start && tot_r) renew_window(t, sh, sh.cursor);
-    if (rd) renew_ready(t, sh, rk, off_r, c);
-    if (rm) t.rm_list[nrm + off_m] = c;
-    nrm += tot_m;
-    __syncthreads();
-    if (tot_r && tid < 64) renew_decide(t, sh, pb, st, tot_r);
-    __syncthreads();
-  }
-  return nrm;
-}
-
-// k_renew_flags and k_renew_scan in one launch
-__global__ void __launch_bounds__(RCHUNK) k_renew_walk(const Tis* __restrict__ T, int pb, int cb) {
-  const Tis& t = T[blockIdx.y];
-  Status* st = t.st;
-  __shared__ RenewSh sh;
-  const int n_old = st->n;
-  const RenewK rk = renew_k(t.prm);
-  if (threadIdx.x == 0) st->n_old = n_old;
-  if (threadIdx.x == 64 && st->force_err) set_err(st, st->force_err);
-  const int nrm = renew_walk(t, sh, rk, pb, cb, n_old);
-  if (threadIdx.x == 0) {
-    st->rng_pos = sh.cursor;
-    st->ndiv = sh.ndiv;
-    st->nrm = nrm;
-  }
-}
-
-// What bounds it is the chain of round trips of its one workgroup: the
-// blocks' counts, the packed cells, their words and the draws, each for up to
-// RCHUNK blocks or ready cells at once, and then the rounds of renew_decide.
-// 20,000 cells past the membrane: 18.6 us (walking the cells 1024 at a time,
-// 64 ready cells a round, 24).
-__global__ void __launch_bounds__(RCHUNK) k_renew_scan(const Tis* __restrict__ T, int pb) {
-  const Tis& t = T[blockIdx.y];
-  Status* st = t.st;
-  __shared__ RenewSh sh;
-  const int tid = threadIdx.x;
-  const int start = t.nmemb + t.nder;
-  const int n_old = st->n;
-  const RenewK rk = renew_k(t.prm);
-  if (tid == 0) { sh.cursor = st->rng_pos; sh.ndiv = 0; st->n_old = n_old; }
-  if (tid == 64 && st->force_err) set_err(st, st->force_err);
-  const int nblk = n_old > start ? (n_old - start + RBLOCK - 1) / RBLOCK : 0;
-  int nrm = 0;
-  for (int b0 = 0; b0 < nblk; b0 += RCHUNK) {
-    const int nb = min(nblk - b0, RCHUNK);
-    const int cr = tid < nb ? t.rd_n[b0 + tid] : 0, cm = tid < nb ? t.rm_n[b0 + tid] : 0;
-    int off_r, off_m, tot_r, tot_m;
-    renew_offsets(sh, cr, cm, &off_r, &off_m, &tot_r, &tot_m);
-    sh.off_r[tid] = off_r;
-    sh.off_m[tid] = off_m;
-    __syncthreads();
-    for (int i = tid; i < tot_m; i += RCHUNK) {
-      const int b = renew_block_of(sh.off_m, nb, i);
-      t.rm_list[nrm + i] = t.rm_pack[(size_t)(b0 + b) * RBLOCK + i - sh.off_m[b]];
-    }
-    nrm += tot_m;
-    for (int r0 = 0; r0 < tot_r; r0 += RCHUNK) {
-      const int m = min(tot_r - r0, RCHUNK);
-      renew_window(t, sh, sh.cursor);
-      if (tid < m) {
-        const int b = renew_block_of(sh.off_r, nb, r0 + tid);
-        renew_ready(t, sh, rk, tid, t.rd_list[(size_t)(b0 + b) * RBLOCK + r0 + tid - sh.off_r[b]]);
-      }
-      __syncthreads();
-      if (tid < 64) renew_decide(t, sh, pb, st, m);
-      __syncthreads();
-    }
-    __syncthreads();   // off_r, off_m and the counts are the next blocks' from here
-  }
-  if (tid == 0) {
-    st->rng_pos = sh.cursor;
-    st->ndiv = sh.ndiv;
-    st->nrm = nrm;
-  }
 }
 
 // ageing and lipid laws (:31-119)
@@ -355,7 +94,7 @@ __device__ __forceinline__ Lipid lipid_rates(const RenewK& k, double ca2p_avg, d
 // cell_divide (:227-270) for division rank k of parent c
 __device__ void divide(const Tis& t, int pb, int cpar, int c, int k, int n_old, long long next_uid) {
   const int d = n_old + k;
-  if (d >= t.cap) { set_err(t.st, ERR_CAPACITY); return; }
+  if (d >= t.cap) { renew_err(t.st, ERR_CAPACITY); return; }
   const P3 p = ld_pos(t, pb, c);
   const double divx = t.div_dir[3 * k], divy = t.div_dir[3 * k + 1], divz = t.div_dir[3 * k + 2];
   const double cav = t.ca2p[cpar][c];
@@ -397,13 +136,10 @@ __device__ void divide(const Tis& t, int pb, int cpar, int c, int k, int n_old, 
   t.pos[pb][2][c] = p.z + divz * 0.5 * delta_L;
 }
 
-// one cell's rule; 1 if it cornifies
-__device__ __forceinline__ int renew_cell(const Tis& t, const RenewK& pm, int pb, int cb, int cpar, int c, int n_old,
-                                          long long next_uid, long long ts) {
-  const RCell r = load_rcell(t, cb, c);
-  const double cav = t.ca2p_avg[c], in_fat = t.in_fat[c], ex_fat = t.ex_fat[c];
-  const uint8_t malig = t.is_malignant[c];
-  const int slot = t.div_slot[c];
+// the rule of a cell that needs no draw; 1 if it cornifies
+__device__ __forceinline__ int renew_cell(const Tis& t, const RenewK& pm, const RCell& r, int c, long long ts) {
+  const double cav = r.ca2p_avg, in_fat = r.in_fat;
+  const uint8_t malig = r.is_malignant;
   const double DT_Cell = pm.DT_Cell;
   switch (r.s) {
     case ALIVE:   // _ALIVE_state_renew :347-358
@@ -415,7 +151,7 @@ __device__ __forceinline__ int renew_cell(const Tis& t, const RenewK& pm, int pb
         const Lipid l = lipid_rates(pm, cav, r.agek);
         const double tmp = l.release * in_fat;
         t.in_fat[c] = in_fat + DT_Cell * (l.make * (1.0 - in_fat) - tmp);
-        t.ex_fat[c] = ex_fat + DT_Cell * tmp;
+        t.ex_fat[c] = r.ex_fat + DT_Cell * tmp;
         t.agek[c] = r.agek + DT_Cell * agek_ALIVE_const(pm, cav, malig);
       }
       break;
@@ -424,15 +160,13 @@ __device__ __forceinline__ int renew_cell(const Tis& t, const RenewK& pm, int pb
       break;
     case FIX: case MUSUME: {
       if (r.s == FIX) {   // _FIX_state_renew :308-324
-        if (r.dermis < 0) { set_err(t.st, ERR_NO_DERMIS); break; }
+        if (r.dermis < 0) { renew_err(t.st, ERR_NO_DERMIS); break; }
       } else if (r.dermis < 0 && r.pair < 0) {   // _MUSUME_state_renew :282-302 (SYSTEM == WHOLE)
         t.state[c] = ALIVE;
         t.cst[3 * c] = ts;   // :287
         break;
       }
-      const int k = needs_draw(pm, r) ? slot : -1;
-      if (k >= 0) divide(t, pb, cpar, c, k, n_old, next_uid);
-      else t.ageb[c] = r.ageb + DT_Cell * ageb_const(pm, cav, malig);
+      t.ageb[c] = r.ageb + DT_Cell * ageb_const(pm, cav, malig);
       break;
     }
     default:
@@ -441,17 +175,185 @@ __device__ __forceinline__ int renew_cell(const Tis& t, const RenewK& pm, int pb
   return 0;
 }
 
-__global__ void __launch_bounds__(256) k_renew_apply(const Tis* __restrict__ T, int pb, int cb, int cpar) {
+// The cells of each block of 256 that need a draw, and those that go, in
+// index order at the block's place of rd_list and rm_pack; the others' rule.
+// No cell's rule touches another cell, and a cell that needs a draw waits for
+// k_renew_tail, so the two parts need no order between them.
+constexpr int RBLOCK = 256;
+
+__global__ void __launch_bounds__(RBLOCK) k_renew_cells(const Tis* __restrict__ T, int cb) {
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;
-  const int n_old = st->n_old;
-  const long long next_uid = st->next_uid;
+  __shared__ int s_rd[4], s_rm[4];
+  const RenewK rk = renew_k(t.prm);
+  const int start = t.nmemb + t.nder;
+  const int n = st->n;
   const long long ts = st->timestep;
-  const RenewK pm = renew_k(t.prm);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   int ncorn = 0;
-  for (int c = t.nmemb + t.nder + blockIdx.x * blockDim.x + threadIdx.x; c < n_old; c += gridDim.x * blockDim.x)
-    ncorn += renew_cell(t, pm, pb, cb, cpar, c, n_old, next_uid, ts);
+  for (int b = blockIdx.x; start + b * RBLOCK < n; b += gridDim.x) {
+    const int c = start + b * RBLOCK + tid;
+    const RCell r = load_rcell(t, cb, c < n ? c : n - 1);
+    const bool rd = c < n && needs_draw(rk, r), rm = c < n && to_remove(rk, r);
+    const unsigned long long mr = __ballot(rd), mm = __ballot(rm);
+    if (lane == 0) { s_rd[wv] = __popcll(mr); s_rm[wv] = __popcll(mm); }
+    __syncthreads();
+    int at_r = b * RBLOCK, at_m = b * RBLOCK, nr = 0, nm = 0;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      if (w < wv) { at_r += s_rd[w]; at_m += s_rm[w]; }
+      nr += s_rd[w]; nm += s_rm[w];
+    }
+    const unsigned long long below = (1ull << lane) - 1;
+    if (rd) t.rd_list[at_r + __popcll(mr & below)] = c;
+    if (rm) t.rm_pack[at_m + __popcll(mm & below)] = c;
+    if (tid == 0) { t.rd_n[b] = nr; t.rm_n[b] = nm; }
+    if (c < n && !rd) ncorn += renew_cell(t, rk, r, c, ts);
+    __syncthreads();   // the counts are the next block's from here
+  }
   if (ncorn) atomicAdd(&st->sw, ncorn);
+}
+
+// the ordered part: one workgroup of RCHUNK lanes decides the divisions of up
+// to RCHUNK ready cells at a time
+constexpr int RCHUNK = 1024;
+struct RenewSh {
+  int ready[RCHUNK], der[RCHUNK], slot[RCHUNK];   // slot: the division's rank, or -1
+  double thr[RCHUNK], rhs[RCHUNK];
+  double rng[2 * RCHUNK];
+  int off_r[RCHUNK], off_m[RCHUNK];
+  int wcnt[16], wrm[16];
+  int ndiv;
+  long long cursor;
+};
+
+// the replay window for the next decisions (the caller synchronises)
+__device__ __forceinline__ void renew_window(const Tis& t, RenewSh& sh, long long cur0) {
+  for (int i = threadIdx.x; i < 2 * RCHUNK; i += RCHUNK) {
+    const long long q = cur0 + i;
+    sh.rng[i] = q < t.rng_n ? t.rng[q] : 2.0;
+  }
+}
+
+// the first wave decides sh.ready[0 .. tot_r) in index order, RENEW_U * 64
+// ready cells per round as long as none of them divides; draws past the window
+// come from memory.  A round is a chain of LDS reads and a ballot, whatever it
+// holds; a division adds its cell's positions and direction.
+constexpr int RENEW_U = 4;
+__device__ __forceinline__ void renew_decide(const Tis& t, RenewSh& sh, int pb, Status* st, int tot_r) {
+  const int lane = threadIdx.x;
+  const long long cur0 = sh.cursor;
+  long long cur = cur0;
+  int ndiv = sh.ndiv;
+  auto draw = [&](long long dpos) {
+    const long long wi = dpos - cur0;
+    return wi < 2 * RCHUNK ? sh.rng[wi] : t.rng[dpos];
+  };
+  int i = 0;
+  while (i < tot_r) {
+    bool act[RENEW_U], dv[RENEW_U];
+#pragma unroll
+    for (int u = 0; u < RENEW_U; u++) {
+      const int idx = i + 64 * u + lane;
+      const long long dpos = cur + 64 * u + lane;
+      act[u] = idx < tot_r;
+      dv[u] = act[u] && dpos < t.rng_n && draw(dpos) * sh.thr[idx] <= sh.rhs[idx];
+    }
+    int f0 = -1;   // the first division's place in the round
+#pragma unroll
+    for (int u = RENEW_U - 1; u >= 0; u--) {
+      const unsigned long long md = __ballot(dv[u]);
+      if (md) f0 = 64 * u + __ffsll((long long)md) - 1;
+    }
+    const int k = f0 < 0 ? min(64 * RENEW_U, tot_r - i) : f0;   // cells of the round that do not divide
+    // the cells up to the first division took their draws
+    if (cur + min(k + (f0 >= 0), tot_r - i) > t.rng_n && lane == 0) renew_err(st, ERR_RNG_EXHAUSTED);
+#pragma unroll
+    for (int u = 0; u < RENEW_U; u++)
+      if (64 * u + lane < k) sh.slot[i + 64 * u + lane] = -1;
+    cur += k;
+    i += k;
+    if (f0 < 0) continue;
+    int att = 0;
+    if (lane == (f0 & 63)) {
+      // div_direction (:192-217) with draws after the decision draw
+      const P3 me = ld_pos(t, pb, sh.ready[i]), dm = ld_pos(t, pb, sh.der[i]);
+      const double nvx = p_diff_x(t, me.x, dm.x);
+      const double nvy = p_diff_y(t, me.y, dm.y);
+      const double nvz = me.z - dm.z;
+      const double norm = sqrt(nvx * nvx + nvy * nvy + nvz * nvz);
+      const double nx = nvx / norm, ny = nvy / norm, nz = nvz / norm;
+      double ox, oy, oz, sum;
+      long long dp = cur + 1;
+      do {
+        if (dp + 1 >= t.rng_n) { renew_err(st, ERR_RNG_EXHAUSTED); ox = 1; oy = 0; oz = 0; att++; break; }
+        const double rand_theta = PI_D * draw(dp);
+        const double cr1 = cos(rand_theta);
+        const double sr1 = sin(rand_theta);
+        const double rand_phi = 2 * PI_D * draw(dp + 1);
+        const double cr2 = cos(rand_phi);
+        const double sr2 = sin(rand_phi);
+        const double rvx = sr1 * cr2;
+        const double rvy = sr1 * sr2;
+        const double rvz = cr1;
+        ox = ny * rvz - nz * rvy;
+        oy = nz * rvx - nx * rvz;
+        oz = nx * rvy - ny * rvx;
+        dp += 2;
+        att++;
+      } while ((sum = ox * ox + oy * oy + oz * oz) < 1.0e-14);
+      sum = sqrt(sum);
+      sh.slot[i] = ndiv;
+      t.div_dir[3 * ndiv + 0] = ox / sum;
+      t.div_dir[3 * ndiv + 1] = oy / sum;
+      t.div_dir[3 * ndiv + 2] = oz / sum;
+    }
+    att = __shfl(att, f0 & 63, 64);
+    ndiv++;
+    cur += 1 + 2 * att;
+    i++;
+  }
+  if (lane == 0) { sh.cursor = cur; sh.ndiv = ndiv; }
+}
+
+// a ready cell, its dermis and the two sides of its division test
+__device__ __forceinline__ void renew_ready(const Tis& t, RenewSh& sh, const RenewK& rk, int k, int c) {
+  sh.ready[k] = c;
+  sh.der[k] = t.dermis[c];
+  sh.thr[k] = t.div_age_thresh[c] * rk.stoch_div_time_ratio;
+  sh.rhs[k] = stoch_corr_coef * rk.DT_Cell * weighted_eps_kb(rk, t.is_malignant[c]) * rk.S2;
+}
+
+// the rule of the k-th ready cell, decided
+__device__ __forceinline__ void renew_ready_rule(const Tis& t, const RenewSh& sh, const RenewK& rk, int pb, int cpar, int k,
+                                                 int n_old, long long next_uid) {
+  const int c = sh.ready[k];
+  if (sh.slot[k] >= 0) divide(t, pb, cpar, c, sh.slot[k], n_old, next_uid);
+  else t.ageb[c] = t.ageb[c] + rk.DT_Cell * ageb_const(rk, t.ca2p_avg[c], t.is_malignant[c]);
+}
+
+// exclusive offsets of the block's values a and b, and their sums
+__device__ __forceinline__ void renew_offsets(RenewSh& sh, int a, int b, int* off_a, int* off_b, int* sum_a, int* sum_b) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  int ta, tb;
+  int oa = group_exclusive_scan<64>(a, lane, &ta), ob = group_exclusive_scan<64>(b, lane, &tb);
+  if (lane == 0) { sh.wcnt[wv] = ta; sh.wrm[wv] = tb; }
+  __syncthreads();
+  int sa = 0, sb = 0;
+#pragma unroll
+  for (int w = 0; w < 16; w++) {
+    if (w < wv) { oa += sh.wcnt[w]; ob += sh.wrm[w]; }
+    sa += sh.wcnt[w]; sb += sh.wrm[w];
+  }
+  *off_a = oa; *off_b = ob; *sum_a = sa; *sum_b = sb;
+}
+
+// the last block whose offset is not past i (off ascends over m blocks)
+__device__ __forceinline__ int renew_block_of(const int* off, int m, int i) {
+  int lo = 0;
+  for (int step = RCHUNK / 2; step > 0; step >>= 1)
+    if (lo + step < m && off[lo + step] <= i) lo += step;
+  return lo;
 }
 
 // CellManager::remove_exec (cellmanager.cpp:338-352): queued slot q_i takes
@@ -479,7 +381,7 @@ __device__ __forceinline__ void remove_cells(const Tis& t, int pb, int zero_zz, 
       ns += __popcll(mk);
     }
     if (threadIdx.x == 0) {
-      if (ns > t.cap) set_err(st, ERR_CAPACITY);
+      if (ns > t.cap) renew_err(st, ERR_CAPACITY);
       st->nstat = min(ns, t.cap);
       st->timestep = ts + 1;
     }
@@ -487,8 +389,8 @@ __device__ __forceinline__ void remove_cells(const Tis& t, int pb, int zero_zz, 
   __syncthreads();
   for (int i = threadIdx.x; i < nrm; i += blockDim.x) {
     const int q = t.rm_list[i];
-    if (q >= N - i) { set_err(st, ERR_REMOVE_ALIAS); continue; }
-    if (t.pair[q] >= 0) set_err(st, ERR_PAIR_REMOVED);
+    if (q >= N - i) { renew_err(st, ERR_REMOVE_ALIAS); continue; }
+    if (t.pair[q] >= 0) renew_err(st, ERR_PAIR_REMOVED);
     const int s = N - 1 - i;
     if (s == q) continue;
     t.state[q] = t.state[s]; t.is_malignant[q] = t.is_malignant[s]; t.touch_air[q] = t.touch_air[s];
@@ -519,7 +421,7 @@ __device__ __forceinline__ void remove_cells(const Tis& t, int pb, int zero_zz, 
     if (p >= N - nrm) {
       const int j = N - 1 - p;
       np = t.rm_list[j];
-      if (np == p || np >= N - j) { set_err(st, ERR_PAIR_REMOVED); continue; }
+      if (np == p || np >= N - j) { renew_err(st, ERR_PAIR_REMOVED); continue; }
     } else {
       t.pair[p] = q;
     }
@@ -532,53 +434,107 @@ __device__ __forceinline__ void remove_cells(const Tis& t, int pb, int zero_zz, 
   }
 }
 
-__global__ void __launch_bounds__(256) k_remove(const Tis* __restrict__ T, int pb, int zero_zz) {
-  const Tis& t = T[blockIdx.y];
-  const int ndiv = t.st->ndiv, nrm = t.st->nrm;
-  remove_cells(t, pb, zero_zz, t.st->n_old + ndiv, ndiv, nrm);
+// pair_disperse (:364-385), from the higher-index partner (:422-428), by one
+// workgroup of RCHUNK lanes; few cells have a partner, so the pair words of
+// four cells per lane are read at a time
+__device__ __forceinline__ void disperse_pair(const Tis& t, int pb, int c, int p) {
+  const double eps_L = t.prm.eps_L, unpair_dist_coef = t.prm.unpair_dist_coef;
+  const double rad_sum = t.radius[c] + t.radius[p];
+  const double unpair_th = unpair_dist_coef * rad_sum;
+  const double snl = t.spr_nat_len[c];
+  if (snl < 2.0 * t.radius[c]) {
+    const double v = snl + t.prm.DT_Cell * eps_L;
+    t.spr_nat_len[c] = v;
+    t.spr_nat_len[p] = v;
+  } else if (dist_sq(t, ld_pos(t, pb, c), ld_pos(t, pb, p)) > unpair_th * unpair_th) {
+    t.spr_nat_len[c] = 0;
+    t.spr_nat_len[p] = 0;
+    t.pair[p] = -1;
+    t.pair[c] = -1;
+  }
 }
-
-// pair_disperse (:364-385), from the higher-index partner (:422-428), by
-// `lanes` lanes of which this is lane `first`
-__device__ __forceinline__ void disperse_pairs(const Tis& t, int pb, int n, int first, int lanes) {
-  for (int c = t.nmemb + t.nder + first; c < n; c += lanes) {
-    const int p = t.pair[c];
-    if (p < 0 || !(c > p)) continue;
-    const double eps_L = t.prm.eps_L, unpair_dist_coef = t.prm.unpair_dist_coef;
-    const double rad_sum = t.radius[c] + t.radius[p];
-    const double unpair_th = unpair_dist_coef * rad_sum;
-    const double snl = t.spr_nat_len[c];
-    if (snl < 2.0 * t.radius[c]) {
-      const double v = snl + t.prm.DT_Cell * eps_L;
-      t.spr_nat_len[c] = v;
-      t.spr_nat_len[p] = v;
-    } else if (dist_sq(t, ld_pos(t, pb, c), ld_pos(t, pb, p)) > unpair_th * unpair_th) {
-      t.spr_nat_len[c] = 0;
-      t.spr_nat_len[p] = 0;
-      t.pair[p] = -1;
-      t.pair[c] = -1;
+__device__ __forceinline__ void disperse_pairs(const Tis& t, int pb, int n) {
+  constexpr int U = 4;
+  for (int c0 = t.nmemb + t.nder + threadIdx.x; c0 < n; c0 += U * RCHUNK) {
+    int p[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) p[u] = t.pair[min(c0 + u * RCHUNK, n - 1)];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int c = c0 + u * RCHUNK;
+      if (c < n && p[u] >= 0 && c > p[u]) disperse_pair(t, pb, c, p[u]);
     }
   }
 }
 
-__global__ void __launch_bounds__(256) k_pair_disperse(const Tis* __restrict__ T, int pb) {
-  const Tis& t = T[blockIdx.y];
-  disperse_pairs(t, pb, t.st->n, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
-}
-
-// k_remove and k_pair_disperse in one launch
-__global__ void __launch_bounds__(RCHUNK) k_remove_pairs(const Tis* __restrict__ T, int pb, int zero_zz) {
-  const Tis& t = T[blockIdx.y];
-  const int ndiv = t.st->ndiv, nrm = t.st->nrm, N = t.st->n_old + ndiv;
-  remove_cells(t, pb, zero_zz, N, ndiv, nrm);
+// What follows a tissue's decisions: the counts, removals and pairs
+__device__ __forceinline__ void renew_end(const Tis& t, const RenewSh& sh, int pb, int zero_zz, int n_old, int nrm) {
+  Status* st = t.st;
+  const int ndiv = sh.ndiv;
+  if (threadIdx.x == 0) {
+    st->rng_pos = sh.cursor;
+    st->ndiv = ndiv;
+    st->nrm = nrm;
+    st->n_old = n_old;
+  }
+  if (threadIdx.x == 64 && st->force_err) set_err(st, st->force_err);
+  remove_cells(t, pb, zero_zz, n_old + ndiv, ndiv, nrm);
   __syncthreads();
-  disperse_pairs(t, pb, N - nrm, threadIdx.x, RCHUNK);
+  disperse_pairs(t, pb, n_old + ndiv - nrm);
 }
 
-// The whole renewal of tissues with few cells, one workgroup per tissue: the
-// five launches above depend on each other, and for few cells each is its own
-// start and a round trip or two.  A tissue of 420 cells: 9.6 us, against 16.8 and
-// four gaps of about 1 us.
+// What bounds it is the chain of round trips of its one workgroup: the
+// blocks' counts, the packed cells, their words and the draws, each for up to
+// RCHUNK blocks or ready cells at once, then the rounds of renew_decide, the
+// removals and the pairs.  With k_renew_cells, 2,000 cells past the membrane:
+// 4.3 + 9.8 us (five launches that waited for each other, the walk 1024 cells
+// at a time: 20.8 and four gaps); 20,000 cells: 5.1 + 26.4 (43.2).
+__global__ void __launch_bounds__(RCHUNK) k_renew_tail(const Tis* __restrict__ T, int pb, int cpar, int zero_zz) {
+  const Tis& t = T[blockIdx.y];
+  Status* st = t.st;
+  __shared__ RenewSh sh;
+  const int tid = threadIdx.x;
+  const int start = t.nmemb + t.nder;
+  const int n_old = st->n;
+  const long long next_uid = st->next_uid;
+  const RenewK rk = renew_k(t.prm);
+  if (tid == 0) { sh.cursor = st->rng_pos; sh.ndiv = 0; }
+  const int nblk = n_old > start ? (n_old - start + RBLOCK - 1) / RBLOCK : 0;
+  int nrm = 0;
+  for (int b0 = 0; b0 < nblk; b0 += RCHUNK) {
+    const int nb = min(nblk - b0, RCHUNK);
+    const int cr = tid < nb ? t.rd_n[b0 + tid] : 0, cm = tid < nb ? t.rm_n[b0 + tid] : 0;
+    int off_r, off_m, tot_r, tot_m;
+    renew_offsets(sh, cr, cm, &off_r, &off_m, &tot_r, &tot_m);
+    sh.off_r[tid] = off_r;
+    sh.off_m[tid] = off_m;
+    __syncthreads();
+    for (int i = tid; i < tot_m; i += RCHUNK) {
+      const int b = renew_block_of(sh.off_m, nb, i);
+      t.rm_list[nrm + i] = t.rm_pack[(size_t)(b0 + b) * RBLOCK + i - sh.off_m[b]];
+    }
+    nrm += tot_m;
+    for (int r0 = 0; r0 < tot_r; r0 += RCHUNK) {
+      const int m = min(tot_r - r0, RCHUNK);
+      renew_window(t, sh, sh.cursor);
+      if (tid < m) {
+        const int b = renew_block_of(sh.off_r, nb, r0 + tid);
+        renew_ready(t, sh, rk, tid, t.rd_list[(size_t)(b0 + b) * RBLOCK + r0 + tid - sh.off_r[b]]);
+      }
+      __syncthreads();
+      if (tid < 64) renew_decide(t, sh, pb, st, m);
+      __syncthreads();
+      if (tid < m) renew_ready_rule(t, sh, rk, pb, cpar, tid, n_old, next_uid);
+      __syncthreads();   // the lists are the next cells' from here
+    }
+    __syncthreads();   // off_r, off_m and the counts are the next blocks' from here
+  }
+  __syncthreads();
+  renew_end(t, sh, pb, zero_zz, n_old, nrm);
+}
+
+// The whole renewal of tissues with few cells, one workgroup per tissue.  A
+// tissue of 420 cells: 9.6 us, against about 3.5 and 7 and the gap.
 __global__ void __launch_bounds__(RCHUNK) k_renew_one(const Tis* __restrict__ T, int pb, int cb, int cpar, int zero_zz) {
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;
@@ -587,26 +543,32 @@ __global__ void __launch_bounds__(RCHUNK) k_renew_one(const Tis* __restrict__ T,
   const int tid = threadIdx.x;
   const int start = t.nmemb + t.nder;
   const int n_old = st->n;
-  const long long next_uid = st->next_uid, ts = st->timestep;
+  const long long next_uid = st->next_uid, ts = st->timestep, cur0 = st->rng_pos;
   const RenewK rk = renew_k(t.prm);
-  if (tid == 0) { s_corn = 0; st->n_old = n_old; }
-  if (tid == 64 && st->force_err) set_err(st, st->force_err);
-  const int nrm = renew_walk(t, sh, rk, pb, cb, n_old);
-  __syncthreads();
-  const int ndiv = sh.ndiv;
-  int ncorn = 0;
-  for (int c = start + tid; c < n_old; c += RCHUNK) ncorn += renew_cell(t, rk, pb, cb, cpar, c, n_old, next_uid, ts);
+  if (tid == 0) { sh.cursor = cur0; sh.ndiv = 0; s_corn = 0; }
+  renew_window(t, sh, cur0);
+  int nrm = 0, ncorn = 0;
+  for (int base = start; base < n_old; base += RCHUNK) {
+    const int c = base + tid;
+    const RCell r = load_rcell(t, cb, min(c, n_old - 1));
+    const bool rd = c < n_old && needs_draw(rk, r), rm = c < n_old && to_remove(rk, r);
+    int off_r, off_m, tot_r, tot_m;
+    renew_offsets(sh, rd, rm, &off_r, &off_m, &tot_r, &tot_m);
+    if (base > start && tot_r) renew_window(t, sh, sh.cursor);
+    if (rd) renew_ready(t, sh, rk, off_r, c);
+    if (rm) t.rm_list[nrm + off_m] = c;
+    nrm += tot_m;
+    __syncthreads();
+    if (tot_r && tid < 64) renew_decide(t, sh, pb, st, tot_r);
+    if (c < n_old && !rd) ncorn += renew_cell(t, rk, r, c, ts);
+    __syncthreads();
+    if (tid < tot_r) renew_ready_rule(t, sh, rk, pb, cpar, tid, n_old, next_uid);
+    __syncthreads();   // the lists are the next cells' from here
+  }
   if (ncorn) atomicAdd(&s_corn, ncorn);
   __syncthreads();
-  if (tid == 0) {
-    st->rng_pos = sh.cursor;
-    st->ndiv = ndiv;
-    st->nrm = nrm;
-    st->sw += s_corn;
-  }
-  remove_cells(t, pb, zero_zz, n_old + ndiv, ndiv, nrm);
-  __syncthreads();
-  disperse_pairs(t, pb, n_old + ndiv - nrm, tid, RCHUNK);
+  if (tid == 0) st->sw += s_corn;
+  renew_end(t, sh, pb, zero_zz, n_old, nrm);
 }
 
 // initialize_sc (:435-443)
@@ -636,24 +598,13 @@ __global__ void __launch_bounds__(256) k_periodic_fix(const Tis* __restrict__ T,
   }
 }
 
-void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_n, int max_free,
-                  int zero_zz) {
+void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_free, int zero_zz) {
   if (max_free <= RENEW_ONE) {
     EPI_LAUNCH(K_RENEW_ONE, k_renew_one, dim3(1, ntis), dim3(RCHUNK), 0, s, dT, pb, cb, cpar, zero_zz);
     return;
   }
-  dim3 g((max_n + 255) / 256, ntis);
-  if (max_free <= RENEW_FEW) {
-    EPI_LAUNCH(K_RENEW_SCAN, k_renew_walk, dim3(1, ntis), dim3(RCHUNK), 0, s, dT, pb, cb);
-    EPI_LAUNCH(K_RENEW_APPLY, k_renew_apply, g, dim3(256), 0, s, dT, pb, cb, cpar);
-    EPI_LAUNCH(K_REMOVE, k_remove_pairs, dim3(1, ntis), dim3(RCHUNK), 0, s, dT, pb, zero_zz);
-    return;
-  }
-  EPI_LAUNCH(K_RENEW_FLAGS, k_renew_flags, g, dim3(RBLOCK), 0, s, dT, cb);
-  EPI_LAUNCH(K_RENEW_SCAN, k_renew_scan, dim3(1, ntis), dim3(RCHUNK), 0, s, dT, pb);
-  EPI_LAUNCH(K_RENEW_APPLY, k_renew_apply, g, dim3(256), 0, s, dT, pb, cb, cpar);
-  EPI_LAUNCH(K_REMOVE, k_remove, dim3(1, ntis), dim3(256), 0, s, dT, pb, zero_zz);
-  EPI_LAUNCH(K_PAIR_DISPERSE, k_pair_disperse, g, dim3(256), 0, s, dT, pb);
+  EPI_LAUNCH(K_RENEW_CELLS, k_renew_cells, dim3((max_free + RBLOCK - 1) / RBLOCK, ntis), dim3(RBLOCK), 0, s, dT, cb);
+  EPI_LAUNCH(K_RENEW_TAIL, k_renew_tail, dim3(1, ntis), dim3(RCHUNK), 0, s, dT, pb, cpar, zero_zz);
 }
 
 void launch_initialize_sc(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int pb, int max_n) {

@@ -10,7 +10,7 @@ struct Tis;
 struct Status;
 
 enum KernelId {
-  K_FORCES, K_FORCES_LONG, K_RENEW_FLAGS, K_RENEW_SCAN, K_RENEW_APPLY, K_REMOVE, K_PAIR_DISPERSE,
+  K_FORCES, K_FORCES_LONG, K_RENEW_CELLS, K_RENEW_TAIL,
   K_INIT_SC, K_PERIODIC_FIX, K_BUCKET_INSERT, K_SWEEP,
   K_FINISH, K_ZZ_SET, K_ZZMAX, K_MAP_CLEAR, K_MAP_STAMP,
   K_EXT_STIM, K_CA_BEGIN, K_CA_VOX, K_CA_CELLS, K_ATP, K_CA_END, K_SW_RESET,
@@ -94,16 +94,11 @@ int launch_forces_rows(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, i
 void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int cap);
 // zero_zz: also clear zzmax, for a build whose insertion takes it.  max_free:
 // the most cells past membrane and dermis of any tissue.  Up to RENEW_ONE the
-// renewal is one launch, a workgroup per tissue: with 160 cells 9.6 us against
-// 12.6 and two gaps for the three launches of RENEW_FEW, with 2,000 cells 20.1
-// (the lipid laws' tanh on one CU) against 17.3.  Up to RENEW_FEW the flags
-// and the ordered walk are one launch and so are the removal and the pairs:
-// with 2,000 cells 10.4 + 3.1 us against 11.6 + 4.7 and two gaps; the walk
-// takes 2.8 us more for each 1,024 cells, and with 7,000 cells 30 against 18.
+// renewal is one launch of a workgroup per tissue (160 cells: 9.6 us against
+// 11.5 with the gap for two launches; with 2,000 cells it took 20.1 against 15,
+// the lipid laws' tanh on one CU)
 constexpr int RENEW_ONE = 768;
-constexpr int RENEW_FEW = 3072;
-void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_n, int max_free,
-                  int zero_zz);
+void launch_renew(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int cpar, int max_free, int zero_zz);
 void launch_initialize_sc(hipStream_t s, const Tis* dT, const int* tlist, int ntis, int pb, int max_n);
 void launch_periodic_fix(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n);
 // the bucket insertion and the rest of the build, for callers that run the

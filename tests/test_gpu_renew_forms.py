@@ -1,6 +1,5 @@
-"""cell_state_renew where its launch form changes (one launch, three, five: the
-counts past the membrane on both sides of each limit) and where its chunks
-end, with many divisions and removals in a step, against the oracle's loop:
+"""cell_state_renew where its launch form changes (one launch or two: the counts
+past the membrane on both sides of the limit) and where its chunks end, with many divisions and removals in a step, against the oracle's loop:
 every cell field, the removal records and the draws consumed are equal."""
 import numpy as np
 import pytest
@@ -9,8 +8,8 @@ from epi_amd import configs
 
 pytestmark = pytest.mark.gpu
 
-# (sheet side, cells past the membrane): limits 768 - 64 and 3072 - 64 of the
-# forms' cell counts, chunks of 1024 and blocks of 256
+# (sheet side, cells past the membrane): limit 768 - 64 of the one
+# launch, chunks of 1024 and blocks of 256
 SHAPES = [(16, 255), (24, 703), (24, 705), (28, 1025), (36, 2049), (44, 3007), (44, 3010), (52, 4400)]
 
 

@@ -86,8 +86,8 @@ const char* kKernelNames[K_COUNT] = {
     "k_finish", "k_zz_set", "k_zzmax", "k_map_clear", "k_map_stamp",
     "k_ext_stim", "k_ca_begin", "k_ca_vox", "k_ca_cells", "k_atp", "k_ca_end", "k_sw_reset",
     "k_rd_snapshot", "k_rd_restore", "k_rd_put_gj", "k_rd_state", "k_rd_seed",
-    "k_rd_step", "k_rd_sums", "k_rd_own", "k_mech_state", "k_mech_seed", "k_mech_bwd_begin",
-    "k_mech_bwd_pairs", "k_mech_bwd_memb", "k_ca_fused", "k_ca_corners", "k_sweep_wave", "k_wl", "k_ca_swap",
+    "k_rd_step", "k_rd_sums", "k_rd_own", "k_mech_state", "k_mech_seed", "k_mech_bwd", "k_mech_sums", "k_mech_plan",
+    "k_ca_fused", "k_ca_corners", "k_sweep_wave", "k_wl", "k_ca_swap",
     "k_out_pack", "k_renew_one"};
 
 // with ready_only, only the pairs whose kernels have finished (the rest stay
@@ -2116,8 +2116,10 @@ int mech_params(epi_ctx* c, const epi_mech_params* prm) {
   HIPCHK(c, hipMemcpyAsync(c->d_tis, c->tis.data(), sizeof(Tis) * c->T, hipMemcpyHostToDevice, c->stream));
   return EPI_OK;
 }
-int mech_step(epi_ctx* c) {
-  launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, max_memb(c), max_n(c), max_list_len(c));
+// one step, its result also into slot `slot` if that is not negative
+int mech_step(epi_ctx* c, int slot = -1) {
+  launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, max_memb(c), max_n(c), max_list_len(c),
+                slot < 0 ? MechSave{} : MechSave{c->mech.d, slot});
   c->pb ^= 1;
   return EPI_OK;
 }
@@ -2136,7 +2138,11 @@ int epi_mech_begin(epi_ctx* c) {
       MechTis& r = m.h[t];
       const size_t cap = c->th[t].cap;
       r.x0[0] = cv.take<double>(3 * cap); r.x0[1] = cv.take<double>(3 * cap);
-      r.lam[0] = cv.take<double>(3 * cap); r.lam[1] = cv.take<double>(3 * cap);
+      for (int b = 0; b < 3; b++) r.lam[b] = cv.take<double>(3 * cap);
+      r.es = c->th[t].ns + 8;   // a row and its pair's spring
+      r.ent = cv.take<int>(cap * (size_t)r.es);
+      r.code = cv.take<uint8_t>(cap * (size_t)r.es);
+      r.ent_n = cv.take<int>(cap);
       r.target = cv.take<double>(3 * cap);
       r.scal = cv.take<double>(5);
     }
@@ -2180,8 +2186,12 @@ int epi_mech_adjoint(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps, in
   if (!m.active) return fail(c, EPI_ERR_INVALID, "no mechanics window is open");
   const int K = std::min(every, n_steps);
   const int nck = (n_steps + K - 1) / K;
+  int other = 1;   // cells past the membrane
+  for (auto& h : c->th) other = std::max(other, h.n_est + 64 - h.nmemb);
+  const int memb = max_memb(c), nblk = mech_bwd_blocks(memb, other);
   size_t need = 0;
-  for (int t = 0; t < c->T; t++) need += align_up(8 * 3 * (size_t)c->th[t].cap * (K + nck), 256) + 512;
+  for (int t = 0; t < c->T; t++)
+    need += align_up(8 * (3 * (size_t)c->th[t].cap * (K + nck) + 4 * (size_t)nblk), 256) + 768;
   if (need > m.work_bytes) {
     if (m.work) (void)hipFree(m.work);
     m.work = nullptr;
@@ -2195,6 +2205,7 @@ int epi_mech_adjoint(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps, in
     const size_t cap = c->th[t].cap, n = (size_t)c->h_st[t].n;
     r.slot = cv.take<double>(3 * cap * K);
     r.ck = cv.take<double>(3 * cap * nck);
+    r.part = cv.take<double>(4 * (size_t)nblk);
     for (int a = 0; a < 3; a++)
       HIPCHK(c, hipMemcpyAsync(r.target + a * cap, targets[t] + a * n, 8 * n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemsetAsync(r.scal, 0, 5 * sizeof(double), c->stream));
@@ -2208,16 +2219,17 @@ int epi_mech_adjoint(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps, in
   std::vector<int> ck_pb(nck);
   const int last0 = (nck - 1) * K;
   for (int s = 0; s < n_steps; s++) {
-    if (s >= last0) {
-      launch_mech_state(c->stream, c->d_tis, m.d, c->T, s - last0, 0, c->pb, mn);
-    } else if (s % K == 0) {
+    if (s == last0) {
+      launch_mech_state(c->stream, c->d_tis, m.d, c->T, 0, 0, c->pb, mn);
+    } else if (s < last0 && s % K == 0) {
       ck_pb[s / K] = c->pb;
       launch_mech_state(c->stream, c->d_tis, m.d, c->T, s / K, 2, c->pb, mn);
     }
-    RCHK(mech_step(c));
+    RCHK(mech_step(c, s >= last0 && s + 1 < n_steps ? s + 1 - last0 : -1));
   }
   int q = 0;
-  launch_mech_seed(c->stream, c->d_tis, m.d, c->T, c->pb, q, mn);
+  launch_mech_seed(c->stream, c->d_tis, m.d, c->T, c->pb, q, mn, nblk);
+  launch_mech_plan(c->stream, c->d_tis, m.d, c->T, c->pb, c->cb, other);
   for (int k = nck - 1; k >= 0; k--) {
     const int s0 = k * K, s1 = std::min(n_steps, s0 + K);
     if (k < nck - 1) {
@@ -2225,16 +2237,15 @@ int epi_mech_adjoint(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps, in
       launch_mech_state(c->stream, c->d_tis, m.d, c->T, k, 3, c->pb, mn);
       // the states before steps s0 .. s1 - 1; the one after s1 - 1 is the
       // next checkpoint and is not recomputed
-      for (int s = s0; s < s1; s++) {
-        launch_mech_state(c->stream, c->d_tis, m.d, c->T, s - s0, 0, c->pb, mn);
-        if (s + 1 < s1) RCHK(mech_step(c));
-      }
+      for (int s = s0; s + 1 < s1; s++) RCHK(mech_step(c, s + 1 - s0));
     }
     for (int s = s1 - 1; s >= s0; s--) {
-      launch_mech_backward_step(c->stream, c->d_tis, m.d, c->T, s - s0, c->pb, c->cb, q, mn);
-      q ^= 1;
+      launch_mech_backward_step(c->stream, c->d_tis, m.d, c->T, s - s0, q, memb, other);
+      q = q == 2 ? 0 : q + 1;
     }
   }
+  launch_mech_sums(c->stream, m.d, c->T, nblk);
+  launch_mech_state(c->stream, c->d_tis, m.d, c->T, 0, 1, c->pb, mn);   // the window's first state
   HIPCHK(c, hipGetLastError());
   RCHK(sync_status(c));
   for (int t = 0; t < c->T; t++) {

@@ -393,7 +393,8 @@ __device__ __forceinline__ void status_out(const Tis& t, const StatusOut& out) {
 }
 
 template <int FCAP>
-__global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, int pb, int cb, StatusOut out) {
+__global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, int pb, int cb, StatusOut out,
+                                                    MechSave save) {
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;
   if (out.host && blockIdx.x == 0) status_out(t, out);
@@ -557,43 +558,50 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
     }
   }
   t.pos[1 - pb][lane][X] = acc;
+  if (save.m) save.m[blockIdx.y].slot[(3LL * save.slot + lane) * t.cap + X] = acc;
 }
 
 // cells whose rows exceed the LDS slots (cap) of k_forces, one lane per cell
-__global__ void __launch_bounds__(256) k_forces_long(const Tis* __restrict__ T, int pb, int cb, int cap) {
+__global__ void __launch_bounds__(256) k_forces_long(const Tis* __restrict__ T, int pb, int cb, int cap,
+                                                     MechSave save) {
   const Tis& t = T[blockIdx.y];
   const int n = t.st->n;
   for (int X = blockIdx.x * blockDim.x + threadIdx.x; X < n; X += gridDim.x * blockDim.x)
-    if (t.nlen[cb][X] > cap) forces_serial(t, pb, cb, X, t.st);
+    if (t.nlen[cb][X] > cap) {
+      forces_serial(t, pb, cb, X, t.st);
+      if (save.m)
+        for (int a = 0; a < 3; a++) save.m[blockIdx.y].slot[(3LL * save.slot + a) * t.cap + X] = t.pos[1 - pb][a][X];
+    }
 }
 
 int launch_forces_rows(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len,
-                       const StatusOut& out) {
+                       const StatusOut& out, const MechSave& save) {
   dim3 g((max_other + F_GROUPS - 1) / F_GROUPS, ntis);
   int cap;
   if (max_len <= 40) {
     cap = 40;
-    EPI_LAUNCH(K_FORCES, k_forces<40>, g, dim3(F_BLOCK), 0, s, dT, pb, cb, out);
+    EPI_LAUNCH(K_FORCES, k_forces<40>, g, dim3(F_BLOCK), 0, s, dT, pb, cb, out, save);
   } else if (max_len <= 48) {
     cap = 48;
-    EPI_LAUNCH(K_FORCES, k_forces<48>, g, dim3(F_BLOCK), 0, s, dT, pb, cb, out);
+    EPI_LAUNCH(K_FORCES, k_forces<48>, g, dim3(F_BLOCK), 0, s, dT, pb, cb, out, save);
   } else {
     cap = FORCES_ROW_CAP;
-    EPI_LAUNCH(K_FORCES, k_forces<FORCES_ROW_CAP>, g, dim3(F_BLOCK), 0, s, dT, pb, cb, out);
+    EPI_LAUNCH(K_FORCES, k_forces<FORCES_ROW_CAP>, g, dim3(F_BLOCK), 0, s, dT, pb, cb, out, save);
   }
   return cap;
 }
 
-void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int cap) {
+void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int cap,
+                        const MechSave& save) {
   dim3 gl((max_other + 255) / 256, ntis);
-  EPI_LAUNCH(K_FORCES_LONG, k_forces_long, gl, dim3(256), 0, s, dT, pb, cb, cap);
+  EPI_LAUNCH(K_FORCES_LONG, k_forces_long, gl, dim3(256), 0, s, dT, pb, cb, cap, save);
 }
 
 void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_memb, int max_other,
-                   int max_len) {
+                   int max_len, const MechSave& save) {
   (void)max_memb;
-  const int cap = launch_forces_rows(s, dT, ntis, pb, cb, max_other, max_len, StatusOut{});
-  if (max_len > cap) launch_forces_long(s, dT, ntis, pb, cb, max_other, cap);
+  const int cap = launch_forces_rows(s, dT, ntis, pb, cb, max_other, max_len, StatusOut{}, save);
+  if (max_len > cap) launch_forces_long(s, dT, ntis, pb, cb, max_other, cap, save);
 }
 
 // ==== frozen mechanics window: the reverse pass ==============================
@@ -603,214 +611,284 @@ void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int m
 // list, its pair, the membrane slots), evaluates the derivative of the
 // active branch of each law at the step's positions, and scatters
 // lam_c1 - lam_c2 through the pair's Jacobian with FP64 atomics.
+//
+// A group of lanes owns a cell (16 a membrane particle, whose 12 dihedrals
+// and six neighbours they take; 4 another cell, over the entries k_mech_plan
+// has packed), and for the same reason as in k_forces the laws and the two
+// dihedral forms each run as one code path: the quotients the common laws
+// share (1 / d^2, 1 / R, d) are taken once, and the operands chosen per lane.
+// A cell's own terms are summed over its lanes before one atomic; so are, for
+// a membrane particle, the terms of its six neighbours, which the dihedrals
+// meet two to three times each (39 atomics a particle instead of 144).  Sums
+// are reduced in another order than the serial reverse's, as a gradient may.
+//
+// One lane per cell before (two launches and a third for the copies): its
+// waves, fewer than two a SIMD, each walked a whole list through every law's
+// own branch.  24 tissues, 105,000 cells, a step: 134 -> 76 us (8 lanes 79, 16
+// lanes 92 with entries that have no law still in the list), 25 of it the
+// atomics, which leave the chip's L2s, and 25 the arithmetic.
+constexpr int MG = 16;   // of a membrane particle
+constexpr int MC = 4;    // of another cell
 
 namespace {
 struct LawD { double coef, ds, deps, dadh, dspr; };
 
-__device__ LawD ljmain_d(double s, double R, double eps) {
-  const double L = POW6(R) / POW3(s);
-  return LawD{4.0 * eps * L * (L - 1) / s, 4.0 * eps * (4.0 * L - 7.0 * L * L) / (s * s), 4.0 * L * (L - 1) / s, 0, 0};
+// What the reverse pass needs to know of an interaction besides the two cells'
+// positions and radii: the law and the one choice inside it that frozen data
+// make.  They hold for a whole window, so k_mech_plan stores them, with the
+// entries that have a law, once per gradient.
+enum : int { CODE_LAW = 15, CODE_1 = 16, CODE_2 = 32 };
+__device__ __forceinline__ int law_code(const Tis& t, int law, const CV& a, const CV& b) {
+  if (law == LAW_ALAIRDE) return law | (a.agek > t.prm.THRESH_SP && b.agek > t.prm.THRESH_SP ? CODE_1 : 0);
+  if (law == LAW_MU_MEMB) return law | (a.pair >= 0 && t.state[a.pair] == FIX ? CODE_1 : a.rdt > 0 ? CODE_2 : 0);
+  return law;
 }
-__device__ LawD adhesion_d(double s, double R, double K, double lj) {
+
+// coef of the law of `code` at squared distance s and radius sum R (snl: the
+// pair spring's natural length) and its derivatives with respect to s and to
+// eps_m, K_TOTAL, Kspring.  Forms as in coef_law.
+__device__ __forceinline__ LawD coef_law_d(const Tis& t, int code, double R, double snl, double s) {
+  const int law = code & CODE_LAW;
+  const double eps = t.m_eps;
   LawD r{0, 0, 0, 0, 0};
-  const double d = sqrt(s);
-  const double x = d / R - 1;
-  if (x + 1 > lj) return r;
-  const double c2 = (lj - 1.0) * (lj - 1.0);
-  const double g = x * (1 - x * x / c2);
-  r.coef = -(K / d) * g;
-  const double dg = (1 - 3 * x * x / c2) / R;
-  r.ds = (K * g / (d * d) - (K / d) * dg) / (2 * d);
+  if (law == LAW_PAIR) {
+    const double d = sqrt(s);
+    r.coef = -(t.prm.Kspring_division * (d - snl)) / d;
+    r.ds = -t.prm.Kspring_division * snl / (2 * d * d * d);
+    return r;
+  }
+  if (law == LAW_DER_DER) {
+    const double d = sqrt(s), D = d + t.prm.delta_R;
+    const double L = POW6(R) / POW6(D);
+    const double dL = -6.0 * L / D;
+    double g, dgd;
+    if (D < R) {
+      g = L * (L - 1) / (d * D);
+      dgd = (2 * L - 1) * dL / (d * D) - L * (L - 1) * (D + d) / ((d * D) * (d * D));
+    } else if (s < R * R) {
+      return r;
+    } else {
+      g = L * (L - 1) / (d * d);
+      dgd = (2 * L - 1) * dL / (d * d) - 2 * L * (L - 1) / (d * d * d);
+    }
+    return LawD{4.0 * eps * g + t.prm.para_ljp2, 4.0 * eps * dgd / (2 * d), 4.0 * g, 0, 0};
+  }
+  const bool memb = law == LAW_MEMB_MEMB;
+  const double cr = memb ? R * t.prm.P_MEMB : R;
+  if (memb && !(s < cr * cr) && !(s < R * R)) {   // stretched MEMB-MEMB
+    const double d = sqrt(s);
+    const double lam = (1.0 + t.prm.P_MEMB) * R;
+    const double m = lam - d;
+    const double L = POW6(cr) / POW6(m);
+    const double dL = 6.0 * L / m;
+    const double q = L * (L - 1.0) / (m * d);
+    const double dq = (2 * L - 1) * dL / (m * d) + L * (L - 1.0) * (d - m) / ((m * d) * (m * d));
+    return LawD{-(t.prm.DER_DER_CONST / R) * ((1.0 - t.prm.P_MEMB) / t.prm.P_MEMB) - 4 * eps * q, -4 * eps * dq / (2 * d),
+                -4 * q, 0, 0};
+  }
+  const double is = 1.0 / s;
+  if (law == LAW_OTHER || s < cr * cr) {   // ljmain
+    const double Q = POW6(cr) * (is * is * is);
+    const double c1 = 4.0 * Q * (Q - 1.0) * is;
+    return LawD{eps * c1, 4.0 * eps * (4.0 * Q - 7.0 * Q * Q) * (is * is), c1, 0, 0};
+  }
+  // K times the unit of the parameter that scales it: ka of K_TOTAL, ks of
+  // Kspring, kc of neither
+  double ka = 0, ks = 0, kc = 0;
+  if (law == LAW_ALAIRDE) {
+    ka = code & CODE_1 ? 1.0 : t.prm.K_DESMOSOME_RATIO;
+  } else if (law == LAW_FIXMU) {
+    ka = t.prm.K_DESMOSOME_RATIO;
+  } else if (law == LAW_FIX_MEMB) {
+    ks = 1.0;
+  } else if (law == LAW_MU_MEMB) {
+    if (code & CODE_1) ks = 1.0;
+    else if (code & CODE_2) kc = t.prm.Kspring_d;
+  } else {
+    kc = t.prm.DER_DER_CONST;
+  }
+  const double K = ka * t.m_kadh + ks * t.m_kspring + kc;
+  const double d = sqrt(s), id = d * is, iR = 1.0 / cr;
+  const double x = d * iR - 1.0;
+  double g = x, dg = iR;   // the anchor and the relaxed membrane
+  if (!memb && law != LAW_FIX_MEMB) {   // adhesion
+    if (x + 1 > t.prm.LJ_THRESH) return r;
+    const double c2 = (t.prm.LJ_THRESH - 1.0) * (t.prm.LJ_THRESH - 1.0);
+    const double y = x * x / c2;
+    g = x * (1 - y);
+    dg = (1 - 3 * y) * iR;
+  }
+  r.coef = -K * id * g;
+  r.ds = 0.5 * K * id * (g * is - id * dg);
+  r.dadh = -ka * id * g;
+  r.dspr = -ks * id * g;
   return r;
 }
 
-// coef of `law` (c1 = a, c2 = b) and its derivatives with respect to the
-// squared distance and to eps_m, K_TOTAL, Kspring
-__device__ LawD coef_law_d(const Tis& t, int law, const CV& a, const CV& b) {
-  const double s = dist_sq(t, a.p, b.p);
-  const double R = a.r + b.r;
-  const double eps = t.m_eps;
-  LawD r{0, 0, 0, 0, 0};
-  switch (law) {
-    case LAW_OTHER:
-      return ljmain_d(s, R, eps);
-    case LAW_DER_DER: {
-      const double d = sqrt(s), D = d + t.prm.delta_R;
-      const double L = POW6(R) / POW6(D);
-      const double dL = -6.0 * L / D;
-      double g, dgd;
-      if (D < R) {
-        g = L * (L - 1) / (d * D);
-        dgd = (2 * L - 1) * dL / (d * D) - L * (L - 1) * (D + d) / ((d * D) * (d * D));
-      } else if (s < R * R) {
-        return r;
-      } else {
-        g = L * (L - 1) / (d * d);
-        dgd = (2 * L - 1) * dL / (d * d) - 2 * L * (L - 1) / (d * d * d);
-      }
-      return LawD{4.0 * eps * g + t.prm.para_ljp2, 4.0 * eps * dgd / (2 * d), 4.0 * g, 0, 0};
-    }
-    case LAW_ALAIRDE:
-      if (s < R * R) return ljmain_d(s, R, eps);
-      {
-        const bool strong = a.agek > t.prm.THRESH_SP && b.agek > t.prm.THRESH_SP;
-        r = adhesion_d(s, R, strong ? t.m_kadh : t.m_kadh * t.prm.K_DESMOSOME_RATIO, t.prm.LJ_THRESH);
-        r.dadh = r.coef / t.m_kadh;
-        return r;
-      }
-    case LAW_FIXMU:
-      if (s < R * R) return ljmain_d(s, R, eps);
-      r = adhesion_d(s, R, t.m_kadh * t.prm.K_DESMOSOME_RATIO, t.prm.LJ_THRESH);
-      r.dadh = r.coef / t.m_kadh;
-      return r;
-    case LAW_MU_MEMB: {
-      if (s < R * R) return ljmain_d(s, R, eps);
-      const bool fixpair = a.pair >= 0 && t.state[a.pair] == FIX;
-      const double spring = fixpair ? t.m_kspring : (a.rdt > 0 ? t.prm.Kspring_d : 0.0);
-      r = adhesion_d(s, R, spring, t.prm.LJ_THRESH);
-      if (fixpair) r.dspr = r.coef / t.m_kspring;
-      return r;
-    }
-    case LAW_FIX_MEMB:
-      if (s < R * R) return ljmain_d(s, R, eps);
-      {
-        const double d = sqrt(s);
-        return LawD{-(t.m_kspring / d) * (d / R - 1.0), -t.m_kspring / (2 * d * d * d), 0, 0,
-                    -(1.0 / d) * (d / R - 1.0)};
-      }
-    case LAW_MEMB_MEMB: {
-      const double cr = R * t.prm.P_MEMB, cr2 = cr * cr;
-      if (s < cr2) {
-        const double L = POW3(cr2) / POW3(s);
-        return LawD{4.0 * eps * L * (L - 1) / s, 4.0 * eps * (4.0 * L - 7.0 * L * L) / (s * s),
-                    4.0 * L * (L - 1) / s, 0, 0};
-      } else if (s < R * R) {
-        const double d = sqrt(s);
-        return LawD{-(t.prm.DER_DER_CONST / d) * (d / cr - 1.0), -t.prm.DER_DER_CONST / (2 * d * d * d), 0, 0, 0};
-      } else {
-        const double d = sqrt(s);
-        const double lam = (1.0 + t.prm.P_MEMB) * R;
-        const double m = lam - d;
-        const double L = POW6(cr) / POW6(m);
-        const double dL = 6.0 * L / m;
-        const double q = L * (L - 1.0) / (m * d);
-        const double dq = (2 * L - 1) * dL / (m * d) + L * (L - 1.0) * (d - m) / ((m * d) * (m * d));
-        return LawD{-(t.prm.DER_DER_CONST / R) * ((1.0 - t.prm.P_MEMB) / t.prm.P_MEMB) - 4 * eps * q, -4 * eps * dq / (2 * d), -4 * q,
-                    0, 0};
-      }
-    }
-    case LAW_PAIR: {
-      const double d = sqrt(s);
-      return LawD{-(t.prm.Kspring_division * (d - a.snl)) / d, -t.prm.Kspring_division * a.snl / (2 * d * d * d), 0, 0, 0};
-    }
-    default:
-      return r;
+struct ParAcc { double eps, adh, spr, bend; };
+__device__ __forceinline__ P3 ld3(const double* v, long long cap, int c) { return P3{v[c], v[cap + c], v[2 * cap + c]}; }
+__device__ __forceinline__ void atomic_add3(double* v, long long cap, int c, P3 g) {
+  atomicAdd(&v[c], g.x);
+  atomicAdd(&v[cap + c], g.y);
+  atomicAdd(&v[2 * cap + c], g.z);
+}
+template <int G>
+__device__ __forceinline__ P3 p3_group_sum(P3 v) {
+#pragma unroll
+  for (int o = 1; o < G; o <<= 1) {
+    v.x += __shfl_xor(v.x, o, G);
+    v.y += __shfl_xor(v.y, o, G);
+    v.z += __shfl_xor(v.z, o, G);
   }
+  return v;
+}
+__device__ __forceinline__ P3 p3_shfl(P3 v, int src) {
+  return P3{__shfl(v.x, src, MG), __shfl(v.y, src, MG), __shfl(v.z, src, MG)};
 }
 
-__device__ __forceinline__ void atomic_add3(double* lam, long long cap, int c, P3 g) {
-  atomicAdd(&lam[c], g.x);
-  atomicAdd(&lam[cap + c], g.y);
-  atomicAdd(&lam[2 * cap + c], g.z);
-}
-__device__ __forceinline__ P3 ld3(const double* lam, long long cap, int c) {
-  return P3{lam[c], lam[cap + c], lam[2 * cap + c]};
-}
-
-struct ParAcc { double eps, adh, spr; };
-
-// scatters the pair's term to ib and returns the one for ia (the caller's
-// cell, whose lanes reduce their terms before one atomic)
-__device__ __forceinline__ P3 pair_bwd(const Tis& t, int law, const CV& a, int ia, const CV& b, int ib,
-                                       const double* lam, double* nl, long long cap, ParAcc& pa) {
-  const LawD ld = coef_law_d(t, law, a, b);
-  const P3 r{p_diff_x(t, a.p.x, b.p.x), p_diff_y(t, a.p.y, b.p.y), a.p.z - b.p.z};
-  const P3 la = ld3(lam, cap, ia), lb = ld3(lam, cap, ib);
-  const P3 av{la.x - lb.x, la.y - lb.y, la.z - lb.z};
-  const double ar = v_dot(av, r);
+// the adjoint term of a pair for its first cell; the second's is its negative
+__device__ __forceinline__ P3 pair_bwd(const Tis& t, int code, P3 a, P3 b, double R, double snl, P3 la, P3 lb,
+                                       ParAcc& pa) {
+  const P3 r = vpsub(t, a, b);
+  const LawD ld = coef_law_d(t, code, R, snl, v_dot(r, r));
+  const P3 av = v_sub(la, lb);
+  const double ar = v_dot(av, r), DT = t.prm.DT_Cell;
   const double k2 = 2 * ld.ds * ar;
-  const P3 g{t.prm.DT_Cell * (ld.coef * av.x + k2 * r.x), t.prm.DT_Cell * (ld.coef * av.y + k2 * r.y),
-             t.prm.DT_Cell * (ld.coef * av.z + k2 * r.z)};
-  atomic_add3(nl, cap, ib, P3{-g.x, -g.y, -g.z});
-  pa.eps += t.prm.DT_Cell * ld.deps * ar;
-  pa.adh += t.prm.DT_Cell * ld.dadh * ar;
-  pa.spr += t.prm.DT_Cell * ld.dspr * ar;
-  return g;
+  pa.eps += DT * ld.deps * ar;
+  pa.adh += DT * ld.dadh * ar;
+  pa.spr += DT * ld.dspr * ar;
+  return P3{DT * (ld.coef * av.x + k2 * r.x), DT * (ld.coef * av.y + k2 * r.y), DT * (ld.coef * av.z + k2 * r.z)};
 }
 
-// adjoint of n = N / |N|
-__device__ __forceinline__ P3 unit_bar(P3 N, P3 nb) {
-  const double nn = v_norm(N);
-  const P3 n = v_div(N, nn);
-  return v_div(v_sub(nb, v_scale(v_dot(nb, n), n)), nn);
+// the wall's term for z (:287-294)
+__device__ __forceinline__ double wall_bwd(const Tis& t, double z, double radius, double lz, ParAcc& pa) {
+  const double L = POW6(radius) / POW6(z), DT = t.prm.DT_Cell;
+  pa.eps += lz * DT * 2.0 * L * (L - 1.0) / z;
+  return lz * DT * 2.0 * t.m_eps * (7.0 * L - 13.0 * L * L) / (z * z);
 }
+
 __device__ __forceinline__ double bend_factor_d(double c) {
   if (c >= 0) return -1.0;
   return -2.0 / ((1.0 + c) * (1.0 + c) * (1.0 + c));
 }
-// y = scale f(d) (v x (n2 - d n1)), d = n1.n2
-__device__ __forceinline__ void bend_pair_bar(P3 n1, P3 n2, P3 v, double scale, P3 ob, P3& vb, P3& n1b, P3& n2b,
-                                              double& db) {
+// v with its part along the unit vector n taken out, over |N|
+__device__ __forceinline__ P3 unit_bar(P3 n, double inv, P3 nb) { return v_scale(inv, v_sub(nb, v_scale(v_dot(nb, n), n))); }
+
+// reverse of tri_bend(second; r, a, b, c) for the adjoint ob = kb lm of its
+// value: bar[0..3] are the adjoints of r, a, b, c; lm . value is returned.
+// With y = f(d) (A2 x rho1 + [2] ab x rho2), d = n1.n2, rho1 = n2 - d n1,
+// rho2 = n1 - d n2 (the normals' own norms, 1, carry no derivative).
+__device__ __forceinline__ double tri_bend_bar(const Tis& t, bool second, P3 rv, P3 av, P3 bv, P3 cv, P3 lm, double kb,
+                                               P3* bar) {
+  const P3 ab = vpsub(t, av, bv), rb = vpsub(t, rv, bv);
+  const P3 rc = vpsub(t, rv, cv);
+  const P3 bc = vpsub(t, p3_sel(second, bv, cv), p3_sel(second, cv, bv));   // c - b of form 1
+  const P3 A1 = p3_sel(second, rc, rb), A2 = p3_sel(second, bc, ab);
+  const P3 B1 = p3_sel(second, rb, ab), B2 = p3_sel(second, ab, bc);
+  const P3 N1 = v_cross(A1, A2), N2 = v_cross(B1, B2);
+  const double inv1 = 1.0 / v_norm(N1), inv2 = 1.0 / v_norm(N2);
+  const P3 n1 = v_scale(inv1, N1), n2 = v_scale(inv2, N2);
   const double d = v_dot(n1, n2);
-  const P3 rho = v_sub(n2, v_scale(d, n1));
-  const P3 oy = v_scale(scale * bend_factor(d), ob);
-  db += scale * bend_factor_d(d) * v_dot(ob, v_cross(v, rho));
-  vb = v_add(vb, v_cross(rho, oy));
-  const P3 rb = v_cross(oy, v);
-  n2b = v_add(n2b, rb);
-  db += -v_dot(rb, n1);
-  n1b = v_add(n1b, v_scale(-d, rb));
-}
-// reverse of tri_bend_1(r, a, b, c); bar[0..3] get the adjoints of r, a, b, c
-__device__ void tri_bend_1_bar(const Tis& t, P3 rv, P3 avp, P3 bv, P3 cv, P3 ob, P3* bar) {
-  const P3 u = vpsub(t, rv, bv), v = vpsub(t, avp, bv), w = vpsub(t, cv, bv);
-  P3 N1 = v_cross(u, v), N2 = v_cross(v, w);
-  P3 t1 = N1, t2 = N2;
-  const P3 n1 = v_normalize(t1), n2 = v_normalize(t2);
-  const double div = v_norm(t1);
-  P3 vb{0, 0, 0}, n1b{0, 0, 0}, n2b{0, 0, 0};
-  double db = 0;
-  bend_pair_bar(n1, n2, v, 1.0 / div, ob, vb, n1b, n2b, db);
+  const P3 rho1 = v_sub(n2, v_scale(d, n1)), rho2 = v_sub(n1, v_scale(d, n2));
+  const double f = bend_factor(d);
+  const P3 oy = v_scale(f * kb, lm);
+  P3 V = v_cross(A2, rho1), ab_b{0, 0, 0}, n1b{0, 0, 0}, n2b = v_cross(oy, A2);
+  P3 A2b = v_cross(rho1, oy);
+  double db = -v_dot(n2b, n1);
+  n1b = v_scale(-d, n2b);
+  if (second) {
+    V = v_add(V, v_cross(ab, rho2));
+    ab_b = v_cross(rho2, oy);
+    const P3 q = v_cross(oy, ab);
+    n1b = v_add(n1b, q);
+    db -= v_dot(q, n2);
+    n2b = v_sub(n2b, v_scale(d, q));
+  }
+  const double val = v_dot(lm, V);
+  db += bend_factor_d(d) * kb * val;
   n1b = v_add(n1b, v_scale(db, n2));
   n2b = v_add(n2b, v_scale(db, n1));
-  const P3 N1b = unit_bar(N1, n1b), N2b = unit_bar(N2, n2b);
-  const P3 ub = v_cross(v, N1b);
-  vb = v_add(vb, v_add(v_cross(N1b, u), v_cross(w, N2b)));
-  const P3 wb = v_cross(N2b, v);
-  bar[0] = v_add(bar[0], ub);
-  bar[1] = v_add(bar[1], vb);
-  bar[3] = v_add(bar[3], wb);
-  bar[2] = v_sub(bar[2], v_add(ub, v_add(vb, wb)));
+  const P3 N1b = unit_bar(n1, inv1, n1b), N2b = unit_bar(n2, inv2, n2b);
+  const P3 A1b = v_cross(A2, N1b);
+  A2b = v_add(A2b, v_cross(N1b, A1));
+  const P3 B1b = v_cross(B2, N2b), B2b = v_cross(N2b, B1);
+  // form 1: A1 = rb, A2 = B1 = ab, B2 = cb; form 2: A1 = rc, A2 = bc, B1 = rb, B2 = ab
+  const P3 rbb = p3_sel(second, B1b, A1b);
+  const P3 abb = p3_sel(second, v_add(ab_b, B2b), v_add(A2b, B1b));
+  const P3 zero{0, 0, 0};
+  const P3 rcb = p3_sel(second, A1b, zero);
+  const P3 bcb = p3_sel(second, A2b, v_scale(-1.0, B2b));   // of b - c
+  bar[0] = v_add(rbb, rcb);
+  bar[1] = abb;
+  bar[2] = v_sub(bcb, v_add(rbb, abb));
+  bar[3] = v_sub(v_scale(-1.0, rcb), bcb);
+  return f * val;
 }
-// reverse of tri_bend_2(r, a, b, c)
-__device__ void tri_bend_2_bar(const Tis& t, P3 rv, P3 avp, P3 bv, P3 cv, P3 ob, P3* bar) {
-  const P3 p = vpsub(t, rv, cv), q = vpsub(t, bv, cv);
-  const P3 u = vpsub(t, rv, bv), v = vpsub(t, avp, bv);
-  P3 N1 = v_cross(p, q), N2 = v_cross(u, v);
-  P3 t1 = N1, t2 = N2;
-  const P3 n1 = v_normalize(t1), n2 = v_normalize(t2);
-  const double div1 = v_norm(t1), div2 = v_norm(t2);
-  P3 qb{0, 0, 0}, vb{0, 0, 0}, n1b{0, 0, 0}, n2b{0, 0, 0};
-  double db = 0;
-  bend_pair_bar(n1, n2, q, 1.0 / div1, ob, qb, n1b, n2b, db);
-  bend_pair_bar(n2, n1, v, 1.0 / div2, ob, vb, n2b, n1b, db);
-  n1b = v_add(n1b, v_scale(db, n2));
-  n2b = v_add(n2b, v_scale(db, n1));
-  const P3 N1b = unit_bar(N1, n1b), N2b = unit_bar(N2, n2b);
-  const P3 pb = v_cross(q, N1b);
-  qb = v_add(qb, v_cross(N1b, p));
-  const P3 ub = v_cross(v, N2b);
-  vb = v_add(vb, v_cross(N2b, u));
-  bar[0] = v_add(bar[0], v_add(pb, ub));
-  bar[1] = v_add(bar[1], vb);
-  bar[2] = v_add(bar[2], v_sub(qb, v_add(ub, vb)));
-  bar[3] = v_sub(bar[3], v_add(pb, qb));
+
+// a membrane particle: its dihedrals (:488-499), its membrane neighbours, the wall
+__device__ __forceinline__ void bwd_membrane(const Tis& t, const double* px, const double* lam, double* nl, int X, int lane,
+                                             ParAcc& pa) {
+  const long long cap = t.cap;
+  const int i = lane < 6 ? lane : lane < 12 ? lane - 6 : 0;   // lanes from 12 on take no term
+  const int ma = t.memb6[6 * X + i];
+  const P3 xp = ld3(px, cap, X), lm = ld3(lam, cap, X);
+  const double xr = t.radius[X];
+  const int mb = __shfl(ma, i == 5 ? 0 : i + 1, MG);
+  const int m2 = __shfl(ma, i >= 4 ? i - 4 : i + 2, MG);
+  const int mc = lane < 6 ? t.memb6[6 * mb + i] : m2;
+  const P3 ap = ld3(px, cap, ma), bp = ld3(px, cap, mb), cp = ld3(px, cap, mc);
+  // the membrane pair first: its operands are done with before the dihedral
+  P3 own{0, 0, 0}, nb{0, 0, 0};
+  if (lane < 6 && t.state[ma] == MEMB && X > ma) {
+    own = pair_bwd(t, LAW_MEMB_MEMB, xp, ap, xr + t.radius[ma], 0.0, lm, ld3(lam, cap, ma), pa);
+    nb = v_scale(-1.0, own);
+  }
+  P3 bar[4];
+  const double val = tri_bend_bar(t, lane >= 6, xp, ap, bp, cp, lm, t.prm.DT_Cell * t.m_kbend, bar);
+  if (lane < 12) {
+    pa.bend += t.prm.DT_Cell * val;
+    own = v_add(own, bar[0]);
+  }
+  if (lane < 6) atomic_add3(nl, cap, mc, bar[3]);
+  // neighbour i of X (lanes 0 to 5): a of the dihedrals i, b of those before
+  // it, c of form 2's two before
+  const int i1 = i == 0 ? 5 : i - 1, i2 = i < 2 ? i + 4 : i - 2;
+  nb = v_add(v_add(nb, v_add(bar[1], p3_shfl(bar[2], i1))), v_add(p3_shfl(bar[1], 6 + i), p3_shfl(bar[2], 6 + i1)));
+  nb = v_add(nb, p3_shfl(bar[3], 6 + i2));
+  if (lane < 6) atomic_add3(nl, cap, ma, nb);
+  if (lane == 12 && xp.z < xr) own.z += wall_bwd(t, xp.z, xr, lm.z, pa);
+  own = v_add(p3_group_sum<MG>(own), lm);
+  if (lane < 3) atomicAdd(&nl[lane * cap + X], lane == 0 ? own.x : lane == 1 ? own.y : own.z);
+}
+
+// the planned interactions of another cell's handler, and a DER cell's wall
+__device__ __forceinline__ void bwd_cell(const Tis& t, const MechTis& m, const double* px, const double* lam, double* nl,
+                                         int X, int lane, ParAcc& pa) {
+  const long long cap = t.cap;
+  const int* ent = m.ent + (size_t)X * m.es;
+  const uint8_t* code = m.code + (size_t)X * m.es;
+  const int o0 = ent[lane], k0 = code[lane];   // in one round trip with the row's length (a row holds es > MC slots)
+  const int len = m.ent_n[X];
+  const P3 xp = ld3(px, cap, X), lx = ld3(lam, cap, X);
+  const double xr = t.radius[X], snl = t.spr_nat_len[X];
+  const bool der = t.state[X] == DER;
+  P3 own{0, 0, 0};
+  for (int e = lane; e < len; e += MC) {
+    const int o = e == lane ? o0 : ent[e], k = e == lane ? k0 : code[e];
+    const P3 g = pair_bwd(t, k, xp, ld3(px, cap, o), xr + t.radius[o], snl, lx, ld3(lam, cap, o), pa);
+    own = v_add(own, g);
+    atomic_add3(nl, cap, o, v_scale(-1.0, g));
+  }
+  if (lane == MC - 1 && der && xp.z < xr) own.z += wall_bwd(t, xp.z, xr, lx.z, pa);
+  own = v_add(p3_group_sum<MC>(own), lx);
+  if (lane < 3) atomicAdd(&nl[lane * cap + X], lane == 0 ? own.x : lane == 1 ? own.y : own.z);
 }
 }  // namespace
 
 // positions between the tissue's current buffer and the window's storage:
 // dir 0 save to slot, 1 restore from slot, 2 save checkpoint, 3 restore
-// checkpoint, 4 restore the snapshot (both buffers), 5 take the snapshot
+// checkpoint (and keep it as slot 0), 4 restore the snapshot (both buffers),
+// 5 take the snapshot
 __global__ void __launch_bounds__(256) k_mech_state(const Tis* __restrict__ T, const MechTis* __restrict__ M,
                                                      int slot, int dir, int pb) {
   const Tis& t = T[blockIdx.y];
@@ -823,6 +901,7 @@ __global__ void __launch_bounds__(256) k_mech_state(const Tis* __restrict__ T, c
         double* st = (dir < 2 ? m.slot : m.ck) + (long long)slot * 3 * cap + a * cap;
         if (dir == 0 || dir == 2) st[c] = t.pos[pb][a][c];
         else t.pos[pb][a][c] = st[c];
+        if (dir == 3) m.slot[a * cap + c] = st[c];
       } else if (dir == 4) {
         t.pos[pb][a][c] = m.x0[0][a * cap + c];
         t.pos[1 - pb][a][c] = m.x0[1][a * cap + c];
@@ -836,12 +915,13 @@ __global__ void __launch_bounds__(256) k_mech_state(const Tis* __restrict__ T, c
 
 // loss = mean over cells of |x - target|^2 (minimum image in x, y) and the seed
 __global__ void __launch_bounds__(256) k_mech_seed(const Tis* __restrict__ T, MechTis* __restrict__ M, int pb,
-                                                    int q) {
+                                                    int q, int nblk) {
   const Tis& t = T[blockIdx.y];
   MechTis& m = M[blockIdx.y];
   const int n = t.st->n;
   const long long cap = t.cap;
   double part = 0;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 4 * nblk; i += gridDim.x * blockDim.x) m.part[i] = 0;
   for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
     const double dx = p_diff_x(t, t.pos[pb][0][c], m.target[c]);
     const double dy = p_diff_y(t, t.pos[pb][1][c], m.target[cap + c]);
@@ -850,146 +930,117 @@ __global__ void __launch_bounds__(256) k_mech_seed(const Tis* __restrict__ T, Me
     m.lam[q][c] = 2 * dx / n;
     m.lam[q][cap + c] = 2 * dy / n;
     m.lam[q][2 * cap + c] = 2 * dz / n;
+    for (int a = 0; a < 3; a++) m.lam[q + 1][a * cap + c] = 0;
   }
   for (int o = 32; o > 0; o >>= 1) part += __shfl_down(part, o, 64);
   if ((threadIdx.x & 63) == 0 && part != 0) atomicAdd(&m.scal[0], part / n);
 }
 
-// restore the state of slot `slot` and start the next adjoint at the identity
-__global__ void __launch_bounds__(256) k_mech_bwd_begin(const Tis* __restrict__ T, MechTis* __restrict__ M, int slot,
-                                                         int pb, int q) {
-  const Tis& t = T[blockIdx.y];
-  MechTis& m = M[blockIdx.y];
-  const int n = t.st->n;
-  const long long cap = t.cap;
-  const double* st = m.slot + (long long)slot * 3 * cap;
-  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x)
-    for (int a = 0; a < 3; a++) {
-      t.pos[pb][a][c] = st[a * cap + c];
-      m.lam[1 - q][a * cap + c] = m.lam[q][a * cap + c];
-    }
-}
-
-// The reverse kernels take one lane per cell.  A cell's own terms are summed
-// by its lane and added with one atomic; the terms of other cells are
-// scattered with atomics and the parameter sums are reduced at the end, so
-// no order is kept (a gradient need not follow the forward's).  (Lane groups
-// per cell measured slower: the laws' branches and the dihedral terms' two
-// code paths then run one after the other within a group.)
-
 // every interaction a cell's handler applies (cell_interaction.cpp:529-641)
-__global__ void __launch_bounds__(256) k_mech_bwd_pairs(const Tis* __restrict__ T, MechTis* __restrict__ M, int pb,
-                                                         int cb, int q) {
+// and its pair's spring, packed by ballots of MG lanes per cell
+__global__ void __launch_bounds__(256) k_mech_plan(const Tis* __restrict__ T, MechTis* __restrict__ M, int pb, int cb) {
   const Tis& t = T[blockIdx.y];
-  MechTis& m = M[blockIdx.y];
+  const MechTis& m = M[blockIdx.y];
   const int n = t.st->n;
-  const long long cap = t.cap;
-  const double* lam = m.lam[q];
-  double* nl = m.lam[1 - q];
-  ParAcc pa{0, 0, 0};
-  for (int X = blockIdx.x * blockDim.x + threadIdx.x; X < n; X += gridDim.x * blockDim.x) {
+  const int lane = threadIdx.x & (MG - 1), sh = threadIdx.x & 63 & ~(MG - 1);
+  for (int X = t.nmemb + blockIdx.x * (256 / MG) + threadIdx.x / MG; X < n; X += gridDim.x * (256 / MG)) {
+    const int* row = t.col[cb] + (size_t)X * t.ns;
     const CV cx = load_cv(t, pb, X);
-    P3 gx{0, 0, 0};
-    if (X < t.nmemb) {
-      for (int i = 0; i < MEMB_ADJ; i++) {
-        const int o = t.memb6[6 * X + i];
-        if (t.state[o] == MEMB && X > o)
-          gx = v_add(gx, pair_bwd(t, LAW_MEMB_MEMB, cx, X, load_cv(t, pb, o), o, lam, nl, cap, pa));
+    const int len = t.nlen[cb][X], all = len + (cx.pair >= 0 && X > cx.pair);
+    int at = 0;
+    for (int e0 = 0; e0 < all; e0 += MG) {
+      const int e = e0 + lane;
+      const int o = e < len ? row[e] : e < all ? cx.pair : X;
+      const CV co = load_cv(t, pb, o);
+      const int law = e < len ? proc_law(cx, X, co, o) : e < all ? (int)LAW_PAIR : (int)LAW_NONE;
+      const unsigned mk = (unsigned)(__ballot(law != LAW_NONE) >> sh) & ((1u << MG) - 1);
+      if (law != LAW_NONE) {
+        const int k = at + __popc(mk & ((1u << lane) - 1));
+        m.ent[(size_t)X * m.es + k] = o;
+        m.code[(size_t)X * m.es + k] = (uint8_t)law_code(t, law, cx, co);
       }
-    } else {
-      const int* row = t.col[cb] + (size_t)X * t.ns;
-      const int len = t.nlen[cb][X];
-      for (int e = 0; e < len; e++) {
-        const int o = row[e];
-        const CV co = load_cv(t, pb, o);
-        const int law = proc_law(cx, X, co, o);
-        if (law != LAW_NONE) gx = v_add(gx, pair_bwd(t, law, cx, X, co, o, lam, nl, cap, pa));
-      }
-      if (cx.pair >= 0 && X > cx.pair)
-        gx = v_add(gx, pair_bwd(t, LAW_PAIR, cx, X, load_cv(t, pb, cx.pair), cx.pair, lam, nl, cap, pa));
+      at += __popc(mk);
     }
-    atomic_add3(nl, cap, X, gx);
-  }
-  for (int o = 32; o > 0; o >>= 1) {
-    pa.eps += __shfl_down(pa.eps, o, 64);
-    pa.adh += __shfl_down(pa.adh, o, 64);
-    pa.spr += __shfl_down(pa.spr, o, 64);
-  }
-  if ((threadIdx.x & 63) == 0) {
-    if (pa.eps != 0) atomicAdd(&m.scal[1], pa.eps);
-    if (pa.adh != 0) atomicAdd(&m.scal[2], pa.adh);
-    if (pa.spr != 0) atomicAdd(&m.scal[3], pa.spr);
+    if (lane == 0) m.ent_n[X] = at;
   }
 }
 
-// the wall (membrane and DER cells, :287-294) and the bending of every
-// membrane particle (:488-499)
-__global__ void __launch_bounds__(256) k_mech_bwd_memb(const Tis* __restrict__ T, MechTis* __restrict__ M, int pb,
-                                                        int q) {
+// One reverse step from the state in slot `slot`: lam[q] (after the step) to
+// lam[q + 1] (before it), which the step before cleared, and lam[q + 2] cleared
+// for the next.  Blocks [0, mblk) take the membrane, the rest the other cells.
+// A block adds its share of the parameters' adjoints to its own words of part.
+__global__ void __launch_bounds__(256) k_mech_bwd(const Tis* __restrict__ T, MechTis* __restrict__ M, int slot, int q,
+                                                   int mblk) {
   const Tis& t = T[blockIdx.y];
   MechTis& m = M[blockIdx.y];
-  const int n = t.st->n;
   const long long cap = t.cap;
+  const double* px = m.slot + (long long)slot * 3 * cap;
   const double* lam = m.lam[q];
-  double* nl = m.lam[1 - q];
-  double peps = 0, pbend = 0;
-  for (int X = blockIdx.x * blockDim.x + threadIdx.x; X < n; X += gridDim.x * blockDim.x) {
-    const bool memb = X < t.nmemb;
-    if (!memb && t.state[X] != DER) continue;
-    const CV cx = load_cv(t, pb, X);
-    if (cx.p.z < cx.r) {
-      const double z = cx.p.z;
-      const double L = POW6(cx.r) / POW6(z);
-      atomicAdd(&nl[2 * cap + X], lam[2 * cap + X] * t.prm.DT_Cell * 2.0 * t.m_eps * (7.0 * L - 13.0 * L * L) / (z * z));
-      peps += lam[2 * cap + X] * t.prm.DT_Cell * 2.0 * L * (L - 1.0) / z;
+  double* nl = m.lam[q == 2 ? 0 : q + 1];
+  double* dead = m.lam[q == 0 ? 2 : q - 1];
+  const bool memb = (int)blockIdx.x < mblk;
+  const int nblk = memb ? mblk : gridDim.x - mblk, bid = memb ? blockIdx.x : blockIdx.x - mblk;
+  ParAcc pa{0, 0, 0, 0};
+  if (memb) {
+    const int lane = threadIdx.x & (MG - 1), step = nblk * (256 / MG);
+    for (int X = bid * (256 / MG) + threadIdx.x / MG; X < t.nmemb; X += step) {
+      if (lane < 3) dead[lane * cap + X] = 0;
+      bwd_membrane(t, px, lam, nl, X, lane, pa);
     }
-    if (!memb) continue;
-    const P3 lm = ld3(lam, cap, X);
-    const P3 ob = v_scale(t.prm.DT_Cell * t.m_kbend, lm);
-    const int* md = t.memb6 + 6 * X;
-    P3 dr{0, 0, 0};
-    for (int i = 0; i < 6; i++) {
-      const int i1 = (i + 1) % 6;
-      const int idx[4] = {X, md[i], md[i1], t.memb6[6 * md[i1] + i]};
-      const P3 pr = ld_pos(t, pb, idx[1]), pbv = ld_pos(t, pb, idx[2]), pc = ld_pos(t, pb, idx[3]);
-      dr = v_add(dr, tri_bend_1(t, cx.p, pr, pbv, pc));
-      P3 bar[4] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-      tri_bend_1_bar(t, cx.p, pr, pbv, pc, ob, bar);
-      for (int k = 0; k < 4; k++) atomic_add3(nl, cap, idx[k], bar[k]);
+  } else {
+    const int lane = threadIdx.x & (MC - 1), step = nblk * (256 / MC), n = t.st->n;
+    for (int X = t.nmemb + bid * (256 / MC) + threadIdx.x / MC; X < n; X += step) {
+      if (lane < 3) dead[lane * cap + X] = 0;
+      bwd_cell(t, m, px, lam, nl, X, lane, pa);
     }
-    for (int i = 0; i < 6; i++) {
-      const int idx[4] = {X, md[i], md[(i + 1) % 6], md[(i + 2) % 6]};
-      const P3 pa = ld_pos(t, pb, idx[1]), pbv = ld_pos(t, pb, idx[2]), pc = ld_pos(t, pb, idx[3]);
-      dr = v_add(dr, tri_bend_2(t, cx.p, pa, pbv, pc));
-      P3 bar[4] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-      tri_bend_2_bar(t, cx.p, pa, pbv, pc, ob, bar);
-      for (int k = 0; k < 4; k++) atomic_add3(nl, cap, idx[k], bar[k]);
-    }
-    pbend += t.prm.DT_Cell * v_dot(lm, dr);
   }
-  for (int o = 32; o > 0; o >>= 1) {
-    peps += __shfl_down(peps, o, 64);
-    pbend += __shfl_down(pbend, o, 64);
+  __shared__ double s_pa[4][4];
+  double v[4] = {pa.eps, pa.adh, pa.spr, pa.bend};
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_down(v[k], o, 64);
+    if ((threadIdx.x & 63) == 0) s_pa[threadIdx.x >> 6][k] = v[k];
   }
-  if ((threadIdx.x & 63) == 0) {
-    if (peps != 0) atomicAdd(&m.scal[1], peps);
-    if (pbend != 0) atomicAdd(&m.scal[4], pbend);
-  }
+  __syncthreads();
+  if (threadIdx.x < 4)
+    m.part[4 * blockIdx.x + threadIdx.x] +=
+        s_pa[0][threadIdx.x] + s_pa[1][threadIdx.x] + s_pa[2][threadIdx.x] + s_pa[3][threadIdx.x];
+}
+
+// the parameters' adjoints of a window from its blocks' sums, one block per tissue
+__global__ void __launch_bounds__(256) k_mech_sums(MechTis* __restrict__ M, int nblk) {
+  MechTis& m = M[blockIdx.y];
+  double v = 0;   // the thread's values all belong to one parameter: 256 is a multiple of 4
+  for (int i = threadIdx.x; i < 4 * nblk; i += 256) v += m.part[i];
+  __shared__ double s_v[4][4];
+  for (int o = 32; o >= 4; o >>= 1) v += __shfl_down(v, o, 64);
+  if ((threadIdx.x & 63) < 4) s_v[threadIdx.x >> 6][threadIdx.x & 3] = v;
+  __syncthreads();
+  if (threadIdx.x < 4)
+    m.scal[1 + threadIdx.x] = s_v[0][threadIdx.x] + s_v[1][threadIdx.x] + s_v[2][threadIdx.x] + s_v[3][threadIdx.x];
 }
 
 void launch_mech_state(hipStream_t s, const Tis* dT, const MechTis* dM, int ntis, int slot, int dir, int pb,
                        int max_n) {
   EPI_LAUNCH(K_MECH_STATE, k_mech_state, dim3((max_n + 255) / 256, ntis), dim3(256), 0, s, dT, dM, slot, dir, pb);
 }
-void launch_mech_seed(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int q, int max_n) {
-  EPI_LAUNCH(K_MECH_SEED, k_mech_seed, dim3((max_n + 255) / 256, ntis), dim3(256), 0, s, dT, dM, pb, q);
+void launch_mech_seed(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int q, int max_n, int nblk) {
+  EPI_LAUNCH(K_MECH_SEED, k_mech_seed, dim3((max_n + 255) / 256, ntis), dim3(256), 0, s, dT, dM, pb, q, nblk);
 }
-void launch_mech_backward_step(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int slot, int pb, int cb, int q,
-                               int max_n) {
-  const dim3 g((max_n + 255) / 256, ntis);
-  EPI_LAUNCH(K_MECH_BWD_BEGIN, k_mech_bwd_begin, g, dim3(256), 0, s, dT, dM, slot, pb, q);
-  EPI_LAUNCH(K_MECH_BWD_PAIRS, k_mech_bwd_pairs, g, dim3(256), 0, s, dT, dM, pb, cb, q);
-  EPI_LAUNCH(K_MECH_BWD_MEMB, k_mech_bwd_memb, g, dim3(256), 0, s, dT, dM, pb, q);
+namespace {
+int mech_blocks(int cells, int lanes) { return (int)(((long long)cells * lanes + 255) / 256); }
+}  // namespace
+int mech_bwd_blocks(int max_memb, int max_other) { return mech_blocks(max_memb, MG) + mech_blocks(max_other, MC); }
+void launch_mech_plan(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int cb, int max_other) {
+  EPI_LAUNCH(K_MECH_PLAN, k_mech_plan, dim3(mech_blocks(max_other, MG), ntis), dim3(256), 0, s, dT, dM, pb, cb);
+}
+void launch_mech_backward_step(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int slot, int q, int max_memb,
+                               int max_other) {
+  EPI_LAUNCH(K_MECH_BWD, k_mech_bwd, dim3(mech_bwd_blocks(max_memb, max_other), ntis), dim3(256), 0, s, dT, dM, slot, q,
+             mech_blocks(max_memb, MG));
+}
+void launch_mech_sums(hipStream_t s, MechTis* dM, int ntis, int nblk) {
+  EPI_LAUNCH(K_MECH_SUMS, k_mech_sums, dim3(1, ntis), dim3(256), 0, s, dM, nblk);
 }
 
 }  // namespace epi

@@ -8,6 +8,7 @@
 namespace epi {
 struct Tis;
 struct Status;
+struct MechTis;
 
 enum KernelId {
   K_FORCES, K_FORCES_LONG, K_RENEW_CELLS, K_RENEW_TAIL,
@@ -15,7 +16,7 @@ enum KernelId {
   K_FINISH, K_ZZ_SET, K_ZZMAX, K_MAP_CLEAR, K_MAP_STAMP,
   K_EXT_STIM, K_CA_BEGIN, K_CA_VOX, K_CA_CELLS, K_ATP, K_CA_END, K_SW_RESET,
   K_RD_SNAPSHOT, K_RD_RESTORE, K_RD_PUT_GJ, K_RD_STATE, K_RD_SEED, K_RD_STEP,
-  K_RD_SUMS, K_RD_OWN, K_MECH_STATE, K_MECH_SEED, K_MECH_BWD_BEGIN, K_MECH_BWD_PAIRS, K_MECH_BWD_MEMB,
+  K_RD_SUMS, K_RD_OWN, K_MECH_STATE, K_MECH_SEED, K_MECH_BWD, K_MECH_SUMS, K_MECH_PLAN,
   K_CA_FUSED, K_CA_CORNERS, K_SWEEP_WAVE, K_WL, K_CA_SWAP, K_OUT_PACK, K_RENEW_ONE, K_COUNT
 };
 
@@ -82,16 +83,25 @@ struct StatusOut {
   unsigned long long value = 0;
 };
 
+// where a force kernel also leaves the new positions: slot `slot` of a
+// mechanics window (m == nullptr: nowhere)
+struct MechSave {
+  MechTis* m = nullptr;
+  int slot = 0;
+};
+
 // Rows of up to FORCES_ROW_CAP entries go to the cooperative kernel (whose
 // LDS slots per cell, 40, 48 or 64, follow max_len), longer ones to a
 // one-lane-per-cell kernel, launched only when max_len exceeds the slots.
 constexpr int FORCES_ROW_CAP = 64;
-void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_memb, int max_other, int max_len);
+void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_memb, int max_other, int max_len,
+                   const MechSave& save = {});
 // the two halves of launch_forces: the cooperative kernel for rows of up to
 // the returned number of slots (chosen from max_len), and the long rows
 int launch_forces_rows(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len,
-                       const StatusOut& out);
-void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int cap);
+                       const StatusOut& out, const MechSave& save = {});
+void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int cap,
+                        const MechSave& save = {});
 // zero_zz: also clear zzmax, for a build whose insertion takes it.  max_free:
 // the most cells past membrane and dermis of any tissue.  Up to RENEW_ONE the
 // renewal is one launch of a workgroup per tissue (160 cells: 9.6 us against
@@ -194,11 +204,14 @@ void launch_rd_seed(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int cp, i
 void launch_rd_backward_substep(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int slot, int q, int qa, int max_n,
                                 long long max_box, int rg);
 // frozen mechanics window (k_mech.hip)
-struct MechTis;
 void launch_mech_state(hipStream_t s, const Tis* dT, const MechTis* dM, int ntis, int slot, int dir, int pb,
                        int max_n);
-void launch_mech_seed(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int q, int max_n);
-void launch_mech_backward_step(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int slot, int pb, int cb, int q,
-                               int max_n);
+// blocks of a reverse step, each with four words of MechTis::part
+int mech_bwd_blocks(int max_memb, int max_other);
+void launch_mech_seed(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int q, int max_n, int nblk);
+void launch_mech_backward_step(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int slot, int q, int max_memb,
+                               int max_other);
+void launch_mech_plan(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int cb, int max_other);
+void launch_mech_sums(hipStream_t s, MechTis* dM, int ntis, int nblk);
 void launch_rd_sums(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int q, long long items);
 }  // namespace epi

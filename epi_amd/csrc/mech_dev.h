@@ -14,7 +14,16 @@ struct MechTis {
   GPtr<double> x0[2];      // snapshot of both position buffers, [0] = current
   GPtr<double> slot;       // positions of the states of one segment (slot-major, 3 * cap each)
   GPtr<double> ck;         // checkpoints (3 * cap each)
-  GPtr<double> lam[2];     // position adjoints (3 * cap each)
+  // position adjoints (3 * cap each) in three rotating buffers: [q] after the
+  // step, [q + 1] before it, [q + 2] cleared for the next, q = step mod 3
+  GPtr<double> lam[3];
+  // the interactions each cell's handler applies, es slots a cell: the other
+  // cell and the law's code (k_mech_plan)
+  GPtr<int> ent;
+  GPtr<uint8_t> code;
+  GPtr<int> ent_n;
+  int es;
+  GPtr<double> part;       // four parameter sums per block of the reverse kernel
   GPtr<double> target;     // 3 * cap: x, y, z
   GPtr<double> scal;       // [0] loss, [1] dL/deps, [2] dL/dK_TOTAL, [3] dL/dKspring, [4] dL/dKBEND
 };

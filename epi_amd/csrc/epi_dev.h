@@ -145,7 +145,7 @@ struct Tis {
   // (x, y, z, radius) of every cell after the periodic fix, written by the
   // bucket insertion: the sweep and the row assembly gather a candidate's
   // position and radius with one 32-byte load instead of four
-  GPtr<double4> pk;
+  GPtr<double4> pk[2]; GPtr<int4> fa;
   // state renewal
   GPtr<double> div_dir;   // per division: its direction
   GPtr<int> rm_list;
@@ -164,6 +164,10 @@ struct Tis {
   Params prm;
 };
 
+// the record of a cell's attributes that the force laws read (Tis::fa)
+__device__ __forceinline__ int4 force_attr(int pair, int dermis, int rest_div_times, uint8_t state, bool strong) {
+  return make_int4(pair, dermis, rest_div_times, state | (strong ? 256 : 0));
+}
 __device__ __forceinline__ void set_err(Status* st, int e) { atomicCAS(&st->err, 0, e); }
 // of a force kernel: kept apart until the next renewal takes it over, so that
 // a step's status never shows an error of the step after it

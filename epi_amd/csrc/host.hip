@@ -88,7 +88,7 @@ const char* kKernelNames[K_COUNT] = {
     "k_rd_snapshot", "k_rd_restore", "k_rd_put_gj", "k_rd_state", "k_rd_seed",
     "k_rd_step", "k_rd_sums", "k_rd_own", "k_mech_state", "k_mech_seed", "k_mech_bwd", "k_mech_sums", "k_mech_plan",
     "k_ca_fused", "k_ca_corners", "k_sweep_wave", "k_wl", "k_ca_swap",
-    "k_out_pack", "k_renew_one"};
+    "k_out_pack", "k_renew_one", "k_force_pack"};
 
 // with ready_only, only the pairs whose kernels have finished (the rest stay
 // pending for a later read-back)
@@ -311,7 +311,8 @@ void carve_tissue(Carver& cv, TH& h, Tis& t) {
   t.bucket_of = cv.take<int>(cap);
   t.bucket = cv.take<int>((size_t)h.nbuckets * BUCKET_HEAD);
   t.bucket_rest = cv.take<int>((size_t)h.nbuckets * bucket_more(h.bcap));
-  t.pk = cv.take<double4>(cap);
+  for (int b = 0; b < 2; b++) t.pk[b] = cv.take<double4>(cap);
+  t.fa = cv.take<int4>(cap);
   t.div_dir = cv.take<double>(3 * cap);
   t.rm_list = cv.take<int>(cap);
   t.rd_list = cv.take<int>(cap + 256);
@@ -1102,6 +1103,7 @@ int epi_rng_mt19937_64(uint64_t seed, double* out, int64_t n) {
 
 int epi_cell_interaction(epi_ctx* c) {
   if (!c) return EPI_ERR_INVALID;
+  launch_force_pack(c->stream, c->d_tis, c->T, c->pb, max_n(c));
   launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, max_memb(c), max_n(c), max_list_len(c));
   HIPCHK(c, hipGetLastError());
   c->pos_pending = true;
@@ -1359,6 +1361,7 @@ int epi_step(epi_ctx* c, int64_t nsteps, epi_driver* drv) {
     const int mn = max_n(c);
     // cell_dynamics (proc.cpp:22-32)
     if (!forces_issued) {
+      launch_force_pack(c->stream, c->d_tis, c->T, c->pb, mn);
       launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, max_memb(c), mn, max_list_len(c));
       c->pb ^= 1;
     }
@@ -2119,7 +2122,7 @@ int mech_params(epi_ctx* c, const epi_mech_params* prm) {
 // one step, its result also into slot `slot` if that is not negative
 int mech_step(epi_ctx* c, int slot = -1) {
   launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, max_memb(c), max_n(c), max_list_len(c),
-                slot < 0 ? MechSave{} : MechSave{c->mech.d, slot});
+                MechSave{slot < 0 ? nullptr : c->mech.d, slot, true});
   c->pb ^= 1;
   return EPI_OK;
 }
@@ -2165,6 +2168,7 @@ int epi_mech_forward(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps) {
   if (!c->mech.active) return fail(c, EPI_ERR_INVALID, "no mechanics window is open");
   RCHK(mech_params(c, prm));
   launch_mech_state(c->stream, c->d_tis, c->mech.d, c->T, 0, 4, c->pb, max_n(c));
+  launch_force_pack(c->stream, c->d_tis, c->T, c->pb, max_n(c));
   for (int s = 0; s < n_steps; s++) RCHK(mech_step(c));
   HIPCHK(c, hipGetLastError());
   return sync_status(c);
@@ -2214,6 +2218,7 @@ int epi_mech_adjoint(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps, in
   RCHK(mech_params(c, prm));
   const int mn = max_n(c);
   launch_mech_state(c->stream, c->d_tis, m.d, c->T, 0, 4, c->pb, mn);
+  launch_force_pack(c->stream, c->d_tis, c->T, c->pb, mn);
   // checkpoint every K steps; the last segment saves its states straight
   // into the slots, so the reverse pass starts without a recompute
   std::vector<int> ck_pb(nck);
@@ -2235,6 +2240,7 @@ int epi_mech_adjoint(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps, in
     if (k < nck - 1) {
       c->pb = ck_pb[k];
       launch_mech_state(c->stream, c->d_tis, m.d, c->T, k, 3, c->pb, mn);
+      launch_force_pack(c->stream, c->d_tis, c->T, c->pb, mn);
       // the states before steps s0 .. s1 - 1; the one after s1 - 1 is the
       // next checkpoint and is not recomputed
       for (int s = s0; s + 1 < s1; s++) RCHK(mech_step(c, s + 1 - s0));

@@ -63,7 +63,7 @@ __device__ __forceinline__ void insert_cells(const Tis& t, int pb, int fix, bool
     const long aix = (long)((0.5 * t.LX - p_diff_x(t, 0.5 * t.LX, x)) / AREA_GRID);
     const long aiy = (long)((0.5 * t.LY - p_diff_y(t, 0.5 * t.LY, y)) / AREA_GRID);
     const long aiz = (long)((min0(z)) / AREA_GRID);
-    t.pk[c] = make_double4(x, y, z, r);
+    t.pk[pb][c] = make_double4(x, y, z, r);
     t.bcnt[c] = 0;
     t.nlo[c] = 0;
     if (aix >= t.ANX || aiy >= t.ANY || aiz >= t.ANZ || aix < 0 || aiy < 0 || aiz < 0) {
@@ -143,8 +143,8 @@ __device__ __forceinline__ void sweep_append(const Tis& t, int c, int o) {
 // a sweep of any size, without lists: each lane counts its buckets' hits, and
 // writes them in order, each time the least cell above the last one
 template <int G>
-__device__ __forceinline__ int sweep_crowded(const Tis& t, int c, const P3& pc, double rc, const SweepAt& at, int lane,
-                                             int* row) {
+__device__ __forceinline__ int sweep_crowded(const Tis& t, const double4* pk, int c, const P3& pc, double rc,
+                                             const SweepAt& at, int lane, int* row) {
   constexpr int NB = 128 / G;
   const int q1 = min(NB * lane + NB, 125);
   auto cell = [&](int b, int m) -> int {
@@ -157,7 +157,7 @@ __device__ __forceinline__ int sweep_crowded(const Tis& t, int c, const P3& pc, 
     const int sz = min(t.bucket[(size_t)b * BUCKET_HEAD], t.bcap);
     for (int m = 0; m < sz; m++) {
       const int o = cell(b, m);
-      cnt += o < c && sweep_hit(t, pc, rc, t.pk[o]);
+      cnt += o < c && sweep_hit(t, pc, rc, pk[o]);
     }
   }
   int total;
@@ -170,7 +170,7 @@ __device__ __forceinline__ int sweep_crowded(const Tis& t, int c, const P3& pc, 
         int best = c;
         for (int m = 0; m < sz; m++) {
           const int o = cell(b, m);
-          if (o > last && o < best && sweep_hit(t, pc, rc, t.pk[o])) best = o;
+          if (o > last && o < best && sweep_hit(t, pc, rc, pk[o])) best = o;
         }
         if (best == c) break;
         if (off < t.ns) row[off] = best;
@@ -183,7 +183,7 @@ __device__ __forceinline__ int sweep_crowded(const Tis& t, int c, const P3& pc, 
 }
 
 template <int G>
-__device__ __forceinline__ void sweep_part(const Tis& t, int nb, int nblk) {
+__device__ __forceinline__ void sweep_part(const Tis& t, int pb, int nb, int nblk) {
   constexpr int NB = 128 / G;   // buckets of a lane
   Status* st = t.st;
   const int n = st->n;
@@ -203,8 +203,9 @@ __device__ __forceinline__ void sweep_part(const Tis& t, int nb, int nblk) {
     return G == 64 ? b : b >> (threadIdx.x & 32) & 0xffffffffull;
   };
   int* const col = t.col[nb];
+  const double4* const pk = t.pk[pb];
   for (int c = t.nmemb + blockIdx.x * (blockDim.x / G) + threadIdx.x / G; c < n; c += groups) {
-    const double4 pq = t.pk[c];
+    const double4 pq = pk[c];
     const P3 pc{pq.x, pq.y, pq.z};
     const double rc = pq.w;
     const long lx = (long)(pc.x / AREA_GRID);
@@ -288,7 +289,7 @@ __device__ __forceinline__ void sweep_part(const Tis& t, int nb, int nblk) {
           const int i = i0 + k * G + lane;
           o[k] = i < nc ? cand[i] : c;
           q[k] = i < nc ? cq[i] : 0;
-          po[k] = t.pk[o[k]];
+          po[k] = pk[o[k]];
         }
 #pragma unroll
         for (int k = 0; k < 2; k++) {
@@ -302,7 +303,7 @@ __device__ __forceinline__ void sweep_part(const Tis& t, int nb, int nblk) {
     }
     int* const row = col + (size_t)c * ns;
     if (nc > SWEEP_C || total > SWEEP_H) {
-      total = sweep_crowded<G>(t, c, pc, rc, at, lane, row);
+      total = sweep_crowded<G>(t, pk, c, pc, rc, at, lane, row);
     } else {
       wave_sync();
       for (int i = lane; i < total; i += G) {
@@ -331,7 +332,7 @@ __global__ void __launch_bounds__(256) k_sweep(const Tis* __restrict__ T, int pb
       return;
     }
   }
-  sweep_part<G>(t, nb, sweep_blocks);
+  sweep_part<G>(t, pb, nb, sweep_blocks);
 }
 
 // Row assembly, gj carry-over and dermis.  A group of KG lanes owns one
@@ -369,7 +370,7 @@ __device__ __forceinline__ void finish_part(const Tis& t, int pb, int nb, int nb
   __shared__ double s_og[K_GROUPS][KCAP];
   const int lane = threadIdx.x & (KG - 1);
   const int grp = threadIdx.x / KG;
-  const double gj_init = t.prm.gj_init;   // read before any store (a store could alias the descriptor)
+  const double gj_init = t.prm.gj_init, THRESH_SP = t.prm.THRESH_SP;   // read before any store (a store could alias the descriptor)
   int mylen = 0;
   const int stride = nblk * K_GROUPS;
   for (int c = blockIdx.x * K_GROUPS + grp; c < n; c += stride) {
@@ -382,6 +383,8 @@ __device__ __forceinline__ void finish_part(const Tis& t, int pb, int nb, int nb
     const long long my_uid = t.uid[c];
     const uint8_t s = t.state[c];
     const P3 pc = ld_pos(t, pb, c);
+    const int pair = t.pair[c], dermis = t.dermis[c], rdt = t.rest_div_times[c];
+    const bool strong = t.agek[c] > THRESH_SP;
     const int na = memb ? 0 : na0;
     const int len = base + na + nbh;
     int* const row = t.col[nb] + (size_t)c * t.ns;
@@ -486,6 +489,7 @@ __device__ __forceinline__ void finish_part(const Tis& t, int pb, int nb, int nb
         if (d < bd) { bd = d; be = e; }   // entries of a lane ascend
       }
     }
+    int found = dermis;
     if (want_dermis) {
 #pragma unroll
       for (int o = 1; o < KG; o <<= 1) {
@@ -493,8 +497,10 @@ __device__ __forceinline__ void finish_part(const Tis& t, int pb, int nb, int nb
         const int e2 = __shfl_xor(be, o, KG);
         if (d2 < bd || (d2 == bd && e2 < be)) { bd = d2; be = e2; }
       }
-      if (lane == 0) t.dermis[c] = be == 0x7fffffff ? -1 : r[be];
+      found = be == 0x7fffffff ? -1 : r[be];
+      if (lane == 0) t.dermis[c] = found;
     }
+    if (lane == 0) t.fa[c] = force_attr(pair, found, rdt, s, strong);   // what the force laws read (k_mech.hip)
     wave_sync();
   }
   // maxlen only grows: a wave that cannot raise it skips the atomic, which

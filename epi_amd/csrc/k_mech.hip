@@ -17,23 +17,38 @@
 
 namespace epi {
 
-struct CV {           // what a force law reads of a cell
+// What a force law reads of a cell, from two records: pk[pb] (position and
+// radius, 32 bytes) and fa (pair, dermis, rest_div_times, and state with
+// whether the age passes THRESH_SP, 16 bytes).  A gather touches two cache
+// lines a lane, where the ten arrays the records are made from touched ten
+// (the address units were busy for half of k_forces).  In a step the bucket
+// insertion writes pk and k_finish fa; force_pack writes both where a force
+// kernel does not follow a build; in a window k_forces writes the next pk.
+// snl is read for a pair's spring alone (load_cv_snl).
+struct CV {
   P3 p;
-  double r, agek, snl;
+  double r, snl;
+  bool strong;   // agek > THRESH_SP
   int pair, dermis, rdt;
   uint8_t s;
 };
 
 __device__ __forceinline__ CV load_cv(const Tis& t, int pb, int c) {
+  const double4 p = t.pk[pb][c];
+  const int4 f = t.fa[c];
   CV v;
-  v.p = ld_pos(t, pb, c);
-  v.r = t.radius[c];
-  v.agek = t.agek[c];
+  v.p = P3{p.x, p.y, p.z};
+  v.r = p.w;
+  v.pair = f.x;
+  v.dermis = f.y;
+  v.rdt = f.z;
+  v.s = (uint8_t)(f.w & 255);
+  v.strong = f.w >> 8;
+  return v;
+}
+__device__ __forceinline__ CV load_cv_snl(const Tis& t, int pb, int c) {
+  CV v = load_cv(t, pb, c);
   v.snl = t.spr_nat_len[c];
-  v.pair = t.pair[c];
-  v.dermis = t.dermis[c];
-  v.rdt = t.rest_div_times[c];
-  v.s = t.state[c];
   return v;
 }
 
@@ -109,7 +124,7 @@ __device__ __forceinline__ double coef_law(const Tis& t, int law, const CV& a, c
   const bool L = law == LAW_OTHER || (memb ? distSq < cr_dist_sq : distSq < rad_sum * rad_sum);
   double K = t.m_kadh * t.prm.K_DESMOSOME_RATIO;   // LAW_FIXMU, LAW_ALAIRDE
   if (law == LAW_ALAIRDE) {
-    if (a.agek > t.prm.THRESH_SP && b.agek > t.prm.THRESH_SP) K = t.m_kadh;
+    if (a.strong && b.strong) K = t.m_kadh;
   } else if (law == LAW_MU_MEMB) {
     // spring_force_to_memb, set at the top of _MUSUME_interaction (:613-620)
     K = 0;
@@ -283,14 +298,14 @@ __device__ void forces_serial(const Tis& t, int pb, int cb, int X, Status* st) {
       }
     }
     if (cx.pair >= 0 && X > cx.pair) {
-      const P3 d = delta(t, LAW_PAIR, cx, load_cv(t, pb, cx.pair), st);
+      const P3 d = delta(t, LAW_PAIR, load_cv_snl(t, pb, X), load_cv(t, pb, cx.pair), st);
       acc.x += d.x; acc.y += d.y; acc.z += d.z;
     }
     int P = cx.pair > X ? cx.pair : -1;
     for (int i = nlo; i < len; i++) {
       const int p = row[i];
       if (P >= 0 && P < p) {
-        const P3 d = delta(t, LAW_PAIR, load_cv(t, pb, P), cx, st);
+        const P3 d = delta(t, LAW_PAIR, load_cv_snl(t, pb, P), cx, st);
         acc.x -= d.x; acc.y -= d.y; acc.z -= d.z;
         P = -1;
       }
@@ -301,13 +316,13 @@ __device__ void forces_serial(const Tis& t, int pb, int cb, int X, Status* st) {
         acc.x -= d.x; acc.y -= d.y; acc.z -= d.z;
       }
       if (p == P) {
-        const P3 d = delta(t, LAW_PAIR, cp, cx, st);
+        const P3 d = delta(t, LAW_PAIR, load_cv_snl(t, pb, p), cx, st);
         acc.x -= d.x; acc.y -= d.y; acc.z -= d.z;
         P = -1;
       }
     }
     if (P >= 0) {
-      const P3 d = delta(t, LAW_PAIR, load_cv(t, pb, P), cx, st);
+      const P3 d = delta(t, LAW_PAIR, load_cv_snl(t, pb, P), cx, st);
       acc.x -= d.x; acc.y -= d.y; acc.z -= d.z;
     }
   }
@@ -341,9 +356,10 @@ __device__ void forces_serial(const Tis& t, int pb, int cb, int X, Status* st) {
 // other) and, on a small tissue, the chain of round trips and the ordered
 // sum.  One copy of the laws with shared divisions, one path for both
 // dihedral forms and one coordinate per summing lane, against every law and
-// form on its own and a leader summing all three: 100 steps of one tissue of
-// 3,900 cells 1490 -> 1073 us, of 24 tissues (with their reverse pass) 30.3 ->
-// 26.9 ms.
+// form on its own and a leader summing all three; then the packed records and
+// the dihedrals' indices asked for early: 100 steps of one tissue of 3,900
+// cells 1490 -> 1083 -> 1043 us, a launch for 24 tissues of 105,000 cells
+// 82.6 -> 63.5 -> 60.1 us (without the laws 50, without the sums 57).
 //
 // FCAP, the LDS slots per cell, is chosen per launch from the longest list
 // built so far: 40 keeps a 128-lane block's LDS small enough for 4 waves per
@@ -420,6 +436,16 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
   if (blockIdx.x == 0 && threadIdx.x == 0 && (long long)gridDim.x * F_GROUPS < n) set_force_err(st, ERR_INVALID);
   if (X >= n) return;
   if (len > FCAP) return;   // k_forces_long
+  // a membrane particle's dihedral of this lane: its cells' indices are asked
+  // for before the laws, so that only their positions are left to wait for
+  int ma = 0, mb = 0, mc = 0;
+  if (memb && lane < 12) {
+    const int* md = t.memb6 + 6 * X;
+    const int i = lane < 6 ? lane : lane - 6;
+    ma = md[i];
+    mb = md[i == 5 ? 0 : i + 1];
+    mc = lane < 6 ? t.memb6[6 * mb + i] : md[i >= 4 ? i - 4 : i + 2];
+  }
   bool hi = false;          // this lane's membrane slot is subtracted (its handler has the higher index)
 #pragma unroll 1
   for (int e = lane; e < len; e += FG) {
@@ -452,7 +478,7 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
       CV a, b;
       a.p = p3_sel(own, cx.p, cq.p); b.p = p3_sel(own, cq.p, cx.p);
       a.r = cx.r; b.r = cq.r;            // the sum of the two radii alone is read
-      a.agek = cx.agek; b.agek = cq.agek;   // and whether both ages pass a threshold
+      a.strong = cx.strong; b.strong = cq.strong;
       a.pair = own ? cx.pair : cq.pair;
       a.rdt = own ? cx.rdt : cq.rdt;
       const P3 d = delta_law<false>(t, law, a, b, st);
@@ -464,11 +490,8 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
     }
   }
   if (memb && lane < 12) {
-    const int* md = t.memb6 + 6 * X;
-    const int i = lane < 6 ? lane : lane - 6;
-    const int ma = md[i], mb = md[(i + 1) % 6];
-    const int mc = lane < 6 ? t.memb6[6 * mb + i] : md[(i + 2) % 6];
-    s_bend[grp][lane] = tri_bend(t, lane >= 6, cx.p, ld_pos(t, pb, ma), ld_pos(t, pb, mb), ld_pos(t, pb, mc));
+    const double4 ap = t.pk[pb][ma], bp = t.pk[pb][mb], cp = t.pk[pb][mc];
+    s_bend[grp][lane] = tri_bend(t, lane >= 6, cx.p, P3{ap.x, ap.y, ap.z}, P3{bp.x, bp.y, bp.z}, P3{cp.x, cp.y, cp.z});
   }
   wave_sync();
   int nhi = 0;
@@ -496,7 +519,10 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
     }
   }
   wave_sync();
-  if (lane >= 3) return;
+  if (lane >= 3) {
+    if (lane == 3 && save.chain) t.pk[1 - pb][X].w = cx.r;
+    return;
+  }
   const double* own = reinterpret_cast<const double*>(s_own[grp].v) + lane;
   const double* oth = reinterpret_cast<const double*>(s_oth[grp].v) + lane;
   double acc = p3_at(cx.p, lane);
@@ -534,9 +560,9 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
     } else {
       // the pair's spring: added after the own list when this cell has the
       // higher index, else subtracted after the partner's list
-      const CV cp = load_cv(t, pb, cx.pair);
-      const bool up = X > cx.pair;
-      const double dp = p3_at(up ? delta(t, LAW_PAIR, cx, cp, st) : delta(t, LAW_PAIR, cp, cx, st), lane);
+      const bool up = X > cx.pair;   // the handler of the pair is the higher index
+      const CV ca = load_cv_snl(t, pb, up ? X : cx.pair), cp = load_cv(t, pb, up ? cx.pair : X);
+      const double dp = p3_at(delta(t, LAW_PAIR, ca, cp, st), lane);
       if (up) {
         acc = sum_slots<false>(acc + dp, oth, nA, len);
       } else {
@@ -558,6 +584,7 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
     }
   }
   t.pos[1 - pb][lane][X] = acc;
+  if (save.chain) reinterpret_cast<double*>(static_cast<double4*>(t.pk[1 - pb]))[4LL * X + lane] = acc;
   if (save.m) save.m[blockIdx.y].slot[(3LL * save.slot + lane) * t.cap + X] = acc;
 }
 
@@ -569,6 +596,7 @@ __global__ void __launch_bounds__(256) k_forces_long(const Tis* __restrict__ T, 
   for (int X = blockIdx.x * blockDim.x + threadIdx.x; X < n; X += gridDim.x * blockDim.x)
     if (t.nlen[cb][X] > cap) {
       forces_serial(t, pb, cb, X, t.st);
+      if (save.chain) t.pk[1 - pb][X] = make_double4(t.pos[1 - pb][0][X], t.pos[1 - pb][1][X], t.pos[1 - pb][2][X], t.radius[X]);
       if (save.m)
         for (int a = 0; a < 3; a++) save.m[blockIdx.y].slot[(3LL * save.slot + a) * t.cap + X] = t.pos[1 - pb][a][X];
     }
@@ -595,6 +623,23 @@ void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, 
                         const MechSave& save) {
   dim3 gl((max_other + 255) / 256, ntis);
   EPI_LAUNCH(K_FORCES_LONG, k_forces_long, gl, dim3(256), 0, s, dT, pb, cb, cap, save);
+}
+
+// the records load_cv reads, from the cells' arrays
+__global__ void __launch_bounds__(256) k_force_pack(const Tis* __restrict__ T, int pb) {
+  const Tis& t = T[blockIdx.y];
+  const double THRESH_SP = t.prm.THRESH_SP;
+  const int n = t.st->n;
+  for (int c = blockIdx.x * blockDim.x + threadIdx.x; c < n; c += gridDim.x * blockDim.x) {
+    const P3 p = P3{t.pos[pb][0][c], t.pos[pb][1][c], t.pos[pb][2][c]};
+    const int4 f = force_attr(t.pair[c], t.dermis[c], t.rest_div_times[c], t.state[c], t.agek[c] > THRESH_SP);
+    t.pk[pb][c] = make_double4(p.x, p.y, p.z, t.radius[c]);
+    t.fa[c] = f;
+  }
+}
+
+void launch_force_pack(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n) {
+  EPI_LAUNCH(K_FORCE_PACK, k_force_pack, dim3((max_n + 255) / 256, ntis), dim3(256), 0, s, dT, pb);
 }
 
 void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_memb, int max_other,
@@ -639,7 +684,7 @@ struct LawD { double coef, ds, deps, dadh, dspr; };
 // entries that have a law, once per gradient.
 enum : int { CODE_LAW = 15, CODE_1 = 16, CODE_2 = 32 };
 __device__ __forceinline__ int law_code(const Tis& t, int law, const CV& a, const CV& b) {
-  if (law == LAW_ALAIRDE) return law | (a.agek > t.prm.THRESH_SP && b.agek > t.prm.THRESH_SP ? CODE_1 : 0);
+  if (law == LAW_ALAIRDE) return law | (a.strong && b.strong ? CODE_1 : 0);
   if (law == LAW_MU_MEMB) return law | (a.pair >= 0 && t.state[a.pair] == FIX ? CODE_1 : a.rdt > 0 ? CODE_2 : 0);
   return law;
 }

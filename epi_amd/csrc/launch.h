@@ -17,7 +17,7 @@ enum KernelId {
   K_EXT_STIM, K_CA_BEGIN, K_CA_VOX, K_CA_CELLS, K_ATP, K_CA_END, K_SW_RESET,
   K_RD_SNAPSHOT, K_RD_RESTORE, K_RD_PUT_GJ, K_RD_STATE, K_RD_SEED, K_RD_STEP,
   K_RD_SUMS, K_RD_OWN, K_MECH_STATE, K_MECH_SEED, K_MECH_BWD, K_MECH_SUMS, K_MECH_PLAN,
-  K_CA_FUSED, K_CA_CORNERS, K_SWEEP_WAVE, K_WL, K_CA_SWAP, K_OUT_PACK, K_RENEW_ONE, K_COUNT
+  K_CA_FUSED, K_CA_CORNERS, K_SWEEP_WAVE, K_WL, K_CA_SWAP, K_OUT_PACK, K_RENEW_ONE, K_FORCE_PACK, K_COUNT
 };
 
 // ints of a context's work-list buffer: the offsets and per-tissue iz_bound
@@ -88,6 +88,7 @@ struct StatusOut {
 struct MechSave {
   MechTis* m = nullptr;
   int slot = 0;
+  bool chain = false;   // and the next force kernel's records (no build between the two)
 };
 
 // Rows of up to FORCES_ROW_CAP entries go to the cooperative kernel (whose
@@ -100,6 +101,8 @@ void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int m
 // the returned number of slots (chosen from max_len), and the long rows
 int launch_forces_rows(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len,
                        const StatusOut& out, const MechSave& save = {});
+// the records the force kernels read, where no build has just written them
+void launch_force_pack(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n);
 void launch_forces_long(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int cap,
                         const MechSave& save = {});
 // zero_zz: also clear zzmax, for a build whose insertion takes it.  max_free:

@@ -623,11 +623,14 @@ int graph_run(epi_ctx* c, const std::vector<long long>& key, F issue) {
 
 // the launch shapes of a solve or window over tissues ids[0..ntis) (nullptr =
 // all), ca_fuse resolved to 0 or 1.  ca_fuse 2 fuses those of at most
-// FUSE_AUTO_CELLS cells (a gated solve of a few tissues is latency-bound,
-// where one launch per sub-step wins; a solve of a whole large batch is
-// throughput-bound, where two leaner ones do)
+// FUSE_AUTO_CELLS cells: with few the time is launches and round trips, where
+// one launch per sub-step wins; a solve of a whole large batch is bound by the
+// address units and the arithmetic, where two leaner ones with taller ATP
+// tiles do.  50 steps of uneven tissues with one solve, fused and not: 138,000
+// cells 47.4 and 49.6 ms, 178,000 60.7 and 61.6, 223,000 74.9 and 74.3,
+// 292,000 99.9 and 94.8.
 Tuning ca_shapes(const epi_ctx* c, const int* ids, int ntis) {
-  constexpr long long FUSE_AUTO_CELLS = 131072;
+  constexpr long long FUSE_AUTO_CELLS = 196608;
   long long cells = 0;
   for (int i = 0; i < ntis; i++) cells += c->th[ids ? ids[i] : i].n_est;
   Tuning tu = c->tu;
@@ -642,8 +645,12 @@ Tuning ca_shapes(const epi_ctx* c, const int* ids, int ntis) {
   // planes through one thread, which the cells beside them wait for (14.1
   // against 10.1 us per sub-step of the large tissue).  They address a plane
   // with 32-bit byte offsets; a tissue of larger planes takes two launches.
+  // One tissue takes one plane a tile (most blocks, shortest chain: two planes
+  // 1.5 % slower at 36,000 cells); several, whose tiles are found in a list,
+  // two (30,000 cells in 4 tissues 18.0 -> 16.8 ms for 50 steps and a solve,
+  // 138,000 in 16 52.7 -> 47.4).
   if (any_wide_plane(c, ids, ntis)) tu.ca_fuse = 0;
-  if (tu.ca_fuse && tu.a_zb > 2) tu.a_zb = 1;
+  if (tu.ca_fuse && tu.a_zb > 2) tu.a_zb = ntis == 1 ? 1 : 2;
   return tu;
 }
 

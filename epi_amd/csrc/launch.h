@@ -29,13 +29,13 @@ struct Tuning {
   int b_zb = 4, b_rows = 4;   // k_ext_stim: z planes per tile, 64-lane rows per block (points per tile)
   int a_zb = 4, a_rows = 4;   // k_atp: the same (a fused solve's tiles are 128 points)
   int ca_group = 8;           // Ca cell kernels: lanes per cell (8, or 16; 4 takes 8)
-  int xcd = 0;                // k_ca_cells, k_atp: XCD-contiguous workgroup order
+  int xcd = 1;                // Ca cells and ATP: XCD-contiguous workgroup order (launches of many workgroups)
   int b_xcd = 0;              // k_ext_stim: its tile list in one contiguous run per XCD
   int sweep_wave = 0;         // k_sweep: 1, one wave per cell (64 lanes instead of 32)
   int side_fork = 0;          // 1: the side stream forks after the whole build
   int rd_group = 8;           // k_rd_step: lanes per cell
-  int ca_fuse = 1;            // Ca solves: ATP of a sub-step and cells of the next in one launch
-                              // (0 never, 1 always, 2 for solves of at most 131072 cells)
+  int ca_fuse = 2;            // Ca solves: ATP of a sub-step and cells of the next in one launch
+                              // (0 never, 1 always, 2 for solves of at most 196608 cells)
   int ca_group_small = 8;     // k_ca_cells lanes per cell in the solves that ca_fuse 2 fuses
   int map_lanes = 16;         // k_map_stamp: lanes per cell (1, 4 or 16, along x of the stamp box)
   int step_graph = 0;         // epi_step: 1 replays the renewal and build from a captured graph

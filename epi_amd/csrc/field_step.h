@@ -126,6 +126,30 @@ __device__ __forceinline__ double fB(const BK& k, double age, double B, bool cor
   return (cornif && age > k.THRESH_DEAD - k.DUR_ALIVE && age <= k.THRESH_DEAD + k.DUR_DEAD ? 1 : 0) - k.kb * B;
 }
 
+// exclusive prefix sum of v over a block of blockDim.x (a multiple of 64,
+// at most 1024) threads; returns the block total in *total
+__device__ __forceinline__ int block_exclusive_scan(int v, int* total) {
+  __shared__ int s_w[16];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  int x = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int y = __shfl_up(x, o, 64);
+    if (lane >= o) x += y;
+  }
+  if (lane == 63) s_w[wv] = x;
+  __syncthreads();
+  int before = 0, all = 0;
+  for (int i = 0; i < nw; i++) {
+    const int w = s_w[i];
+    if (i < wv) before += w;
+    all += w;
+  }
+  __syncthreads();
+  *total = all;
+  return before + x - v;
+}
+
 // The B stencil's iz_bound = (int)((zzmax + FAC_MAP * R_max) * inv_dz)
 // (ext_stim.cpp:22) from the device's zzmax.  One outside [0, NZ] sweeps
 // nothing and is reported as ERR_OUT_OF_GRID; the sweep's NX NY iz_bound

@@ -42,30 +42,6 @@ __global__ void __launch_bounds__(128) k_map_stamp(const Tis* __restrict__ T, in
 // chunks fastest.  No lane covers a point outside its tissue except in the
 // last plane chunk, and no block is launched for a tissue that has no work.
 
-// exclusive prefix sum of v over a block of blockDim.x (a multiple of 64,
-// at most 1024) threads; returns the block total in *total
-__device__ __forceinline__ int block_exclusive_scan(int v, int* total) {
-  __shared__ int s_w[16];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = blockDim.x >> 6;
-  int x = v;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int y = __shfl_up(x, o, 64);
-    if (lane >= o) x += y;
-  }
-  if (lane == 63) s_w[wv] = x;
-  __syncthreads();
-  int before = 0, all = 0;
-  for (int i = 0; i < nw; i++) {
-    const int w = s_w[i];
-    if (i < wv) before += w;
-    all += w;
-  }
-  __syncthreads();
-  *total = all;
-  return before + x - v;
-}
-
 // The B stencil's list, once zzmax is on the device: per tissue iz_bound into
 // izb[i], and ceil(NX NY / bs) ceil(iz_bound / zb) tiles.  One block.
 __global__ void __launch_bounds__(256) k_wl_b(const Tis* __restrict__ T, int ntis, int bs, int zb,
@@ -920,27 +896,36 @@ void launch_map_stamp(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n,
     EPI_LAUNCH(K_MAP_STAMP, k_map_stamp<1>, dim3((max_n + 127) / 128, ntis), dim3(128), 0, s, dT, pb);
 }
 
+namespace {
+// a grid-stride walk over the list: the grid is sized from the host's estimate
+// (the last known zzmax), one block per tile (a cap at the blocks the CUs hold
+// at once left a tail of blocks waiting: 376-383 against 328-338 us on the
+// 256-tissue batch), and a multiple of 8 so that the XCD split applies
+unsigned ext_stim_blocks(long long tiles_est) {
+  return (unsigned)((std::min(std::max(tiles_est, 1LL), 1LL << 24) + 7) / 8 * 8);
+}
+}  // namespace
+
+void launch_ext_stim_list(hipStream_t s, const Tis* dT, int ntis, int bp, long long tiles_est, const int* d_wl,
+                          const Tuning& tu) {
+  by_zb(tu.b_zb, [&](auto zbc) {
+    EPI_LAUNCH(K_EXT_STIM, k_ext_stim<decltype(zbc)::value>, dim3(ext_stim_blocks(tiles_est)), dim3(64 * tu.b_rows), 0, s, dT,
+               d_wl, d_wl + ntis + 1, ntis, bp, tu.b_xcd);
+  });
+}
+
 void launch_ext_stim(hipStream_t s, const Tis* dT, int ntis, int bp, long long tiles_est, int* d_wl,
                      const Tuning& tu) {
   const int bs = 64 * tu.b_rows;
-  // a grid-stride walk over the list: the grid is sized from the host's
-  // estimate (the last known zzmax), one block per tile (a cap at the blocks
-  // the CUs hold at once left a tail of blocks waiting: 376-383 against
-  // 328-338 us on the 256-tissue batch), and a multiple of 8 so that the XCD
-  // split applies
-  const long long cap = 1LL << 24;
-  long long g = std::min(std::max(tiles_est, 1LL), cap);
-  g = (g + 7) / 8 * 8;
-  by_zb(tu.b_zb, [&](auto zbc) {
-    constexpr int zb = decltype(zbc)::value;
-    if (ntis == 1) {
-      EPI_LAUNCH(K_EXT_STIM, k_ext_stim_one<zb>, dim3((unsigned)g), dim3(bs), 0, s, dT, bp, tu.b_xcd);
-      return;
-    }
-    EPI_LAUNCH(K_WL, k_wl_b, dim3(1), dim3(256), 0, s, dT, ntis, bs, zb, d_wl, d_wl + ntis + 1);
-    EPI_LAUNCH(K_EXT_STIM, k_ext_stim<zb>, dim3((unsigned)g), dim3(bs), 0, s, dT, d_wl, d_wl + ntis + 1, ntis, bp,
-               tu.b_xcd);
-  });
+  if (ntis == 1) {
+    by_zb(tu.b_zb, [&](auto zbc) {
+      EPI_LAUNCH(K_EXT_STIM, k_ext_stim_one<decltype(zbc)::value>, dim3(ext_stim_blocks(tiles_est)), dim3(bs), 0, s, dT, bp,
+                 tu.b_xcd);
+    });
+    return;
+  }
+  EPI_LAUNCH(K_WL, k_wl_b, dim3(1), dim3(256), 0, s, dT, ntis, bs, tu.b_zb, d_wl, d_wl + ntis + 1);
+  launch_ext_stim_list(s, dT, ntis, bp, tiles_est, d_wl, tu);
 }
 
 static unsigned ca_lane_blocks(int max_n) { return ((unsigned)max_n * BL + 255) / 256; }

@@ -147,6 +147,9 @@ void launch_map_stamp(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n,
 // the B stencil over a work list of (tissue, tile) built on the device from
 // zzmax (d_wl: 2 ntis + 1 ints); tiles_est sizes the grid (any value covers
 // the list: the blocks walk it grid-stride)
+// k_ext_stim over a list that is in d_wl already: ntis + 1 offsets, ntis iz_bounds
+void launch_ext_stim_list(hipStream_t s, const Tis* dT, int ntis, int bp, long long tiles_est, const int* d_wl,
+                          const Tuning& tu);
 void launch_ext_stim(hipStream_t s, const Tis* dT, int ntis, int bp, long long tiles_est, int* d_wl,
                      const Tuning& tu);
 // a solve's or window's set-up: packed entries, pairs, laws' constants (and

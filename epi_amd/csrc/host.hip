@@ -412,6 +412,12 @@ int max_free(const epi_ctx* c) {
   for (auto& h : c->th) m = std::max(m, h.n_est + 64 - h.nmemb - h.nder);
   return m;
 }
+// cells past the membrane: those whose neighbourhood is swept
+int max_swept(const epi_ctx* c) {
+  int m = 1;
+  for (auto& h : c->th) m = std::max(m, h.n_est + 64 - h.nmemb);
+  return m;
+}
 int max_memb(const epi_ctx* c) {
   int m = 0;
   for (auto& h : c->th) m = std::max(m, h.nmemb);
@@ -1145,7 +1151,7 @@ int epi_cell_pos_periodic_fix(epi_ctx* c) {
 int epi_connect_cell(epi_ctx* c) {
   if (!c) return EPI_ERR_INVALID;
   const int nb = 1 - c->cb;
-  launch_connect(c->stream, c->d_tis, c->T, c->pb, nb, max_n(c), c->tu.sweep_wave);
+  launch_connect(c->stream, c->d_tis, c->T, c->pb, nb, max_n(c), max_swept(c), c->tu.sweep_wave);
   c->len_known = false;
   HIPCHK(c, hipGetLastError());
   c->cb = nb;
@@ -1287,7 +1293,7 @@ int epi_ca_substep(epi_ctx* c, int32_t iz_bound) {
 // and B sweep: epi_step joins it after issuing the next step's forces, which
 // read neither.
 constexpr int BUILD_FIELD_TISSUES = 1;
-hipError_t issue_build(epi_ctx* c, int mn, int mfree, int nb, int izb, bool side, bool join = true) {
+hipError_t issue_build(epi_ctx* c, int mn, int mfree, int swept, int nb, int izb, bool side, bool join = true) {
   hipError_t e = hipSuccess;
   auto chk = [&](hipError_t r) { if (e == hipSuccess) e = r; };
   launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, mfree, 1);
@@ -1295,7 +1301,7 @@ hipError_t issue_build(epi_ctx* c, int mn, int mfree, int nb, int izb, bool side
   if (!side) {
     long long tiles = 1;
     for (int t = 0; t < c->T; t++) tiles = std::max(tiles, b_tiles_of(c, t, BUILD_FIELD_BS));
-    launch_connect_field(c->stream, c->d_tis, c->T, c->pb, nb, c->bp, mn, tiles, c->tu);
+    launch_connect_field(c->stream, c->d_tis, c->T, c->pb, nb, c->bp, mn, swept, tiles, c->tu);
     chk(hipGetLastError());
     return e;
   }
@@ -1303,7 +1309,7 @@ hipError_t issue_build(epi_ctx* c, int mn, int mfree, int nb, int izb, bool side
   // beside the sweep) or after the whole build (1: the sweep runs alone and
   // the maps beside the next forces)
   if (!c->tu.side_fork) chk(hipEventRecord(c->ev_fork, c->stream));
-  launch_connect_rest(c->stream, c->d_tis, c->T, c->pb, nb, mn, c->tu.sweep_wave);
+  launch_connect_rest(c->stream, c->d_tis, c->T, c->pb, nb, mn, swept, c->tu.sweep_wave);
   if (c->tu.side_fork) chk(hipEventRecord(c->ev_fork, c->stream));
   chk(hipStreamWaitEvent(c->side_stream, c->ev_fork, 0));
   launch_map_stamp(c->side_stream, c->d_tis, c->T, c->pb, mn, c->tu);
@@ -1330,7 +1336,7 @@ int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
   const bool side = c->T > BUILD_FIELD_TISSUES || (g_prof.mask & seg);
   if (!c->tu.step_graph || (g_prof.mask & seg)) {
     *joined = !side;
-    HIPCHK(c, issue_build(c, mn, max_free(c), nb, izb, side, false));
+    HIPCHK(c, issue_build(c, mn, max_free(c), max_swept(c), nb, izb, side, false));
     return EPI_OK;
   }
   *joined = true;   // a captured graph rejoins its forked stream
@@ -1342,7 +1348,7 @@ int run_build(epi_ctx* c, int mn, int nb, int izb, bool* joined) {
   const int mfree = max_free(c) <= RENEW_ONE ? RENEW_ONE : mr;
   const std::vector<long long> key = {1, mfree > RENEW_ONE, c->pb, c->cb, c->cp, c->bp, nb, mr, izb, max_gsize(c),
                                       max_nx(c), max_ny(c), tu.b_zb, tu.b_rows, tu.map_lanes, tu.sweep_wave, tu.side_fork};
-  return graph_run(c, key, [&] { return issue_build(c, mr, mfree, nb, izb, side); });
+  return graph_run(c, key, [&] { return issue_build(c, mr, mfree, mr, nb, izb, side); });
 }
 
 int epi_step(epi_ctx* c, int64_t nsteps, epi_driver* drv) {
@@ -2197,8 +2203,7 @@ int epi_mech_adjoint(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps, in
   if (!m.active) return fail(c, EPI_ERR_INVALID, "no mechanics window is open");
   const int K = std::min(every, n_steps);
   const int nck = (n_steps + K - 1) / K;
-  int other = 1;   // cells past the membrane
-  for (auto& h : c->th) other = std::max(other, h.n_est + 64 - h.nmemb);
+  const int other = max_swept(c);
   const int memb = max_memb(c), nblk = mech_bwd_blocks(memb, other);
   size_t need = 0;
   for (int t = 0; t < c->T; t++)

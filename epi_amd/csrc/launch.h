@@ -31,7 +31,7 @@ struct Tuning {
   int ca_group = 8;           // Ca cell kernels: lanes per cell (8, or 16; 4 takes 8)
   int xcd = 1;                // Ca cells and ATP: XCD-contiguous workgroup order (launches of many workgroups)
   int b_xcd = 0;              // k_ext_stim: its tile list in one contiguous run per XCD
-  int sweep_wave = 0;         // k_sweep: 1, one wave per cell (64 lanes instead of 32)
+  int sweep_wave = 0;         // k_sweep: 1, one wave per cell whatever the number of cells (0: only for few)
   int side_fork = 0;          // 1: the side stream forks after the whole build
   int rd_group = 8;           // k_rd_step: lanes per cell
   int ca_fuse = 2;            // Ca solves: ATP of a sub-step and cells of the next in one launch
@@ -119,14 +119,15 @@ void launch_periodic_fix(hipStream_t s, const Tis* dT, int ntis, int pb, int max
 // applies the periodic fix, takes zzmax (cleared by launch_renew) and empties
 // the voxel maps with that many more blocks
 void launch_connect_insert(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n, unsigned clear_blocks);
-void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave);
+void launch_connect_rest(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int max_swept,
+                         int sweep_wave);
 // the rest of the build of a step with the stamping of the voxel maps as
 // further blocks of the sweep and the B stencil as further blocks of k_finish:
 // up to b_tiles tiles of BUILD_FIELD_BS points per tissue
 constexpr int BUILD_FIELD_BS = 128;
-void launch_connect_field(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int bp, int max_n, long long b_tiles,
-                          const Tuning& tu);
-void launch_connect(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int sweep_wave);
+void launch_connect_field(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int bp, int max_n, int max_swept,
+                          long long b_tiles, const Tuning& tu);
+void launch_connect(hipStream_t s, const Tis* dT, int ntis, int pb, int nb, int max_n, int max_swept, int sweep_wave);
 void launch_zzmax(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n);
 // A snapshot's output record (CellManager::output's fields): a header of
 // OUT_HDR bytes whose first int is the device's cell count, then m >= n

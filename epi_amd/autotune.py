@@ -12,8 +12,10 @@ The shapes it chooses (see epi_set_tuning in include/epi_amd.h):
                only solves of a few tissues, when the whole set runs faster
                unfused), with its own lanes per cell and z planes per thread
   k_map_stamp  lanes per cell (1, 4, 16)
-  k_sweep      32 lanes per cell or one wave per cell (sweep_wave 0, 1)
-  whole steps  where the side stream forks (side_fork 0, 1)
+  k_sweep      32 lanes per cell (64 where the cells are few) or one wave per
+               cell (sweep_wave 0, 1)
+  whole steps  where the side stream forks (side_fork 0, 1; sets of several
+               tissues)
 
 With CA_FUSE 2 the fused small solves use CA_GROUP_SMALL lanes per cell
 (default 8, the best width on a latency-bound single-tissue solve).

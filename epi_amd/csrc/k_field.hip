@@ -337,7 +337,7 @@ __device__ __forceinline__ Corner corner_load(const CaArg& a, int k, uint4 q) {
   const unsigned f = q.z;
   const bool hx = k & 1, hy = k & 2, hz = k & 4;
   const int dx = hx ? ((f & CQ_XP) ? 1 - a.NX : 1) : ((f & CQ_XM) ? a.NX - 1 : -1);
-  const int wy = (a.NY - 1) * a.XP;   // a plane has fewer than 2^31 points (epi_create)
+  const int wy = (a.NY - 1) * a.XP;   // only fused launches take corners so, and their planes are below 4 GB
   const int dy = hy ? ((f & CQ_YP) ? -wy : a.XP) : ((f & CQ_YM) ? wy : -a.XP);
   const long long dz = hz ? ((f & CQ_ZP) ? 0 : a.PL) : ((f & CQ_ZM) ? a.PL : -a.PL);
   const bool plain = f & CQ_PLAIN;

@@ -426,28 +426,30 @@ int epi_calc_ext_stim_noalloc(const epi_bfield_view* views, int32_t ngrids, int3
  * results.  The stencils walk a list of tiles over every tissue of a launch;
  * a tile is 64 *_ROWS consecutive points of a tissue's x-y plane (the block)
  * by *_ZB z planes.  Values: *_ZB in {1, 2, 4, 8, 16} (z planes per tile),
- * *_ROWS in {1, 2, 4} (64-lane rows per block), CA_GROUP in {4, 8, 16} (lanes per
- * cell in the Ca cell kernel), XCD in {0, 1} (1: the Ca cell and ATP kernels
- * number their workgroups so that each of the 8 XCDs runs one contiguous run
- * of cells / grid rows), RD_GROUP in {8, 16} (lanes per cell in the reverse
- * cell kernel of reaction-diffusion windows), CA_FUSE in {0, 1, 2} (1: a Ca
- * solve launches the ATP update of a sub-step and the cells of the next one
- * together, the cells computing their ATP corners themselves; 2: only for
- * solves of at most 131072 cells in total), MAP_LANES in
- * {1, 4, 16} (lanes per cell in the voxel-map stamp, splitting its voxels),
- * CA_GROUP_SMALL in {4, 8, 16} (lanes per cell in the solves CA_FUSE 2
- * fuses; those solves' ATP tiles are one plane deep when ATP_ZB is above 2), STEP_GRAPH in {0, 1} (0, the default: epi_step launches the
- * renewal and neighbour-build kernels of a step one by one; 1: it replays
- * them, side stream included, and every whole Ca solve (set-up, sub-steps,
- * averages) from HIP graphs captured once per launch key; whether a step
- * solves is still decided on the host from the step's status read-back),
+ * *_ROWS in {1, 2, 4} (64-lane rows per block; a one-tissue step's B sweep
+ * takes 128 points whatever B_ROWS), CA_GROUP in {4, 8, 16} (lanes per cell in
+ * the Ca cell kernels; 4 takes 8), XCD in {0, 1} (1: solves whose launches
+ * have at least 2048 workgroups number them so that each of the 8 XCDs runs
+ * one contiguous run of cells / of ATP tiles), RD_GROUP in {8, 16} (lanes per
+ * cell in the reverse cell kernel of reaction-diffusion windows), CA_FUSE in
+ * {0, 1, 2} (1: a Ca solve or window launches the ATP update of a sub-step and
+ * the cells of the next one together, the cells computing their ATP corners
+ * themselves; 2: only for solves of at most 196608 cells in total; a fused
+ * launch's ATP tiles are one plane deep for one tissue and two for several
+ * when ATP_ZB is above 2), MAP_LANES in {1, 4, 16} (lanes per cell in the
+ * voxel-map stamp, along x), CA_GROUP_SMALL in {4, 8, 16} (lanes per cell in
+ * the solves CA_FUSE 2 fuses), STEP_GRAPH in {0, 1} (0, the default: epi_step
+ * launches the renewal and neighbour-build kernels of a step one by one; 1: it
+ * replays them, side stream included, and every whole Ca solve (set-up,
+ * sub-steps, averages) from HIP graphs captured once per launch key; whether a
+ * step solves is still decided on the host from the step's status read-back),
  * B_XCD in {0, 1} (1: the B stencil's tile list is cut into one contiguous
- * run per XCD), SWEEP_WAVE in {0, 1} (lanes per cell of the neighbour
- * sweep: 0, 32 lanes of five buckets each; 1, one wave of two buckets per
- * lane, for small tissues), SIDE_FORK in {0, 1} (where a step's voxel maps
- * and B sweep fork onto the side stream: 0, after the bucket insertion, beside
- * the neighbour sweep; 1, after the whole build, beside the next step's
- * forces).  EPI_ERR_INVALID for other keys or values. */
+ * run per XCD), SWEEP_WAVE in {0, 1} (lanes per cell of the neighbour sweep:
+ * 0, 64 where at most 8192 cells are swept and 32 otherwise; 1, 64), SIDE_FORK
+ * in {0, 1} (where a step of several tissues forks its voxel maps and B sweep
+ * onto the side stream: 0, after the bucket insertion, beside the neighbour
+ * sweep; 1, after the whole build, beside the next step's forces; one tissue
+ * uses no side stream).  EPI_ERR_INVALID for other keys or values. */
 enum {
     EPI_TUNE_B_ZB = 0, EPI_TUNE_B_ROWS = 1, EPI_TUNE_ATP_ZB = 2, EPI_TUNE_ATP_ROWS = 3,
     EPI_TUNE_CA_GROUP = 4, EPI_TUNE_XCD = 5, EPI_TUNE_RD_GROUP = 6, EPI_TUNE_CA_FUSE = 7,

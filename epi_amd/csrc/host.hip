@@ -1137,7 +1137,7 @@ int epi_cell_state_renew(epi_ctx* c) {
   if (c->pos_pending) return fail(c, EPI_ERR_INVALID, "pos_copy must follow cell_interaction");
   launch_renew(c->stream, c->d_tis, c->T, c->pb, c->cb, c->cp, max_free(c), 0);
   HIPCHK(c, hipGetLastError());
-  for (auto& v : c->dev_ts) v++;   // k_remove advances each tissue's timestep
+  for (auto& v : c->dev_ts) v++;   // the renewal advances each tissue's timestep
   return EPI_OK;
 }
 

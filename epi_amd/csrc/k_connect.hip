@@ -42,7 +42,7 @@ __device__ __forceinline__ void zzmax_add(Status* st, double m) {
 // what it reads or nothing, and that would otherwise be three launches on the
 // side stream before the stamping (zz_set, zzmax, clear: 12 us of a step of
 // 420 cells with their gaps): calc_zzmax over the same cells (the maximum was
-// cleared by k_remove), and, in the blocks from cell_blocks on, the emptying of
+// cleared by the renewal), and, in the blocks from cell_blocks on, the emptying of
 // the voxel maps, which nothing reads between the last step's B sweep or solve
 // and this step's stamping.
 __device__ __forceinline__ void insert_cells(const Tis& t, int pb, int fix, bool step, int nblocks) {

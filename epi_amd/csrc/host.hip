@@ -2155,7 +2155,7 @@ int epi_mech_begin(epi_ctx* c) {
       const size_t cap = c->th[t].cap;
       r.x0[0] = cv.take<double>(3 * cap); r.x0[1] = cv.take<double>(3 * cap);
       for (int b = 0; b < 3; b++) r.lam[b] = cv.take<double>(3 * cap);
-      r.es = c->th[t].ns + 8;   // a row and its pair's spring
+      r.es = 2 * c->th[t].ns + 8;   // both roles of a row's entries, and the pair's spring
       r.ent = cv.take<int>(cap * (size_t)r.es);
       r.code = cv.take<uint8_t>(cap * (size_t)r.es);
       r.ent_n = cv.take<int>(cap);
@@ -2246,7 +2246,7 @@ int epi_mech_adjoint(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps, in
   }
   int q = 0;
   launch_mech_seed(c->stream, c->d_tis, m.d, c->T, c->pb, q, mn, nblk);
-  launch_mech_plan(c->stream, c->d_tis, m.d, c->T, c->pb, c->cb, other);
+  launch_mech_plan(c->stream, c->d_tis, m.d, c->T, c->pb, c->cb, mn);
   for (int k = nck - 1; k >= 0; k--) {
     const int s0 = k * K, s1 = std::min(n_steps, s0 + K);
     if (k < nck - 1) {

@@ -654,24 +654,26 @@ void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int m
 // and dermis frozen.  Which interactions apply depends only on that frozen
 // data, so the reverse pass enumerates them from each handler cell (its own
 // list, its pair, the membrane slots), evaluates the derivative of the
-// active branch of each law at the step's positions, and scatters
-// lam_c1 - lam_c2 through the pair's Jacobian with FP64 atomics.
+// active branch of each law at the step's positions, and takes
+// lam_c1 - lam_c2 through the pair's Jacobian.
 //
 // A group of lanes owns a cell (16 a membrane particle, whose 12 dihedrals
-// and six neighbours they take; 4 another cell, over the entries k_mech_plan
-// has packed), and for the same reason as in k_forces the laws and the two
-// dihedral forms each run as one code path: the quotients the common laws
-// share (1 / d^2, 1 / R, d) are taken once, and the operands chosen per lane.
-// A cell's own terms are summed over its lanes before one atomic; so are, for
-// a membrane particle, the terms of its six neighbours, which the dihedrals
-// meet two to three times each (39 atomics a particle instead of 144).  Sums
+// and six neighbours they take; 4 another cell), over the interactions that
+// k_mech_plan has packed, and for the same reason as in k_forces the laws and
+// the two dihedral forms each run as one code path: the quotients the common
+// laws share (1 / d^2, 1 / R, d) are taken once, and the operands chosen per
+// lane.  An interaction is evaluated from both of its cells, each keeping its
+// own side, so that the cells past the membrane need no atomics: those leave
+// the chip's L2s, which cost more than evaluating a law twice.  A membrane
+// particle's terms of its six neighbours, which the dihedrals meet two to three
+// times each, are summed before an atomic (39 a particle instead of 144).  Sums
 // are reduced in another order than the serial reverse's, as a gradient may.
 //
 // One lane per cell before (two launches and a third for the copies): its
 // waves, fewer than two a SIMD, each walked a whole list through every law's
-// own branch.  24 tissues, 105,000 cells, a step: 134 -> 76 us (8 lanes 79, 16
-// lanes 92 with entries that have no law still in the list), 25 of it the
-// atomics, which leave the chip's L2s, and 25 the arithmetic.
+// own branch.  24 tissues, 105,000 cells, a step: 134 us; lane groups over the
+// handlers' entries with atomics for the other cell 76 (8 lanes a cell 79; of
+// it the atomics 25); both sides evaluated 63.
 constexpr int MG = 16;   // of a membrane particle
 constexpr int MC = 4;    // of another cell
 
@@ -682,7 +684,7 @@ struct LawD { double coef, ds, deps, dadh, dspr; };
 // positions and radii: the law and the one choice inside it that frozen data
 // make.  They hold for a whole window, so k_mech_plan stores them, with the
 // entries that have a law, once per gradient.
-enum : int { CODE_LAW = 15, CODE_1 = 16, CODE_2 = 32 };
+enum : int { CODE_LAW = 15, CODE_1 = 16, CODE_2 = 32, CODE_OWN = 64 };   // CODE_OWN: this cell is the handler
 __device__ __forceinline__ int law_code(const Tis& t, int law, const CV& a, const CV& b) {
   if (law == LAW_ALAIRDE) return law | (a.strong && b.strong ? CODE_1 : 0);
   if (law == LAW_MU_MEMB) return law | (a.pair >= 0 && t.state[a.pair] == FIX ? CODE_1 : a.rdt > 0 ? CODE_2 : 0);
@@ -791,7 +793,9 @@ __device__ __forceinline__ P3 p3_shfl(P3 v, int src) {
   return P3{__shfl(v.x, src, MG), __shfl(v.y, src, MG), __shfl(v.z, src, MG)};
 }
 
-// the adjoint term of a pair for its first cell; the second's is its negative
+// the adjoint term of an interaction for one of its two cells, at a; the
+// formula is the same from either side (r and la - lb change sign together).
+// The parameters' sums take it once, with the handler.
 __device__ __forceinline__ P3 pair_bwd(const Tis& t, int code, P3 a, P3 b, double R, double snl, P3 la, P3 lb,
                                        ParAcc& pa) {
   const P3 r = vpsub(t, a, b);
@@ -799,9 +803,10 @@ __device__ __forceinline__ P3 pair_bwd(const Tis& t, int code, P3 a, P3 b, doubl
   const P3 av = v_sub(la, lb);
   const double ar = v_dot(av, r), DT = t.prm.DT_Cell;
   const double k2 = 2 * ld.ds * ar;
-  pa.eps += DT * ld.deps * ar;
-  pa.adh += DT * ld.dadh * ar;
-  pa.spr += DT * ld.dspr * ar;
+  const double once = code & CODE_OWN ? DT * ar : 0.0;
+  pa.eps += ld.deps * once;
+  pa.adh += ld.dadh * once;
+  pa.spr += ld.dspr * once;
   return P3{DT * (ld.coef * av.x + k2 * r.x), DT * (ld.coef * av.y + k2 * r.y), DT * (ld.coef * av.z + k2 * r.z)};
 }
 
@@ -870,23 +875,45 @@ __device__ __forceinline__ double tri_bend_bar(const Tis& t, bool second, P3 rv,
   return f * val;
 }
 
+// this lane's share of a cell's planned interactions
+template <int G>
+__device__ __forceinline__ P3 planned_bwd(const Tis& t, const MechTis& m, const double* px, const double* lam, int X, P3 xp,
+                                          P3 lx, double xr, int lane, ParAcc& pa) {
+  const long long cap = t.cap;
+  const int* ent = m.ent + (size_t)X * m.es;
+  const uint8_t* code = m.code + (size_t)X * m.es;
+  const int o0 = ent[lane], k0 = code[lane];   // in one round trip with the row's length (a row holds es > G slots)
+  const int len = m.ent_n[X];
+  P3 own{0, 0, 0};
+  for (int e = lane; e < len; e += G) {
+    const int o = e == lane ? o0 : ent[e], k = e == lane ? k0 : code[e];
+    // a pair's spring has the natural length of its handler, the higher index
+    const double snl = (k & CODE_LAW) == LAW_PAIR ? t.spr_nat_len[max(X, o)] : 0.0;
+    own = v_add(own, pair_bwd(t, k, xp, ld3(px, cap, o), xr + t.radius[o], snl, lx, ld3(lam, cap, o), pa));
+  }
+  return own;
+}
+
 // a membrane particle: its dihedrals (:488-499), its membrane neighbours, the wall
-__device__ __forceinline__ void bwd_membrane(const Tis& t, const double* px, const double* lam, double* nl, int X, int lane,
-                                             ParAcc& pa) {
+__device__ __forceinline__ void bwd_membrane(const Tis& t, const MechTis& m, const double* px, const double* lam, double* nl,
+                                             int X, int lane, ParAcc& pa) {
   const long long cap = t.cap;
   const int i = lane < 6 ? lane : lane < 12 ? lane - 6 : 0;   // lanes from 12 on take no term
   const int ma = t.memb6[6 * X + i];
   const P3 xp = ld3(px, cap, X), lm = ld3(lam, cap, X);
   const double xr = t.radius[X];
+  P3 own = planned_bwd<MG>(t, m, px, lam, X, xp, lm, xr, lane, pa);
+  if (lane == 12 && xp.z < xr) own.z += wall_bwd(t, xp.z, xr, lm.z, pa);
   const int mb = __shfl(ma, i == 5 ? 0 : i + 1, MG);
   const int m2 = __shfl(ma, i >= 4 ? i - 4 : i + 2, MG);
   const int mc = lane < 6 ? t.memb6[6 * mb + i] : m2;
   const P3 ap = ld3(px, cap, ma), bp = ld3(px, cap, mb), cp = ld3(px, cap, mc);
-  // the membrane pair first: its operands are done with before the dihedral
-  P3 own{0, 0, 0}, nb{0, 0, 0};
+  // the membrane pair before the dihedral: its operands are done with by then
+  P3 nb{0, 0, 0};
   if (lane < 6 && t.state[ma] == MEMB && X > ma) {
-    own = pair_bwd(t, LAW_MEMB_MEMB, xp, ap, xr + t.radius[ma], 0.0, lm, ld3(lam, cap, ma), pa);
-    nb = v_scale(-1.0, own);
+    const P3 g = pair_bwd(t, LAW_MEMB_MEMB | CODE_OWN, xp, ap, xr + t.radius[ma], 0.0, lm, ld3(lam, cap, ma), pa);
+    own = v_add(own, g);
+    nb = v_scale(-1.0, g);
   }
   P3 bar[4];
   const double val = tri_bend_bar(t, lane >= 6, xp, ap, bp, cp, lm, t.prm.DT_Cell * t.m_kbend, bar);
@@ -901,32 +928,22 @@ __device__ __forceinline__ void bwd_membrane(const Tis& t, const double* px, con
   nb = v_add(v_add(nb, v_add(bar[1], p3_shfl(bar[2], i1))), v_add(p3_shfl(bar[1], 6 + i), p3_shfl(bar[2], 6 + i1)));
   nb = v_add(nb, p3_shfl(bar[3], 6 + i2));
   if (lane < 6) atomic_add3(nl, cap, ma, nb);
-  if (lane == 12 && xp.z < xr) own.z += wall_bwd(t, xp.z, xr, lm.z, pa);
   own = v_add(p3_group_sum<MG>(own), lm);
   if (lane < 3) atomicAdd(&nl[lane * cap + X], lane == 0 ? own.x : lane == 1 ? own.y : own.z);
 }
 
-// the planned interactions of another cell's handler, and a DER cell's wall
+// the planned interactions of another cell, and a DER cell's wall; nothing
+// else reaches the cell's adjoint, so it is stored, not added
 __device__ __forceinline__ void bwd_cell(const Tis& t, const MechTis& m, const double* px, const double* lam, double* nl,
                                          int X, int lane, ParAcc& pa) {
   const long long cap = t.cap;
-  const int* ent = m.ent + (size_t)X * m.es;
-  const uint8_t* code = m.code + (size_t)X * m.es;
-  const int o0 = ent[lane], k0 = code[lane];   // in one round trip with the row's length (a row holds es > MC slots)
-  const int len = m.ent_n[X];
   const P3 xp = ld3(px, cap, X), lx = ld3(lam, cap, X);
-  const double xr = t.radius[X], snl = t.spr_nat_len[X];
+  const double xr = t.radius[X];
   const bool der = t.state[X] == DER;
-  P3 own{0, 0, 0};
-  for (int e = lane; e < len; e += MC) {
-    const int o = e == lane ? o0 : ent[e], k = e == lane ? k0 : code[e];
-    const P3 g = pair_bwd(t, k, xp, ld3(px, cap, o), xr + t.radius[o], snl, lx, ld3(lam, cap, o), pa);
-    own = v_add(own, g);
-    atomic_add3(nl, cap, o, v_scale(-1.0, g));
-  }
+  P3 own = planned_bwd<MC>(t, m, px, lam, X, xp, lx, xr, lane, pa);
   if (lane == MC - 1 && der && xp.z < xr) own.z += wall_bwd(t, xp.z, xr, lx.z, pa);
   own = v_add(p3_group_sum<MC>(own), lx);
-  if (lane < 3) atomicAdd(&nl[lane * cap + X], lane == 0 ? own.x : lane == 1 ? own.y : own.z);
+  if (lane < 3) nl[lane * cap + X] = lane == 0 ? own.x : lane == 1 ? own.y : own.z;
 }
 }  // namespace
 
@@ -981,30 +998,44 @@ __global__ void __launch_bounds__(256) k_mech_seed(const Tis* __restrict__ T, Me
   if ((threadIdx.x & 63) == 0 && part != 0) atomicAdd(&m.scal[0], part / n);
 }
 
-// every interaction a cell's handler applies (cell_interaction.cpp:529-641)
-// and its pair's spring, packed by ballots of MG lanes per cell
+// Every interaction a cell takes part in, as its handler or as the other cell
+// (cell_interaction.cpp:529-641; rows are symmetric but for the membrane's six
+// slots, which bwd_membrane takes), and its pair's spring, packed by ballots of
+// MG lanes per cell.  A row's entry has two where both cells are DER.
 __global__ void __launch_bounds__(256) k_mech_plan(const Tis* __restrict__ T, MechTis* __restrict__ M, int pb, int cb) {
   const Tis& t = T[blockIdx.y];
   const MechTis& m = M[blockIdx.y];
   const int n = t.st->n;
   const int lane = threadIdx.x & (MG - 1), sh = threadIdx.x & 63 & ~(MG - 1);
-  for (int X = t.nmemb + blockIdx.x * (256 / MG) + threadIdx.x / MG; X < n; X += gridDim.x * (256 / MG)) {
+  for (int X = blockIdx.x * (256 / MG) + threadIdx.x / MG; X < n; X += gridDim.x * (256 / MG)) {
+    const bool memb = X < t.nmemb;
     const int* row = t.col[cb] + (size_t)X * t.ns;
     const CV cx = load_cv(t, pb, X);
-    const int len = t.nlen[cb][X], all = len + (cx.pair >= 0 && X > cx.pair);
+    const int len = t.nlen[cb][X], all = len + (!memb && cx.pair >= 0);
     int at = 0;
-    for (int e0 = 0; e0 < all; e0 += MG) {
+    for (int e0 = memb ? MEMB_ADJ : 0; e0 < all; e0 += MG) {
       const int e = e0 + lane;
       const int o = e < len ? row[e] : e < all ? cx.pair : X;
       const CV co = load_cv(t, pb, o);
-      const int law = e < len ? proc_law(cx, X, co, o) : e < all ? (int)LAW_PAIR : (int)LAW_NONE;
-      const unsigned mk = (unsigned)(__ballot(law != LAW_NONE) >> sh) & ((1u << MG) - 1);
-      if (law != LAW_NONE) {
-        const int k = at + __popc(mk & ((1u << lane) - 1));
-        m.ent[(size_t)X * m.es + k] = o;
-        m.code[(size_t)X * m.es + k] = (uint8_t)law_code(t, law, cx, co);
+      int code[2] = {LAW_NONE, LAW_NONE};   // as the handler, as the other cell
+      if (e < len) {
+        const int own = memb ? (int)LAW_NONE : proc_law(cx, X, co, o);
+        const int oth = o < t.nmemb ? (int)LAW_NONE : proc_law(co, o, cx, X);
+        if (own != LAW_NONE) code[0] = law_code(t, own, cx, co) | CODE_OWN;
+        if (oth != LAW_NONE) code[1] = law_code(t, oth, co, cx);
+      } else if (e < all) {
+        code[0] = LAW_PAIR | (X > o ? CODE_OWN : 0);
       }
-      at += __popc(mk);
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        const unsigned mk = (unsigned)(__ballot(code[k] != LAW_NONE) >> sh) & ((1u << MG) - 1);
+        if (code[k] != LAW_NONE) {
+          const int slot = at + __popc(mk & ((1u << lane) - 1));
+          m.ent[(size_t)X * m.es + slot] = o;
+          m.code[(size_t)X * m.es + slot] = (uint8_t)code[k];
+        }
+        at += __popc(mk);
+      }
     }
     if (lane == 0) m.ent_n[X] = at;
   }
@@ -1030,7 +1061,7 @@ __global__ void __launch_bounds__(256) k_mech_bwd(const Tis* __restrict__ T, Mec
     const int lane = threadIdx.x & (MG - 1), step = nblk * (256 / MG);
     for (int X = bid * (256 / MG) + threadIdx.x / MG; X < t.nmemb; X += step) {
       if (lane < 3) dead[lane * cap + X] = 0;
-      bwd_membrane(t, px, lam, nl, X, lane, pa);
+      bwd_membrane(t, m, px, lam, nl, X, lane, pa);
     }
   } else {
     const int lane = threadIdx.x & (MC - 1), step = nblk * (256 / MC), n = t.st->n;
@@ -1076,8 +1107,8 @@ namespace {
 int mech_blocks(int cells, int lanes) { return (int)(((long long)cells * lanes + 255) / 256); }
 }  // namespace
 int mech_bwd_blocks(int max_memb, int max_other) { return mech_blocks(max_memb, MG) + mech_blocks(max_other, MC); }
-void launch_mech_plan(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int cb, int max_other) {
-  EPI_LAUNCH(K_MECH_PLAN, k_mech_plan, dim3(mech_blocks(max_other, MG), ntis), dim3(256), 0, s, dT, dM, pb, cb);
+void launch_mech_plan(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int cb, int max_n) {
+  EPI_LAUNCH(K_MECH_PLAN, k_mech_plan, dim3(mech_blocks(max_n, MG), ntis), dim3(256), 0, s, dT, dM, pb, cb);
 }
 void launch_mech_backward_step(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int slot, int q, int max_memb,
                                int max_other) {

@@ -218,7 +218,7 @@ int mech_bwd_blocks(int max_memb, int max_other);
 void launch_mech_seed(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int q, int max_n, int nblk);
 void launch_mech_backward_step(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int slot, int q, int max_memb,
                                int max_other);
-void launch_mech_plan(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int cb, int max_other);
+void launch_mech_plan(hipStream_t s, const Tis* dT, MechTis* dM, int ntis, int pb, int cb, int max_n);
 void launch_mech_sums(hipStream_t s, MechTis* dM, int ntis, int nblk);
 void launch_rd_sums(hipStream_t s, const Tis* dT, RdTis* dR, int ntis, int q, long long items);
 }  // namespace epi

@@ -17,8 +17,8 @@ struct MechTis {
   // position adjoints (3 * cap each) in three rotating buffers: [q] after the
   // step, [q + 1] before it, [q + 2] cleared for the next, q = step mod 3
   GPtr<double> lam[3];
-  // the interactions each cell's handler applies, es slots a cell: the other
-  // cell and the law's code (k_mech_plan)
+  // the interactions each cell takes part in, es slots a cell: the other cell
+  // and the law's code (k_mech_plan)
   GPtr<int> ent;
   GPtr<uint8_t> code;
   GPtr<int> ent_n;

@@ -28,6 +28,18 @@ __host__ __device__ __forceinline__ AtpK atp_k(const Params& pm) {
   return AtpK{pm.DT_Ca, pm.Da, pm.STIM11, pm.Kaa, pm.AIR_STIM};
 }
 
+// ATP_refresh's update of one point (ca2p.cpp:302-338) from its value, its
+// six neighbours (mirror z, periodic x and y) and their masks.  Every path
+// that advances an ATP point goes through this one expression.
+__device__ __forceinline__ double atp_new(const AtpK& k, double catp, double cxm, double cxp, double cym,
+                                          double cyp, double czm, double czp, double mxm, double mxp, double mym,
+                                          double myp, double mzm, double mzp, double diffu, double air, double inv_dx) {
+  const double fa = k.STIM11 * min0(diffu) - catp * k.Kaa;
+  return catp + k.DT_Ca * (k.Da * (mxm * (cxm - catp) + mxp * (cxp - catp) + mym * (cym - catp) + myp * (cyp - catp)
+                                   + mzm * (czm - catp) + mzp * (czp - catp))
+                           * inv_dx * inv_dx + fa + air * k.AIR_STIM);
+}
+
 // ca2p_by_ext_stim (:59-63) of a cell's mean B
 __device__ __forceinline__ double ca2p_by_ext(const CaK& k, double B) {
   return k.kbc * B * B * k.Cout / (k.Hb + B * B);

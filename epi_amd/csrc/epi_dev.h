@@ -32,6 +32,9 @@ enum { OK = 0, ERR_CAPACITY = 1, ERR_STRONG_INTERACTION = 2, ERR_NO_DERMIS = 3,
 constexpr int MEMB_ADJ = 6;                // define.h:147-153 (TRI_MEMB)
 constexpr int MAX_CONN = 400;              // define.h:80, cell_connection.cpp:30
 constexpr int N3 = 200;                    // cell_connection.cpp:28
+// the fewest slots of a list row: kernels read a row's first chunk before they
+// know its length, and check that it fits
+constexpr int ROW_SLOTS_MIN = 64;
 // A bucket is a head of eight words, its count and its first seven cells (two
 // 16-byte loads), and the rest of its slots elsewhere: the five heads that a
 // sweep reads of a column lie in two or three cache lines.  Words between two

@@ -795,9 +795,7 @@ int epi_create(int32_t ntissues, const epi_geometry* geos, epi_ctx** out) {
     h.g = g;
     h.nmemb = g.nmx * g.nmy;
     h.cap = g.max_cells;
-    // a row holds at least 64 slots: the Ca cell kernel reads its first list
-    // chunk (up to 64 entries) before it knows the length
-    h.ns = g.row_stride > 0 ? std::max(64, std::min(g.row_stride, MAX_CONN)) : MAX_CONN;
+    h.ns = g.row_stride > 0 ? std::max(ROW_SLOTS_MIN, std::min(g.row_stride, MAX_CONN)) : MAX_CONN;
     h.bcap = g.bucket_cap > 0 ? std::min(g.bucket_cap, N3) : N3;
     h.NX = g.nx; h.NY = g.ny; h.NZ = g.nz;
     h.XP = (int)align_up(g.nx + 1, 16);

@@ -221,6 +221,7 @@ template <int RG>
 __device__ __forceinline__ void rd_cells_part(const Tis& t, const RdTis& r, int bid, int nblk, int slot, int q,
                                               int qa) {
   constexpr int REP = 32 / RG;
+  static_assert(RG * REP <= ROW_SLOTS_MIN, "the entries read before the length lie inside a row");
   constexpr int OWN = 64 / RG;   // owned voxels a lane takes in one go
   const int start = t.nmemb + t.nder;
   const long long cap = t.cap, ns = t.ns;
@@ -288,7 +289,7 @@ __device__ __forceinline__ void rd_cells_part(const Tis& t, const RdTis& r, int 
     int o[REP];
     uint8_t kd[REP], so[REP];
     double gv[REP], lgv[REP], uo[REP], po[REP];
-    // every load unconditional (a row holds ns >= 32 slots; a masked entry
+    // every load unconditional (a row holds ns >= ROW_SLOTS_MIN slots; a masked entry
     // reads cell 0), masked with integer masks afterwards, so that no load
     // sits in a branch that waits for it
     int x[REP];

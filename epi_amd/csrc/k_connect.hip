@@ -348,7 +348,7 @@ __global__ void __launch_bounds__(256) k_sweep(const Tis* __restrict__ T, int pb
 // minimum over the group.  Longer rows take the same steps through global
 // memory.
 // The time is the chain of round trips: the cell's words; the rows' first
-// KPRE entries (unconditional: a row holds at least 32 slots) with the
+// KPRE entries (unconditional: a row has ROW_SLOTS_MIN slots) with the
 // previous row's length and values; the uids of both.  The launch also does
 // what the next build needs of this one (every cell's row is its own from
 // here, the uids are kept beside the rows they number, the buckets are
@@ -358,6 +358,7 @@ constexpr int KCAP = 64;   // rows (and previous rows) longer than this take the
 constexpr int KPRE = 2;    // entries of each row a lane asks for before it knows the lengths
 constexpr int K_BLOCK = 128;
 constexpr int K_GROUPS = K_BLOCK / KG;
+static_assert(KPRE * KG <= ROW_SLOTS_MIN, "the entries read before the length lie inside a row");
 
 __device__ __forceinline__ void finish_part(const Tis& t, int pb, int nb, int nblk) {
   Status* st = t.st;

@@ -15,6 +15,7 @@
 #include "launch.h"
 #include "epi_group.h"
 #include "ca_laws.h"
+#include "ca_corner.h"
 #include "rd_dev.h"
 #include "field_step.h"
 
@@ -212,18 +213,6 @@ __device__ __forceinline__ unsigned xcd_order(unsigned L, unsigned G, int on) {
   return x * q + min(x, r) + (L >> 3);
 }
 
-// ATP_refresh's update of one point (ca2p.cpp:302-338) from its value, its
-// six neighbours (mirror z, periodic x and y) and their masks.  Every path
-// that advances an ATP point goes through this one expression.
-__device__ __forceinline__ double atp_new(const AtpK& k, double catp, double cxm, double cxp, double cym,
-                                          double cyp, double czm, double czp, double mxm, double mxp, double mym,
-                                          double myp, double mzm, double mzp, double diffu, double air, double inv_dx) {
-  const double fa = k.STIM11 * min0(diffu) - catp * k.Kaa;
-  return catp + k.DT_Ca * (k.Da * (mxm * (cxm - catp) + mxp * (cxp - catp) + mym * (cym - catp) + myp * (cyp - catp)
-                                   + mzm * (czm - catp) + mzp * (czp - catp))
-                           * inv_dx * inv_dx + fa + air * k.AIR_STIM);
-}
-
 // diff_u of a sub-step by Ca parity: the sub-step at parity cp writes it and
 // its ATP update reads it, so a fused launch (ATP of one sub-step beside the
 // cells of the next) reads one buffer while it writes the other.
@@ -276,45 +265,19 @@ __host__ __device__ __forceinline__ CaArg ca_arg(const Tis& t, int cpc, int cpa,
 // each AFM cell keeps, for all of its sub-steps, its ca2p_by_ext_stim and, of
 // its eight grid_avg8 corners, the point, its voxel word, neighbour masks and
 // where the stencil wraps.  One lane per (cell, corner), after k_ca_vox.
-constexpr unsigned CQ_XM = 1u << 6, CQ_XP = 1u << 7, CQ_YM = 1u << 8, CQ_YP = 1u << 9;   // x = 0, x = NX - 1, ...
-constexpr unsigned CQ_ZM = 1u << 10, CQ_ZP = 1u << 11;   // z = 0 (mirror), z = NZ - 1 (self)
-constexpr unsigned CQ_PLAIN = 1u << 30;   // not updated inside the solve: read as it is
-constexpr unsigned CQ_SLOW = 1u << 31;    // a mask byte above 1: word and masks come from the maps
-
 __global__ void __launch_bounds__(256) k_ca_corners(const Tis* __restrict__ T, const int* tlist, int bp) {
   const Tis& t = T[tlist ? tlist[blockIdx.y] : blockIdx.y];
   const int n = t.st->n;
   const int start = t.nmemb + t.nder;
   const int izb = ca_iz_bound(t);
-  const int NX = t.NX, NY = t.NY, NZ = t.NZ;
   const CaK ck = ca_k(t.prm);
   for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < 8LL * n;
        i += (long long)gridDim.x * blockDim.x) {
     const int c = (int)(i >> 3), k = (int)(i & 7);
     if (c < start || !is_afm(t.state[c])) continue;
-    int j = t.lat[3 * c] + (k & 1), kk = t.lat[3 * c + 1] + ((k >> 1) & 1);
-    const int l = t.lat[3 * c + 2] + (k >> 2);
-    const long long raw = gidx(t, j, kk, l);
-    const double b = t.bf[bp][raw];
-    if (j == NX) j = 0;
-    if (kk == NY) kk = 0;
-    const long long v = gidx(t, j, kk, l);
-    unsigned word = 0, bits = CQ_PLAIN;
-    if (l < izb && izb <= NZ) {
-      const int px = j == 0 ? NX - 1 : j - 1, nx = j == NX - 1 ? 0 : j + 1;
-      const int py = kk == 0 ? NY - 1 : kk - 1, ny = kk == NY - 1 ? 0 : kk + 1;
-      const int pz = l == 0 ? 1 : l - 1, nz = l + 1 == NZ ? NZ - 1 : l + 1;
-      const uint8_t m[6] = {t.cmap2[gidx(t, px, kk, l)], t.cmap2[gidx(t, nx, kk, l)], t.cmap2[gidx(t, j, py, l)],
-                            t.cmap2[gidx(t, j, ny, l)], t.cmap2[gidx(t, j, kk, pz)], t.cmap2[gidx(t, j, kk, nz)]};
-      bits = (j == 0 ? CQ_XM : 0) | (j == NX - 1 ? CQ_XP : 0) | (kk == 0 ? CQ_YM : 0) | (kk == NY - 1 ? CQ_YP : 0) |
-             (l == 0 ? CQ_ZM : 0) | (l + 1 == NZ ? CQ_ZP : 0);
-      for (int q = 0; q < 6; q++) {
-        if (m[q] > 1) bits |= CQ_SLOW;
-        bits |= (unsigned)(m[q] & 1) << q;
-      }
-      word = t.vox[v];
-    }
-    t.ca_cq[i] = make_uint4((unsigned)v, word, bits, (unsigned)raw);
+    const int x = t.lat[3 * c], y = t.lat[3 * c + 1], z = t.lat[3 * c + 2];
+    const double b = t.bf[bp][gidx(t, x + (k & 1), y + ((k >> 1) & 1), z + (k >> 2))];
+    t.ca_cq[i] = corner_word(t, izb, x, y, z, k);
     // grid_avg8 (utils.h:18-23) of B in its order: 000 100 010 001 110 101 011 111
     const double sum = __shfl(b, 0, 8) + __shfl(b, 1, 8) + __shfl(b, 2, 8) + __shfl(b, 4, 8) + __shfl(b, 3, 8) +
                        __shfl(b, 5, 8) + __shfl(b, 6, 8) + __shfl(b, 7, 8);
@@ -322,61 +285,11 @@ __global__ void __launch_bounds__(256) k_ca_corners(const Tis* __restrict__ T, c
   }
 }
 
-// The ATP value of a cell's corner `k` (binary x, y, z; its lane is k) after
-// the ATP update that runs beside this launch, computed from the buffer before
-// it (the grid kernel's expression, atp_new).  The corners of a cell are the
-// points of a cube, so three of a corner's six stencil neighbours are the
-// cube's other corners and come from their lanes; the other three, the point
-// itself and the owner's diff_u are loaded, without branches, so that the
-// loads of the cell's entries can be issued behind them.  A corner that the
-// update leaves alone takes its value from the buffer after it, in `ox`.
-struct Corner { double c0, ox, oy, oz, diffu; };
-__device__ __forceinline__ Corner corner_load(const CaArg& a, int k, uint4 q) {
-  const double* __restrict__ A = a.A0;
-  const long long v = q.x;
-  const unsigned f = q.z;
-  const bool hx = k & 1, hy = k & 2, hz = k & 4;
-  const int dx = hx ? ((f & CQ_XP) ? 1 - a.NX : 1) : ((f & CQ_XM) ? a.NX - 1 : -1);
-  const int wy = (a.NY - 1) * a.XP;   // only fused launches take corners so, and their planes are below 4 GB
-  const int dy = hy ? ((f & CQ_YP) ? -wy : a.XP) : ((f & CQ_YM) ? wy : -a.XP);
-  const long long dz = hz ? ((f & CQ_ZP) ? 0 : a.PL) : ((f & CQ_ZM) ? a.PL : -a.PL);
-  const bool plain = f & CQ_PLAIN;
-  const unsigned cell1 = q.y & 0x7fffffffu;
-  Corner r;
-  r.c0 = A[v];
-  r.ox = *(plain ? a.A1 + v : A + v + dx);
-  r.oy = A[plain ? v : v + dy];
-  r.oz = A[plain ? v : v + dz];
-  r.diffu = a.dfo[cell1 ? cell1 - 1 : 0];
-  return r;
-}
+// corner_new of the cell's corner `k` (its lane is k): the cube's other corners
+// come from their lanes
 __device__ __forceinline__ double corner_value(const Tis& t, const CaArg& a, int k, uint4 q, const Corner& r) {
-  const unsigned f = q.z;
-  const bool hx = k & 1, hy = k & 2, hz = k & 4;
   const double c0 = r.c0;
-  const double ix = __shfl_xor(c0, 1, 64), iy = __shfl_xor(c0, 2, 64), iz = __shfl_xor(c0, 4, 64);
-  // next_z(NZ - 1) is the point itself (utils.cpp:32-72); such a point is the
-  // upper corner (oz above) or, with its cell at the grid's top, the lower one
-  const double izn = !hz && (f & CQ_ZP) ? c0 : iz;
-  unsigned word = q.y;
-  double diffu = (word & 0x7fffffffu) ? r.diffu : 0.0;
-  double m[6];
-#pragma unroll
-  for (int b = 0; b < 6; b++) m[b] = (double)((f >> b) & 1);
-  if (f & CQ_SLOW) {
-    const uint8_t* __restrict__ cm2 = a.cm2;
-    const long long v = q.x, wy = (long long)(a.NY - 1) * a.XP;
-    m[0] = cm2[v + ((f & CQ_XM) ? a.NX - 1 : -1)];
-    m[1] = cm2[v + ((f & CQ_XP) ? 1 - a.NX : 1)];
-    m[2] = cm2[v + ((f & CQ_YM) ? wy : -(long long)a.XP)];
-    m[3] = cm2[v + ((f & CQ_YP) ? -wy : a.XP)];
-    m[4] = cm2[v + ((f & CQ_ZM) ? a.PL : -a.PL)];
-    m[5] = cm2[v + ((f & CQ_ZP) ? 0 : a.PL)];
-  }
-  const double nv = atp_new(atp_k(t.prm), c0, hx ? ix : r.ox, hx ? r.ox : ix, hy ? iy : r.oy, hy ? r.oy : iy,
-                            hz ? iz : r.oz, hz ? r.oz : izn, m[0], m[1], m[2], m[3], m[4], m[5], diffu,
-                            (double)(word >> 31), t.inv_dx);
-  return (f & CQ_PLAIN) ? r.ox : nv;
+  return corner_new(atp_k(t.prm), t.inv_dx, a, k, q, r, __shfl_xor(c0, 1, 64), __shfl_xor(c0, 2, 64), __shfl_xor(c0, 4, 64));
 }
 
 // dead_IP3_calc (:156-173) and supra_calc (:182-222).  A group of CG lanes (8
@@ -417,6 +330,7 @@ __device__ __forceinline__ void ca_cells_part(const Tis& t, const CaArg& a, unsi
   constexpr int C_GROUPS = C_BLOCK / CG;
   constexpr int CCAP = 32;          // entries per chunk: more than nearly every cell has
   constexpr int EPL = CCAP / CG;    // of them per lane
+  static_assert(CG >= 8 && EPL * CG == CCAP && CCAP <= ROW_SLOTS_MIN, "eight corner lanes, whole chunks inside a row");
   // per-entry terms for the summing lanes, corners, and the per-cell values
   // and quotients; rows padded so that the groups of a wave read different banks
   __shared__ double2 s_a[C_GROUPS][CCAP + 1];
@@ -429,7 +343,7 @@ __device__ __forceinline__ void ca_cells_part(const Tis& t, const CaArg& a, unsi
   // First round trip: the cell's own words, its first chunk's entries and its
   // corners' words, beside the cell count (a device value).  A cell past the
   // count reads allocated, stale slots and leaves once the count is in; a row
-  // holds ns >= CCAP slots, and entries past len are masked.
+  // holds ns >= ROW_SLOTS_MIN slots, and entries past len are masked.
   const uint8_t s = a.state[c];
   const int len = a.cn[c];
   const double2 uc = a.up[c];
@@ -450,11 +364,11 @@ __device__ __forceinline__ void ca_cells_part(const Tis& t, const CaArg& a, unsi
   // Second round trip: the corners' points and the entries' pairs.  A DEAD
   // cell has no corners (its words may never have been written): point 0, as
   // it lies.
-  if (dead) q = make_uint4(0u, 0u, CQ_PLAIN, 0u);
+  if (dead) q = corner_none();
   Corner cr;
   double raw = 0;
   if (REC) cr = corner_load(a, lane & 7, q);
-  else raw = a.A0[q.w];
+  else raw = a.A0[corner_raw(q)];
   double2 w[EPL];
 #pragma unroll
   for (int i = 0; i < EPL; i++) w[i] = a.up[lane + i * CG < len ? en[i] >> 2 : c];

@@ -368,6 +368,7 @@ __device__ void forces_serial(const Tis& t, int pb, int cb, int X, Status* st) {
 constexpr int FG = 16;
 constexpr int F_BLOCK = 128;
 constexpr int F_GROUPS = F_BLOCK / FG;
+static_assert(FG <= ROW_SLOTS_MIN, "a lane's first entry lies inside its cell's row");
 
 // a group's LDS slots, padded by 8 bytes so that the summing lanes of a
 // wave's groups read different banks
@@ -431,7 +432,7 @@ __global__ void __launch_bounds__(F_BLOCK) k_forces(const Tis* __restrict__ T, i
   const bool memb = X < t.nmemb;
   const int nA = memb ? 0 : t.nlo[X];
   const int* row = t.col[cb] + (size_t)X * t.ns;
-  const int q0 = row[lane];   // a row holds ns >= 64 > FG slots
+  const int q0 = row[lane];   // a row holds ns >= ROW_SLOTS_MIN > FG slots
   const int n = st->n;
   if (blockIdx.x == 0 && threadIdx.x == 0 && (long long)gridDim.x * F_GROUPS < n) set_force_err(st, ERR_INVALID);
   if (X >= n) return;

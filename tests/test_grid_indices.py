@@ -1,0 +1,42 @@
+"""The grid index arithmetic of the kernels, built for the host from the same
+headers and run on sparse grids (CPU only): the eight grid_avg8 corners
+(utils.h:18-23) of a cell in a Ca solve (ca_corner.h) against the seven-point
+ATP update (ca2p.cpp:302-338) written out -- inside the grid, at its periodic
+seams, at the mirrored bottom, the top plane and iz_bound."""
+import ctypes as C
+import itertools
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("grid") / "libgrid.so")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", os.path.join(HERE, "native", "grid_index_check.cpp"), "-o", out], check=True)
+    return C.CDLL(out)
+
+
+def corners(lib, nx, ny, nz, izb, x, y, z, mask, seed):
+    out, want = np.full(8, -1.0), np.full(8, -2.0)
+    raw, raw_want = np.full(8, -1, np.int64), np.full(8, -2, np.int64)
+    rc = lib.corner_check(nx, ny, nz, izb, x, y, z, mask, seed,
+                          *(a.ctypes.data_as(C.c_void_p) for a in (out, want, raw, raw_want)))
+    if rc:
+        pytest.skip("no address space for the grid")
+    # the two sides add the same dozen terms of order 1 in another order
+    assert np.allclose(out, want, rtol=1e-13, atol=1e-14), (x, y, z, out, want)
+    assert np.array_equal(raw, raw_want), (x, y, z)
+
+
+@pytest.mark.parametrize("nx,ny,nz,izb", [(5, 7, 6, 4), (2, 3, 2, 2), (33, 16, 9, 9), (15, 15, 4, 1), (16, 31, 3, 0)])
+@pytest.mark.parametrize("mask", [1, 2])
+def test_every_corner_of_small_grids(lib, nx, ny, nz, izb, mask):
+    at = lambda n: sorted({0, 1, n // 2, n - 2, n - 1})
+    for i, (x, y, z) in enumerate(itertools.product(at(nx), at(ny), at(nz))):
+        corners(lib, nx, ny, nz, izb, x, y, z, mask, i)

@@ -13,17 +13,19 @@ namespace epi {
 // A corner's word: x the point, wrapped in x and y; y its voxel word (Tis::vox);
 // z the masks of its six stencil neighbours (bits 0-5: x-, x+, y-, y+, z-, z+)
 // and the flags below; w the point as it lies (a periodic copy at x = NX or
-// y = NY).
+// y = NY).  A grid's points may pass 2^32 (42 bytes a point of grid arrays:
+// 180 GB), so z also holds bits 32-39 of both points (in bits 12-19 of x's, in
+// bits 20-27 of w's); 2^40 points are more than any card holds.
 constexpr unsigned CQ_XM = 1u << 6, CQ_XP = 1u << 7, CQ_YM = 1u << 8, CQ_YP = 1u << 9;   // x = 0, x = NX - 1, ...
 constexpr unsigned CQ_ZM = 1u << 10, CQ_ZP = 1u << 11;   // z = 0 (mirror), z = NZ - 1 (self)
 constexpr unsigned CQ_PLAIN = 1u << 30;   // not updated inside the solve: read as it is
 constexpr unsigned CQ_SLOW = 1u << 31;    // a mask byte above 1: the masks come from the map
 
 __device__ __forceinline__ uint4 corner_pack(long long v, unsigned word, unsigned bits, long long raw) {
-  return make_uint4((unsigned)v, word, bits, (unsigned)raw);
+  return make_uint4((unsigned)v, word, bits | (unsigned)(v >> 32) << 12 | (unsigned)(raw >> 32) << 20, (unsigned)raw);
 }
-__device__ __forceinline__ long long corner_at(uint4 q) { return q.x; }
-__device__ __forceinline__ long long corner_raw(uint4 q) { return q.w; }
+__device__ __forceinline__ long long corner_at(uint4 q) { return (long long)(q.z >> 12 & 0xffu) << 32 | q.x; }
+__device__ __forceinline__ long long corner_raw(uint4 q) { return (long long)(q.z >> 20 & 0xffu) << 32 | q.w; }
 // of a cell that has no corners: point 0, as it lies
 __device__ __forceinline__ uint4 corner_none() { return make_uint4(0u, 0u, CQ_PLAIN, 0u); }
 

@@ -129,8 +129,7 @@ struct Tis {
   // diff_u of the Ca sub-steps at parity 1 (parity 0 writes diff_u itself)
   GPtr<double> ca_dfu;
   // per AFM cell and grid_avg8 corner (binary x, y, z), during a solve: the
-  // corner's point wrapped in x and y, its voxel word, the masks of its six
-  // stencil neighbours and the CQ_ flags, and the point as it lies
+  // corner's point, voxel word, masks and flags (ca_corner.h)
   GPtr<uint4> ca_cq;
   GPtr<double> ca_bx;   // ca2p_by_ext_stim per AFM cell (B does not change during a solve)
   GPtr<long long> uid; GPtr<long long> old_uid[2]; GPtr<int> src_row;

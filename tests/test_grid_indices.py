@@ -40,3 +40,16 @@ def test_every_corner_of_small_grids(lib, nx, ny, nz, izb, mask):
     at = lambda n: sorted({0, 1, n // 2, n - 2, n - 1})
     for i, (x, y, z) in enumerate(itertools.product(at(nx), at(ny), at(nz))):
         corners(lib, nx, ny, nz, izb, x, y, z, mask, i)
+
+
+@pytest.mark.parametrize("nx,ny,nz,izb", [
+    (1600, 1600, 1680, 1680),    # 4.35 G points in planes of 21 MB
+    (23200, 23200, 8, 8),        # 4.85 G points in planes of 4.3 GB
+    (1040, 1040, 8100, 4000),    # 8.9 G points, the top half above iz_bound
+])
+def test_corners_of_grids_past_32_bit_indices(lib, nx, ny, nz, izb):
+    first = (1 << 32) // ((nx + 1 + 15) // 16 * 16 * (ny + 1))   # the plane that holds point 2^32
+    for i, (x, y, z) in enumerate(itertools.product((0, nx - 1), (0, ny // 2, ny - 1),
+                                                    {1, first - 1, first, first + 1, nz - 2, nz - 1})):
+        if z < nz:
+            corners(lib, nx, ny, nz, izb, x, y, z, 1, i)

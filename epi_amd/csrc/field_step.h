@@ -94,7 +94,9 @@ __device__ __forceinline__ void map_stamp_part(const Tis& t, int pb, int bid, in
         const bool in1 = distSq < normal_radSq, in2 = afm && distSq < cradSq;
         const bool mark = afm ? in1 && in2 : in1;
         if (in2 || mark) {
-          const long long v = (long long)m * PL + ipy * XP + ipx;
+          // a plane has fewer than 2^32 points (a grid of three such planes does
+          // not fit the card), so the place within it is unsigned 32 bits
+          const long long v = (long long)m * PL + ((unsigned)ipy * (unsigned)XP + (unsigned)ipx);
           // the voxel, and its copies in the planes x = NX, y = NY
           for (int copy = 0; copy < 4; copy++) {
             if (((copy & 1) && ipx != 0) || ((copy & 2) && ipy != 0)) continue;

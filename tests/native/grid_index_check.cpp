@@ -1,12 +1,14 @@
 // Host build of the grid index arithmetic of the Ca corners
-// (epi_amd/csrc/ca_corner.h), for tests/test_grid_indices.py.  The grids are sparse: a
-// reservation of address space whose pages exist once written, so that grids
-// far larger than the memory of this machine can be addressed.
+// (epi_amd/csrc/ca_corner.h) and of the voxel-map stamp
+// (epi_amd/csrc/field_step.h), for tests/test_grid_indices.py.  The grids are
+// sparse: a reservation of address space whose pages exist once written, so that
+// grids far larger than the memory of this machine can be addressed.
 #include <algorithm>
 #include <sys/mman.h>
 
 #include "device_on_host.h"
 #include "../../epi_amd/csrc/ca_corner.h"
+#include "../../epi_amd/csrc/field_step.h"
 
 using namespace epi;
 
@@ -114,4 +116,83 @@ extern "C" int corner_check(int NX, int NY, int NZ, int izb, int x, int y, int z
                                (w >> 31) * ak.AIR_STIM);
   }
   return 0;
+}
+
+// setup_map_lat's stamp (map.cpp:39-166) of n cells by `lanes` lanes a cell: the
+// number of voxels of the cells' boxes, their periodic copies included, whose
+// maps differ from the loops written out, or -1 if the grid cannot be reserved.
+// Cell 0 is not looked at (an empty voxel of the sparse map reads 0).
+extern "C" long long stamp_check(int NX, int NY, int NZ, double lx, double ly, double lz, int n, const double* x,
+                                 const double* y, const double* z, const double* radius, const uint8_t* state, int lanes) {
+  Tis t;
+  std::memset(&t, 0, sizeof t);
+  t.NX = NX; t.NY = NY; t.NZ = NZ;
+  t.XP = (NX + 1 + 15) / 16 * 16;
+  t.PL = (long long)t.XP * (NY + 1);
+  t.LX = lx; t.LY = ly; t.LZ = lz;
+  t.dx = lx / NX; t.dy = ly / NY; t.dz = lz / NZ;
+  t.inv_dx = NX / lx; t.inv_dy = NY / ly; t.inv_dz = NZ / lz;
+  t.irx = (int)(1.4 * NX / lx); t.iry = (int)(1.4 * NY / ly); t.irz = (int)(1.4 * NZ / lz);
+  t.prm.FAC_MAP = 2.0;
+  t.cap = n;
+  Status st{};
+  st.n = n;
+  t.st = &st;
+  Sparse<int> m1(t.PL * (NZ + 1));
+  Sparse<uint8_t> m2(t.PL * (NZ + 1));
+  if (!m1.p || !m2.p) return -1;
+  t.cmap1 = m1.p; t.cmap2 = m2.p;
+  t.pos[0][0] = const_cast<double*>(x); t.pos[0][1] = const_cast<double*>(y); t.pos[0][2] = const_cast<double*>(z);
+  t.radius = const_cast<double*>(radius);
+  t.state = const_cast<uint8_t*>(state);
+  int* lat = new int[3 * n];
+  t.lat = lat;
+  blockDim.x = lanes;
+  for (int l = 0; l < lanes; l++) {
+    threadIdx.x = l;
+    if (lanes == 16) map_stamp_part<16>(t, 0, 0, 1);
+    else if (lanes == 4) map_stamp_part<4>(t, 0, 0, 1);
+    else map_stamp_part<1>(t, 0, 0, 1);
+  }
+  long long bad = st.err != 0;
+  auto wrap = [](long v, int N) { return (int)((v % N + N) % N); };
+  auto diff = [](double a, double b, double L) {
+    const double d = a - b;
+    return d > 0.5 * L ? d - L : d <= -0.5 * L ? d + L : d;
+  };
+  struct Cell { int i, j, k; };
+  auto lattice = [&](int c) { return Cell{wrap((long)(x[c] * t.inv_dx), NX), wrap((long)(y[c] * t.inv_dy), NY),
+                                          wrap((long)(z[c] * t.inv_dz), NZ)}; };
+  for (int c = 0; c < n; c++) {
+    const Cell at = lattice(c);
+    bad += lat[3 * c] != at.i || lat[3 * c + 1] != at.j || lat[3 * c + 2] != at.k;
+    if (c == 0) continue;
+    const int f = is_afm(state[c]) ? 2 : 1;
+    for (int k = std::max(at.k - f * t.irz, 1); k <= std::min(at.k + f * t.irz, NZ - 1); k++)
+      for (int j = at.j - f * t.iry; j <= at.j + f * t.iry; j++)
+        for (int i = at.i - f * t.irx; i <= at.i + f * t.irx; i++) {
+          // the owner and the mask of voxel (i, j, k) from every cell
+          int own = 0, mask = 0;
+          for (int o = 1; o < n; o++) {
+            const bool afm = is_afm(state[o]);
+            const int g = afm ? 2 : 1;
+            const Cell ao = lattice(o);
+            auto off = [](int a, int b, int N) { const int d = ((a - b) % N + N) % N; return d > N / 2 ? d - N : d; };
+            const int ii = ao.i + off(i, ao.i, NX), jj = ao.j + off(j, ao.j, NY);
+            if (std::abs(ii - ao.i) > g * t.irx || std::abs(jj - ao.j) > g * t.iry || std::abs(k - ao.k) > g * t.irz) continue;
+            const double dx = diff(ii * t.dx, x[o], lx), dy = diff(jj * t.dy, y[o], ly), dz = k * t.dz - z[o];
+            const double d2 = dx * dx + dy * dy + dz * dz, r = radius[o];
+            if (d2 < r * r) own = o;
+            if (afm && d2 < (2.0 * r) * (2.0 * r)) mask = 1;
+          }
+          const long long wi = wrap(i, NX), wj = wrap(j, NY);
+          for (int copy = 0; copy < 4; copy++) {
+            if (((copy & 1) && wi != 0) || ((copy & 2) && wj != 0)) continue;
+            const long long v = (long long)k * t.PL + (wj + (copy & 2 ? NY : 0)) * (long long)t.XP + wi + (copy & 1 ? NX : 0);
+            bad += m1.p[v] != own || m2.p[v] != mask;
+          }
+        }
+  }
+  delete[] lat;
+  return bad;
 }

@@ -2,7 +2,8 @@
 headers and run on sparse grids (CPU only): the eight grid_avg8 corners
 (utils.h:18-23) of a cell in a Ca solve (ca_corner.h) against the seven-point
 ATP update (ca2p.cpp:302-338) written out -- inside the grid, at its periodic
-seams, at the mirrored bottom, the top plane and iz_bound."""
+seams, at the mirrored bottom, the top plane and iz_bound -- and the voxel-map
+stamp (field_step.h) against setup_map_lat's loops (map.cpp:39-166)."""
 import ctypes as C
 import itertools
 import os
@@ -53,3 +54,25 @@ def test_corners_of_grids_past_32_bit_indices(lib, nx, ny, nz, izb):
                                                     {1, first - 1, first, first + 1, nz - 2, nz - 1})):
         if z < nz:
             corners(lib, nx, ny, nz, izb, x, y, z, 1, i)
+
+
+@pytest.mark.parametrize("nx,ny,nz,lx,ly,lz", [
+    (16, 20, 12, 12.8, 14.0, 10.0),
+    (46400, 46400, 2, 5800.0, 5800.0, 10.0),   # a plane of 2.15 G points: row offsets past 2^31
+])
+@pytest.mark.parametrize("lanes", [1, 4, 16])
+def test_stamp(lib, nx, ny, nz, lx, ly, lz, lanes):
+    from epi_amd.configs import ALIVE, DEAD, FIX, MEMB
+    x = [1.0, 0.01, lx - 0.01, 3.3, lx / 2, 2.2]
+    y = [1.0, 0.02, ly - 0.03, ly - 0.6, ly - 1.9, ly / 2]
+    z = [lz / 2 + 0.1] * len(x)
+    state = np.array([MEMB, ALIVE, DEAD, FIX, ALIVE, MEMB], np.uint8)
+    xs, ys, zs = (np.array(a, np.float64) for a in (x, y, z))
+    r = np.full(len(x), 1.4)
+    p = lambda a: a.ctypes.data_as(C.c_void_p)
+    lib.stamp_check.restype = C.c_longlong
+    bad = lib.stamp_check(nx, ny, nz, C.c_double(lx), C.c_double(ly), C.c_double(lz), len(x), p(xs), p(ys), p(zs), p(r),
+                          p(state), lanes)
+    if bad < 0:
+        pytest.skip("no address space for the grid")
+    assert bad == 0

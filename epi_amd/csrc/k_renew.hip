@@ -534,7 +534,9 @@ __global__ void __launch_bounds__(RCHUNK) k_renew_tail(const Tis* __restrict__ T
 }
 
 // The whole renewal of tissues with few cells, one workgroup per tissue.  A
-// tissue of 420 cells: 9.6 us, against about 3.5 and 7 and the gap.
+// tissue of 420 cells: 9.6 us, against about 3.5 and 7 and the gap.  A tissue is
+// sent here by the count of the last status read-back; renewals called one after
+// the other without one may have outgrown a chunk.
 __global__ void __launch_bounds__(RCHUNK) k_renew_one(const Tis* __restrict__ T, int pb, int cb, int cpar, int zero_zz) {
   const Tis& t = T[blockIdx.y];
   Status* st = t.st;

@@ -76,7 +76,7 @@ struct Status {
   int sw;                 // cornifications since the last Ca solve (uint8 wrap)
   int ndiv;               // divisions in the last renewal
   int nrm;                // removals in the last renewal
-  int maxlen;             // longest neighbour list of the last build
+  int maxlen;             // longest neighbour list of any build or epi_set_lists
   int stamp_z;            // highest z plane ever stamped into the voxel maps
   long long rng_pos;      // replay cursor
   long long next_uid;

@@ -391,7 +391,8 @@ int put_status(epi_ctx* c, int t) {
   return EPI_OK;
 }
 
-// the longest neighbour list any build has made (maxlen only grows), or
+// the longest neighbour list that a build has made or a caller set (maxlen only
+// grows), or
 // INT_MAX when a build has run since the last status read
 int max_list_len(const epi_ctx* c) {
   if (!c->len_known) return INT_MAX;
@@ -1796,6 +1797,7 @@ int epi_set_lists(epi_ctx* c, int32_t t, const int32_t* ptr, const int32_t* conn
   const TH& h = c->th[t];
   const int n = c->h_st[t].n;
   std::vector<int> col((size_t)n * h.ns, 0), nl(n), nlo(n, 0), srow(n);
+  int longest = 0;
   std::vector<double> g((size_t)n * h.ns, c->tis[t].prm.gj_init);
   std::vector<long long> u(n);
   RCHK(download(c, u.data(), ti.uid, n));
@@ -1803,6 +1805,7 @@ int epi_set_lists(epi_ctx* c, int32_t t, const int32_t* ptr, const int32_t* conn
     const int len = ptr[i + 1] - ptr[i];
     if (len > h.ns || len >= MAX_CONN) return fail(c, EPI_ERR_CAPACITY, "list too long");
     nl[i] = len;
+    longest = std::max(longest, len);
     srow[i] = i;
     int k = i < h.nmemb ? MEMB_ADJ : 0;
     int lo = 0;
@@ -1826,7 +1829,10 @@ int epi_set_lists(epi_ctx* c, int32_t t, const int32_t* ptr, const int32_t* conn
   RCHK(upload(c, ti.nlo, nlo.data(), n));
   RCHK(upload(c, ti.src_row, srow.data(), n));
   RCHK(upload(c, ti.old_uid[c->cb], u.data(), n));
-  return EPI_OK;
+  // the force kernels' slots follow the longest list (max_list_len)
+  if (longest <= c->h_st[t].maxlen) return EPI_OK;
+  c->h_st[t].maxlen = longest;
+  return put_status(c, t);
 }
 
 int epi_set_maps(epi_ctx* c, int32_t t, const int32_t* cmap1, const uint8_t* cmap2, const int32_t* lat) {

@@ -2158,11 +2158,6 @@ int epi_mech_begin(epi_ctx* c) {
       MechTis& r = m.h[t];
       const size_t cap = c->th[t].cap;
       r.x0[0] = cv.take<double>(3 * cap); r.x0[1] = cv.take<double>(3 * cap);
-      for (int b = 0; b < 3; b++) r.lam[b] = cv.take<double>(3 * cap);
-      r.es = 2 * c->th[t].ns + 8;   // both roles of a row's entries, and the pair's spring
-      r.ent = cv.take<int>(cap * (size_t)r.es);
-      r.code = cv.take<uint8_t>(cap * (size_t)r.es);
-      r.ent_n = cv.take<int>(cap);
       r.target = cv.take<double>(3 * cap);
       r.scal = cv.take<double>(5);
     }
@@ -2209,9 +2204,28 @@ int epi_mech_adjoint(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps, in
   const int nck = (n_steps + K - 1) / K;
   const int other = max_swept(c);
   const int memb = max_memb(c), nblk = mech_bwd_blocks(memb, other);
-  size_t need = 0;
-  for (int t = 0; t < c->T; t++)
-    need += align_up(8 * (3 * (size_t)c->th[t].cap * (K + nck) + 4 * (size_t)nblk), 256) + 768;
+  // what a gradient alone needs, taken with the first: the segment's states, the
+  // checkpoints, the adjoints and the plan, whose rows hold both roles of the
+  // longest list's entries and the pair's spring (rows of 400 entries, the most a
+  // list may have, would be 4 kB a cell)
+  auto carve = [&](Carver& cv) {
+    for (int t = 0; t < c->T; t++) {
+      MechTis& r = m.h[t];
+      const TH& h = c->th[t];
+      const size_t cap = h.cap;
+      r.es = std::max(2 * (c->len_known ? std::min(c->h_st[t].maxlen, h.ns) : h.ns) + 8, MECH_ROW_MIN);
+      r.slot = cv.take<double>(3 * cap * K);
+      r.ck = cv.take<double>(3 * cap * nck);
+      for (int b = 0; b < 3; b++) r.lam[b] = cv.take<double>(3 * cap);
+      r.ent = cv.take<int>(cap * (size_t)r.es);
+      r.code = cv.take<uint8_t>(cap * (size_t)r.es);
+      r.ent_n = cv.take<int>(cap);
+      r.part = cv.take<double>(4 * (size_t)nblk);
+    }
+  };
+  Carver dry{nullptr, 0, true};
+  carve(dry);
+  const size_t need = align_up(dry.off, 256);
   if (need > m.work_bytes) {
     if (m.work) (void)hipFree(m.work);
     m.work = nullptr;
@@ -2219,13 +2233,11 @@ int epi_mech_adjoint(epi_ctx* c, const epi_mech_params* prm, int32_t n_steps, in
     if (hipMalloc(&m.work, need) != hipSuccess) return fail(c, EPI_ERR_HIP, "window work allocation failed");
     m.work_bytes = need;
   }
-  Carver cv{m.work, 0, false};
+  Carver real{m.work, 0, false};
+  carve(real);
   for (int t = 0; t < c->T; t++) {
     MechTis& r = m.h[t];
     const size_t cap = c->th[t].cap, n = (size_t)c->h_st[t].n;
-    r.slot = cv.take<double>(3 * cap * K);
-    r.ck = cv.take<double>(3 * cap * nck);
-    r.part = cv.take<double>(4 * (size_t)nblk);
     for (int a = 0; a < 3; a++)
       HIPCHK(c, hipMemcpyAsync(r.target + a * cap, targets[t] + a * n, 8 * n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemsetAsync(r.scal, 0, 5 * sizeof(double), c->stream));

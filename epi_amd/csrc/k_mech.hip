@@ -677,6 +677,7 @@ void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int m
 // it the atomics 25); both sides evaluated 63.
 constexpr int MG = 16;   // of a membrane particle
 constexpr int MC = 4;    // of another cell
+static_assert(MG <= MECH_ROW_MIN && MC <= MECH_ROW_MIN, "a lane's first slot lies inside its cell's plan row");
 
 namespace {
 struct LawD { double coef, ds, deps, dadh, dspr; };
@@ -883,7 +884,7 @@ __device__ __forceinline__ P3 planned_bwd(const Tis& t, const MechTis& m, const 
   const long long cap = t.cap;
   const int* ent = m.ent + (size_t)X * m.es;
   const uint8_t* code = m.code + (size_t)X * m.es;
-  const int o0 = ent[lane], k0 = code[lane];   // in one round trip with the row's length (a row holds es > G slots)
+  const int o0 = ent[lane], k0 = code[lane];   // in one round trip with the row's length (a row has MECH_ROW_MIN slots)
   const int len = m.ent_n[X];
   P3 own{0, 0, 0};
   for (int e = lane; e < len; e += G) {

@@ -10,6 +10,10 @@
 
 namespace epi {
 
+// the fewest slots of a plan row: lanes ask for a row's first slots before they
+// know its length
+constexpr int MECH_ROW_MIN = 16;
+
 struct MechTis {
   GPtr<double> x0[2];      // snapshot of both position buffers, [0] = current
   GPtr<double> slot;       // positions of the states of one segment (slot-major, 3 * cap each)
@@ -18,7 +22,8 @@ struct MechTis {
   // step, [q + 1] before it, [q + 2] cleared for the next, q = step mod 3
   GPtr<double> lam[3];
   // the interactions each cell takes part in, es slots a cell: the other cell
-  // and the law's code (k_mech_plan)
+  // and the law's code (k_mech_plan).  lam, the plan and part are a gradient's
+  // alone and lie in its work memory
   GPtr<int> ent;
   GPtr<uint8_t> code;
   GPtr<int> ent_n;

@@ -5,7 +5,7 @@ The shapes it chooses (see epi_set_tuning in include/epi_amd.h):
   k_ext_stim   z planes per tile (1, 2, 4, 8, 16) x 64-lane rows per block (1, 2, 4),
                then its tile list in one run per XCD or not (b_xcd 0, 1)
   k_atp        the same shapes
-  k_ca_cells   lanes per cell (4, 8, 16)
+  k_ca_cells   lanes per cell (8, 16; 4 is accepted and runs as 8)
   k_ca_cells + k_atp   XCD-contiguous workgroup order (0, 1); in fused mode,
                the fused launch's (its ATP tiles in one run per XCD)
   Ca solve     ATP of a sub-step and cells of the next in one launch (1; 2 =
@@ -19,6 +19,11 @@ The shapes it chooses (see epi_set_tuning in include/epi_amd.h):
 
 With CA_FUSE 2 the fused small solves use CA_GROUP_SMALL lanes per cell
 (default 8, the best width on a latency-bound single-tissue solve).
+
+A step of one tissue stamps the maps and sweeps B inside other launches, in
+blocks of a fixed size and with no side stream: of the shapes above it takes
+map_lanes, b_zb and b_xcd, as timed here on launches of their own, and not
+b_rows or side_fork.
 
 A launch shape changes timing only: every grid point is computed on its own
 and the Ca cell kernel sums each list in list order whatever its group size,
@@ -35,6 +40,8 @@ import time
 
 STENCIL_SHAPES = list(itertools.product((1, 2, 4, 8, 16), (1, 2, 4)))
 CA_GROUPS = (4, 8, 16)
+# where the tuner starts: every candidate kernel a launch of its own, so that each
+# can be timed alone.  Not the library's defaults (those are Tuning's, launch.h).
 DEFAULT = {"b_zb": 4, "b_rows": 4, "atp_zb": 4, "atp_rows": 4, "ca_group": 16, "xcd": 0, "ca_fuse": 0, "map_lanes": 1,
            "b_xcd": 0, "sweep_wave": 0, "side_fork": 0}
 

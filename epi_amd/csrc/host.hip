@@ -456,9 +456,9 @@ int izb_est(const epi_ctx* c, bool ca) {
   return m;
 }
 
-// tiles of the B stencil's work list (k_ext_stim) from the last known
-// zzmax, one plane more than it gives, for sizing the grid
-// tiles of bs points of the B stencil in tissue t, from the last known zzmax
+// tiles of bs points of the B stencil in tissue t, and of its work list over all
+// tissues (k_ext_stim): from the last known zzmax, one plane more than it gives,
+// for sizing the grid
 long long b_tiles_of(const epi_ctx* c, int t, int bs) {
   const Tis& ti = c->tis[t];
   const double zz = c->h_st ? c->h_st[t].zzmax : 0.0;
@@ -655,7 +655,9 @@ Tuning ca_shapes(const epi_ctx* c, const int* ids, int ntis) {
   // One tissue takes one plane a tile (most blocks, shortest chain: two planes
   // 1.5 % slower at 36,000 cells); several, whose tiles are found in a list,
   // two (30,000 cells in 4 tissues 18.0 -> 16.8 ms for 50 steps and a solve,
-  // 138,000 in 16 52.7 -> 47.4).
+  // 138,000 in 16 52.7 -> 47.4; a sub-step of 8 tissues of 6,100 cells 11.5 -> 10.7
+  // us, of 4 of 9,100 11.0 -> 10.6, but of 4 of 6,100 7.0 -> 7.6, of 2 of 9,100
+  // 7.1 -> 7.5: the number of tissues stands in for the number of tiles).
   if (any_wide_plane(c, ids, ntis)) tu.ca_fuse = 0;
   if (tu.ca_fuse && tu.a_zb > 2) tu.a_zb = ntis == 1 ? 1 : 2;
   return tu;
@@ -971,7 +973,7 @@ int epi_load_cells(epi_ctx* c, int32_t t, const epi_cell_input* in) {
     if (pair[i] >= 0 && pair[pair[i]] != i) return fail(c, EPI_ERR_INVALID, "pairs must be mutual");
   std::vector<int> m6;
   memb_init_host(h.g.nmx, h.nmemb, m6);
-  // the gather in k_forces_memb needs a symmetric adjacency of distinct cells
+  // the gather in k_forces needs a symmetric adjacency of distinct cells
   for (int j = 0; j < h.nmemb; j++)
     for (int a = 0; a < 6; a++) {
       const int q = m6[6 * j + a];
@@ -1116,7 +1118,7 @@ int epi_rng_mt19937_64(uint64_t seed, double* out, int64_t n) {
 int epi_cell_interaction(epi_ctx* c) {
   if (!c) return EPI_ERR_INVALID;
   launch_force_pack(c->stream, c->d_tis, c->T, c->pb, max_n(c));
-  launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, max_memb(c), max_n(c), max_list_len(c));
+  launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, max_n(c), max_list_len(c));
   HIPCHK(c, hipGetLastError());
   c->pos_pending = true;
   return EPI_OK;
@@ -1282,12 +1284,15 @@ int epi_ca_substep(epi_ctx* c, int32_t iz_bound) {
 // connect_cell (:154), and, on the side stream forked after the insertion,
 // setup_map_lat's stamping and calc_ext_stim (:156-157), which read only the
 // fixed positions, states and radii (and the B field) that the rest of the
-// build leaves alone.  The build, the longer
-// chain, is issued first.
+// build leaves alone.  The build, the longer chain, is issued first.
 // Up to BUILD_FIELD_TISSUES tissues there is no side stream (unless `side`):
 // the stamping is further blocks of the sweep and the B sweep further blocks of
 // k_finish.  Recording and waiting for the two events took the host 25 us a
-// step, and such a step is bound by what the host issues.
+// step, and such a step is bound by what the host issues.  Sets: 32 uneven ones
+// of 292,000 cells are 1.5 % slower without the stream; 2, 4, 8 and 16 tissues
+// of 420 cells would take 40, 42, 45 and 52 us a step without it against 49, 50,
+// 53 and 59 with it, of 6,100 cells 64, 87, 128 and 210 against 66, 92, 133 and
+// 220, so the line could lie higher for sets of small tissues.
 // With join false the main stream does not wait for the side stream's maps
 // and B sweep: epi_step joins it after issuing the next step's forces, which
 // read neither.
@@ -1374,7 +1379,7 @@ int epi_step(epi_ctx* c, int64_t nsteps, epi_driver* drv) {
     // cell_dynamics (proc.cpp:22-32)
     if (!forces_issued) {
       launch_force_pack(c->stream, c->d_tis, c->T, c->pb, mn);
-      launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, max_memb(c), mn, max_list_len(c));
+      launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, mn, max_list_len(c));
       c->pb ^= 1;
     }
     forces_issued = false;
@@ -2138,7 +2143,7 @@ int mech_params(epi_ctx* c, const epi_mech_params* prm) {
 }
 // one step, its result also into slot `slot` if that is not negative
 int mech_step(epi_ctx* c, int slot = -1) {
-  launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, max_memb(c), max_n(c), max_list_len(c),
+  launch_forces(c->stream, c->d_tis, c->T, c->pb, c->cb, max_n(c), max_list_len(c),
                 MechSave{slot < 0 ? nullptr : c->mech.d, slot, true});
   c->pb ^= 1;
   return EPI_OK;

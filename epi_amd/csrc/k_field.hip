@@ -896,15 +896,14 @@ void launch_cells(hipStream_t s, const Tis* dT, const CaList& cl, int cp, int ap
 
 // blocks that walk a list of `tiles` tiles: one per tile (as launch_ext_stim),
 // a multiple of 8 (the XCD split)
-unsigned walk_blocks(long long tiles, int bs) {
-  (void)bs;
+unsigned walk_blocks(long long tiles) {
   const long long cap = 1LL << 24;
   long long g = std::min(std::max(tiles, 1LL), cap);
   return (unsigned)((g + 7) / 8 * 8);
 }
 
 void launch_atp(hipStream_t s, const Tis* dT, const CaList& cl, int cp, int ap, const Tuning& tu) {
-  const dim3 g(walk_blocks(cl.atiles, cl.abs));
+  const dim3 g(walk_blocks(cl.atiles));
   by_zb(tu.a_zb, [&](auto zbc) {
     constexpr int zb = decltype(zbc)::value;
     const auto k1 = k_atp<zb, true, unsigned>, kn = k_atp<zb, false, unsigned>,
@@ -917,7 +916,7 @@ void launch_atp(hipStream_t s, const Tis* dT, const CaList& cl, int cp, int ap, 
 void launch_fused(hipStream_t s, const Tis* dT, const CaList& cl, int cp, int ap, const Tuning& tu, const RdTis* sv,
                   int slot) {
   const unsigned cblocks = tu.xcd ? (unsigned)(cl.ncb + 7) / 8 * 8 : (unsigned)cl.ncb;
-  const dim3 g(cblocks + walk_blocks(cl.atiles, F_BLOCK));
+  const dim3 g(cblocks + walk_blocks(cl.atiles));
   by_cells(cl, tu, sv, [&](auto cg, auto one, auto save) {
     constexpr int CG = decltype(cg)::value;
     constexpr bool ONE = decltype(one)::value, SAVE = decltype(save)::value;

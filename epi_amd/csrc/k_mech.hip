@@ -643,9 +643,8 @@ void launch_force_pack(hipStream_t s, const Tis* dT, int ntis, int pb, int max_n
   EPI_LAUNCH(K_FORCE_PACK, k_force_pack, dim3((max_n + 255) / 256, ntis), dim3(256), 0, s, dT, pb);
 }
 
-void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_memb, int max_other,
-                   int max_len, const MechSave& save) {
-  (void)max_memb;
+void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len,
+                   const MechSave& save) {
   const int cap = launch_forces_rows(s, dT, ntis, pb, cb, max_other, max_len, StatusOut{}, save);
   if (max_len > cap) launch_forces_long(s, dT, ntis, pb, cb, max_other, cap, save);
 }

@@ -95,7 +95,7 @@ struct MechSave {
 // LDS slots per cell, 40, 48 or 64, follow max_len), longer ones to a
 // one-lane-per-cell kernel, launched only when max_len exceeds the slots.
 constexpr int FORCES_ROW_CAP = 64;
-void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_memb, int max_other, int max_len,
+void launch_forces(hipStream_t s, const Tis* dT, int ntis, int pb, int cb, int max_other, int max_len,
                    const MechSave& save = {});
 // the two halves of launch_forces: the cooperative kernel for rows of up to
 // the returned number of slots (chosen from max_len), and the long rows

@@ -384,12 +384,12 @@ int epi_rd_end(epi_ctx* ctx);
  * forbid hipMalloc): calc_ext_stim (ext_stim.cpp:18-69) over grids the caller
  * holds, with no context, through the same kernels as epi_calc_ext_stim,
  * with epi5_MT's parameters (epi_params_default).
- * The sweep's grid descriptors, per-grid status and tile work list live in
- * one static device array per GPU of EPI_NOALLOC_SCRATCH_BYTES, held until
+ * The sweep's grid descriptors and tile work list live in one static device
+ * array per GPU of epi_noalloc_scratch_bytes(), held until
  * the process ends, so a call takes at most EPI_NOALLOC_MAX_GRIDS grids.
  * Calls that overlap on one GPU (on different streams, or from different
  * threads) race on that array.  The call allocates nothing (no hipMalloc,
- * hipFree or allocating library routine): it queues four kernels on `stream`
+ * hipFree or allocating library routine): it queues two kernels on `stream`
  * (a hipStream_t; NULL = the null stream) and returns.
  *
  * Layout: grid point (j, k, l), 0 <= j <= nx, 0 <= k <= ny, 0 <= l <= nz, is

@@ -2014,19 +2014,21 @@ int epi_rd_adjoint(epi_ctx* c, const epi_rd_params* prm, int32_t n_sub, int32_t 
   if (!rd.active) return fail(c, EPI_ERR_INVALID, "no reaction-diffusion window is open");
   const int K = std::min(every, n_sub);
   const int nck = (n_sub + K - 1) / K;
-  // segment slots (K states) and checkpoints (nck, both buffers)
-  size_t need = 0;
-  {
-    Carver dry{nullptr, 0, true};
+  // segment slots (K states, of the ATP grid the cells' averages alone) and
+  // checkpoints (nck, both buffers); the same carving sizes and places them
+  auto carve = [&](Carver& cv) {
     for (int t = 0; t < c->T; t++) {
-      const size_t cap = c->th[t].cap, ns = c->th[t].ns, box = (size_t)rd.h[t].box;
-      dry.take<double>(K * cap); dry.take<double>(K * cap); dry.take<double>(K * cap);
-      dry.take<double>(K * cap * ns); dry.take<double>(K * box);
-      dry.take<double>(2 * nck * cap); dry.take<double>(2 * nck * cap); dry.take<double>(nck * cap);
-      dry.take<double>(nck * cap * ns); dry.take<double>(2 * nck * box);
+      RdTis& r = rd.h[t];
+      const size_t cap = c->th[t].cap, ns = c->th[t].ns, box = (size_t)r.box;
+      r.su = cv.take<double>(K * cap); r.sp = cv.take<double>(K * cap); r.sh = cv.take<double>(K * cap);
+      r.sg = cv.take<double>(K * cap * ns); r.sAv = cv.take<double>(K * cap);
+      r.cu = cv.take<double>(2 * nck * cap); r.cp_ = cv.take<double>(2 * nck * cap); r.ch = cv.take<double>(nck * cap);
+      r.cg = cv.take<double>(nck * cap * ns); r.cA = cv.take<double>(2 * nck * box);
     }
-    need = align_up(dry.off, 256);
-  }
+  };
+  Carver dry{nullptr, 0, true};
+  carve(dry);
+  const size_t need = align_up(dry.off, 256);
   if (need > rd.work_bytes) {
     if (rd.work) (void)hipFree(rd.work);
     rd.work = nullptr;
@@ -2034,14 +2036,10 @@ int epi_rd_adjoint(epi_ctx* c, const epi_rd_params* prm, int32_t n_sub, int32_t 
     if (hipMalloc(&rd.work, need) != hipSuccess) return fail(c, EPI_ERR_HIP, "window work allocation failed");
     rd.work_bytes = need;
   }
-  Carver cv{rd.work, 0, false};
+  Carver real{rd.work, 0, false};
+  carve(real);
   for (int t = 0; t < c->T; t++) {
-    RdTis& r = rd.h[t];
-    const size_t cap = c->th[t].cap, ns = c->th[t].ns, box = (size_t)r.box;
-    r.su = cv.take<double>(K * cap); r.sp = cv.take<double>(K * cap); r.sh = cv.take<double>(K * cap);
-    r.sg = cv.take<double>(K * cap * ns); r.sAv = cv.take<double>(K * cap);
-    r.cu = cv.take<double>(2 * nck * cap); r.cp_ = cv.take<double>(2 * nck * cap); r.ch = cv.take<double>(nck * cap);
-    r.cg = cv.take<double>(nck * cap * ns); r.cA = cv.take<double>(2 * nck * box);
+    const RdTis& r = rd.h[t];
     HIPCHK(c, hipMemcpyAsync(r.target, targets[t], 8 * (size_t)c->h_st[t].n, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemsetAsync(r.scal, 0, 4 * sizeof(double), c->stream));
   }

@@ -1968,7 +1968,7 @@ int epi_rd_begin(epi_ctx* c, const double* zzmax) {
       r.kpa_in = cv.take<double>(cap); r.scal = cv.take<double>(4);
       const Tis& ti = c->tis[t];
       r.oc = (4 * ti.irx + 1) * (4 * ti.iry + 1) * (4 * ti.irz + 1);
-      r.own = cv.take<int>(cap * (size_t)r.oc); r.own_n = cv.take<int>(cap);
+      r.own = cv.take<unsigned>(cap * (size_t)r.oc); r.own_n = cv.take<int>(cap);
       r.nafm = 0;
     }
   };

@@ -301,8 +301,8 @@ __device__ __forceinline__ void rd_cells_part(const Tis& t, const RdTis& r, int 
     }
     // with them the cell's remaining words and its first voxels' indices
     const int no = own0;
-    const int* ov = r.own + (size_t)c * r.oc;
-    int v[OWN];
+    const unsigned* ov = r.own + (size_t)c * r.oc;
+    unsigned v[OWN];
 #pragma unroll
     for (int k = 0; k < OWN; k++) v[k] = ov[lane + k * RG < no ? lane + k * RG : 0];
     const int ix = t.lat[3 * c], iy = t.lat[3 * c + 1], iz = t.lat[3 * c + 2];
@@ -484,14 +484,14 @@ __global__ void __launch_bounds__(256) k_rd_own(const Tis* __restrict__ T, RdTis
       const unsigned me = (unsigned)c + 1;
       const int ix = t.lat[3 * c], iy = t.lat[3 * c + 1], iz = t.lat[3 * c + 2];
       const int z0 = max(iz - 2 * t.irz, 1), z1 = min(min(iz + 2 * t.irz, t.NZ - 1), r.izb - 1);
-      int* ov = r.own + (size_t)c * r.oc;
+      unsigned* ov = r.own + (size_t)c * r.oc;
       for (int l = z0; l <= z1; l++)
         for (int b = 0; b < bx * by; b++) {
           const int jx = (ix - 2 * t.irx + b % bx + t.NX) % t.NX;
           const int ky = (iy - 2 * t.iry + b / bx + t.NY) % t.NY;
           const long long v = gidx(t, jx, ky, l);
           if ((t.vox[v] & 0x7fffffffu) != me) continue;
-          if (m < r.oc) ov[m] = (int)v;
+          if (m < r.oc) ov[m] = (unsigned)v;
           m++;
         }
       if (m > r.oc) { set_err(t.st, ERR_CAPACITY); m = r.oc; }

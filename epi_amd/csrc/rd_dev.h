@@ -30,8 +30,9 @@ struct RdTis {
   GPtr<double> lA[3];
   GPtr<double> gkpa, gdu, gdp;      // dL/dkpa per cell; each cell's share of dL/ddu and dL/ddp
   // the voxels each AFM cell owns in the window's frozen voxel map (its fa
-  // source), up to oc per cell, in stamp-box order
-  GPtr<int> own;
+  // source), up to oc per cell, in stamp-box order.  A window's box has fewer
+  // than 2^32 points (at 97 bytes a point more do not fit a card)
+  GPtr<unsigned> own;
   GPtr<int> own_n;
   int oc;
   GPtr<double> scal;                // [0] loss, [1] dL/ddu, [2] dL/ddp, [3] dL/dgj0

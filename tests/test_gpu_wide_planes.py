@@ -80,3 +80,34 @@ def test_large_grids(nx, ny, nz, lz, y0, top):
     if free.value < 1.05 * BYTES_PER_POINT * points:
         pytest.skip("not enough free memory on the card")
     check(*specs(3, nx, ny, nz, lz, 0.0, y0, top))
+
+
+def gradient(spec, n_sub):
+    from epi_amd import native
+    g = native.Tissue(spec["geometry"])
+    g.set_params({"Da": 0.1})
+    g.load(spec)
+    g.setup_map_lat()
+    g.set.rd_begin(g.calc_zzmax())
+    target = g.get_cells()["ca2p"] * 0.97
+    loss, grads = g.set.rd_adjoint([dict(du=0.01, dp=0.1, gj0=0.99)], n_sub, n_sub, [target])
+    g.close()
+    return loss[0], grads[0]
+
+
+def test_window_box_past_2_31_points():
+    """the voxels that a cell owns in a window: 32 bits, unsigned"""
+    from epi_amd import native
+    nx, ny, nz, lz, top = 1600, 1616, 850, 106.25, 102.75   # iz_bound 844: the box holds 2.2 G points
+    points = (nx + 16) // 16 * 16 * (ny + 1) * (nz + 1)
+    free, total = C.c_size_t(), C.c_size_t()
+    assert native.load_library().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    # the context, the window's snapshot and three adjoint grids, one checkpoint
+    if free.value < 1.05 * (BYTES_PER_POINT + 56) * points:
+        pytest.skip("not enough free memory on the card")
+    small, large = specs(6, nx, ny, nz, lz, 0.0, 0.0, top)
+    ref, got = gradient(small, 4), gradient(large, 4)
+    assert ref[0] > 0 and got[0] == pytest.approx(ref[0], rel=1e-12)
+    for k in ("du", "dp", "gj0"):     # FP64 atomics in another order
+        assert got[1][k] == pytest.approx(ref[1][k], rel=1e-9), k
+    assert np.allclose(got[1]["kpa"], ref[1]["kpa"], rtol=1e-9, atol=1e-9 * np.max(np.abs(ref[1]["kpa"])))
